@@ -61,10 +61,10 @@ struct nuto_ctx
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;
     std::string err;
-    // the constrained solves' vectors and the pinned word their reductions are read through, kept
+    // the constrained solves' vectors, and the pinned states with the events of their arrival, kept
     // between solves (a Newton step solves once per iteration); grown when a solve needs more
     DevBuf solveWork;
-    double* solveHost = nullptr;
+    SolveBuffers solveBuf;
     // cells
     bool cellsSet = false;
     int coordType = 0, dim = 0, nCells = 0, nCoordNodes = 0;
@@ -93,16 +93,18 @@ struct nuto_ctx
     // hex8 gradient-damage node kernel (prepared lazily from the node graph)
     GdmHex8Plan gdm;
     bool gdmTried = false;
-    // constraint equations per dof type slot (Constraints::Add) and the unit constraint matrix
-    // built from them for the monolithic system (C and C^T, CSR, device)
+    // constraint equations per dof type slot (Constraints::Add) and, built from them for the monolithic
+    // system (device): C^T of the unit constraint matrix (CSR over the independent dofs), each dof's row
+    // in it, the dependent dofs per node, and the equations' terms (ConstraintView)
     struct Equations
     {
         std::vector<int> dep, termPtr{0}, termDof;
         std::vector<double> coef;
     } cons[2];
     bool consBuilt = false;
-    int nInd = 0, nEq = 0;
-    DevBuf cRow, cCol, cVal, ctRow, ctCol, ctVal, consDep;
+    int nInd = 0, nEq = 0, nTermDofs = 0;
+    DevBuf consRev, consMask, ctRow, ctCol, ctVal, consDep;
+    DevBuf consPtr, consDof, consVal, consTDof, consTPtr, consTDep, consTVal;
     // per-block views of the monolithic matrix (nuto_block_pattern / nuto_block_values), built on
     // first use per (slot i, slot j): the block's CSR row pointers and, per row, where the block's
     // run starts in the monolithic row
@@ -850,8 +852,11 @@ int nuto_destroy(nuto_ctx* ctx)
         return NUTO_ERR_ARGUMENT;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
-    if (ctx->solveHost)
-        (void)hipHostFree(ctx->solveHost);
+    if (ctx->solveBuf.host)
+        (void)hipHostFree(ctx->solveBuf.host);
+    for (hipEvent_t e : ctx->solveBuf.arrived)
+        if (e)
+            (void)hipEventDestroy(e);
     if (ctx->own)
         (void)hipStreamDestroy(ctx->own);
     delete ctx;
@@ -1328,89 +1333,131 @@ namespace
 // puts the independent dofs first (ascending), then the dependent ones (equation order); column i
 // < nInd_s holds a 1 at independent dof jk(i), and the row of each dependent dof holds -coef at the
 // independent column of each term with |coef| > 1e-18 (setFromTriplets: duplicates summed in order).
+// Its transpose is kept as CSR, rows ascending in each column of C.
 void BuildConstraints(nuto_ctx* ctx)
 {
     if (ctx->consBuilt)
         return;
     const int nSlots = ctx->f[1].set ? 2 : 1;
-    int n[2] = {ctx->f[0].nDofs, nSlots > 1 ? ctx->f[1].nDofs : 0};
-    Require(n[0] + n[1] == ctx->nRows, NUTO_ERR_STATE, "dof counts do not match the pattern");
-    std::vector<std::vector<std::pair<int, double>>> rows(ctx->nRows);
-    std::vector<int> depAll;
-    int rowOff = 0, colOff = 0;
+    const int n[2] = {ctx->f[0].nDofs, nSlots > 1 ? ctx->f[1].nDofs : 0};
+    const int nRows = ctx->nRows;
+    Require(n[0] + n[1] == nRows, NUTO_ERR_STATE, "dof counts do not match the pattern");
+    std::vector<int> rev(nRows, 0), eqOf(nRows, -1), dep;
+    int rowOff = 0;
+    for (int s = 0; s < nSlots; s++)
+    {
+        for (int d : ctx->cons[s].dep)
+        {
+            eqOf[rowOff + d] = (int)dep.size();
+            dep.push_back(rowOff + d);
+        }
+        rowOff += n[s];
+    }
+    int nInd = 0;
+    for (int r = 0; r < nRows; r++)
+        rev[r] = eqOf[r] < 0 ? nInd++ : -1;
+    // the equations' terms, duplicates merged, by ascending dof (= ascending column of C)
+    std::vector<int> ptr{0}, dof;
+    std::vector<double> val;
+    rowOff = 0;
     for (int s = 0; s < nSlots; s++)
     {
         const nuto_ctx::Equations& q = ctx->cons[s];
-        std::vector<char> isDep(n[s], 0);
-        for (int d : q.dep)
-            isDep[d] = 1;
-        std::vector<int> rev(n[s], -1);
-        int nIndS = 0;
-        for (int g = 0; g < n[s]; g++)
-            if (!isDep[g])
-            {
-                rev[g] = nIndS;
-                rows[rowOff + g].push_back({colOff + nIndS, 1.0});
-                nIndS++;
-            }
+        std::vector<std::pair<int, double>> row;
         for (size_t e = 0; e < q.dep.size(); e++)
         {
-            depAll.push_back(rowOff + q.dep[e]);
-            auto& row = rows[rowOff + q.dep[e]];
+            row.clear();
             for (int t = q.termPtr[e]; t < q.termPtr[e + 1]; t++)
             {
                 if (!(std::fabs(q.coef[t]) > 1.e-18))
                     continue;
-                const int c = colOff + rev[q.termDof[t]];
-                bool merged = false;
-                for (auto& kv : row)
-                    if (kv.first == c)
-                    {
-                        kv.second += -q.coef[t];
-                        merged = true;
-                    }
-                if (!merged)
-                    row.push_back({c, -q.coef[t]});
+                const int g = rowOff + q.termDof[t];
+                auto same = std::find_if(row.begin(), row.end(), [&](const auto& kv) { return kv.first == g; });
+                if (same != row.end())
+                    same->second += -q.coef[t];
+                else
+                    row.push_back({g, -q.coef[t]});
             }
+            std::sort(row.begin(), row.end());
+            for (const auto& kv : row)
+            {
+                dof.push_back(kv.first);
+                val.push_back(kv.second);
+            }
+            ptr.push_back((int)dof.size());
         }
         rowOff += n[s];
-        colOff += nIndS;
     }
-    const int nInd = colOff;
-    std::vector<int> cr(ctx->nRows + 1, 0), cc;
-    std::vector<double> cv;
-    std::vector<std::vector<std::pair<int, double>>> cols(nInd);
-    for (int r = 0; r < ctx->nRows; r++)
-    {
-        std::sort(rows[r].begin(), rows[r].end());
-        for (auto& kv : rows[r])
-        {
-            cc.push_back(kv.first);
-            cv.push_back(kv.second);
-            cols[kv.first].push_back({r, kv.second});
-        }
-        cr[r + 1] = (int)cc.size();
-    }
-    std::vector<int> tr(nInd + 1, 0), tc;
-    std::vector<double> tv;
+    // C^T: row j = independent dof j's own 1 and the dependent rows it is a term of, rows ascending
+    std::vector<int> tr(nInd + 1, 0);
+    for (int r = 0; r < nRows; r++)
+        if (rev[r] >= 0)
+            tr[rev[r] + 1] = 1;
+    for (int g : dof)
+        tr[rev[g] + 1]++;
     for (int j = 0; j < nInd; j++)
+        tr[j + 1] += tr[j];
+    std::vector<int> tc(tr[nInd]), at(tr.begin(), tr.end() - 1);
+    std::vector<double> tv(tr[nInd]);
+    for (int r = 0; r < nRows; r++)
     {
-        for (auto& kv : cols[j])
+        if (rev[r] >= 0)
         {
-            tc.push_back(kv.first);
-            tv.push_back(kv.second);
+            tc[at[rev[r]]] = r;
+            tv[at[rev[r]]++] = 1.0;
+            continue;
         }
-        tr[j + 1] = (int)tc.size();
+        for (int k = ptr[eqOf[r]]; k < ptr[eqOf[r] + 1]; k++)
+        {
+            const int j = rev[dof[k]];
+            tc[at[j]] = r;
+            tv[at[j]++] = val[k];
+        }
     }
-    Upload(ctx, ctx->cRow, cr.data(), cr.size(), "constraints");
-    Upload(ctx, ctx->cCol, cc.data(), cc.size(), "constraints");
-    Upload(ctx, ctx->cVal, cv.data(), cv.size(), "constraints");
+    // the independent dofs with terms and the dependent rows they collect
+    std::vector<int> tDof, tPtr{0}, tDep;
+    std::vector<double> tVal;
+    if (!dof.empty())
+        for (int r = 0; r < nRows; r++)
+        {
+            const int j = rev[r];
+            if (j < 0 || tr[j + 1] - tr[j] < 2)
+                continue;
+            tDof.push_back(r);
+            for (int k = tr[j]; k < tr[j + 1]; k++)
+                if (tc[k] != r)
+                {
+                    tDep.push_back(tc[k]);
+                    tVal.push_back(tv[k]);
+                }
+            tPtr.push_back((int)tDep.size());
+        }
+    // dependent rows per dof node: bit i the i-th slot-0 row, the bits after them the slot-1 rows
+    const int c0 = ctx->f[0].ncomp, c1 = nSlots > 1 ? ctx->f[1].ncomp : 0;
+    std::vector<unsigned char> mask(ctx->f[0].nNodes, 0);
+    for (int d : dep)
+    {
+        if (d < n[0])
+            mask[d / c0] |= (unsigned char)(1 << (d % c0));
+        else
+            mask[(d - n[0]) / c1] |= (unsigned char)(1 << (c0 + (d - n[0]) % c1));
+    }
+    Upload(ctx, ctx->consRev, rev.data(), rev.size(), "constraints");
+    Upload(ctx, ctx->consMask, mask.data(), mask.size(), "constraints");
     Upload(ctx, ctx->ctRow, tr.data(), tr.size(), "constraints");
     Upload(ctx, ctx->ctCol, tc.data(), tc.size(), "constraints");
     Upload(ctx, ctx->ctVal, tv.data(), tv.size(), "constraints");
-    Upload(ctx, ctx->consDep, depAll.data(), depAll.size(), "constraints");
+    Upload(ctx, ctx->consDep, dep.data(), dep.size(), "constraints");
+    Upload(ctx, ctx->consPtr, ptr.data(), ptr.size(), "constraints");
+    Upload(ctx, ctx->consDof, dof.data(), dof.size(), "constraints");
+    Upload(ctx, ctx->consVal, val.data(), val.size(), "constraints");
+    Upload(ctx, ctx->consTDof, tDof.data(), tDof.size(), "constraints");
+    Upload(ctx, ctx->consTPtr, tPtr.data(), tPtr.size(), "constraints");
+    Upload(ctx, ctx->consTDep, tDep.data(), tDep.size(), "constraints");
+    Upload(ctx, ctx->consTVal, tVal.data(), tVal.size(), "constraints");
     ctx->nInd = nInd;
-    ctx->nEq = (int)depAll.size();
+    ctx->nEq = (int)dep.size();
+    ctx->nTermDofs = (int)tDof.size();
     ctx->consBuilt = true;
 }
 
@@ -1426,17 +1473,35 @@ NodeRows KNodeRows(const nuto_ctx* ctx)
     return r;
 }
 
-// The context's solve workspace, at least ReducedSolver::WorkDoubles(n_rows, n_independent) doubles
-// (allocated once, or again when the constraints leave more independent dofs), and its pinned word.
-// The size depends on the context only, so a solve inside a Newton step never reallocates it.
-double* SolveWork(nuto_ctx* ctx)
+// The solver of the context's system for the matrix values K, with the workspace, the pinned states and
+// their events that the context keeps between solves (allocated once, or again for a larger system)
+ReducedSolver MakeSolver(nuto_ctx* ctx, const double* K)
 {
-    const size_t need = ReducedSolver::WorkDoubles(ctx->nRows, ctx->nInd) * sizeof(double);
+    const size_t need = ReducedSolver::WorkDoubles(ctx->nRows) * sizeof(double);
+    SolveBuffers& b = ctx->solveBuf;
     if (ctx->solveWork.bytes < need)
         Check(ctx->solveWork.Alloc(need), "solver buffers");
-    if (!ctx->solveHost)
-        Check(hipHostMalloc(&ctx->solveHost, 8 * sizeof(double), hipHostMallocDefault), "solver buffers");
-    return ctx->solveWork.As<double>();
+    b.work = ctx->solveWork.As<double>();
+    if (!b.host)
+        Check(hipHostMalloc(&b.host, 2 * sizeof(KrylovState), hipHostMallocDefault), "solver buffers");
+    for (hipEvent_t& e : b.arrived)
+        if (!e)
+            Check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "solver events");
+    const Csr Kc{ctx->nRows, ctx->rowPtr.As<int>(), ctx->col.As<int>(), K};
+    const Csr Ct{ctx->nInd, ctx->ctRow.As<int>(), ctx->ctCol.As<int>(), ctx->ctVal.As<double>()};
+    ConstraintView c;
+    c.nEq = ctx->nEq;
+    c.nTermDofs = ctx->nTermDofs;
+    c.dep = ctx->consDep.As<int>();
+    c.ptr = ctx->consPtr.As<int>();
+    c.dof = ctx->consDof.As<int>();
+    c.val = ctx->consVal.As<double>();
+    c.tDof = ctx->consTDof.As<int>();
+    c.tPtr = ctx->consTPtr.As<int>();
+    c.tDep = ctx->consTDep.As<int>();
+    c.tVal = ctx->consTVal.As<double>();
+    return ReducedSolver(ctx->stream, Kc, Ct, ctx->consRev.As<int>(), ctx->consMask.As<unsigned char>(), c,
+                         KNodeRows(ctx), b);
 }
 
 void SolveConstrained(nuto_ctx* ctx, const double* K, const double* f, const double* rhsOld, const double* rhsNew,
@@ -1450,18 +1515,9 @@ void SolveConstrained(nuto_ctx* ctx, const double* K, const double* f, const dou
     Require(!trial || ctx->nEq == 0 || rhsNew, NUTO_ERR_ARGUMENT, "rhs_new is NULL");
     const long long n = ctx->nRows;
     const int m = ctx->nInd;
-    Csr Kc{ctx->nRows, ctx->rowPtr.As<int>(), ctx->col.As<int>(), K};
-    Csr Cc{ctx->nRows, ctx->cRow.As<int>(), ctx->cCol.As<int>(), ctx->cVal.As<double>()};
-    Csr Ct{m, ctx->ctRow.As<int>(), ctx->ctCol.As<int>(), ctx->ctVal.As<double>()};
-    ReducedSolver rs(ctx->stream, Kc, Cc, Ct, n, m, KNodeRows(ctx), SolveWork(ctx), ctx->solveHost);
-    double* delta = rs.Extra();
-    double* g = delta + n;
-    double* invd = g + n;
-    double* b = invd + m;
-    double* u = b + m;
-    if (m > 0)
-        hipLaunchKernelGGL(kDiagCtKC, dim3((m + 255) / 256), dim3(256), 0, ctx->stream, m, Ct.row, Ct.col, Ct.val,
-                           Kc.row, Kc.col, Kc.val, invd);
+    ReducedSolver rs = MakeSolver(ctx, K);
+    double* delta = rs.Vec(10);
+    double* g = rs.Vec(11);
     const double* rhs = f;
     if (trial)
     {
@@ -1474,17 +1530,14 @@ void SolveConstrained(nuto_ctx* ctx, const double* K, const double* f, const dou
         rs.Axpby(n, 1.0, f, 1.0, g);
         rhs = g;
     }
-    rs.Spmv(Ct, rhs, b);
     Check(hipGetLastError(), "solver setup");
     const double tol = opt && opt->tolerance > 0.0 ? opt->tolerance : 2.220446049250313e-16;
     const int maxIt = opt && opt->max_iterations > 0 ? opt->max_iterations : 2 * m;
     int iters = 0;
     double rel = 0.0;
-    if (method == NUTO_SOLVER_CG)
-        Check(rs.Cg(b, invd, u, tol, maxIt, iters, rel), "conjugate gradients");
-    else
-        Check(rs.Bicgstab(b, invd, u, tol, maxIt, iters, rel), "BiCGSTAB");
-    rs.Spmv(Cc, u, x);  // x = C u
+    const bool cg = method == NUTO_SOLVER_CG;
+    Check(rs.Solve(cg, rhs, tol, maxIt, iters, rel), cg ? "conjugate gradients" : "BiCGSTAB");
+    rs.Axpby(n, 1.0, rs.Vec(0), 0.0, x);  // x = C u
     if (trial)
         rs.Axpby(n, -1.0, delta, 1.0, x);  // the negative increment: C u - delta
     Check(hipGetLastError(), "solver result");
@@ -1513,31 +1566,25 @@ void QuasistaticStep(nuto_ctx* ctx, double* x, double* kappa, const double* rhsO
     const nuto_solver_options lin = o ? o->linear : nuto_solver_options{NUTO_SOLVER_BICGSTAB, 0.0, 0};
     BuildConstraints(ctx);
     const long long n = ctx->nRows;
-    const int m = ctx->nInd;
     const long long nU = ctx->f[0].nDofs;
     const bool two = ctx->params.kind == kGradientDamage;
     double* hist = ctx->params.kind == kLinearElastic ? nullptr : kappa;
 
-    DevBuf K, R, dx, xk, x0, ctr;
+    DevBuf K, R, dx, xk, x0;
     Check(K.Alloc((size_t)ctx->nnz * 8), "Newton buffers");
     Check(R.Alloc((size_t)n * 8), "Newton buffers");
     Check(dx.Alloc((size_t)n * 8), "Newton buffers");
     Check(xk.Alloc((size_t)n * 8), "Newton buffers");
     Check(x0.Alloc((size_t)n * 8), "Newton buffers");
-    Check(ctr.Alloc((size_t)std::max(m, 1) * 8), "Newton buffers");
-    Csr Kc{ctx->nRows, ctx->rowPtr.As<int>(), ctx->col.As<int>(), K.As<double>()};
-    Csr Cc{ctx->nRows, ctx->cRow.As<int>(), ctx->cCol.As<int>(), ctx->cVal.As<double>()};
-    Csr Ct{m, ctx->ctRow.As<int>(), ctx->ctCol.As<int>(), ctx->ctVal.As<double>()};
     // the norms use the solve workspace's reduction slots between solves (all on one stream, each
     // read before the next solve starts)
-    ReducedSolver rs(ctx->stream, Kc, Cc, Ct, n, m, KNodeRows(ctx), SolveWork(ctx), ctx->solveHost);
+    ReducedSolver rs = MakeSolver(ctx, K.As<double>());
 
     auto E = [&](const double* v) -> const double* { return two ? v + nU : nullptr; };
     // QuasistaticSolver::Norm: |C^T v|
     auto Norm = [&](const double* v) {
-        rs.Spmv(Ct, v, ctr.As<double>());
         hipError_t err = hipSuccess;
-        const double d = m > 0 ? rs.Dot(m, ctr.As<double>(), ctr.As<double>(), err) : 0.0;
+        const double d = rs.ReducedNorm2(v, err);
         Check(err, "residual norm");
         return std::sqrt(d);
     };

@@ -1,0 +1,120 @@
+"""Device solves stopped at a given iteration against the same iteration in numpy.
+
+The host queues several iterations before it reads the state of an earlier one, so a limit below,
+at and beyond a queued group must stop at exactly that iteration; rows longer than 128 columns leave
+the part of the K product that is loaded ahead. Conjugate gradients and BiCGSTAB with the diagonal
+preconditioner are restated densely on C^T K C. Tolerance: at most 9 iterations on systems with
+condition numbers below 1e4, each step's rounding (1e-16) amplified by at most the condition number,
+with 3 digits to spare: 1e-9 of the largest entry.
+"""
+import numpy as np
+import pytest
+
+import nuto_amd as N
+from pairs import Pair, make_mesh, to_dev
+from test_gpu_parity import le_params
+
+pytestmark = pytest.mark.gpu
+
+
+def cg(A, b, k):
+    d = 1.0 / np.diag(A)
+    x, r = np.zeros_like(b), b.copy()
+    z = d * r
+    p, rz = z.copy(), r @ z
+    for _ in range(k):
+        q = A @ p
+        a = rz / (p @ q)
+        x, r = x + a * p, r - a * q
+        z = d * r
+        rz, old = r @ z, rz
+        p = z + (rz / old) * p
+    return x, np.linalg.norm(r) / np.linalg.norm(b)
+
+
+def bicgstab(A, b, k):
+    d = 1.0 / np.diag(A)
+    x, r, r0 = np.zeros_like(b), b.copy(), b.copy()
+    p = v = np.zeros_like(b)
+    rho = alpha = w = 1.0
+    for _ in range(k):
+        rho, old = r0 @ r, rho
+        p = r + (rho / old) * (alpha / w) * (p - w * v)
+        y = d * p
+        v = A @ y
+        alpha = rho / (r0 @ v)
+        s = r - alpha * v
+        z = d * s
+        t = A @ z
+        w = (t @ s) / (t @ t)
+        x = x + alpha * y + w * z
+        r = s - w * t
+    return x, np.linalg.norm(r) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("element,n,terms", [("quad4", (1, 1), False), ("quad4", (7, 3), True), ("hex8", (2, 3, 2), False),
+                                             ("hex20", (2, 1, 2), True), ("hex20", (1, 2, 1), False)])
+@pytest.mark.parametrize("method", [N.SOLVER_CG, N.SOLVER_BICGSTAB])
+def test_stops_at_the_limit(element, n, terms, method):
+    ct = N.QUAD4 if element == "quad4" else N.HEX8
+    dt = {"quad4": N.QUAD4, "hex8": N.HEX8, "hex20": N.HEX20}[element]
+    X, C = make_mesh(ct, n, (1.0, 1.2, 0.9))
+    dim = N.DIM[ct]
+    p = Pair(ct, dt, X, C, *le_params(dim), two_fields=False)
+    ctx = p.context()
+    K = ctx.build_matrix(to_dev(np.zeros(p.n_u)))
+    rp, ci = ctx.pattern()
+    dense = np.zeros((p.n_u, p.n_u))
+    dense[np.repeat(np.arange(p.n_u), np.diff(rp)), ci] = K.cpu().numpy()
+    xs = np.zeros((p.nn, dim))
+    xs[p.ranks[:, :C.shape[1]].ravel()] = X[C.ravel(), :dim]
+    xs[np.setdiff1d(np.arange(p.nn), p.ranks[:, :C.shape[1]])] = 1.0  # edge nodes: not clamped here
+    left = np.nonzero(xs[:, 0] < 1e-12)[0]
+    eqs = [(int(dim * r + c), []) for r in left for c in range(dim)]
+    if terms:
+        free = np.setdiff1d(np.arange(p.n_u), [q[0] for q in eqs])
+        eqs.append((int(free[3]), [(int(free[0]), -0.5), (int(free[-1]), 0.25), (int(free[0]), 0.1)]))
+        eqs.append((int(free[5]), [(int(free[0]), -0.3)]))
+    ctx.set_constraints(0, eqs)
+    ind = np.setdiff1d(np.arange(p.n_u), [q[0] for q in eqs])
+    Cm = np.zeros((p.n_u, len(ind)))
+    Cm[ind, np.arange(len(ind))] = 1.0
+    for dep, ts in eqs:
+        for g, coef in ts:
+            Cm[dep, np.searchsorted(ind, g)] -= coef
+    f = np.random.default_rng(3).uniform(-1.0, 1.0, p.n_u)
+    A, b = Cm.T @ dense @ Cm, Cm.T @ f
+    for k in [k for k in (1, 3, 4, 5, 8, 9) if k < len(ind) // 2]:
+        x, info = ctx.solve(K, to_dev(f), method=method, tol=1e-300, max_iter=k)
+        want, rel = (cg if method == N.SOLVER_CG else bicgstab)(A, b, k)
+        want = Cm @ want
+        assert info["iterations"] == k
+        assert np.abs(x.cpu().numpy() - want).max() <= 1e-9 * np.abs(want).max()
+        assert abs(info["relative_residual"] - rel) <= 1e-9 * max(rel, 1.0)
+    # to convergence, and a right-hand side of zero
+    x, info = ctx.solve(K, to_dev(f), method=method, tol=1e-13)
+    want = Cm @ np.linalg.solve(A, b)
+    assert np.abs(x.cpu().numpy() - want).max() <= 1e-9 * np.abs(want).max()
+    x, info = ctx.solve(K, to_dev(np.zeros(p.n_u)), method=method)
+    assert info["iterations"] == 0 and info["relative_residual"] == 0.0 and not x.cpu().numpy().any()
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_bicgstab_restart(seed):
+    """A lower triangular matrix on one quad4 cell (all its dofs are coupled) with f = e_0: after the
+    first iteration the residual has no entry at dof 0, so rho = 0 and the solver must restart."""
+    X, C = make_mesh(N.QUAD4, (1, 1), (1.0, 1.0, 1.0))
+    p = Pair(N.QUAD4, N.QUAD4, X, C, *le_params(2), two_fields=False)
+    ctx = p.context()
+    rp, ci = ctx.pattern()
+    assert len(ci) == 64
+    rng = np.random.default_rng(seed)
+    A = np.tril(rng.uniform(-0.5, 0.5, (8, 8)), -1) + np.diag(rng.uniform(1.0, 2.0, 8))
+    K = to_dev(A[np.repeat(np.arange(8), np.diff(rp)), ci])
+    ctx.set_constraints(0, [])
+    f = np.zeros(8)
+    f[0] = 1.0
+    x, info = ctx.solve(K, to_dev(f), method=N.SOLVER_BICGSTAB, tol=1e-13, max_iter=200)
+    want = np.linalg.solve(A, f)
+    assert info["iterations"] < 200 and info["relative_residual"] <= 1e-13
+    assert np.abs(x.cpu().numpy() - want).max() <= 1e-9 * np.abs(want).max()
