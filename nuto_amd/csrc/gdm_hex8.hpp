@@ -339,7 +339,6 @@ __device__ inline int NodeOfBlock(const GdmHex8Tables& T)
 struct NodeFetch
 {
     int cell, la, slot;
-    int q;  // dof node of (r, j)
     double v[4];  // u0 u1 u2 e of node j of cell r
     double g[gdm8::kGeo];  // geometry of cell r at IP j
     double sr[gdm8::kSr];  // pre-pass state of cell r at IP j
@@ -359,7 +358,6 @@ __device__ inline void FetchNode(const RowArgs& A, const GdmHex8Tables& T, int p
     f.la = T.nodeLa[pr];
     f.slot = T.nodeSlot[pr * 8 + j];
     f.kh = 0.0;
-    f.q = 0;
     if (CLAMP || f.cell >= 0)
     {
         const int cl = CLAMP && f.cell < 0 ? 0 : f.cell;
@@ -387,7 +385,6 @@ __device__ inline void FetchNode(const RowArgs& A, const GdmHex8Tables& T, int p
         {
             const int hist = T.nodeHist ? T.nodeHist[pr] : f.cell;
             const int q = A.dconn[(size_t)f.cell * 8 + j];
-            f.q = q;
             f.kh = A.kappa[(size_t)hist + (size_t)j * A.kappaLd];
             f.v[0] = A.u[(size_t)q * 3];
             f.v[1] = A.u[(size_t)q * 3 + 1];
@@ -653,7 +650,7 @@ struct NodeLds
 
 // The rows of node p (one 64-lane workgroup); `state` is the workgroup's LDS (NodeLds::kState doubles):
 // records [i][r][kSt]; after phase B: partial blocks, R sums and the slot map.
-template <bool WR, bool WK, bool FULLDMG, int MODE>
+template <bool WR, bool FULLDMG, int MODE>
 __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int pos, double* state)
 {
     using namespace gdm8;
@@ -696,21 +693,17 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
         PreRecord<FULLDMG, kSt, false>(f.sr, f.g, la, j, P, rec, Rv);
         if (!valid)
             Rv[0] = Rv[1] = Rv[2] = Rv[3] = 0.0;
-        if (WK)
-        {
-            StoreRecord<kSt>(state + (r * 8 + j) * kSt, rec);
-            __syncthreads();
-            // lane (r, b) works on cell r, whose J^-1 the group holds
-            const double inv[3][3] = {{f.g[0], f.g[1], f.g[2]}, {f.g[3], f.g[4], f.g[5]}, {f.g[6], f.g[7], f.g[8]}};
-            PhaseBAffine<FULLDMG, kSt>(state, r, j, inv, acc);
-        }
+        StoreRecord<kSt>(state + (r * 8 + j) * kSt, rec);
+        __syncthreads();
+        // lane (r, b) works on cell r, whose J^-1 the group holds
+        const double inv[3][3] = {{f.g[0], f.g[1], f.g[2]}, {f.g[3], f.g[4], f.g[5]}, {f.g[6], f.g[7], f.g[8]}};
+        PhaseBAffine<FULLDMG, kSt>(state, r, j, inv, acc);
     }
     else if constexpr (PRE)
     {
         double rec[kSt];
         if (valid)
             PreRecord<FULLDMG, kSt>(f.sr, f.g, la, j, P, rec, Rv);
-        if (WK)
         {
             // pass 0: IPs 0..3 (records of lanes j < 4)
             if (valid && j < 4)
@@ -760,7 +753,6 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
                 Rv[2] = s * bt[2];
                 Rv[3] = s * (Na * (eN - eq) + P.c * (ga[0] * ge[0] + ga[1] * ge[1] + ga[2] * ge[2]));
             }
-            if (WK)
             {
                 double m[6];
                 GdmMisesDerivative(st, P, m);
@@ -804,10 +796,10 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
     if constexpr (!PRE)
     {
         __syncthreads();
-        if (WK && valid)
+        if (valid)
             PhaseB<FULLDMG, kSt>(state, r, j, 0, 8, acc);
     }
-    if (WK && (valid || AFF) && FULLDMG)
+    if ((valid || AFF) && FULLDMG)
     {
         // uu = lambda' S + mu' S^T + mu' tr(S) I
         const double lam = (m3K - m2G) * kThird, mu = 0.5 * m2G;
@@ -838,7 +830,6 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
     double* rcell = state + 8 * 8 * kPs;  // [4][r]: R terms summed over the IPs of cell r
     // slotOf[q][r] = local index b of neighbour q in cell r, 0xFF if q is not a node of cell r
     unsigned char(*slotOf)[kMaxInc] = reinterpret_cast<unsigned char(*)[kMaxInc]>(rcell + 40);
-    if (WK)
     {
         reinterpret_cast<unsigned int*>(slotOf)[lane] = 0xFFFFFFFFu;  // 64 x 4 bytes = the whole map
 #pragma unroll
@@ -852,7 +843,7 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
             rcell[k * 8 + r] = Rv[k];
     }
     __syncthreads();
-    if (WK && valid)
+    if (valid)
         slotOf[f.slot][r] = (unsigned char)j;
     __syncthreads();
 
@@ -860,7 +851,6 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
     // (only the cells that hold q are read: the lanes of absent (cell, q) pairs sit out that step, so
     // the LDS reads are the 64 partial blocks, not 8 per neighbour). Row layout: the three
     // displacement rows of p are consecutive in the CSR (4 nA columns each), then the eeq row.
-    if (WK)
     {
         const int q = lane >> 1, h = lane & 1;
         double sum[8];
@@ -917,7 +907,7 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
 }
 
 // MODE >= 1 targets 4 waves per SIMD (<= 128 VGPRs; the LDS of modes 1 and 2 allows 16 workgroups per CU)
-template <bool WR, bool WK, bool FULLDMG, int MODE>
+template <bool WR, bool FULLDMG, int MODE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE >= 1 ? 4 : 1)))
 kGdmHex8Node(const RowArgs A, const GdmHex8Tables T)
 {
@@ -925,7 +915,7 @@ kGdmHex8Node(const RowArgs A, const GdmHex8Tables T)
     const int pos = NodeOfBlock(T);
     if (pos < 0)
         return;
-    NodeBody<WR, WK, FULLDMG, MODE>(A, T, pos, state);
+    NodeBody<WR, FULLDMG, MODE>(A, T, pos, state);
 }
 
 // Pre-pass: the state of every (cell, IP) once, for the node kernel (which would otherwise evaluate
@@ -1151,7 +1141,7 @@ struct GdmHex8Plan
     int xcdMap = 1;   // contiguous node ranges per XCD (env NUTO_AMD_GDM_XCD_MAP=0 switches it off)
     DevBuf nodeHead, nodeCell, nodeHist, nodeLa, nodeSlot, geo;
     DevBuf posOf;        // node -> table position (Morton order; NUTO_AMD_GDM_ORDER=0: node order, empty)
-    DevBuf ipState;      // pre-pass state records (NUTO_AMD_GDM_PREPASS=0: recompute in the node kernel)
+    DevBuf ipState;      // pre-pass state records, or cell vectors (Work)
     DevBuf geoCell;      // affine meshes: IP 0's geometry record per cell
     DevBuf extra;        // nodes beyond the kernel's bounds (more than 8 cells or 32 neighbours)
     int nExtra = 0;      // ... assembled by the generic row-owner kernel
@@ -1306,7 +1296,7 @@ struct GdmHex8Plan
                 return false;
             }
         }
-        if (prepass && (err = ipState.Alloc((size_t)nCells * 8 * gdm8::kSr * sizeof(double))) != hipSuccess)
+        if ((err = ipState.Alloc((size_t)nCells * 8 * gdm8::kSr * sizeof(double))) != hipSuccess)
         {
             Release();
             return false;
@@ -1330,14 +1320,12 @@ struct GdmHex8Plan
     }
 
     template <bool FULLDMG, int MODE>
-    void LaunchNodes(const RowArgs& a, const GdmHex8Tables& t, bool wr, bool wk, int grid_, hipStream_t stream)
+    void LaunchNodes(const RowArgs& a, const GdmHex8Tables& t, bool wr, int grid_, hipStream_t stream)
     {
-        if (wr && wk)
-            hipLaunchKernelGGL((kGdmHex8Node<true, true, FULLDMG, MODE>), dim3(grid_), dim3(64), 0, stream, a, t);
-        else if (wr)
-            hipLaunchKernelGGL((kGdmHex8Node<true, false, FULLDMG, MODE>), dim3(grid_), dim3(64), 0, stream, a, t);
+        if (wr)
+            hipLaunchKernelGGL((kGdmHex8Node<true, FULLDMG, MODE>), dim3(grid_), dim3(64), 0, stream, a, t);
         else
-            hipLaunchKernelGGL((kGdmHex8Node<false, true, FULLDMG, MODE>), dim3(grid_), dim3(64), 0, stream, a, t);
+            hipLaunchKernelGGL((kGdmHex8Node<false, FULLDMG, MODE>), dim3(grid_), dim3(64), 0, stream, a, t);
     }
 
     // doubles of the pre-pass state records (written in full by kGdmHex8Ip before the node kernel reads them)
@@ -1347,7 +1335,7 @@ struct GdmHex8Plan
     }
 
     template <bool FULLDMG>
-    void LaunchT(const RowArgs& a, bool wr, bool wk, double* state, hipStream_t stream)
+    void LaunchT(const RowArgs& a, bool wr, double* state, hipStream_t stream)
     {
         GdmHex8Tables t = Tables();
         if (prepass)
@@ -1358,46 +1346,51 @@ struct GdmHex8Plan
             {
                 if (nCells > 0)
                     hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, true>), ipGrid, dim3(64), 0, stream, a, t, state);
-                LaunchNodes<FULLDMG, 2>(a, t, wr, wk, grid, stream);
+                LaunchNodes<FULLDMG, 2>(a, t, wr, grid, stream);
             }
             else
             {
                 if (nCells > 0)
                     hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, false>), ipGrid, dim3(64), 0, stream, a, t, state);
-                LaunchNodes<FULLDMG, 1>(a, t, wr, wk, grid, stream);
+                LaunchNodes<FULLDMG, 1>(a, t, wr, grid, stream);
             }
         }
         else
-            LaunchNodes<FULLDMG, 0>(a, t, wr, wk, grid, stream);
+            LaunchNodes<FULLDMG, 0>(a, t, wr, grid, stream);
     }
 
-    // state: device memory of StateDoubles() doubles for the pre-pass records (nullptr: the plan's own)
-    void Launch(const RowArgs& a, bool wr, bool wk, hipStream_t stream, double* state = nullptr)
+    // K (and R, wr). state: device memory of StateDoubles() doubles for the pre-pass records (nullptr: the
+    // plan's own)
+    void Launch(const RowArgs& a, bool wr, hipStream_t stream, double* state = nullptr)
     {
         if (nNodes > 0)
         {
-            if (!state && ipState.p)
-                state = ipState.As<double>();
+            if (!state)
+                state = Work();
             if (a.P.damage_application == 0)
-                LaunchT<true>(a, wr, wk, state, stream);
+                LaunchT<true>(a, wr, state, stream);
             else
-                LaunchT<false>(a, wr, wk, state, stream);
+                LaunchT<false>(a, wr, state, stream);
         }
-        LaunchExtras(a, wr, wk, stream);
+        LaunchExtras(a, wr, stream);
     }
 
-    // R and K rows of the nodes beyond the node kernel's bounds (the generic row-owner body)
-    void LaunchExtras(const RowArgs& a, bool wr, bool wk, hipStream_t stream)
+    // The plan's device memory: the pre-pass records of a matrix assembly (StateDoubles), or the cell
+    // vectors of a residual or an adjoint (32 doubles per cell, less than the records)
+    double* Work() const
+    {
+        return ipState.As<double>();
+    }
+
+    // K (and R) rows of the nodes beyond the node kernel's bounds (the generic row-owner body)
+    void LaunchExtras(const RowArgs& a, bool wr, hipStream_t stream)
     {
         if (nExtra > 0)
         {
             const dim3 grid((unsigned)((nExtra + 63) / 64));
             const int* list = extra.As<int>();
-            if (wr && wk)
+            if (wr)
                 hipLaunchKernelGGL((kAssembleRowsList<kGradientDamage, 3, 8, 8, 8, 4, true, true>), grid, dim3(64), 0,
-                                   stream, a, list, nExtra);
-            else if (wr)
-                hipLaunchKernelGGL((kAssembleRowsList<kGradientDamage, 3, 8, 8, 8, 4, true, false>), grid, dim3(64), 0,
                                    stream, a, list, nExtra);
             else
                 hipLaunchKernelGGL((kAssembleRowsList<kGradientDamage, 3, 8, 8, 8, 4, false, true>), grid, dim3(64), 0,
@@ -1418,9 +1411,9 @@ struct GdmHex8Plan
         t.order = posOf.p ? posOf.As<int>() : nullptr;  // launch index = node
         // per-mesh launches recompute the IP state in the node kernel (no pre-pass over the mesh's cells)
         if (a.P.damage_application == 0)
-            LaunchNodes<true, 0>(a, t, true, true, end - first, stream);
+            LaunchNodes<true, 0>(a, t, true, end - first, stream);
         else
-            LaunchNodes<false, 0>(a, t, true, true, end - first, stream);
+            LaunchNodes<false, 0>(a, t, true, end - first, stream);
     }
 };
 

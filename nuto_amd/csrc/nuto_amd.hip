@@ -17,7 +17,7 @@
 #include "assemble_rows.hpp"
 #include "elements.hpp"
 #include "gdm_hex8.hpp"
-#include "gdm_hex8_vjp.hpp"
+#include "gdm_hex8_vectors.hpp"
 #include "batch.hpp"
 #include "cell_fields.hpp"
 #include "cell_gram.hpp"
@@ -754,7 +754,10 @@ void Assemble(nuto_ctx* ctx, const double* u, const double* e, const double* kap
     if (nodeKernel && ctx->gdm.Usable(ctx->params.kind, ctx->coordType, ctx->f[0].type, ctx->nip))
     {
         RowArgs a = MakeRowArgs(ctx, u, e, kappa, R, K);
-        ctx->gdm.Launch(a, wr, wk, ctx->stream);
+        if (wk)
+            ctx->gdm.Launch(a, wr, ctx->stream);
+        else
+            LaunchGdmHex8Vector<false>(ctx->gdm, a, nullptr, R, nullptr, ctx->gdm.Work(), ctx->stream);
         Check(hipGetLastError(), "gdm hex8 launch");
         SyncCheck(ctx, "gdm hex8 kernel");
         return;
@@ -1220,7 +1223,7 @@ int nuto_build_vector_matrix_noalloc(nuto_ctx* ctx, const double* u, const doubl
         double* state = ScratchOf(ctx->device);
         Require(state != nullptr, NUTO_ERR_DEVICE, "device scratch address not resolved");
         RowArgs a = MakeRowArgs(ctx, u, e, kappa, R, K);
-        ctx->gdm.Launch(a, true, true, ctx->stream, state);
+        ctx->gdm.Launch(a, true, ctx->stream, state);
         Check(hipGetLastError(), "gdm hex8 launch");
         SyncCheck(ctx, "gdm hex8 kernel");
     });
@@ -1696,11 +1699,10 @@ int nuto_vjp(nuto_ctx* ctx, const double* u, const double* e, const double* kapp
         if (!ctx->tabValid)
             BuildTables(ctx);
         PrepareGdm(ctx);
-        // nodes beyond the node kernel's bounds (more than 8 cells or 32 neighbours) get the list kernel
         Require(ctx->gdm.Usable(ctx->params.kind, ctx->coordType, ctx->f[0].type, ctx->nip), NUTO_ERR_UNSUPPORTED,
                 "the adjoint needs hex8 cells and dofs and 2x2x2 Gauss points");
         RowArgs a = MakeRowArgs(ctx, u, e, kappa, nullptr, nullptr);
-        LaunchGdmHex8Vjp(ctx->gdm, a, lambda, d_state, d_theta, ctx->stream);
+        LaunchGdmHex8Vector<true>(ctx->gdm, a, lambda, d_state, d_theta, ctx->gdm.Work(), ctx->stream);
         Check(hipGetLastError(), "vjp launch");
         SyncCheck(ctx, "vjp kernel");
     });
@@ -2077,7 +2079,7 @@ void LaunchBatch(nuto_batch* b, int mode, const double* u, const double* e, cons
             if (mode == 3)
             {
                 if (IsGdm(b))
-                    g.ctx->gdm.Launch(a, true, true, b->stream);
+                    g.ctx->gdm.Launch(a, true, b->stream);
                 else if (kind == kLinearElastic)
                     LaunchRange<kLinearElastic>(a, g.type, 0, g.nNodes, b->stream);
                 else
@@ -2096,7 +2098,7 @@ void LaunchBatch(nuto_batch* b, int mode, const double* u, const double* e, cons
                     LaunchRange<kLocalDamage>(a, g.type, first, end, b->stream);
             }
             if (IsGdm(b))
-                g.ctx->gdm.LaunchExtras(a, true, true, b->stream);
+                g.ctx->gdm.LaunchExtras(a, true, b->stream);
         }
     }
     Check(hipGetLastError(), "batch launch");
@@ -2116,7 +2118,8 @@ void LaunchVjp(nuto_batch* b, const double* u, const double* e, const double* ka
     for (BatchGroup& g : b->groups)
     {
         RowArgs a = MakeRowArgs(g.ctx, u + g.uOff, e + g.eOff, kappa + g.hOff, nullptr, nullptr);
-        LaunchGdmHex8Vjp(g.ctx->gdm, a, lam + g.ROff, dstate + g.ROff, dtheta ? dtheta + g.tOff : nullptr, b->stream);
+        LaunchGdmHex8Vector<true>(g.ctx->gdm, a, lam + g.ROff, dstate + g.ROff, dtheta ? dtheta + g.tOff : nullptr,
+                                  g.ctx->gdm.Work(), b->stream);
     }
     Check(hipGetLastError(), "batch vjp launch");
 }
