@@ -61,6 +61,12 @@ constexpr int kGeo = 10;     // doubles per (cell, IP) geometry record: J^-1 (ro
 // (tensor strain) the stress, t = s omega' kappa' d sigma / d omega and m = d eps_eq / d eps are all
 // of the form alpha [1, 1, 1, 0, 0, 0] + beta e'', so B_a^T of each is alpha g_a + beta (e'' g_a)
 constexpr int kSr = 18;
+// with the decreasing nonlocal interaction two more, the factor g and g' omega' kappa' (padded to an odd
+// number of 16-byte chunks)
+template <bool DEC>
+constexpr int kSrOf = DEC ? 22 : kSr;
+constexpr int rGi = 18;   // g(omega)
+constexpr int rDg = 19;   // dg / d omega * d omega / d kappa * d kappa / d eeq
 constexpr int rEps = 0;   // e'' (6)
 constexpr int rSig = 6;   // s alpha_sigma, s beta_sigma
 constexpr int rT = 8;     // alpha_t, beta_t (s included)
@@ -310,7 +316,7 @@ struct GdmHex8Tables
     const unsigned char* nodeLa;    // [pos][8]: local index of the node in that cell
     const unsigned char* nodeSlot;  // [pos][8][8]: neighbour slot (column block) of local node j
     const double* geo;              // [cell][ip][kGeo] geometry records
-    const double* ipState;          // [cell][ip][kSr] pre-pass state records (nullptr: recompute)
+    const double* ipState;          // [cell][ip][kSrOf] pre-pass state records (nullptr: recompute)
     const double* geoCell;          // [cell][kGeo] IP 0's geometry record (affine meshes, else nullptr)
     int xcdMap;                     // 1: contiguous node ranges per XCD
     int pBegin, pEnd;               // launch indices [pBegin, pEnd)
@@ -336,12 +342,13 @@ __device__ inline int NodeOfBlock(const GdmHex8Tables& T)
 }
 
 // Inputs of lane (r, j) of node p.
+template <bool DEC>
 struct NodeFetch
 {
     int cell, la, slot;
     double v[4];  // u0 u1 u2 e of node j of cell r
     double g[gdm8::kGeo];  // geometry of cell r at IP j
-    double sr[gdm8::kSr];  // pre-pass state of cell r at IP j
+    double sr[gdm8::kSrOf<DEC>];  // pre-pass state of cell r at IP j
     double th[3];
     double kh;  // history kappa of cell r at IP j
 };
@@ -350,9 +357,10 @@ struct NodeFetch
 // CLAMP: lanes past the node's last incident cell (f.cell < 0) load cell 0's records instead of
 // skipping the loads, so that every lane runs the same straight-line code (their results are
 // never used: the slot map of the reduction leaves absent cells out).
-template <bool PRE, bool GEO0 = false, bool CLAMP = false>
-__device__ inline void FetchNode(const RowArgs& A, const GdmHex8Tables& T, int pos, int r, int j, NodeFetch& f)
+template <bool PRE, bool GEO0, bool CLAMP, bool DEC>
+__device__ inline void FetchNode(const RowArgs& A, const GdmHex8Tables& T, int pos, int r, int j, NodeFetch<DEC>& f)
 {
+    constexpr int kN = gdm8::kSrOf<DEC>, kUse = DEC ? 20 : gdm8::kSr;  // record stride, doubles read
     const size_t pr = (size_t)pos * 8 + r;
     f.cell = T.nodeCell[pr];
     f.la = T.nodeLa[pr];
@@ -372,9 +380,9 @@ __device__ inline void FetchNode(const RowArgs& A, const GdmHex8Tables& T, int p
         }
         if constexpr (PRE)
         {
-            const double2* sp = reinterpret_cast<const double2*>(T.ipState + ((size_t)cl * 8 + j) * gdm8::kSr);
+            const double2* sp = reinterpret_cast<const double2*>(T.ipState + ((size_t)cl * 8 + j) * kN);
 #pragma unroll
-            for (int k = 0; k < gdm8::kSr / 2; k++)
+            for (int k = 0; k < kUse / 2; k++)
             {
                 const double2 v = sp[k];
                 f.sr[2 * k] = v.x;
@@ -421,9 +429,11 @@ __device__ inline double GroupSum0(double v)
 }
 
 // geometry and pre-pass state records of (cell, ip)
+template <bool DEC>
 __device__ inline void LoadIpRecords(const GdmHex8Tables& T, int cell, int ip, double g[gdm8::kGeo],
-                                     double sr[gdm8::kSr])
+                                     double sr[gdm8::kSrOf<DEC>])
 {
+    constexpr int kN = gdm8::kSrOf<DEC>, kUse = DEC ? 20 : gdm8::kSr;
     const double2* gr = reinterpret_cast<const double2*>(T.geo + ((size_t)cell * 8 + ip) * gdm8::kGeo);
 #pragma unroll
     for (int k = 0; k < gdm8::kGeo / 2; k++)
@@ -432,9 +442,9 @@ __device__ inline void LoadIpRecords(const GdmHex8Tables& T, int cell, int ip, d
         g[2 * k] = v.x;
         g[2 * k + 1] = v.y;
     }
-    const double2* sp = reinterpret_cast<const double2*>(T.ipState + ((size_t)cell * 8 + ip) * gdm8::kSr);
+    const double2* sp = reinterpret_cast<const double2*>(T.ipState + ((size_t)cell * 8 + ip) * kN);
 #pragma unroll
-    for (int k = 0; k < gdm8::kSr / 2; k++)
+    for (int k = 0; k < kUse / 2; k++)
     {
         const double2 v = sp[k];
         sr[2 * k] = v.x;
@@ -447,7 +457,9 @@ __device__ inline void LoadIpRecords(const GdmHex8Tables& T, int cell, int ip, d
 // R terms s B_a^T sigma, s (N_a (eeq - eps_eq) + c g_a . grad eeq).
 // WITHINV false: the record omits J^-1 (affine cells keep one J^-1 per cell) and the other terms
 // start at 0 instead of 9.
-template <bool FULLDMG, int kSt, bool WITHINV = true>
+// DEC: the nonlocal term carries g(omega), and K_ee the term c (grad eeq . g_a) g' omega' kappa' N_b, which
+// joins s N_a N_b.
+template <bool FULLDMG, int kSt, bool WITHINV, bool DEC>
 __device__ inline void PreRecord(const double* sr, const double* g, int la, int ip, const LawParams& P, double rec[kSt],
                                  double Rv[4])
 {
@@ -465,7 +477,9 @@ __device__ inline void PreRecord(const double* sr, const double* g, int la, int 
 #pragma unroll
     for (int i = 0; i < 3; i++)
         Rv[i] = sr[rSig] * ga[i] + sr[rSig + 1] * Eg[i];
-    Rv[3] = Na * sr[rRe] + (ga[0] * sr[rGe] + ga[1] * sr[rGe + 1] + ga[2] * sr[rGe + 2]);
+    const double gdot = ga[0] * sr[rGe] + ga[1] * sr[rGe + 1] + ga[2] * sr[rGe + 2];
+    Rv[3] = Na * sr[rRe] + (DEC ? sr[DEC ? rGi : 0] * gdot : gdot);
+    const double cs = DEC ? P.c * s * sr[DEC ? rGi : 0] : P.c * s;
     if constexpr (WITHINV)
     {
 #pragma unroll
@@ -479,14 +493,14 @@ __device__ inline void PreRecord(const double* sr, const double* g, int la, int 
     {
         rec[o + sHa + i] = sr[rC1] * ga[i];
         rec[o + sVa + i] = sr[rT] * ga[i] + sr[rT + 1] * Eg[i];
-        rec[o + sCg + i] = P.c * s * ga[i];
+        rec[o + sCg + i] = cs * ga[i];
         if (!FULLDMG)
             rec[o + sKa + i] = sr[rC2] * ga[i];
     }
 #pragma unroll
     for (int i = 0; i < 6; i++)
         rec[o + sMn + i] = -Na * ((i < 3 ? sr[rM] : 0.0) + sr[rM + 1] * sr[rEps + i]);
-    rec[o + sSn] = s * Na;
+    rec[o + sSn] = DEC ? s * Na + sr[DEC ? rDg : 0] * gdot : s * Na;
 #pragma unroll
     for (int k = o + (FULLDMG ? sSn + 1 : sKa + 3); k < kSt; k++)
         rec[k] = 0.0;  // padding
@@ -650,7 +664,7 @@ struct NodeLds
 
 // The rows of node p (one 64-lane workgroup); `state` is the workgroup's LDS (NodeLds::kState doubles):
 // records [i][r][kSt]; after phase B: partial blocks, R sums and the slot map.
-template <bool WR, bool FULLDMG, int MODE>
+template <bool WR, bool FULLDMG, int MODE, bool DEC>
 __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int pos, double* state)
 {
     using namespace gdm8;
@@ -665,8 +679,9 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
     const int4 head = T.nodeHead[pos];
     const int p = head.x, ru0 = head.y, L = head.z, re0 = head.w;
     const int nA = L >> 2;
-    NodeFetch f;
-    FetchNode<PRE, AFF, AFF>(A, T, pos, r, j, f);
+    static_assert(PRE || !DEC, "the decreasing interaction needs the pre-pass");
+    NodeFetch<DEC> f;
+    FetchNode<PRE, AFF, AFF, DEC>(A, T, pos, r, j, f);
     const bool valid = f.cell >= 0;  // r < number of cells incident to p
     const int la = f.la;
 
@@ -690,7 +705,7 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
         // every lane, absent cells included (their records and blocks are never read; their R terms
         // are zeroed)
         double rec[kSt];
-        PreRecord<FULLDMG, kSt, false>(f.sr, f.g, la, j, P, rec, Rv);
+        PreRecord<FULLDMG, kSt, false, DEC>(f.sr, f.g, la, j, P, rec, Rv);
         if (!valid)
             Rv[0] = Rv[1] = Rv[2] = Rv[3] = 0.0;
         StoreRecord<kSt>(state + (r * 8 + j) * kSt, rec);
@@ -703,7 +718,7 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
     {
         double rec[kSt];
         if (valid)
-            PreRecord<FULLDMG, kSt>(f.sr, f.g, la, j, P, rec, Rv);
+            PreRecord<FULLDMG, kSt, true, DEC>(f.sr, f.g, la, j, P, rec, Rv);
         {
             // pass 0: IPs 0..3 (records of lanes j < 4)
             if (valid && j < 4)
@@ -715,9 +730,9 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
             // pass 1: IPs 4..7; lanes j >= 4 rebuild their records from the (cached) state records
             if (valid && j >= 4)
             {
-                double g2[kGeo], sr2[kSr], Rd[4];
-                LoadIpRecords(T, f.cell, j, g2, sr2);
-                PreRecord<FULLDMG, kSt>(sr2, g2, la, j, P, rec, Rd);
+                double g2[kGeo], sr2[kSrOf<DEC>], Rd[4];
+                LoadIpRecords<DEC>(T, f.cell, j, g2, sr2);
+                PreRecord<FULLDMG, kSt, true, DEC>(sr2, g2, la, j, P, rec, Rd);
                 StoreRecord<kSt>(state + (r * 4 + j - 4) * kSt, rec);
             }
             __syncthreads();
@@ -907,7 +922,7 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
 }
 
 // MODE >= 1 targets 4 waves per SIMD (<= 128 VGPRs; the LDS of modes 1 and 2 allows 16 workgroups per CU)
-template <bool WR, bool FULLDMG, int MODE>
+template <bool WR, bool FULLDMG, int MODE, bool DEC>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE >= 1 ? 4 : 1)))
 kGdmHex8Node(const RowArgs A, const GdmHex8Tables T)
 {
@@ -915,7 +930,7 @@ kGdmHex8Node(const RowArgs A, const GdmHex8Tables T)
     const int pos = NodeOfBlock(T);
     if (pos < 0)
         return;
-    NodeBody<WR, FULLDMG, MODE>(A, T, pos, state);
+    NodeBody<WR, FULLDMG, MODE, DEC>(A, T, pos, state);
 }
 
 // Pre-pass: the state of every (cell, IP) once, for the node kernel (which would otherwise evaluate
@@ -926,11 +941,12 @@ kGdmHex8Node(const RowArgs A, const GdmHex8Tables T)
 // records are contiguous blocks in memory; both pass through LDS so that every global load and
 // store of them is 16 contiguous bytes per lane across the wave (the address and data paths, not
 // the arithmetic, bound this kernel).
-template <bool FULLDMG, bool AFF>
+template <bool FULLDMG, bool AFF, bool DEC>
 __global__ void __launch_bounds__(64) kGdmHex8Ip(const RowArgs A, const GdmHex8Tables T, double* __restrict__ out)
 {
     using namespace gdm8;
-    __shared__ __align__(16) double stage[64 * kSr];  // the block's geometry, then its records
+    constexpr int kN = kSrOf<DEC>;
+    __shared__ __align__(16) double stage[64 * kN];  // the block's geometry, then its records
     const int lane = threadIdx.x;
     const int j = lane & 7, r = lane >> 3;
     const long long cell0 = (long long)blockIdx.x * 8;
@@ -1000,7 +1016,7 @@ __global__ void __launch_bounds__(64) kGdmHex8Ip(const RowArgs A, const GdmHex8T
             bm = h * P.K2;
         }
         const double ct = s * st.dom * st.dk;
-        double rec[kSr];
+        double rec[kN];
         rec[rEps] = st.eps[0];
         rec[rEps + 1] = st.eps[1];
         rec[rEps + 2] = st.eps[2];
@@ -1019,14 +1035,22 @@ __global__ void __launch_bounds__(64) kGdmHex8Ip(const RowArgs A, const GdmHex8T
         rec[rGe] = s * P.c * st.ge[0];
         rec[rGe + 1] = s * P.c * st.ge[1];
         rec[rGe + 2] = s * P.c * st.ge[2];
-        // record (r, j) at row r * 8 + j: 9 chunks (odd), consecutive lanes on distinct bank groups
-        StoreRecord<kSr>(stage + lane * kSr, rec);
+        if constexpr (DEC)
+        {
+            double gi, dgi;
+            NonlocalFactor(P, st.om, gi, dgi);
+            rec[rGi] = gi;
+            rec[rDg] = dgi * st.dom * st.dk;
+            rec[kN - 2] = rec[kN - 1] = 0.0;
+        }
+        // record (r, j) at row r * 8 + j: 9 or 11 chunks (odd), consecutive lanes on distinct bank groups
+        StoreRecord<kN>(stage + lane * kN, rec);
     }
     __syncthreads();
     {
-        constexpr int kPerCell = 8 * kSr / 2;  // 16-byte chunks of records per cell
+        constexpr int kPerCell = 8 * kN / 2;  // 16-byte chunks of records per cell
         const double2* src = reinterpret_cast<const double2*>(stage);
-        double2* dst = reinterpret_cast<double2*>(out + cell0 * 8 * kSr);
+        double2* dst = reinterpret_cast<double2*>(out + cell0 * 8 * kN);
 #pragma unroll
         for (int i = 0; i < (8 * kPerCell + 63) / 64; i++)
         {
@@ -1147,6 +1171,7 @@ struct GdmHex8Plan
     int nExtra = 0;      // ... assembled by the generic row-owner kernel
     bool prepass = true;
     bool affine = false;  // every cell affine: MODE 2 of the node kernel
+    bool decreasing = false;  // NonlocalInteraction::Decreasing: longer pre-pass records
     int nCells = 0;
 
     void Release()
@@ -1168,7 +1193,7 @@ struct GdmHex8Plan
     // used) when the mesh exceeds the kernel's bounds; a HIP failure is returned through `err`.
     bool Prepare(int kind, int coordType, int dofType, int nip, const NodeGraph& g, int nCells, const int* cellIds,
                  int nCoord, const double* x, const double* y, const double* z, const int* cconn, const double* tab,
-                 const int* rowPtr, int nRows, hipStream_t stream, hipError_t& err)
+                 const int* rowPtr, int nRows, bool decreasingInteraction, hipStream_t stream, hipError_t& err)
     {
         Release();
         err = hipSuccess;
@@ -1296,7 +1321,8 @@ struct GdmHex8Plan
                 return false;
             }
         }
-        if ((err = ipState.Alloc((size_t)nCells * 8 * gdm8::kSr * sizeof(double))) != hipSuccess)
+        decreasing = decreasingInteraction;
+        if ((err = ipState.Alloc((size_t)nCells * 8 * RecordDoubles() * sizeof(double))) != hipSuccess)
         {
             Release();
             return false;
@@ -1319,44 +1345,51 @@ struct GdmHex8Plan
                              xcdMap, 0, nNodes, nullptr};
     }
 
-    template <bool FULLDMG, int MODE>
+    template <bool FULLDMG, int MODE, bool DEC>
     void LaunchNodes(const RowArgs& a, const GdmHex8Tables& t, bool wr, int grid_, hipStream_t stream)
     {
         if (wr)
-            hipLaunchKernelGGL((kGdmHex8Node<true, FULLDMG, MODE>), dim3(grid_), dim3(64), 0, stream, a, t);
+            hipLaunchKernelGGL((kGdmHex8Node<true, FULLDMG, MODE, DEC>), dim3(grid_), dim3(64), 0, stream, a, t);
         else
-            hipLaunchKernelGGL((kGdmHex8Node<false, FULLDMG, MODE>), dim3(grid_), dim3(64), 0, stream, a, t);
+            hipLaunchKernelGGL((kGdmHex8Node<false, FULLDMG, MODE, DEC>), dim3(grid_), dim3(64), 0, stream, a, t);
+    }
+
+    // doubles of a pre-pass record
+    int RecordDoubles() const
+    {
+        return decreasing ? gdm8::kSrOf<true> : gdm8::kSrOf<false>;
     }
 
     // doubles of the pre-pass state records (written in full by kGdmHex8Ip before the node kernel reads them)
     size_t StateDoubles() const
     {
-        return prepass ? (size_t)nCells * 8 * gdm8::kSr : 0;
+        return prepass ? (size_t)nCells * 8 * RecordDoubles() : 0;
     }
 
-    template <bool FULLDMG>
+    template <bool FULLDMG, bool DEC>
     void LaunchT(const RowArgs& a, bool wr, double* state, hipStream_t stream)
     {
         GdmHex8Tables t = Tables();
-        if (prepass)
+        t.ipState = state;
+        const dim3 ipGrid((unsigned)(((long long)nCells * 8 + 63) / 64));
+        if (affine)
         {
-            t.ipState = state;
-            const dim3 ipGrid((unsigned)(((long long)nCells * 8 + 63) / 64));
-            if (affine)
-            {
-                if (nCells > 0)
-                    hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, true>), ipGrid, dim3(64), 0, stream, a, t, state);
-                LaunchNodes<FULLDMG, 2>(a, t, wr, grid, stream);
-            }
-            else
-            {
-                if (nCells > 0)
-                    hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, false>), ipGrid, dim3(64), 0, stream, a, t, state);
-                LaunchNodes<FULLDMG, 1>(a, t, wr, grid, stream);
-            }
+            if (nCells > 0)
+                hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, true, DEC>), ipGrid, dim3(64), 0, stream, a, t, state);
+            LaunchNodes<FULLDMG, 2, DEC>(a, t, wr, grid, stream);
         }
         else
-            LaunchNodes<FULLDMG, 0>(a, t, wr, grid, stream);
+        {
+            if (nCells > 0)
+                hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, false, DEC>), ipGrid, dim3(64), 0, stream, a, t, state);
+            LaunchNodes<FULLDMG, 1, DEC>(a, t, wr, grid, stream);
+        }
+    }
+
+    // the matrix of the plan's interaction can be assembled by the node kernel
+    bool Matrix() const
+    {
+        return prepass || !decreasing;
     }
 
     // K (and R, wr). state: device memory of StateDoubles() doubles for the pre-pass records (nullptr: the
@@ -1367,10 +1400,25 @@ struct GdmHex8Plan
         {
             if (!state)
                 state = Work();
-            if (a.P.damage_application == 0)
-                LaunchT<true>(a, wr, state, stream);
+            const bool full = a.P.damage_application == 0;
+            if (!prepass)
+            {
+                if (full)
+                    LaunchNodes<true, 0, false>(a, Tables(), wr, grid, stream);
+                else
+                    LaunchNodes<false, 0, false>(a, Tables(), wr, grid, stream);
+            }
+            else if (decreasing)
+            {
+                if (full)
+                    LaunchT<true, true>(a, wr, state, stream);
+                else
+                    LaunchT<false, true>(a, wr, state, stream);
+            }
+            else if (full)
+                LaunchT<true, false>(a, wr, state, stream);
             else
-                LaunchT<false>(a, wr, state, stream);
+                LaunchT<false, false>(a, wr, state, stream);
         }
         LaunchExtras(a, wr, stream);
     }
@@ -1411,9 +1459,9 @@ struct GdmHex8Plan
         t.order = posOf.p ? posOf.As<int>() : nullptr;  // launch index = node
         // per-mesh launches recompute the IP state in the node kernel (no pre-pass over the mesh's cells)
         if (a.P.damage_application == 0)
-            LaunchNodes<true, 0>(a, t, true, end - first, stream);
+            LaunchNodes<true, 0, false>(a, t, true, end - first, stream);
         else
-            LaunchNodes<false, 0>(a, t, true, end - first, stream);
+            LaunchNodes<false, 0, false>(a, t, true, end - first, stream);
     }
 };
 

@@ -165,12 +165,15 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
     }
     else
     {
+        double gi = 1.0, dgi;
+        if (P.interaction != 0)
+            NonlocalFactor(P, st.om, gi, dgi);
 #pragma unroll
         for (int i = 0; i < 6; i++)
             sig[i] = s * st.sig[i];
 #pragma unroll
         for (int i = 0; i < 3; i++)
-            grad[i] = s * P.c * st.ge[i];
+            grad[i] = s * P.c * gi * st.ge[i];
         value = s * (st.eN - st.eq);
     }
     // sigma g_a = (sigma J^-T) dN_a/dxi: the reference-space terms of this point, then the node's sums

@@ -659,7 +659,14 @@ void PrepareGdm(nuto_ctx* ctx)
     ctx->gdm.Prepare(ctx->params.kind, ctx->coordType, ctx->f[0].type, ctx->nip, ctx->graph, ctx->nCells,
                      ctx->hasCellIds ? ctx->hcellId.data() : nullptr, ctx->nCoordNodes, ctx->x.As<double>(),
                      ctx->y.As<double>(), ctx->z.As<double>(), ctx->cconn.As<int>(), ctx->tab.As<double>(),
-                     ctx->rowPtr.As<int>(), ctx->nRows, ctx->stream, err);
+                     ctx->rowPtr.As<int>(), ctx->nRows, ctx->params.interaction != 0, ctx->stream, err);
+    if (err == hipErrorOutOfMemory && ctx->params.interaction != 0)
+    {
+        // no room for the tables and records: the generic kernel, which takes this interaction too
+        (void)hipGetLastError();
+        ctx->gdm.Release();
+        err = hipSuccess;
+    }
     Check(err, "hex8 node tables");
     ctx->gdmTried = true;
 }
@@ -747,11 +754,11 @@ void Assemble(nuto_ctx* ctx, const double* u, const double* e, const double* kap
     const bool wr = R != nullptr, wk = K != nullptr;
     if (!wr && !wk)
         return;
-    // the node kernel takes the Constant nonlocal interaction only: no tables for other cases
-    const bool nodeKernel = !ForceGeneric() && ctx->params.interaction == 0;
+    const bool nodeKernel = !ForceGeneric();
     if (nodeKernel)
         PrepareGdm(ctx);
-    if (nodeKernel && ctx->gdm.Usable(ctx->params.kind, ctx->coordType, ctx->f[0].type, ctx->nip))
+    if (nodeKernel && ctx->gdm.Usable(ctx->params.kind, ctx->coordType, ctx->f[0].type, ctx->nip) &&
+        (!wk || ctx->gdm.Matrix()))
     {
         RowArgs a = MakeRowArgs(ctx, u, e, kappa, R, K);
         if (wk)
@@ -1099,8 +1106,7 @@ int nuto_build_pattern(nuto_ctx* ctx, long long* nnz, int* n_rows)
         ctx->patternBuilt = true;
         // gradient damage with the integrand and the rule already set: the IP tables and the node
         // kernel's tables now, so that assemblies (nuto_build_vector_matrix_noalloc) allocate nothing
-        if (ctx->integrandSet && ctx->ruleSet && ctx->params.kind == kGradientDamage &&
-            ctx->params.interaction == 0 && !ForceGeneric())
+        if (ctx->integrandSet && ctx->ruleSet && ctx->params.kind == kGradientDamage && !ForceGeneric())
         {
             if (!ctx->tabValid)
                 BuildTables(ctx);

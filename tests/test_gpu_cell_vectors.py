@@ -9,8 +9,9 @@ import numpy as np
 import pytest
 
 import nuto_amd as N
+import oracle as O
 from nuto_amd import synthetic as S
-from pairs import check_values, to_dev
+from pairs import Pair, check_values, make_mesh, to_dev
 from test_gpu_adjoint import gdm_pair, kt_lambda
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +48,30 @@ def test_gradient_damage(n, jitter, app):
                 val.append(lam @ p.orc.assemble(u, e, kap, want_k=False)["R"])
             fd[k, c] = (val[0] - val[1]) / (2 * h)
     assert (np.abs(got - fd) <= 1e-6 * np.abs(fd).max(axis=1, keepdims=True)).all()
+
+
+@pytest.mark.parametrize("n,jitter", [((1, 1, 1), 0.0), ((3, 3, 1), 0.1), ((5, 3, 3), 0.0), ((4, 3, 3), 0.1)])
+@pytest.mark.parametrize("app", [N.FULL, N.UNILATERAL])
+@pytest.mark.parametrize("r", [0.005, 0.0])
+def test_decreasing_interaction(n, jitter, app, r):
+    """R and K of the decreasing nonlocal interaction (node kernel and cell vectors) against the oracle,
+    also with a factor that reaches zero at omega = 1, and the residual alone."""
+    X, C = make_mesh(N.HEX8, n, lengths=tuple(float(v) for v in n), jitter=jitter)
+    dev = N.gradient_damage_params(damage_application=app, interaction=N.DECREASING, interaction_r=r)
+    orc = O.Params(kind=1, dim=3, E=30000.0, nu=0.2, k=10.0, kappa0=1e-4, beta=100.0, alpha=0.99, c=4.0,
+                   damage_application=app, interaction=1, interaction_r=r, interaction_eta=5.0)
+    p = Pair(N.HEX8, N.HEX8, X, C, dev, orc, True)
+    th = S.material_fields(p.ncells)
+    p.orc.set_theta(*th)
+    u, e, kap = p.inputs()
+    ref = p.orc.assemble(u, e, kap)
+    ctx = p.context()
+    ctx.set_material_fields(*th)
+    state = [to_dev(v) for v in (u, e, kap)]
+    R, K = ctx.build_vector_matrix(*state)
+    check_values(R.cpu().numpy(), ref["R"], ref["R_bound"], "R")
+    check_values(K.cpu().numpy(), ref["val"], ref["bound"], "K")
+    check_values(ctx.build_vector(*state).cpu().numpy(), ref["R"], ref["R_bound"], "R alone")
+    assert np.array_equal(ctx.build_matrix(*state).cpu().numpy(), K.cpu().numpy())
+    with pytest.raises(N.NutoError):
+        ctx.vjp(*state, R)
