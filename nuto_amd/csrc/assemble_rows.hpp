@@ -51,6 +51,10 @@ struct RowArgs
     double* K;
 };
 
+// The strain of a local-damage point decides whether it loads (kappa' is 1 where the equivalent strain
+// equals the history, as it does right after an update). Every kernel that forms that strain goes through
+// the functions of this file and Mises3, which name each fused multiply-add: left to the compiler, a b + c d
+// is contracted one way in one kernel and the other way in the next, and the last bit differs.
 template <int DIM>
 __device__ inline double Inverse(const double J[DIM][DIM], double inv[DIM][DIM])
 {
@@ -66,20 +70,22 @@ __device__ inline double Inverse(const double J[DIM][DIM], double inv[DIM][DIM])
     }
     else
     {
-        const double c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
-        const double c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
-        const double c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
-        const double det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
+        // a b - c d with the second product rounded first
+        auto minor = [](double x, double y, double z, double w) { return fma(x, y, -(z * w)); };
+        const double c00 = minor(J[1][1], J[2][2], J[1][2], J[2][1]);
+        const double c01 = minor(J[1][2], J[2][0], J[1][0], J[2][2]);
+        const double c02 = minor(J[1][0], J[2][1], J[1][1], J[2][0]);
+        const double det = fma(J[0][2], c02, fma(J[0][1], c01, J[0][0] * c00));
         const double id = 1.0 / det;
         inv[0][0] = c00 * id;
         inv[1][0] = c01 * id;
         inv[2][0] = c02 * id;
-        inv[0][1] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
-        inv[1][1] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
-        inv[2][1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
-        inv[0][2] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
-        inv[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
-        inv[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
+        inv[0][1] = minor(J[0][2], J[2][1], J[0][1], J[2][2]) * id;
+        inv[1][1] = minor(J[0][0], J[2][2], J[0][2], J[2][0]) * id;
+        inv[2][1] = minor(J[0][1], J[2][0], J[0][0], J[2][1]) * id;
+        inv[0][2] = minor(J[0][1], J[1][2], J[0][2], J[1][1]) * id;
+        inv[1][2] = minor(J[0][2], J[1][0], J[0][0], J[1][2]) * id;
+        inv[2][2] = minor(J[0][0], J[1][1], J[0][1], J[1][0]) * id;
         return det;
     }
 }
@@ -96,6 +102,44 @@ __device__ inline void Grad(const double* dNd, int b, const double inv[DIM][DIM]
             s += dNd[b * DIM + i] * inv[i][j];
         g[j] = s;
     }
+}
+
+// eps += B_b u_b (Voigt 2D [xx, yy, xy], 3D [xx, yy, zz, yz, zx, xy], engineering shear)
+template <int DIM>
+__device__ inline void AddStrain(const double g[DIM], const double* u, double* eps)
+{
+    if constexpr (DIM == 2)
+    {
+        eps[0] = fma(g[0], u[0], eps[0]);
+        eps[1] = fma(g[1], u[1], eps[1]);
+        eps[2] = fma(g[1], u[0], fma(g[0], u[1], eps[2]));
+    }
+    else
+    {
+        eps[0] = fma(g[0], u[0], eps[0]);
+        eps[1] = fma(g[1], u[1], eps[1]);
+        eps[2] = fma(g[2], u[2], eps[2]);
+        eps[3] = fma(g[2], u[1], fma(g[1], u[2], eps[3]));
+        eps[4] = fma(g[2], u[0], fma(g[0], u[2], eps[4]));
+        eps[5] = fma(g[1], u[0], fma(g[0], u[1], eps[5]));
+    }
+}
+
+// the strain of the displacement gradient R J^-1, R = sum u_n dN_n/dxi^T (row-major)
+__device__ inline void StrainOfGradient(const double* R, const double inv[3][3], double eps[6])
+{
+    double H[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            H[i][k] = fma(R[3 * i + 2], inv[2][k], fma(R[3 * i + 1], inv[1][k], R[3 * i] * inv[0][k]));
+    eps[0] = H[0][0];
+    eps[1] = H[1][1];
+    eps[2] = H[2][2];
+    eps[3] = H[1][2] + H[2][1];
+    eps[4] = H[0][2] + H[2][0];
+    eps[5] = H[0][1] + H[1][0];
 }
 
 // Rows of dof node p (p < pEnd <= A.nNodes): one lane per node, incident cells in group order.
@@ -199,21 +243,7 @@ __device__ inline void AssembleRowsBody(const RowArgs& A, int p, int pEnd)
                 {
                     double g[DIM];
                     Grad<DIM, NND>(dNd, b, inv, g);
-                    if constexpr (DIM == 2)
-                    {
-                        eps[0] += g[0] * U[b][0];
-                        eps[1] += g[1] * U[b][1];
-                        eps[2] += g[1] * U[b][0] + g[0] * U[b][1];
-                    }
-                    else
-                    {
-                        eps[0] += g[0] * U[b][0];
-                        eps[1] += g[1] * U[b][1];
-                        eps[2] += g[2] * U[b][2];
-                        eps[3] += g[2] * U[b][1] + g[1] * U[b][2];
-                        eps[4] += g[2] * U[b][0] + g[0] * U[b][2];
-                        eps[5] += g[1] * U[b][0] + g[0] * U[b][1];
-                    }
+                    AddStrain<DIM>(g, U[b], eps);
                     if constexpr (KIND == kGradientDamage)
                     {
                         eN += Nd[b] * EE[b];
@@ -456,71 +486,6 @@ __global__ void __launch_bounds__(64) kAssembleRowsList(const RowArgs A, const i
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (i < n)
         AssembleRowsBody<KIND, DIM, NNC, NND, NIP, BH, WR, WK>(A, nodes[i], A.nNodes);
-}
-
-// History update (GradientDamage::Update, GradientDamage.h:122-125, or EvolutionImplicit::Update,
-// LocalIsotropicDamage.h:130-133): one lane per (cell, ip).
-template <int KIND, int DIM, int NNC, int NND, int NIP>
-__global__ void __launch_bounds__(256) kUpdateHistory(const RowArgs A, double* kappa)
-{
-    constexpr int S = 1 + NNC * DIM + NND + NND * DIM;
-    const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= (long long)A.nCells * NIP)
-        return;
-    const int cell = (int)(gid / NIP), ip = (int)(gid % NIP);
-    const double* t = A.tab + ip * S;
-    const double* dNc = t + 1;
-    const double* Nd = dNc + NNC * DIM;
-    const double* dNd = Nd + NND;
-    const int cid = A.cellId ? A.cellId[cell] : cell;
-    double& kh = kappa[(size_t)cid + (size_t)ip * A.kappaLd];
-    double val;
-    if constexpr (KIND == kGradientDamage)
-    {
-        val = 0.0;
-        for (int b = 0; b < NND; b++)
-            val += Nd[b] * A.e[A.dconn[(size_t)cell * NND + b]];
-    }
-    else
-    {
-        double X[NNC][DIM];
-        for (int k = 0; k < NNC; k++)
-        {
-            const int n = A.cconn[(size_t)cell * NNC + k];
-            X[k][0] = A.x[n];
-            X[k][1] = A.y[n];
-            if constexpr (DIM == 3)
-                X[k][2] = A.z[n];
-        }
-        double J[DIM][DIM];
-        for (int i = 0; i < DIM; i++)
-            for (int j = 0; j < DIM; j++)
-            {
-                double s = 0.0;
-                for (int k = 0; k < NNC; k++)
-                    s += X[k][i] * dNc[k * DIM + j];
-                J[i][j] = s;
-            }
-        double inv[DIM][DIM];
-        Inverse<DIM>(J, inv);
-        double eps[6] = {0, 0, 0, 0, 0, 0};
-        for (int b = 0; b < NND; b++)
-        {
-            const int q = A.dconn[(size_t)cell * NND + b];
-            double g[DIM];
-            Grad<DIM, NND>(dNd, b, inv, g);
-            const double u0 = A.u[(size_t)q * DIM], u1 = A.u[(size_t)q * DIM + 1], u2 = A.u[(size_t)q * DIM + 2];
-            eps[0] += g[0] * u0;
-            eps[1] += g[1] * u1;
-            eps[2] += g[2] * u2;
-            eps[3] += g[2] * u1 + g[1] * u2;
-            eps[4] += g[2] * u0 + g[0] * u2;
-            eps[5] += g[1] * u0 + g[0] * u1;
-        }
-        double d[6];
-        val = Mises3(eps, A.P.nu, A.P.k, d);
-    }
-    kh = kh < val ? val : kh;
 }
 
 }  // namespace nuto_amd

@@ -1,11 +1,10 @@
-// Outputs of a cell group besides R and K: the diagonally lumped mass matrix and fields at the
-// integration points.
+// Outputs of a cell group besides R and K: the diagonally lumped mass matrix and the names of the fields
+// at the integration points (cell_points.hpp).
 //
 // kLumpedMass: SimpleAssembler::BuildDiagonallyLumpedMatrix (SimpleAssembler.cpp:67-98) with the
 //   integrand DynamicMomentumBalance::Hessian2 = N^T N rho (DynamicMomentumBalance.h:22-30) on dof
 //   type slot 0. Row-owner form like the assembly kernel: one lane per dof node, its incident cells
 //   in group order, so the per-node sum runs in cell order without atomics.
-// kEvalIp: Cell::Eval (Cell.h:80-93) of the integrand's fields, one lane per (cell, IP).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -108,133 +107,6 @@ __global__ void __launch_bounds__(64) kLumpedMass(const RowArgs A, double rho, d
 #pragma unroll
     for (int c = 0; c < DIM; c++)
         M[(size_t)p * DIM + c] = acc;
-}
-
-// Field `field` at every (cell, IP), written to out[(cell * NIP + ip) * ncomp + comp] (cells in
-// group order, IPs in rule order).
-template <int KIND, int DIM, int NNC, int NND, int NIP>
-__global__ void __launch_bounds__(256) kEvalIp(const RowArgs A, int field, double* __restrict__ out)
-{
-    constexpr int S = 1 + NNC * DIM + NND + NND * DIM;
-    constexpr int NV = DIM == 2 ? 3 : 6;
-    const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= (long long)A.nCells * NIP)
-        return;
-    const int cell = (int)(gid / NIP), ip = (int)(gid % NIP);
-    const double* t = A.tab + ip * S;
-    const double* dNc = t + 1;
-    const double* Nd = dNc + NNC * DIM;
-    const double* dNd = Nd + NND;
-    double inv[DIM][DIM];
-    CellJacobian<DIM, NNC>(A, cell, dNc, inv);
-    double eps[NV];
-#pragma unroll
-    for (int i = 0; i < NV; i++)
-        eps[i] = 0.0;
-    double eN = 0.0;
-    for (int b = 0; b < NND; b++)
-    {
-        const int q = A.dconn[(size_t)cell * NND + b];
-        double g[DIM];
-        Grad<DIM, NND>(dNd, b, inv, g);
-        if constexpr (DIM == 2)
-        {
-            const double u0 = A.u[(size_t)q * 2], u1 = A.u[(size_t)q * 2 + 1];
-            eps[0] += g[0] * u0;
-            eps[1] += g[1] * u1;
-            eps[2] += g[1] * u0 + g[0] * u1;
-        }
-        else
-        {
-            const double u0 = A.u[(size_t)q * 3], u1 = A.u[(size_t)q * 3 + 1], u2 = A.u[(size_t)q * 3 + 2];
-            eps[0] += g[0] * u0;
-            eps[1] += g[1] * u1;
-            eps[2] += g[2] * u2;
-            eps[3] += g[2] * u1 + g[1] * u2;
-            eps[4] += g[2] * u0 + g[0] * u2;
-            eps[5] += g[1] * u0 + g[0] * u1;
-        }
-        if constexpr (KIND == kGradientDamage)
-            eN += Nd[b] * A.e[q];
-    }
-    double* o = out + (size_t)gid * (field <= kIpStress ? NV : 1);
-    if (field == kIpStrain)
-    {
-#pragma unroll
-        for (int i = 0; i < NV; i++)
-            o[i] = eps[i];
-        return;
-    }
-    const LawParams& P = A.P;
-    const double E = A.thE ? A.thE[cell] : P.E;
-    if constexpr (KIND == kLinearElastic)
-    {
-        // field == kIpStress (the caller rejects the damage fields for linear elasticity)
-        if constexpr (DIM == 2)
-        {
-            double C11, C12, C33;
-            if (P.plane_state == 0)
-            {
-                const double f = E / (1.0 - P.nu * P.nu);
-                C11 = f;
-                C12 = f * P.nu;
-                C33 = f * 0.5 * (1.0 - P.nu);
-            }
-            else
-            {
-                const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
-                C11 = f * (1.0 - P.nu);
-                C12 = f * P.nu;
-                C33 = E / (2.0 * (1.0 + P.nu));
-            }
-            o[0] = C11 * eps[0] + C12 * eps[1];
-            o[1] = C12 * eps[0] + C11 * eps[1];
-            o[2] = C33 * eps[2];
-        }
-        else
-        {
-            const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
-            const double lam = f * P.nu, mu = E / (2.0 * (1.0 + P.nu));
-            const double tr = eps[0] + eps[1] + eps[2];
-            for (int i = 0; i < 3; i++)
-                o[i] = lam * tr + 2.0 * mu * eps[i];
-            for (int i = 3; i < 6; i++)
-                o[i] = mu * eps[i];
-        }
-    }
-    else if constexpr (DIM == 3)
-    {
-        double d[6];
-        const double eq = Mises3(eps, P.nu, P.k, d);
-        if (field == kIpEqStrain)
-        {
-            o[0] = eq;
-            return;
-        }
-        const int cid = A.cellId ? A.cellId[cell] : cell;
-        const double kh = A.kappa[(size_t)cid + (size_t)ip * A.kappaLd];
-        const double drive = KIND == kGradientDamage ? eN : eq;
-        const double kap = kh < drive ? drive : kh;
-        if (field == kIpKappa)
-        {
-            o[0] = kap;
-            return;
-        }
-        const double k0 = A.thE ? A.thFt[cell] / E : P.kappa0;
-        const double beta = A.thE ? A.thFt[cell] / A.thGf[cell] : P.beta;
-        double om, dom;
-        DamageExp(kap, k0, beta, P.alpha, om, dom);
-        if (field == kIpDamage)
-        {
-            o[0] = om;
-            return;
-        }
-        DamageStress3 ds;
-        ElasticDamage3(eps, om, E, P.nu, P.damage_application, ds);
-#pragma unroll
-        for (int i = 0; i < 6; i++)
-            o[i] = ds.sig[i];
-    }
 }
 
 }  // namespace nuto_amd

@@ -120,13 +120,8 @@ __device__ inline void CellIpRecords(const RowArgs& A, int c1, int cellBase, dou
                     Jm[r][m] = jg[3 * r + m];
             const double detJ = Inverse<3>(Jm, inv);
             const double s = detJ * A.tab[ip * S];
-            double H[3][3];
-#pragma unroll
-            for (int r = 0; r < 3; r++)
-#pragma unroll
-                for (int m = 0; m < 3; m++)
-                    H[r][m] = jg[9 + 3 * r] * inv[0][m] + jg[9 + 3 * r + 1] * inv[1][m] + jg[9 + 3 * r + 2] * inv[2][m];
-            const double eps[6] = {H[0][0], H[1][1], H[2][2], H[1][2] + H[2][1], H[0][2] + H[2][0], H[0][1] + H[1][0]};
+            double eps[6];
+            StrainOfGradient(jg + 9, inv, eps);
             double* rec = sIp[cl][i];
 #pragma unroll
             for (int r = 0; r < 3; r++)

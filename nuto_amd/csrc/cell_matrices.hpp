@@ -147,13 +147,8 @@ __global__ void __launch_bounds__(64) kCellMatrices(const RowArgs A, int c0, int
 
         // strain (Voigt [xx, yy, zz, yz, zx, xy], engineering shear) from the displacement gradient
         // H = (U^T dNd) J^-1, H_ik = du_i / dx_k
-        double H[3][3];
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int k = 0; k < 3; k++)
-                H[i][k] = jg[9 + 3 * i] * inv[0][k] + jg[9 + 3 * i + 1] * inv[1][k] + jg[9 + 3 * i + 2] * inv[2][k];
-        const double eps[6] = {H[0][0], H[1][1], H[2][2], H[1][2] + H[2][1], H[0][2] + H[2][0], H[0][1] + H[1][0]};
+        double eps[6];
+        StrainOfGradient(jg + 9, inv, eps);
 
         // law: stress, isotropic tangent (c1 tr + 2 c2 eps, shear c2 gamma), rank-one damage term
         double sig[6], c1, c2;

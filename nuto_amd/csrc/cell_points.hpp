@@ -1,0 +1,367 @@
+// Integration-point work of a cell without its matrix: the cell's vector R_e (Cell::Integrate of
+// MomentumBalance::Gradient or GradientDamage::Gradient, Cell.h:105-119), the history update
+// (GradientDamage::Update, GradientDamage.h:122-125; EvolutionImplicit::Update,
+// LocalIsotropicDamage.h:130-133) and the fields of Cell::Eval (Cell.h:80-93).
+//
+// One wave takes 64 / NIP cells: their coordinates and node values go to LDS once, lane (cell, IP) forms
+// the point's state, and for R_e lane (cell, node) adds the points in rule order from LDS. A point is
+// evaluated once; the row-owner kernel evaluates it for every node of its cell. The sum over the cells is
+// kGatherCellVectors. Bound by the latency of the gathers and the two passes over LDS.
+// Measured on 47,880 ten-node tetrahedra with local damage: residual 267 us by the row-owner kernel, 22 +
+// 10 us (gather) here; history 15 -> 13 us, stresses 17 -> 15 us (one lane per point with its own gathers
+// before). 2993 waves, three per SIMD: the chain of loads, not a rate, is what is left.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "assemble_rows.hpp"
+#include "cell_fields.hpp"
+
+namespace nuto_amd
+{
+
+enum PointOutput : int
+{
+    kPointVector,   // R_e[cell][node][F]
+    kPointHistory,  // kappa[cellId + ip * ld] = max(history, driving strain)
+    kPointField     // field[(cell * NIP + ip) * components]
+};
+
+// o[DIM i + m] = s sum_k sigma_ik J^-1_mk: sigma g_a = (this) dN_a/dxi
+template <int DIM>
+__device__ inline void PointTerms(double s, const double* sig, const double inv[DIM][DIM], double* o)
+{
+    double t[DIM][DIM];
+    if constexpr (DIM == 2)
+    {
+        t[0][0] = sig[0];
+        t[1][1] = sig[1];
+        t[0][1] = t[1][0] = sig[2];
+    }
+    else
+    {
+        t[0][0] = sig[0];
+        t[1][1] = sig[1];
+        t[2][2] = sig[2];
+        t[1][2] = t[2][1] = sig[3];
+        t[0][2] = t[2][0] = sig[4];
+        t[0][1] = t[1][0] = sig[5];
+    }
+#pragma unroll
+    for (int i = 0; i < DIM; i++)
+#pragma unroll
+        for (int m = 0; m < DIM; m++)
+        {
+            double v = 0.0;
+#pragma unroll
+            for (int k = 0; k < DIM; k++)
+                v += t[i][k] * inv[m][k];
+            o[DIM * i + m] = s * v;
+        }
+}
+
+template <int KIND, int DIM, int NNC, int NND, int NIP, int OUT>
+__global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, double* __restrict__ out)
+{
+    constexpr int CPW = 64 / NIP;                       // cells per wave
+    constexpr bool GD = KIND == kGradientDamage;
+    constexpr int F = GD ? DIM + 1 : DIM;               // values per node
+    constexpr int S = 1 + NNC * DIM + NND + NND * DIM;  // IP table row: w, dNc, N, dNd
+    constexpr int NV = DIM == 2 ? 3 : 6;
+    constexpr int SX = NNC * DIM | 1, SU = NND * F | 1;  // odd strides: consecutive cells on other banks
+    constexpr int PR = GD ? DIM * DIM + DIM + 1 : (DIM == 2 ? 5 : 9);  // doubles per point in LDS (odd)
+    // the strain: the gradient H = (sum u_n dN_n/dxi^T) J^-1 as the cell-matrix kernels form it, or the sum
+    // of B_n u_n as the row-owner kernel does, whichever assembles this rule's matrix: a history that was
+    // just updated then counts as loading there too (kappa' is 1 where the two are equal)
+    constexpr bool kSumForm = DIM == 2 || GD || NIP > 27;
+    static_assert(CPW >= 1, "a wave holds a cell's points");
+    constexpr int IN = CPW * (SX + SU), RES = CPW * NIP * PR;
+    __shared__ double pool[IN > RES ? IN : RES];  // the cells' nodes, then the points' results
+    double* sX = pool;
+    double* sU = pool + CPW * SX;
+    double* sP = pool;
+    const int lane = (int)threadIdx.x;
+    const int cell0 = (int)blockIdx.x * CPW;
+    const int nc = A.nCells - cell0 < CPW ? A.nCells - cell0 : CPW;
+    const LawParams& P = A.P;
+    constexpr bool kGeometry = !(GD && OUT == kPointHistory);  // its history needs eeq only
+    // every node number, then every node value is loaded before the first of them is waited for
+    constexpr int ITX = kGeometry ? (CPW * NNC + 63) / 64 : 0, ITU = (CPW * NND + 63) / 64;
+    {
+        int nx[ITX + 1], nu[ITU];
+        double x[ITX + 1][DIM], v[ITU][F];
+#pragma unroll
+        for (int i = 0; i < ITX; i++)
+            nx[i] = A.cconn[(size_t)cell0 * NNC + (lane + 64 * i < nc * NNC ? lane + 64 * i : 0)];
+#pragma unroll
+        for (int i = 0; i < ITU; i++)
+            nu[i] = A.dconn[(size_t)cell0 * NND + (lane + 64 * i < nc * NND ? lane + 64 * i : 0)];
+#pragma unroll
+        for (int i = 0; i < ITX; i++)
+        {
+            x[i][0] = A.x[nx[i]];
+            x[i][1] = A.y[nx[i]];
+            if constexpr (DIM == 3)
+                x[i][2] = A.z[nx[i]];
+        }
+#pragma unroll
+        for (int i = 0; i < ITU; i++)
+        {
+#pragma unroll
+            for (int k = 0; k < DIM; k++)
+                v[i][k] = A.u[(size_t)nu[i] * DIM + k];
+            if constexpr (GD)
+                v[i][DIM] = A.e[nu[i]];
+        }
+#pragma unroll
+        for (int i = 0; i < ITX; i++)
+        {
+            const int k = lane + 64 * i;
+            if (k < nc * NNC)
+            {
+#pragma unroll
+                for (int m = 0; m < DIM; m++)
+                    sX[k / NNC * SX + k % NNC * DIM + m] = x[i][m];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < ITU; i++)
+        {
+            const int k = lane + 64 * i;
+            if (k < nc * NND)
+            {
+#pragma unroll
+                for (int m = 0; m < F; m++)
+                    sU[k / NND * SU + k % NND * F + m] = v[i][m];
+            }
+        }
+    }
+    __syncthreads();
+
+    const int cl = lane / NIP, ip = lane - cl * NIP;
+    double o[PR];  // the point's results
+    if (cl < nc)
+    {
+        const int cell = cell0 + cl;
+        const double* t = A.tab + ip * S;
+        const double* dNc = t + 1;
+        const double* Nd = dNc + NNC * DIM;
+        const double* dNd = Nd + NND;
+        const double* U = sU + cl * SU;
+        double eN = 0.0;
+        if constexpr (GD)
+        {
+#pragma unroll
+            for (int b = 0; b < NND; b++)
+                eN += Nd[b] * U[b * F + DIM];
+        }
+        double eps[NV], inv[DIM][DIM], ge[3] = {0.0, 0.0, 0.0}, s = 0.0;
+        if constexpr (kGeometry)
+        {
+            double J[DIM][DIM];
+#pragma unroll
+            for (int i = 0; i < DIM; i++)
+#pragma unroll
+                for (int k = 0; k < DIM; k++)
+                    J[i][k] = 0.0;
+#pragma unroll
+            for (int n = 0; n < NNC; n++)
+#pragma unroll
+                for (int i = 0; i < DIM; i++)
+                {
+                    const double x = sX[cl * SX + n * DIM + i];
+#pragma unroll
+                    for (int k = 0; k < DIM; k++)
+                        J[i][k] += x * dNc[n * DIM + k];
+                }
+            s = Inverse<DIM>(J, inv) * t[0];
+            if constexpr (kSumForm)
+            {
+#pragma unroll
+                for (int i = 0; i < NV; i++)
+                    eps[i] = 0.0;
+#pragma unroll
+                for (int b = 0; b < NND; b++)
+                {
+                    double g[DIM];
+                    Grad<DIM, NND>(dNd, b, inv, g);
+                    const double* u = U + b * F;
+                    AddStrain<DIM>(g, u, eps);
+                    if constexpr (GD)
+                    {
+#pragma unroll
+                        for (int i = 0; i < 3; i++)
+                            ge[i] += g[i] * u[DIM];
+                    }
+                }
+            }
+            else
+            {
+                double R[9];
+#pragma unroll
+                for (int i = 0; i < 9; i++)
+                    R[i] = 0.0;
+#pragma unroll
+                for (int n = 0; n < NND; n++)
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+                    {
+                        const double u = U[n * F + i];
+#pragma unroll
+                        for (int k = 0; k < 3; k++)
+                            R[3 * i + k] += u * dNd[n * 3 + k];
+                    }
+                StrainOfGradient(R, inv, eps);
+            }
+        }
+
+        const double E = A.thE ? A.thE[cell] : P.E;
+        if constexpr (KIND == kLinearElastic)
+        {
+            double sig[NV];
+            if constexpr (DIM == 2)
+            {
+                double C11, C12, C33;
+                if (P.plane_state == 0)
+                {
+                    const double f = E / (1.0 - P.nu * P.nu);
+                    C11 = f;
+                    C12 = f * P.nu;
+                    C33 = f * 0.5 * (1.0 - P.nu);
+                }
+                else
+                {
+                    const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
+                    C11 = f * (1.0 - P.nu);
+                    C12 = f * P.nu;
+                    C33 = E / (2.0 * (1.0 + P.nu));
+                }
+                sig[0] = C11 * eps[0] + C12 * eps[1];
+                sig[1] = C12 * eps[0] + C11 * eps[1];
+                sig[2] = C33 * eps[2];
+            }
+            else
+            {
+                const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
+                const double lam = f * P.nu, mu = E / (2.0 * (1.0 + P.nu));
+                const double tr = eps[0] + eps[1] + eps[2];
+                for (int i = 0; i < 3; i++)
+                    sig[i] = lam * tr + 2.0 * mu * eps[i];
+                for (int i = 3; i < 6; i++)
+                    sig[i] = mu * eps[i];
+            }
+            if constexpr (OUT == kPointVector)
+                PointTerms<DIM>(s, sig, inv, o);
+            else
+            {
+                // strain or stress (the caller rejects the damage fields)
+#pragma unroll
+                for (int i = 0; i < NV; i++)
+                    o[i] = field == kIpStrain ? eps[i] : sig[i];
+            }
+        }
+        else
+        {
+            const int cid = A.cellId ? A.cellId[cell] : cell;
+            const size_t at = (size_t)cid + (size_t)ip * A.kappaLd;
+            double d[6], eq = 0.0;
+            if constexpr (kGeometry)
+                eq = Mises3(eps, P.nu, P.k, d);
+            const double drive = GD ? eN : eq;
+            const double kh = A.kappa[at];
+            const double kap = kh < drive ? drive : kh;
+            if constexpr (OUT == kPointHistory)
+            {
+                out[at] = kap;
+                return;
+            }
+            double om = 0.0, dom = 0.0;
+            DamageStress3 ds;
+            if (OUT == kPointVector || field == kIpStress || field == kIpDamage)
+            {
+                const double k0 = A.thE ? A.thFt[cell] / E : P.kappa0;
+                const double beta = A.thE ? A.thFt[cell] / A.thGf[cell] : P.beta;
+                DamageExp(kap, k0, beta, P.alpha, om, dom);
+                ElasticDamage3(eps, om, E, P.nu, P.damage_application, ds);
+            }
+            if constexpr (OUT == kPointVector)
+            {
+                PointTerms<DIM>(s, ds.sig, inv, o);
+                if constexpr (GD)
+                {
+                    double gi, dgi;
+                    NonlocalFactor(P, om, gi, dgi);
+                    const double c = s * P.c * gi;
+#pragma unroll
+                    for (int k = 0; k < 3; k++)
+                        o[9 + k] = c * (ge[0] * inv[k][0] + ge[1] * inv[k][1] + ge[2] * inv[k][2]);
+                    o[12] = s * (eN - eq);
+                }
+            }
+            else if (field <= kIpStress)
+            {
+#pragma unroll
+                for (int i = 0; i < 6; i++)
+                    o[i] = field == kIpStrain ? eps[i] : ds.sig[i];
+            }
+            else
+                o[0] = field == kIpKappa ? kap : (field == kIpDamage ? om : eq);
+        }
+    }
+    if constexpr (OUT == kPointHistory)
+        return;
+    __syncthreads();  // the results overwrite the nodes
+    if (cl < nc)
+    {
+#pragma unroll
+        for (int i = 0; i < PR; i++)
+            sP[lane * PR + i] = o[i];
+    }
+    __syncthreads();
+    if constexpr (OUT == kPointField)
+    {
+        // the block's values are contiguous: written with consecutive lanes on consecutive doubles
+        const int w = field <= kIpStress ? NV : 1;
+        double* dst = out + (size_t)cell0 * NIP * w;
+        for (int k = lane; k < nc * NIP * w; k += 64)
+            dst[k] = sP[(k / w) * PR + k % w];
+        return;
+    }
+    // R_e: the points' reference-space terms against dN_a/dxi (and N_a), in rule order
+    for (int k = lane; k < nc * NND; k += 64)
+    {
+        const int c = k / NND, a = k - c * NND;
+        double r[F];
+#pragma unroll
+        for (int i = 0; i < F; i++)
+            r[i] = 0.0;
+        for (int q = 0; q < NIP; q++)
+        {
+            const double* pt = sP + (c * NIP + q) * PR;
+            const double* Nd = A.tab + q * S + 1 + NNC * DIM;
+            const double* dN = Nd + NND + a * DIM;
+            double d[DIM];
+#pragma unroll
+            for (int m = 0; m < DIM; m++)
+                d[m] = dN[m];
+#pragma unroll
+            for (int i = 0; i < DIM; i++)
+#pragma unroll
+                for (int m = 0; m < DIM; m++)
+                    r[i] += pt[i * DIM + m] * d[m];
+            if constexpr (GD)
+            {
+#pragma unroll
+                for (int m = 0; m < DIM; m++)
+                    r[DIM] += pt[9 + m] * d[m];
+                r[DIM] += pt[12] * Nd[a];
+            }
+        }
+        double* dst = out + ((size_t)cell0 * NND + k) * F;
+#pragma unroll
+        for (int i = 0; i < F; i++)
+            dst[i] = r[i];
+    }
+}
+
+}  // namespace nuto_amd

@@ -43,6 +43,7 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
     using namespace gdm8;
     constexpr int kPerCell = AFF ? kGeo / 2 : 8 * kGeo / 2;  // 16-byte chunks of geometry per cell
     __shared__ __align__(16) double stage[16 * kPerCell];
+    __shared__ double sE[64];  // eeq of the cells' nodes
     const int lane = (int)threadIdx.x, r = lane >> 3;
     const CornerLane c = CornerOf(lane);
     const long long cell0 = (long long)blockIdx.x * 8;
@@ -87,6 +88,7 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
             l[i] = lam[(size_t)q * 3 + i];
         l[3] = lam[(size_t)A.nU + q];
     }
+    sE[8 * r + c.node] = v[3];
     __syncthreads();
     double g[kGeo];
     {
@@ -107,7 +109,20 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
 #pragma unroll
     for (int i = 0; i < 3; i++)
         NodesToPoint(c, v[i], unused, Hu[i]);
-    NodesToPoint(c, v[3], eN, he);
+    NodesToPoint(c, v[3], unused, he);
+    // kappa' jumps where eeq meets the history, as it does at every loading point after an update: eeq is bit
+    // for bit the value that the update and the matrix kernels form (N_n from ShapeAt's products, the nodes
+    // added in order), so that all take the same side and a residual does not change with the update
+    {
+        const double near = 1.0 + kGauss, far = 1.0 - kGauss;
+        const double fx[2] = {c.hx < 0.0 ? near : far, c.hx < 0.0 ? far : near};
+        const double fy[2] = {c.hy < 0.0 ? near : far, c.hy < 0.0 ? far : near};
+        const double fz[2] = {c.hz < 0.0 ? near : far, c.hz < 0.0 ? far : near};
+        eN = 0.0;
+#pragma unroll
+        for (int n = 0; n < 8; n++)
+            eN = fma(0.125 * fx[((n + 1) >> 1) & 1] * fy[(n >> 1) & 1] * fz[n >> 2], sE[8 * r + n], eN);
+    }
     GdmIp st;
     GdmIpState<FULLDMG>(Hu, he, eN, inv, kh, m3K, m2G, k0, beta, P, st);
 

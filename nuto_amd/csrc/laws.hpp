@@ -87,8 +87,9 @@ __device__ __host__ inline double Mises3(const double e[6], double nu, double k,
     const double K2 = 3.0 / (k * (1.0 + nu) * (1.0 + nu));
     const double I1 = e[0] + e[1] + e[2];
     const double a = e[0] - e[1], b = e[1] - e[2], cc = e[2] - e[0];
-    const double J2 = (a * a + b * b + cc * cc) * (1.0 / 6.0) + 0.25 * (e[3] * e[3] + e[4] * e[4] + e[5] * e[5]);
-    const double A = sqrt(K1 * K1 * I1 * I1 + K2 * J2);
+    const double sh = fma(e[5], e[5], fma(e[4], e[4], e[3] * e[3]));
+    const double J2 = fma(0.25, sh, fma(cc, cc, fma(b, b, a * a)) * (1.0 / 6.0));
+    const double A = sqrt(fma(K1 * K1 * I1, I1, K2 * J2));
     if (A == 0.0)
     {
         d[0] = d[1] = d[2] = K1;
@@ -106,7 +107,7 @@ __device__ __host__ inline double Mises3(const double e[6], double nu, double k,
         d[4] = h * K2 * 0.5 * e[4];
         d[5] = h * K2 * 0.5 * e[5];
     }
-    return K1 * I1 + A;
+    return fma(K1, I1, A);
 }
 
 // LinearElasticDamage<3>::Stress and DstressDomega (LinearElasticDamage.h:65-91)

@@ -22,6 +22,8 @@
 #include "cell_fields.hpp"
 #include "cell_gram.hpp"
 #include "cell_mfma.hpp"
+#include "cell_points.hpp"
+#include "cell_vectors.hpp"
 #include "cell_matrices.hpp"
 #include "solve.hpp"
 #include "mesh.hpp"
@@ -239,6 +241,18 @@ void InvalidatePattern(nuto_ctx* ctx)
     ctx->gdmTried = false;
     ctx->consBuilt = false;
     ctx->maxAdj = -1;
+}
+
+// Staging of the cells' vectors (every dof of every cell); false when it cannot be allocated (the error
+// state is cleared). It only grows: two-phase matrix assemblies stage their vectors there too.
+bool TryVectorStage(nuto_ctx* ctx)
+{
+    const size_t bytes = (size_t)ctx->nCells * NodesOf(ctx->f[0].type) *
+                         (ctx->f[0].ncomp + (ctx->f[1].set ? ctx->f[1].ncomp : 0)) * sizeof(double);
+    if (ctx->reStage.bytes >= bytes || ctx->reStage.Alloc(bytes) == hipSuccess)
+        return true;
+    (void)hipGetLastError();
+    return false;
 }
 
 // IP tables: per IP w, dNc[nnC][dim], N[nnD], dNd[nnD][dim] (shape tables of the coordinate
@@ -508,12 +522,33 @@ void LaunchTwoPhaseT(nuto_ctx* ctx, const RowArgs& a, bool wr, int c0, int c1, i
     Check(hipGetLastError(), "two-phase assembly launch");
 }
 
+template <int KIND, int DIM, int NNC, int NND, int NIP, int OUT>
+void LaunchPoints(nuto_ctx* ctx, const RowArgs& a, int field, double* out)
+{
+    constexpr int CPW = 64 / NIP;
+    if (a.nCells > 0)
+        hipLaunchKernelGGL((kCellPoints<KIND, DIM, NNC, NND, NIP, OUT>), dim3((unsigned)((a.nCells + CPW - 1) / CPW)),
+                           dim3(64), 0, ctx->stream, a, field, out);
+}
+
 template <int KIND, int DIM, int NNC, int NND, int NIP, int BH>
 void LaunchRowsT(nuto_ctx* ctx, const RowArgs& a, bool wr, bool wk)
 {
     const int n = a.nNodes;
     if (n == 0)
         return;
+    // a vector alone: the cells' vectors, then the sum per node; the single-pass kernel serves when they
+    // do not fit in device memory
+    if (!wk && !ForceGeneric() && TryVectorStage(ctx))
+    {
+        constexpr int F = KIND == kGradientDamage ? DIM + 1 : DIM;
+        double* cv = ctx->reStage.As<double>();
+        LaunchPoints<KIND, DIM, NNC, NND, NIP, kPointVector>(ctx, a, 0, cv);
+        LaunchGatherCellVectors<NND, DIM, F>(a, cv, a.R, ctx->stream);
+        Check(hipGetLastError(), "vector assembly launch");
+        SyncCheck(ctx, "vector assembly");
+        return;
+    }
     // (the staging kernels keep every IP's state in LDS: rules up to 27 points)
     if constexpr (DIM == 3 && KIND != kGradientDamage && NND * 3 <= 64 && NIP <= 27)
     {
@@ -541,11 +576,7 @@ void LaunchHistoryT(nuto_ctx* ctx, const RowArgs& a, double* kappa)
 {
     if constexpr (KIND != kLinearElastic && DIM == 3)
     {
-        const long long n = (long long)a.nCells * NIP;
-        if (n == 0)
-            return;
-        hipLaunchKernelGGL((kUpdateHistory<KIND, DIM, NNC, NND, NIP>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                           ctx->stream, a, kappa);
+        LaunchPoints<KIND, DIM, NNC, NND, NIP, kPointHistory>(ctx, a, 0, kappa);
         Check(hipGetLastError(), "history launch");
     }
 }
@@ -564,11 +595,7 @@ void LaunchLumpedT(nuto_ctx* ctx, const RowArgs& a, double rho, double* M)
 template <int KIND, int DIM, int NNC, int NND, int NIP>
 void LaunchEvalT(nuto_ctx* ctx, const RowArgs& a, int field, double* out)
 {
-    const long long n = (long long)a.nCells * NIP;
-    if (n == 0)
-        return;
-    hipLaunchKernelGGL((kEvalIp<KIND, DIM, NNC, NND, NIP>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                       ctx->stream, a, field, out);
+    LaunchPoints<KIND, DIM, NNC, NND, NIP, kPointField>(ctx, a, field, out);
     Check(hipGetLastError(), "ip field launch");
     SyncCheck(ctx, "ip field kernel");
 }
@@ -1104,6 +1131,7 @@ int nuto_build_pattern(nuto_ctx* ctx, long long* nnz, int* n_rows)
         ctx->nnz = nz;
         ctx->nRows = (int)(rp.size() - 1);
         ctx->patternBuilt = true;
+        (void)TryVectorStage(ctx);  // here, so that vector assemblies allocate nothing
         // gradient damage with the integrand and the rule already set: the IP tables and the node
         // kernel's tables now, so that assemblies (nuto_build_vector_matrix_noalloc) allocate nothing
         if (ctx->integrandSet && ctx->ruleSet && ctx->params.kind == kGradientDamage && !ForceGeneric())

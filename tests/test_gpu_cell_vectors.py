@@ -13,6 +13,7 @@ import oracle as O
 from nuto_amd import synthetic as S
 from pairs import Pair, check_values, make_mesh, to_dev
 from test_gpu_adjoint import gdm_pair, kt_lambda
+from test_gpu_parity import gdm_params, ld_params, le_params
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +76,82 @@ def test_decreasing_interaction(n, jitter, app, r):
     assert np.array_equal(ctx.build_matrix(*state).cpu().numpy(), K.cpu().numpy())
     with pytest.raises(N.NutoError):
         ctx.vjp(*state, R)
+
+
+def test_adjoint_at_the_updated_history():
+    """kappa' jumps where eeq meets the history, which is every loading point after an update: the adjoint
+    and the tangent must take the same side there (K^T lambda of the device's K, within 1e-12 of |K|^T |lambda|)."""
+    p, th = gdm_pair((5, 4, 3), N.FULL, jitter=0.1)
+    u, e, kap = p.inputs()
+    ctx = p.context()
+    ctx.set_material_fields(*th)
+    state = [to_dev(v) for v in (u, e, kap)]
+    ctx.update_history(*state)
+    lam = S.uniform(0x52, p.n_u + p.n_e, -1.0, 1.0)
+    rp, ci = ctx.pattern()
+    val = ctx.build_matrix(*state).cpu().numpy()
+    kt, kb = kt_lambda(dict(row_ptr=rp, col=ci, val=val, bound=np.abs(val)), lam, len(lam))
+    got = ctx.vjp(*state, to_dev(lam))[0].cpu().numpy()
+    assert (np.abs(got - kt) <= 1e-12 * kb + 1e-300).all()
+
+
+# (coordinate element, dof element, cells, rule); a wave takes 64, 16, 8, 4, 2 or 1 cells
+GENERIC = [(N.QUAD4, N.QUAD4, (1, 1), (0, 1)), (N.QUAD4, N.QUAD4, (5, 4), (0, 2)), (N.QUAD4, N.QUAD4, (3, 3), (0, 5)),
+           (N.HEX8, N.HEX8, (3, 3, 1), (0, 2)), (N.HEX8, N.HEX8, (1, 1, 1), (0, 3)), (N.HEX8, N.HEX8, (2, 1, 1), (0, 4)),
+           (N.HEX8, N.HEX20, (3, 1, 1), (0, 3)), (N.TET4, N.TET4, (1, 1, 1), (1, 1)), (N.TET4, N.TET4, (3, 2, 2), (1, 1)),
+           (N.TET4, N.TET10, (3, 1, 1), (1, 2))]
+
+
+@pytest.mark.parametrize("ct,dt,n,rule", GENERIC)
+@pytest.mark.parametrize("kind", ["elastic", "local", "gradient"])
+def test_generic_vectors_history_and_fields(ct, dt, n, rule, kind, monkeypatch):
+    """The residual alone (cell vectors, and the single-pass kernel) against the oracle; kappa of the field
+    output equals the updated history bit for bit."""
+    dim = N.DIM[ct]
+    if (kind != "elastic" and dim == 2) or (kind == "gradient" and (ct, dt) != (N.HEX8, N.HEX8)):
+        pytest.skip("not provided")
+    X, C = make_mesh(ct, n, lengths=tuple(float(v) for v in n) + (0.0,) * (3 - len(n)), jitter=0.0 if dim == 2 else 0.1)
+    par = {"elastic": lambda: le_params(dim), "local": ld_params, "gradient": gdm_params}[kind]()
+    p = Pair(ct, dt, X, C, *par, two_fields=kind == "gradient", rule=rule)
+    u, e, kap = p.inputs()
+    ctx = p.context()
+    state = [to_dev(u), to_dev(e), to_dev(kap) if kind != "elastic" else None]
+    ref = p.orc.assemble(u, e, kap)
+    R = ctx.build_vector(*state)
+    check_values(R.cpu().numpy(), ref["R"], ref["R_bound"], "R")
+    monkeypatch.setenv("NUTO_AMD_GENERIC", "1")
+    check_values(ctx.build_vector(*state).cpu().numpy(), ref["R"], ref["R_bound"], "R, single pass")
+    monkeypatch.delenv("NUTO_AMD_GENERIC")
+    stress = ctx.eval_ip(N.IP_STRESS, *state)
+    assert stress.shape == (p.ncells, p.nip, 3 if dim == 2 else 6)
+    if kind == "elastic":
+        return
+    kappa, before = ctx.eval_ip(N.IP_KAPPA, *state), state[2].clone()
+    ctx.update_history(*state)
+    assert np.array_equal(state[2].view(p.nip, p.ncells).T.cpu().numpy(), kappa[:, :, 0].cpu().numpy())
+    assert (state[2] >= before).all() and (state[2] > before).any()
+    # the residual depends on max(history, driving strain): unchanged by the update
+    assert np.array_equal(ctx.build_vector(*state).cpu().numpy(), R.cpu().numpy())
+    ctx.update_history(*state)
+    assert np.array_equal(state[2].view(p.nip, p.ncells).T.cpu().numpy(), kappa[:, :, 0].cpu().numpy())
+
+
+@pytest.mark.parametrize("ct,dt,n,rule,forms", [(N.HEX8, N.HEX8, (4, 3, 3), (0, 2), "0123"), (N.HEX8, N.HEX8, (2, 2, 2), (0, 4), "0"),
+                                                (N.HEX8, N.HEX20, (3, 2, 2), (0, 3), "0123"), (N.TET4, N.TET4, (3, 3, 3), (1, 1), "0123"),
+                                                (N.TET4, N.TET10, (2, 2, 2), (1, 2), "0123")])
+def test_local_damage_loads_at_the_updated_history(ct, dt, n, rule, forms, monkeypatch):
+    """Right after a history update every point it raised is loading: the tangent there equals the tangent
+    at a history lower by 1e-10 of itself (omega differs by at most 1e-8 of the entries' magnitude), in every
+    form of the cell matrices."""
+    X, C = make_mesh(ct, n, lengths=tuple(float(v) for v in n), jitter=0.1)
+    p = Pair(ct, dt, X, C, *ld_params(), two_fields=False, rule=rule)
+    u, _, kap = p.inputs()
+    ctx = p.context()
+    du, dk = to_dev(u), to_dev(kap)
+    ctx.update_history(du, None, dk)
+    low = dk * (1.0 - 1e-10)
+    for form in forms:
+        monkeypatch.setenv("NUTO_AMD_CELL_GRAM", form)
+        K, want = (ctx.build_matrix(du, None, k).cpu().numpy() for k in (dk, low))
+        # points that the update did not raise (history above the strain) load in neither
+        assert np.abs(K - want).max() <= 1e-7 * np.abs(want).max()
