@@ -1,15 +1,14 @@
 // Hex8 gradient-damage R+K kernel (the hot path): one 64-lane workgroup per dof node p.
 //
-// Lanes are (r, j) with r = the r-th cell incident to p (group order) and j = 0..7.
-//   phase A  lane (r, ip=j): the integration-point state of cell r at IP ip (Jacobian, strain,
-//            nonlocal strain, damage, stress, equivalent-strain derivative) -> LDS record
-//   phase B  lane (r, b=j):  the 4x4 block (a_r, b) of cell r's element matrix for p's rows
-//            (a_r = local index of p), summed over the 8 IPs in order (Cell.h:108-117)
+// Lanes are (r, m) with r = the r-th cell incident to p (group order) and m = a corner of the cell
+// (hex8_lanes.hpp): the integration point there and the column node b there.
+//   blocks   lane (r, m): the 4x4 block (a_r, b) of cell r's element matrix for p's rows (a_r = local index
+//            of p), summed over the 8 IPs (Cell.h:108-117) by exchanges between the 8 lanes: CellBlock
 //   reduce   slot q of p's neighbourhood = sum over r (cell order, the order setFromTriplets
 //            uses, SimpleAssembler.cpp:149-155) of the blocks that land on q
 //   write    p's three displacement rows (contiguous) and its eeq row, coalesced, written once.
-// R is reduced the same way (cells in order, IPs in order). No atomics: the result is
-// deterministic, and every nonzero and R entry is written exactly once per assembly.
+// R is reduced the same way (its IP terms over the lanes, then the cells in order). No atomics: the
+// result is deterministic, and every nonzero and R entry is written exactly once per assembly.
 //
 // Block algebra (per IP, weight s = detJ * w; g = dN/dX; FULL damage application):
 //   uu = lambda' S + mu' S^T + mu' tr(S) I with S = sum_ip s (1-omega) g_a g_b^T,
@@ -20,14 +19,22 @@
 // UNILATERAL damage application keeps the volumetric factor per IP, so uu is accumulated in the
 // general form c1 g_a g_b^T + c2 g_b g_a^T + c2 (g_a . g_b) I.
 //
+// Modes: 2 (every cell affine: one J^-1 per cell), 1 (J^-1 per IP), both with the IP states from the
+// pre-pass kGdmHex8Ip; 0 evaluates the IP states in the node kernel (launches over one mesh of a batch).
+//
+// What bounds it: the FP64 and exchange instructions of the vector units, 701 per wave in mode 2 (334
+// FP64), with the latency of the record gather and of the reduction's LDS reads behind them (4 waves per
+// SIMD: 9.3 KB of LDS per workgroup). Summing the blocks from records in LDS instead (each lane reading
+// the 8 points' records of its cell) took 732 instructions and kept the LDS busy 78 % of the time.
+// Measured, R + K: 1,000,000 affine cells 2.39 -> 2.08 ms, 146,969 jittered cells 0.479 -> 0.374 ms.
+//
 // Usable when every node has at most 8 incident cells and at most 32 neighbours (structured hex
 // meshes: 8 and 27) and the coordinate and dof layers share their nodes; other meshes use the
 // generic row-owner kernel.
 //
-// Gathers are three dependent loads deep: per-node incidence tables padded to 8 cells (cell,
-// local index, history column, neighbour slots), then the cell's dof node ranks, its history and
-// its geometry, then the node values. The geometry of every (cell, IP) - J^-1 and detJ * w
-// (Jacobian.h:35-47, Cell.h:108-117) - depends on the coordinates only; it is computed once per
+// Gathers are two dependent loads deep: per-node incidence tables padded to 8 cells (cell, local index,
+// neighbour slots), then the cell's geometry and state records. The geometry of every (cell, IP) - J^-1 and
+// detJ * w (Jacobian.h:35-47, Cell.h:108-117) - depends on the coordinates only; it is computed once per
 // pattern by kGdmHex8Geometry with the same arithmetic and stored (80 bytes per IP).
 #pragma once
 
@@ -40,6 +47,7 @@
 
 #include "assemble_rows.hpp"
 #include "devbuf.hpp"
+#include "hex8_lanes.hpp"
 #include "laws.hpp"
 #include "mesh.hpp"
 #include "morton.hpp"
@@ -51,11 +59,6 @@ namespace gdm8
 {
 constexpr int kMaxInc = 8;   // incident cells per node
 constexpr int kMaxAdj = 32;  // neighbours per node
-// doubles per (ip, cell) record: 26 for FULL damage application, 30 with the UNILATERAL terms.
-// Records are 13 (15) 16-byte chunks long: an odd count, so 16 consecutive records start on 16
-// distinct 4-bank groups.
-template <bool FULLDMG>
-constexpr int kStOf = FULLDMG ? 26 : 30;
 constexpr int kGeo = 10;     // doubles per (cell, IP) geometry record: J^-1 (row-major), detJ * w
 // per (cell, IP) state record of the pre-pass (kGdmHex8Ip): with e'' = [e0, e1, e2, e3/2, e4/2, e5/2]
 // (tensor strain) the stress, t = s omega' kappa' d sigma / d omega and m = d eps_eq / d eps are all
@@ -69,8 +72,8 @@ constexpr int rGi = 18;   // g(omega)
 constexpr int rDg = 19;   // dg / d omega * d omega / d kappa * d kappa / d eeq
 constexpr int rEps = 0;   // e'' (6)
 constexpr int rSig = 6;   // s alpha_sigma, s beta_sigma
-constexpr int rT = 8;     // alpha_t, beta_t (s included)
-constexpr int rM = 10;    // s alpha_m, s beta_m
+constexpr int rT = 8;     // alpha_t, beta_t (s and kValueScale included)
+constexpr int rM = 10;    // s alpha_m, s beta_m (kGradScale included, as in the next two)
 constexpr int rC1 = 12;   // FULL: s (1 - omega); UNILATERAL: s (3K (1 - omega H) - 2G (1 - omega)) / 3
 constexpr int rC2 = 13;   // UNILATERAL: s G (1 - omega); FULL: 0
 constexpr int rRe = 14;   // s (eeq - eps_eq)
@@ -78,26 +81,7 @@ constexpr int rGe = 15;   // s c grad eeq (3)
 constexpr int kPs = 17;      // doubles per partial block (odd: 64 lanes spread over the banks)
 constexpr int kTab = 57;     // per-IP table row: w, dNc[8][3], N[8], dNd[8][3]
 
-// record layout
-constexpr int sInv = 0;   // J^-1 (9)
-constexpr int sHa = 9;    // FULL: s (1-omega) g_a; UNILATERAL: c1 g_a (3)
-constexpr int sVa = 12;   // B_a^T t (3)
-constexpr int sMn = 15;   // -N_a s d eps_eq / d eps (6)
-constexpr int sCg = 21;   // c s g_a (3)
-constexpr int sSn = 24;   // s N_a (1)
-constexpr int sKa = 25;   // UNILATERAL: c2 g_a (3)
-constexpr int kRed = 1160;  // doubles after phase B: partial blocks 64 x kPs, R sums 32, 8 unused, slot map 32
-
-// value of lane (lane & ~7) + n within each group of 8 lanes (ds_swizzle bit mode:
-// and-mask 0x18 keeps the group, or-mask n selects the lane)
-template <int n>
-__device__ inline double GroupLane(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_ds_swizzle((int)(b & 0xffffffffLL), 0x18 | (n << 5));
-    const int hi = __builtin_amdgcn_ds_swizzle((int)(b >> 32), 0x18 | (n << 5));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
+constexpr int kRed = 1160;  // doubles of the reduction: partial blocks 64 x kPs, R sums 32, 8 unused, slot map 32
 
 constexpr double kGauss = 0.57735026918962573;  // sqrt(1/3), the 2-point Gauss abscissa
 constexpr double kThird = 1.0 / 3.0;
@@ -119,31 +103,6 @@ __device__ inline void ShapeAt(int n, int ip, double d[3], double& N)
 }
 
 // g = J^-T d  (dN/dX = dN/dxi J^-1, Jacobian.h:100-103)
-// Shape data of a hex8 node at the 2x2x2 Gauss point whose corner differs from the node's in the
-// axes of the set bits of t: f_k = 1 - g if bit k of t is set, else 1 + g (g = sqrt(1/3)), and
-// [|dN/dxi_0|, |dN/dxi_1|, |dN/dxi_2|, N] = [f1 f2, f0 f2, f0 f1, f0 f1 f2] / 8, with the products
-// taken in ShapeAt's order (so the values are bitwise ShapeAt's, up to the gradient signs).
-struct ShapeRelTable
-{
-    double v[8][4];
-};
-constexpr ShapeRelTable MakeShapeRel()
-{
-    ShapeRelTable t{};
-    for (int k = 0; k < 8; k++)
-    {
-        const double f0 = (k & 1) ? 1.0 - kGauss : 1.0 + kGauss;
-        const double f1 = (k & 2) ? 1.0 - kGauss : 1.0 + kGauss;
-        const double f2 = (k & 4) ? 1.0 - kGauss : 1.0 + kGauss;
-        t.v[k][0] = 0.125 * f1 * f2;
-        t.v[k][1] = 0.125 * f0 * f2;
-        t.v[k][2] = 0.125 * f0 * f1;
-        t.v[k][3] = 0.125 * f0 * f1 * f2;
-    }
-    return t;
-}
-__constant__ ShapeRelTable kShapeRel = MakeShapeRel();
-
 __device__ inline void GradOf(const double d[3], const double inv[3][3], double g[3])
 {
 #pragma unroll
@@ -254,57 +213,6 @@ __device__ inline void GdmMisesDerivative(const GdmIp& o, const LawParams& P, do
     }
 }
 
-// Hu, he, eN of cell r at IP ip from the node values held by the 8 lanes of the cell
-// (node n by lane (r, n)): Hu = sum_n u_n dN_n/dxi^T, he = sum_n e_n dN_n/dxi, eN = sum_n N_n e_n
-__device__ inline void GatherGradients(const double v[4], int ip, double Hu[3][3], double he[3], double& eN)
-{
-    using namespace gdm8;
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-    {
-        he[i] = 0.0;
-#pragma unroll
-        for (int k = 0; k < 3; k++)
-            Hu[i][k] = 0.0;
-    }
-    eN = 0.0;
-#pragma unroll
-    for (int n = 0; n < 8; n++)
-    {
-        double d[3], Nv;
-        ShapeAt(n, ip, d, Nv);
-        double U[3], en;
-        switch (n)
-        {
-#define NUTO_GROUP_LANE(N)                                                                                 \
-    case N:                                                                                                \
-        U[0] = GroupLane<N>(v[0]);                                                                         \
-        U[1] = GroupLane<N>(v[1]);                                                                         \
-        U[2] = GroupLane<N>(v[2]);                                                                         \
-        en = GroupLane<N>(v[3]);                                                                           \
-        break;
-            NUTO_GROUP_LANE(0)
-            NUTO_GROUP_LANE(1)
-            NUTO_GROUP_LANE(2)
-            NUTO_GROUP_LANE(3)
-            NUTO_GROUP_LANE(4)
-            NUTO_GROUP_LANE(5)
-            NUTO_GROUP_LANE(6)
-            NUTO_GROUP_LANE(7)
-#undef NUTO_GROUP_LANE
-        }
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int k = 0; k < 3; k++)
-                Hu[i][k] += U[i] * d[k];
-        he[0] += en * d[0];
-        he[1] += en * d[1];
-        he[2] += en * d[2];
-        eN += Nv * en;
-    }
-}
-
 // Per-node tables of the node kernel (built once per pattern, see GdmHex8Plan::Prepare), stored in
 // traversal order: position s holds the node order[s] (nodes sorted along a Morton curve).
 struct GdmHex8Tables
@@ -341,299 +249,209 @@ __device__ inline int NodeOfBlock(const GdmHex8Tables& T)
     return T.order ? T.order[i] : i;
 }
 
-// Inputs of lane (r, j) of node p.
-template <bool DEC>
-struct NodeFetch
+// The pre-pass state record of an integration point (kSrOf doubles)
+template <bool FULLDMG, bool DEC>
+__device__ inline void StateRecord(const GdmIp& st, double s, double m3K, double m2G, const LawParams& P, double* rec)
 {
-    int cell, la, slot;
-    double v[4];  // u0 u1 u2 e of node j of cell r
-    double g[gdm8::kGeo];  // geometry of cell r at IP j
-    double sr[gdm8::kSrOf<DEC>];  // pre-pass state of cell r at IP j
-    double th[3];
-    double kh;  // history kappa of cell r at IP j
-};
-
-// GEO0: the cell's geometry record (IP 0's) in every lane of the group (affine cells).
-// CLAMP: lanes past the node's last incident cell (f.cell < 0) load cell 0's records instead of
-// skipping the loads, so that every lane runs the same straight-line code (their results are
-// never used: the slot map of the reduction leaves absent cells out).
-template <bool PRE, bool GEO0, bool CLAMP, bool DEC>
-__device__ inline void FetchNode(const RowArgs& A, const GdmHex8Tables& T, int pos, int r, int j, NodeFetch<DEC>& f)
-{
-    constexpr int kN = gdm8::kSrOf<DEC>, kUse = DEC ? 20 : gdm8::kSr;  // record stride, doubles read
-    const size_t pr = (size_t)pos * 8 + r;
-    f.cell = T.nodeCell[pr];
-    f.la = T.nodeLa[pr];
-    f.slot = T.nodeSlot[pr * 8 + j];
-    f.kh = 0.0;
-    if (CLAMP || f.cell >= 0)
+    using namespace gdm8;
+    const double eV = st.I1 * kThird;
+    const double sV = (1.0 - st.om * st.H) * m3K * eV;
+    double am = P.K1, bm = 0.0;  // m = am [1,1,1,0,0,0] + bm e'' (A == 0: m = K1 [1,1,1,0,0,0])
+    if (st.Am != 0.0)
     {
-        const int cl = CLAMP && f.cell < 0 ? 0 : f.cell;
-        const double2* gr = reinterpret_cast<const double2*>(
-            GEO0 ? T.geoCell + (size_t)cl * gdm8::kGeo : T.geo + ((size_t)cl * 8 + j) * gdm8::kGeo);
-#pragma unroll
-        for (int k = 0; k < gdm8::kGeo / 2; k++)
-        {
-            const double2 v = gr[k];
-            f.g[2 * k] = v.x;
-            f.g[2 * k + 1] = v.y;
-        }
-        if constexpr (PRE)
-        {
-            const double2* sp = reinterpret_cast<const double2*>(T.ipState + ((size_t)cl * 8 + j) * kN);
-#pragma unroll
-            for (int k = 0; k < kUse / 2; k++)
-            {
-                const double2 v = sp[k];
-                f.sr[2 * k] = v.x;
-                f.sr[2 * k + 1] = v.y;
-            }
-        }
-        else
-        {
-            const int hist = T.nodeHist ? T.nodeHist[pr] : f.cell;
-            const int q = A.dconn[(size_t)f.cell * 8 + j];
-            f.kh = A.kappa[(size_t)hist + (size_t)j * A.kappaLd];
-            f.v[0] = A.u[(size_t)q * 3];
-            f.v[1] = A.u[(size_t)q * 3 + 1];
-            f.v[2] = A.u[(size_t)q * 3 + 2];
-            f.v[3] = A.e[q];
-        }
-        if (A.thE)
-        {
-            f.th[0] = A.thE[cl];
-            f.th[1] = A.thFt[cl];
-            f.th[2] = A.thGf[cl];
-        }
+        const double h = 0.5 / st.Am;
+        am = P.K1 + h * (2.0 * P.K1 * P.K1 * st.I1) - h * P.K2 * st.I1 * kThird;
+        bm = h * P.K2;
+    }
+    const double ct = kValueScale * s * st.dom * st.dk, sg = kGradScale * s;
+    rec[rEps] = st.eps[0];
+    rec[rEps + 1] = st.eps[1];
+    rec[rEps + 2] = st.eps[2];
+    rec[rEps + 3] = 0.5 * st.eps[3];
+    rec[rEps + 4] = 0.5 * st.eps[4];
+    rec[rEps + 5] = 0.5 * st.eps[5];
+    rec[rSig] = s * (sV - st.d2G * eV);
+    rec[rSig + 1] = s * st.d2G;
+    rec[rT] = -ct * (m3K * st.H - m2G) * eV;
+    rec[rT + 1] = -ct * m2G;
+    rec[rM] = sg * am;
+    rec[rM + 1] = sg * bm;
+    rec[rC1] = FULLDMG ? sg * (1.0 - st.om) : sg * (m3K * (1.0 - st.om * st.H) - st.d2G) * kThird;
+    rec[rC2] = FULLDMG ? 0.0 : 0.5 * sg * st.d2G;
+    rec[rRe] = s * (st.eN - st.eq);
+    rec[rGe] = s * P.c * st.ge[0];
+    rec[rGe + 1] = s * P.c * st.ge[1];
+    rec[rGe + 2] = s * P.c * st.ge[2];
+    if constexpr (DEC)
+    {
+        double gi, dgi;
+        NonlocalFactor(P, st.om, gi, dgi);
+        rec[rGi] = gi;
+        rec[rDg] = dgi * st.dom * st.dk;
+        rec[kSrOf<DEC> - 2] = rec[kSrOf<DEC> - 1] = 0.0;
     }
 }
 
-// v of lane i + dpp-selected lane (CTRL: a DPP control word; out-of-row reads give 0)
-template <int CTRL>
-__device__ inline double DppMov(double v)
+// Material of a cell (per-cell fields: E, kappa0 = f_t / E, beta = f_t / G_f)
+__device__ inline void GdmMaterial(const RowArgs& A, int cell, double& E, double& k0, double& beta)
 {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    E = A.P.E;
+    k0 = A.P.kappa0;
+    beta = A.P.beta;
+    if (A.thE)
+    {
+        E = A.thE[cell];
+        k0 = A.thFt[cell] / E;
+        beta = A.thFt[cell] / A.thGf[cell];
+    }
 }
 
-// sum over the 8 lanes of a group, ((t0 + t1) + (t2 + t3)) + ((t4 + t5) + (t6 + t7)), valid in
-// the group's lane 0 (DPP: no LDS instruction)
+// The state of (cell, c.ip) from the node values v = (u, eeq) of node c.node in each lane of the cell's
+// group; sE: 8 doubles of LDS of the group (written by the caller before a barrier: eeq in local node order)
+template <bool FULLDMG>
+__device__ inline void GdmCellState(const RowArgs& A, const CornerLane& c, int cell, const double v[4], const double* sE,
+                                    const double inv[3][3], GdmIp& st, double& m3K, double& m2G)
+{
+    double E, k0, beta;
+    GdmMaterial(A, cell, E, k0, beta);
+    m3K = A.P.cK * E;
+    m2G = A.P.cG * E;
+    const int hist = A.cellId ? A.cellId[cell] : cell;
+    const double kh = A.kappa[(size_t)hist + (size_t)c.ip * A.kappaLd];
+    double Hu[3][3], he[3], inv0[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+    {
+        NodesToPoint(c, v[i], Hu[i]);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            inv0[i][k] = kGradScale * inv[i][k];
+    }
+    NodesToPoint(c, v[3], he);
+    GdmIpState<FULLDMG>(Hu, he, NodeSum(c, sE), inv0, kh, m3K, m2G, k0, beta, A.P, st);
+}
+
+// v of lane i + dpp-selected lane (CTRL: a DPP control word; out-of-row reads give 0): the sum over the
+// 8 lanes of a group, ((t0 + t1) + (t2 + t3)) + ((t4 + t5) + (t6 + t7)), valid in the group's lane 0
 __device__ inline double GroupSum0(double v)
 {
-    v += DppMov<0xB1>(v);   // quad_perm [1, 0, 3, 2]: lane i ^ 1
-    v += DppMov<0x4E>(v);   // quad_perm [2, 3, 0, 1]: lane i ^ 2
-    v += DppMov<0x104>(v);  // row_shl:4: lane i + 4
+    v += LaneDpp<kDppXor1>(v);
+    v += LaneDpp<kDppXor2>(v);
+    v += LaneDpp<0x104>(v);  // row_shl:4: lane i + 4
     return v;
 }
 
-// geometry and pre-pass state records of (cell, ip)
-template <bool DEC>
-__device__ inline void LoadIpRecords(const GdmHex8Tables& T, int cell, int ip, double g[gdm8::kGeo],
-                                     double sr[gdm8::kSrOf<DEC>])
-{
-    constexpr int kN = gdm8::kSrOf<DEC>, kUse = DEC ? 20 : gdm8::kSr;
-    const double2* gr = reinterpret_cast<const double2*>(T.geo + ((size_t)cell * 8 + ip) * gdm8::kGeo);
-#pragma unroll
-    for (int k = 0; k < gdm8::kGeo / 2; k++)
-    {
-        const double2 v = gr[k];
-        g[2 * k] = v.x;
-        g[2 * k + 1] = v.y;
-    }
-    const double2* sp = reinterpret_cast<const double2*>(T.ipState + ((size_t)cell * 8 + ip) * kN);
-#pragma unroll
-    for (int k = 0; k < kUse / 2; k++)
-    {
-        const double2 v = sp[k];
-        sr[2 * k] = v.x;
-        sr[2 * k + 1] = v.y;
-    }
-}
-
-// Terms of row node a (local index la) at IP ip of a cell from its pre-pass state record: the LDS
-// record for phase B (J^-1, s(1-w) g_a or c1 g_a, B_a^T t, -N_a s m, c s g_a, s N_a, c2 g_a) and the
-// R terms s B_a^T sigma, s (N_a (eeq - eps_eq) + c g_a . grad eeq).
-// WITHINV false: the record omits J^-1 (affine cells keep one J^-1 per cell) and the other terms
-// start at 0 instead of 9.
+// Block (a_r, c.node) of cell r for the rows of node a (local index la), summed over the cell's IPs, from
+// the state record sr and geometry g of this lane's IP: acc[4 i + k], i = row component (0..2
+// displacement rows, 3 eeq row), k = column component. Each term is a field over the IPs (formed here from
+// a's shape data) times N_b or dN_b/dxi, summed to the 8 nodes b by the group's exchanges; with one J^-1
+// per cell (AFF) S = (sum s (1-w) g_a dN_b/dxi^T) J^-1, otherwise J^-1 goes into the field. Rv: the R terms
+// of node a at this IP, s B_a^T sigma and s (N_a (eeq - eps_eq) + c g_a . grad eeq).
 // DEC: the nonlocal term carries g(omega), and K_ee the term c (grad eeq . g_a) g' omega' kappa' N_b, which
 // joins s N_a N_b.
-template <bool FULLDMG, int kSt, bool WITHINV, bool DEC>
-__device__ inline void PreRecord(const double* sr, const double* g, int la, int ip, const LawParams& P, double rec[kSt],
-                                 double Rv[4])
+template <bool FULLDMG, bool AFF, bool DEC>
+__device__ inline void CellBlock(const CornerLane& c, const double* sr, const double* g, int la, double m3K, double m2G,
+                                 const LawParams& P, double acc[16], double Rv[4])
 {
     using namespace gdm8;
-    constexpr int o = WITHINV ? 0 : -sHa;  // index shift of the terms after J^-1
     const double inv[3][3] = {{g[0], g[1], g[2]}, {g[3], g[4], g[5]}, {g[6], g[7], g[8]}};
     const double s = g[9];
     double da[3], Na, ga[3];
-    ShapeAt(la, ip, da, Na);
+    ShapeAt(la, c.ip, da, Na);
     GradOf(da, inv, ga);
-    // e'' g_a: B_a^T of the Voigt vector e''
-    const double Eg[3] = {sr[rEps] * ga[0] + sr[rEps + 5] * ga[1] + sr[rEps + 4] * ga[2],
-                          sr[rEps + 5] * ga[0] + sr[rEps + 1] * ga[1] + sr[rEps + 3] * ga[2],
-                          sr[rEps + 4] * ga[0] + sr[rEps + 3] * ga[1] + sr[rEps + 2] * ga[2]};
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-        Rv[i] = sr[rSig] * ga[i] + sr[rSig + 1] * Eg[i];
+    const double E[3][3] = {{sr[rEps], sr[rEps + 5], sr[rEps + 4]},
+                            {sr[rEps + 5], sr[rEps + 1], sr[rEps + 3]},
+                            {sr[rEps + 4], sr[rEps + 3], sr[rEps + 2]}};
     const double gdot = ga[0] * sr[rGe] + ga[1] * sr[rGe + 1] + ga[2] * sr[rGe + 2];
+    const double cs = kGradScale * P.c * (DEC ? s * sr[DEC ? rGi : 0] : s);
     Rv[3] = Na * sr[rRe] + (DEC ? sr[DEC ? rGi : 0] * gdot : gdot);
-    const double cs = DEC ? P.c * s * sr[DEC ? rGi : 0] : P.c * s;
-    if constexpr (WITHINV)
-    {
-#pragma unroll
-        for (int a = 0; a < 3; a++)
-#pragma unroll
-            for (int b = 0; b < 3; b++)
-                rec[sInv + 3 * a + b] = inv[a][b];
-    }
 #pragma unroll
     for (int i = 0; i < 3; i++)
     {
-        rec[o + sHa + i] = sr[rC1] * ga[i];
-        rec[o + sVa + i] = sr[rT] * ga[i] + sr[rT + 1] * Eg[i];
-        rec[o + sCg + i] = cs * ga[i];
-        if (!FULLDMG)
-            rec[o + sKa + i] = sr[rC2] * ga[i];
+        // e'' g_a: B_a^T of the Voigt vector e''
+        const double Eg = E[i][0] * ga[0] + E[i][1] * ga[1] + E[i][2] * ga[2];
+        Rv[i] = sr[rSig] * ga[i] + sr[rSig + 1] * Eg;
+        acc[4 * i + 3] = ValuesToNode(sr[rT] * ga[i] + sr[rT + 1] * Eg);  // ue: (B_a^T t) N_b
     }
-#pragma unroll
-    for (int i = 0; i < 6; i++)
-        rec[o + sMn + i] = -Na * ((i < 3 ? sr[rM] : 0.0) + sr[rM + 1] * sr[rEps + i]);
-    rec[o + sSn] = DEC ? s * Na + sr[DEC ? rDg : 0] * gdot : s * Na;
-#pragma unroll
-    for (int k = o + (FULLDMG ? sSn + 1 : sKa + 3); k < kSt; k++)
-        rec[k] = 0.0;  // padding
-}
-
-template <int kSt>
-__device__ inline void StoreRecord(double* dst, const double rec[kSt])
-{
-#pragma unroll
-    for (int k = 0; k < kSt; k += 2)
-        *reinterpret_cast<double2*>(dst + k) = make_double2(rec[k], rec[k + 1]);
-}
-
-// Adds one IP's contribution to block (a, b): h = the record's terms after J^-1 (c1 g_a, B_a^T t,
-// -N_a m, c g_a, N_a, [c2 g_a]), gb = g_b, Nb = N_b.
-template <bool FULLDMG>
-__device__ inline void AccumulateIp(const double* h, const double gb[3], double Nb, double acc[16])
-{
-    using namespace gdm8;
-    const double* ha = h;
-#pragma unroll
-    for (int ii = 0; ii < 3; ii++)
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-            acc[ii * 4 + c] += ha[ii] * gb[c];
-    if (!FULLDMG)
+    double p[3];
     {
-        const double* ka = h + (sKa - sHa);
-        const double d = ka[0] * gb[0] + ka[1] * gb[1] + ka[2] * gb[2];
+        // eu: -N_a s (B_b^T m), m = alpha [1, 1, 1, 0, 0, 0] + beta e''
+        const double am = -Na * sr[rM], bm = -Na * sr[rM + 1];
 #pragma unroll
-        for (int ii = 0; ii < 3; ii++)
+        for (int i = 0; i < 3; i++)
         {
 #pragma unroll
-            for (int c = 0; c < 3; c++)
-                acc[ii * 4 + c] += gb[ii] * ka[c];
-            acc[ii * 5] += d;
+            for (int k = 0; k < 3; k++)
+                p[k] = am * inv[k][i] + bm * (E[i][0] * inv[k][0] + E[i][1] * inv[k][1] + E[i][2] * inv[k][2]);
+            acc[12 + i] = PointsToNode<false>(c, p, 0.0);
         }
     }
-    const double* va = h + (sVa - sHa);
-    acc[3] += va[0] * Nb;
-    acc[7] += va[1] * Nb;
-    acc[11] += va[2] * Nb;
-    // B_b^T (-N_a m) and the eeq-eeq entry, each term fused into the accumulator
-    const double* mn = h + (sMn - sHa);
-    acc[12] = fma(gb[1], mn[5], fma(gb[2], mn[4], fma(gb[0], mn[0], acc[12])));
-    acc[13] = fma(gb[0], mn[5], fma(gb[2], mn[3], fma(gb[1], mn[1], acc[13])));
-    acc[14] = fma(gb[0], mn[4], fma(gb[1], mn[3], fma(gb[2], mn[2], acc[14])));
-    const double* cg = h + (sCg - sHa);
-    acc[15] = fma(cg[2], gb[2], fma(cg[1], gb[1], fma(cg[0], gb[0], fma(h[sSn - sHa], Nb, acc[15]))));
-}
-
-// Phase B: lane (r, b) accumulates block (a_r, b) over IPs ip0 .. ip0 + n - 1 (records at
-// state[(r * n + i) * kSt], i = ip - ip0), in IP order. The records of one cell are adjacent, so
-// the record stores of consecutive lanes (r, i) hit consecutive records: with an odd number of
-// 16-byte chunks per record (kSt / 2 odd) any 16 of them fall on distinct 4-bank groups.
-template <bool FULLDMG, int kSt>
-__device__ inline void PhaseB(const double* state, int r, int b, int ip0, int n, double acc[16])
-{
-    using namespace gdm8;
-#pragma unroll 1
-    for (int i = 0; i < n; i++)
-    {
-        const int ip = ip0 + i;
-        double db[3], Nb;
-        ShapeAt(b, ip, db, Nb);
-        const double* st = state + (r * n + i) * kSt;
-        constexpr int kRd = FULLDMG ? 26 : 28;
-        double rec[kRd];
+    // ee: s N_a N_b + c s g_a . g_b
 #pragma unroll
-        for (int k = 0; k < kRd; k += 2)
+    for (int k = 0; k < 3; k++)
+        p[k] = cs * (ga[0] * inv[k][0] + ga[1] * inv[k][1] + ga[2] * inv[k][2]);
+    acc[15] = PointsToNode<true>(c, p, kValueScale * (DEC ? s * Na + sr[DEC ? rDg : 0] * gdot : s * Na));
+    // S = sum h g_a g_b^T for the factor h of the displacement block
+    auto gram = [&](double h, double S[3][3]) {
+#pragma unroll
+        for (int i = 0; i < 3; i++)
         {
-            const double2 v = *reinterpret_cast<const double2*>(st + k);
-            rec[k] = v.x;
-            rec[k + 1] = v.y;
+            const double f = h * ga[i];
+            if constexpr (AFF)
+            {
+                double d[3];
+                ValuesToGradients(c, f, d);
+                GradOf(d, inv, S[i]);
+            }
+            else
+            {
+#pragma unroll
+                for (int j = 0; j < 3; j++)
+                {
+#pragma unroll
+                    for (int k = 0; k < 3; k++)
+                        p[k] = f * inv[k][j];
+                    S[i][j] = PointsToNode<false>(c, p, 0.0);
+                }
+            }
         }
-        const double inv[3][3] = {{rec[0], rec[1], rec[2]}, {rec[3], rec[4], rec[5]}, {rec[6], rec[7], rec[8]}};
-        double gb[3];
-        GradOf(db, inv, gb);
-        AccumulateIp<FULLDMG>(rec + sHa, gb, Nb, acc);
+    };
+    double S[3][3];
+    if constexpr (FULLDMG)
+    {
+        // uu = lambda' S + mu' S^T + mu' tr(S) I
+        gram(sr[rC1], S);
+        const double lam = (m3K - m2G) * kThird, mu = 0.5 * m2G;
+        const double tr = mu * (S[0][0] + S[1][1] + S[2][2]);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+            {
+                acc[4 * i + k] = lam * S[i][k] + mu * S[k][i];
+                if (i == k)
+                    acc[4 * i + k] += tr;
+            }
+    }
+    else
+    {
+        // uu = S1 + S2^T + tr(S2) I with the factors c1 and c2
+        gram(sr[rC2], S);
+        const double tr = S[0][0] + S[1][1] + S[2][2];
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                acc[4 * i + k] = S[k][i] + (i == k ? tr : 0.0);
+        gram(sr[rC1], S);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                acc[4 * i + k] += S[i][k];
     }
 }
 
-// Phase B of affine cells (MODE 2): lane (r, b) visits the IPs of cell r in the order
-// ip = t ^ m(b), m(b) = b's corner (bit k set: + side along axis k). Node b's shape data at that
-// IP depends on t only (kShapeRel, uniform over the wave); the signs of b's gradient are folded
-// into J^-1 once, so g_b is bitwise GradOf's. The 8 lanes of a cell read 8 different records:
-// 16 consecutive lanes read 16 consecutive records (distinct 4-bank groups).
-template <bool FULLDMG, int kSt>
-__device__ inline void PhaseBAffine(const double* state, int r, int b, const double inv[3][3], double acc[16])
-{
-    using namespace gdm8;
-    const int sx = ((b + 1) >> 1) & 1, sy = (b >> 1) & 1, sz = b >> 2;
-    const int m = sx | (sy << 1) | (sz << 2);
-    double sinv[3][3];
-#pragma unroll
-    for (int c = 0; c < 3; c++)
-    {
-        sinv[0][c] = sx ? inv[0][c] : -inv[0][c];
-        sinv[1][c] = sy ? inv[1][c] : -inv[1][c];
-        sinv[2][c] = sz ? inv[2][c] : -inv[2][c];
-    }
-    const double* cellRec = state + r * 8 * kSt;
-#pragma unroll 2
-    for (int t = 0; t < 8; t++)
-    {
-        const double d0 = kShapeRel.v[t][0], d1 = kShapeRel.v[t][1], d2 = kShapeRel.v[t][2], Nb = kShapeRel.v[t][3];
-        const double* st = cellRec + (t ^ m) * kSt;
-        constexpr int kRd = FULLDMG ? 16 : 20;
-        double rec[kRd];
-#pragma unroll
-        for (int k = 0; k < kRd; k += 2)
-        {
-            const double2 v = *reinterpret_cast<const double2*>(st + k);
-            rec[k] = v.x;
-            rec[k + 1] = v.y;
-        }
-        double gb[3];
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-            gb[c] = d0 * sinv[0][c] + d1 * sinv[1][c] + d2 * sinv[2][c];
-        AccumulateIp<FULLDMG>(rec, gb, Nb, acc);
-    }
-}
-
-// One workgroup per node. Workgroups are dispatched round-robin over the 8 XCDs; with
-// xcdMap the node of block b is chosen so that each XCD processes a contiguous range of nodes
-// (neighbouring nodes share cells and node data, which then stay in that XCD's L2).
-// MODE 0: the node kernel evaluates the IP states itself (8 records per cell in LDS).
-// MODE 1: the IP states come from kGdmHex8Ip; phase B runs in two passes of 4 IPs so that only 32
-//         records are in LDS at once (9.3 KB per workgroup: 4 waves per SIMD at <= 128 VGPRs).
-// MODE 2: as 1 for meshes of affine cells (J^-1 and detJ w equal at the 8 IPs of every cell, e.g.
-//         bricks): IP 0's geometry for all IPs; records without J^-1 (18 doubles); all 8 IPs in one
-//         pass (9.3 KB).
 // K is written once and not read again here: streaming (non-temporal) stores keep the records,
 // which are re-read, in the caches.
 typedef double D2v __attribute__((ext_vector_type(2)));
@@ -653,197 +471,91 @@ __device__ inline void StoreRows(double* dst, const double* src, int n, int lane
         __builtin_nontemporal_store(src[n - 1], dst + n - 1);
 }
 
-template <bool FULLDMG, int MODE>
-struct NodeLds
-{
-    static constexpr int kSt = MODE == 2 ? (FULLDMG ? 18 : 22) : gdm8::kStOf<FULLDMG>;
-    static constexpr int kRecIps = MODE == 1 ? 4 : 8;                         // IPs of the records in LDS at a time
-    static constexpr int kRecs = 8 * kRecIps * kSt;                           // records
-    static constexpr int kState = kRecs > gdm8::kRed ? kRecs : gdm8::kRed;   // doubles of LDS per workgroup
-};
-
-// The rows of node p (one 64-lane workgroup); `state` is the workgroup's LDS (NodeLds::kState doubles):
-// records [i][r][kSt]; after phase B: partial blocks, R sums and the slot map.
+// The rows of node p (one 64-lane workgroup); `state` is the workgroup's LDS (kRed doubles): partial
+// blocks, R sums and the slot map.
 template <bool WR, bool FULLDMG, int MODE, bool DEC>
 __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int pos, double* state)
 {
     using namespace gdm8;
     constexpr bool PRE = MODE >= 1, AFF = MODE == 2;
-    constexpr int kSt = NodeLds<FULLDMG, MODE>::kSt;
+    constexpr int kN = kSrOf<DEC>, kUse = DEC ? 20 : kSr;  // record stride, doubles read
+    static_assert(PRE || !DEC, "the decreasing interaction needs the pre-pass");
 
     const int lane = threadIdx.x;
-    const int r = lane >> 3, j = lane & 7;
+    const int r = lane >> 3, m = lane & 7;
+    const CornerLane c = CornerOf(lane);
     const LawParams& P = A.P;
     // node p at table position pos; its rows: 3 displacement rows (consecutive in the CSR) and the
     // eeq row, each 4 nA long
     const int4 head = T.nodeHead[pos];
     const int p = head.x, ru0 = head.y, L = head.z, re0 = head.w;
     const int nA = L >> 2;
-    static_assert(PRE || !DEC, "the decreasing interaction needs the pre-pass");
-    NodeFetch<DEC> f;
-    FetchNode<PRE, AFF, AFF, DEC>(A, T, pos, r, j, f);
-    const bool valid = f.cell >= 0;  // r < number of cells incident to p
-    const int la = f.la;
-
-    // material of the cell (per-cell fields: E, kappa0 = f_t / E, beta = f_t / G_f)
-    double E = P.E, k0 = P.kappa0, beta = P.beta;
-    if (A.thE && valid)
-    {
-        E = f.th[0];
-        k0 = f.th[1] / E;
-        beta = f.th[1] / f.th[2];
-    }
-    const double m3K = P.cK * E, m2G = P.cG * E;
+    const size_t pr = (size_t)pos * 8 + r;
+    const int cellOr = T.nodeCell[pr];
+    const int la = T.nodeLa[pr];
+    const int slot = T.nodeSlot[pr * 8 + c.node];
+    const bool valid = cellOr >= 0;  // r < number of cells incident to p
+    // lanes past the node's last cell work on cell 0: their blocks are never read, their R terms are zeroed
+    const int cell = valid ? cellOr : 0;
 
     double Rv[4] = {0.0, 0.0, 0.0, 0.0};
     double acc[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-        acc[i] = 0.0;
-    if constexpr (AFF)
+    if (A.nCells > 0)
     {
-        // every lane, absent cells included (their records and blocks are never read; their R terms
-        // are zeroed)
-        double rec[kSt];
-        PreRecord<FULLDMG, kSt, false, DEC>(f.sr, f.g, la, j, P, rec, Rv);
+        double g[kGeo], sr[kN], m3K, m2G;
+        {
+            const double2* gr = reinterpret_cast<const double2*>(AFF ? T.geoCell + (size_t)cell * kGeo
+                                                                     : T.geo + ((size_t)cell * 8 + c.ip) * kGeo);
+#pragma unroll
+            for (int k = 0; k < kGeo / 2; k++)
+            {
+                const double2 v = gr[k];
+                g[2 * k] = v.x;
+                g[2 * k + 1] = v.y;
+            }
+        }
+        if constexpr (PRE)
+        {
+            const double2* sp = reinterpret_cast<const double2*>(T.ipState + ((size_t)cell * 8 + c.ip) * kN);
+#pragma unroll
+            for (int k = 0; k < kUse / 2; k++)
+            {
+                const double2 v = sp[k];
+                sr[2 * k] = v.x;
+                sr[2 * k + 1] = v.y;
+            }
+            const double E = A.thE ? A.thE[cell] : P.E;
+            m3K = P.cK * E;
+            m2G = P.cG * E;
+        }
+        else
+        {
+            const int q = A.dconn[(size_t)cell * 8 + c.node];
+            const double v[4] = {A.u[(size_t)q * 3], A.u[(size_t)q * 3 + 1], A.u[(size_t)q * 3 + 2], A.e[q]};
+            state[8 * r + c.node] = v[3];
+            __syncthreads();
+            const double inv[3][3] = {{g[0], g[1], g[2]}, {g[3], g[4], g[5]}, {g[6], g[7], g[8]}};
+            GdmIp st;
+            GdmCellState<FULLDMG>(A, c, cell, v, state + 8 * r, inv, st, m3K, m2G);
+            StateRecord<FULLDMG, DEC>(st, g[9], m3K, m2G, P, sr);
+        }
+        CellBlock<FULLDMG, AFF, DEC>(c, sr, g, la, m3K, m2G, P, acc, Rv);
         if (!valid)
             Rv[0] = Rv[1] = Rv[2] = Rv[3] = 0.0;
-        StoreRecord<kSt>(state + (r * 8 + j) * kSt, rec);
-        __syncthreads();
-        // lane (r, b) works on cell r, whose J^-1 the group holds
-        const double inv[3][3] = {{f.g[0], f.g[1], f.g[2]}, {f.g[3], f.g[4], f.g[5]}, {f.g[6], f.g[7], f.g[8]}};
-        PhaseBAffine<FULLDMG, kSt>(state, r, j, inv, acc);
-    }
-    else if constexpr (PRE)
-    {
-        double rec[kSt];
-        if (valid)
-            PreRecord<FULLDMG, kSt, true, DEC>(f.sr, f.g, la, j, P, rec, Rv);
-        {
-            // pass 0: IPs 0..3 (records of lanes j < 4)
-            if (valid && j < 4)
-                StoreRecord<kSt>(state + (r * 4 + j) * kSt, rec);
-            __syncthreads();
-            if (valid)
-                PhaseB<FULLDMG, kSt>(state, r, j, 0, 4, acc);
-            __syncthreads();
-            // pass 1: IPs 4..7; lanes j >= 4 rebuild their records from the (cached) state records
-            if (valid && j >= 4)
-            {
-                double g2[kGeo], sr2[kSrOf<DEC>], Rd[4];
-                LoadIpRecords<DEC>(T, f.cell, j, g2, sr2);
-                PreRecord<FULLDMG, kSt, true, DEC>(sr2, g2, la, j, P, rec, Rd);
-                StoreRecord<kSt>(state + (r * 4 + j - 4) * kSt, rec);
-            }
-            __syncthreads();
-            if (valid)
-                PhaseB<FULLDMG, kSt>(state, r, j, 4, 4, acc);
-        }
-    }
-    else
-    {
-        if (valid)
-        {
-            const int ip = j;
-            double Hu[3][3], he[3], eN;
-            GatherGradients(f.v, ip, Hu, he, eN);
-            const double inv[3][3] = {{f.g[0], f.g[1], f.g[2]}, {f.g[3], f.g[4], f.g[5]}, {f.g[6], f.g[7], f.g[8]}};
-            const double s = f.g[9];
-            GdmIp st;
-            GdmIpState<FULLDMG>(Hu, he, eN, inv, f.kh, m3K, m2G, k0, beta, P, st);
-            const double* sig = st.sig;
-            const double* dsw = st.dsw;
-            const double* ge = st.ge;
-            const double om = st.om, dom = st.dom, dk = st.dk, H = st.H, d2G = st.d2G, eq = st.eq;
-
-            double da[3], Na, ga[3];
-            ShapeAt(la, ip, da, Na);
-            GradOf(da, inv, ga);
-            if (WR)
-            {
-                double bt[3];
-                BTv3(ga, sig, bt);
-                Rv[0] = s * bt[0];
-                Rv[1] = s * bt[1];
-                Rv[2] = s * bt[2];
-                Rv[3] = s * (Na * (eN - eq) + P.c * (ga[0] * ge[0] + ga[1] * ge[1] + ga[2] * ge[2]));
-            }
-            {
-                double m[6];
-                GdmMisesDerivative(st, P, m);
-                double* rp = state + (r * 8 + ip) * kSt;
-                double rec[kSt];
-#pragma unroll
-                for (int a = 0; a < 3; a++)
-#pragma unroll
-                    for (int b = 0; b < 3; b++)
-                        rec[sInv + 3 * a + b] = inv[a][b];
-                const double ct = s * dom * dk;
-                double t6[6], va[3];
-#pragma unroll
-                for (int i = 0; i < 6; i++)
-                {
-                    t6[i] = ct * dsw[i];
-                    rec[sMn + i] = -Na * s * m[i];
-                }
-                BTv3(ga, t6, va);
-                const double c1 = FULLDMG ? s * (1.0 - om) : s * (m3K * (1.0 - om * H) - d2G) * kThird;
-#pragma unroll
-                for (int i = 0; i < 3; i++)
-                {
-                    rec[sHa + i] = c1 * ga[i];
-                    rec[sVa + i] = va[i];
-                    rec[sCg + i] = P.c * s * ga[i];
-                    if (!FULLDMG)
-                        rec[sKa + i] = 0.5 * s * d2G * ga[i];
-                }
-                rec[sSn] = s * Na;
-                if (FULLDMG)
-                    rec[25] = 0.0;
-                else
-                    rec[28] = rec[29] = 0.0;
-#pragma unroll
-                for (int k = 0; k < kSt; k += 2)
-                    *reinterpret_cast<double2*>(rp + k) = make_double2(rec[k], rec[k + 1]);
-            }
-        }
-    }
-    if constexpr (!PRE)
-    {
-        __syncthreads();
-        if (valid)
-            PhaseB<FULLDMG, kSt>(state, r, j, 0, 8, acc);
-    }
-    if ((valid || AFF) && FULLDMG)
-    {
-        // uu = lambda' S + mu' S^T + mu' tr(S) I
-        const double lam = (m3K - m2G) * kThird, mu = 0.5 * m2G;
-        const double S[3][3] = {{acc[0], acc[1], acc[2]}, {acc[4], acc[5], acc[6]}, {acc[8], acc[9], acc[10]}};
-        const double tr = S[0][0] + S[1][1] + S[2][2];
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int c = 0; c < 3; c++)
-            {
-                if (i == c)
-                    acc[i * 4 + c] = lam * S[i][c] + mu * S[c][i] + mu * tr;
-                else
-                    acc[i * 4 + c] = lam * S[i][c] + mu * S[c][i];
-            }
     }
     // R: per cell over its IPs (butterfly within the cell's 8 lanes), then over the cells in order
     if (WR)
     {
 #pragma unroll
         for (int k = 0; k < 4; k++)
-            Rv[k] = GroupSum0(Rv[k]);  // stored by lane j == 0
+            Rv[k] = GroupSum0(Rv[k]);  // stored by lane m == 0
     }
     __syncthreads();
 
-    // ---- partial blocks, R sums and the slot map to LDS (the records are dead now) ------------------
-    double* part = state;               // [r][b][kPs]
+    // ---- partial blocks, R sums and the slot map to LDS ----------------------------------------------
+    double* part = state;               // [r][m][kPs]
     double* rcell = state + 8 * 8 * kPs;  // [4][r]: R terms summed over the IPs of cell r
-    // slotOf[q][r] = local index b of neighbour q in cell r, 0xFF if q is not a node of cell r
+    // slotOf[q][r] = lane m of neighbour q in cell r, 0xFF if q is not a node of cell r
     unsigned char(*slotOf)[kMaxInc] = reinterpret_cast<unsigned char(*)[kMaxInc]>(rcell + 40);
     {
         reinterpret_cast<unsigned int*>(slotOf)[lane] = 0xFFFFFFFFu;  // 64 x 4 bytes = the whole map
@@ -851,7 +563,7 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
         for (int i = 0; i < 16; i++)
             part[lane * kPs + i] = acc[i];
     }
-    if (WR && j == 0)
+    if (WR && m == 0)
     {
 #pragma unroll
         for (int k = 0; k < 4; k++)
@@ -859,7 +571,7 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
     }
     __syncthreads();
     if (valid)
-        slotOf[f.slot][r] = (unsigned char)j;
+        slotOf[slot][r] = (unsigned char)m;
     __syncthreads();
 
     // ---- reduce: lane (q, half) sums its 8 block entries over the cells in order and writes them ----
@@ -926,7 +638,7 @@ template <bool WR, bool FULLDMG, int MODE, bool DEC>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE >= 1 ? 4 : 1)))
 kGdmHex8Node(const RowArgs A, const GdmHex8Tables T)
 {
-    __shared__ __align__(16) double state[NodeLds<FULLDMG, MODE>::kState];
+    __shared__ __align__(16) double state[gdm8::kRed];
     const int pos = NodeOfBlock(T);
     if (pos < 0)
         return;
@@ -947,13 +659,13 @@ __global__ void __launch_bounds__(64) kGdmHex8Ip(const RowArgs A, const GdmHex8T
     using namespace gdm8;
     constexpr int kN = kSrOf<DEC>;
     __shared__ __align__(16) double stage[64 * kN];  // the block's geometry, then its records
+    __shared__ double sE[64];  // eeq of the cells' nodes
     const int lane = threadIdx.x;
-    const int j = lane & 7, r = lane >> 3;
+    const int r = lane >> 3;
+    const CornerLane c = CornerOf(lane);
     const long long cell0 = (long long)blockIdx.x * 8;
     const int nc = (int)(A.nCells - cell0 < 8 ? A.nCells - cell0 : 8);  // cells of this block, >= 1
-    const bool valid = r < nc;  // uniform within each 8-lane group
-    const int cell = valid ? (int)(cell0 + r) : 0;
-    const LawParams& P = A.P;
+    const int cell = (int)cell0 + (r < nc ? r : 0);  // groups past the last cell repeat the first (not stored)
     {
         constexpr int kPerCell = AFF ? kGeo / 2 : 8 * kGeo / 2;  // 16-byte chunks of geometry per cell
         const double2* src =
@@ -962,32 +674,18 @@ __global__ void __launch_bounds__(64) kGdmHex8Ip(const RowArgs A, const GdmHex8T
 #pragma unroll
         for (int i = 0; i < (8 * kPerCell + 63) / 64; i++)
         {
-            const int c = lane + 64 * i;
-            if (c < nc * kPerCell)
-                dst[c] = src[c];
+            const int k = lane + 64 * i;
+            if (k < nc * kPerCell)
+                dst[k] = src[k];
         }
     }
-    double v[4] = {0.0, 0.0, 0.0, 0.0}, g[kGeo];
-    double kh = 0.0, E = P.E, k0 = P.kappa0, beta = P.beta;
-    if (valid)
-    {
-        const int q = A.dconn[(size_t)cell * 8 + j];
-        v[0] = A.u[(size_t)q * 3];
-        v[1] = A.u[(size_t)q * 3 + 1];
-        v[2] = A.u[(size_t)q * 3 + 2];
-        v[3] = A.e[q];
-        const int hist = A.cellId ? A.cellId[cell] : cell;
-        kh = A.kappa[(size_t)hist + (size_t)j * A.kappaLd];
-        if (A.thE)
-        {
-            E = A.thE[cell];
-            k0 = A.thFt[cell] / E;
-            beta = A.thFt[cell] / A.thGf[cell];
-        }
-    }
+    const int q = A.dconn[(size_t)cell * 8 + c.node];
+    const double v[4] = {A.u[(size_t)q * 3], A.u[(size_t)q * 3 + 1], A.u[(size_t)q * 3 + 2], A.e[q]};
+    sE[8 * r + c.node] = v[3];
     __syncthreads();
+    double g[kGeo];
     {
-        const double2* gs = reinterpret_cast<const double2*>(stage + (AFF ? r : r * 8 + j) * kGeo);
+        const double2* gs = reinterpret_cast<const double2*>(stage + (AFF ? r : r * 8 + c.ip) * kGeo);
 #pragma unroll
         for (int k = 0; k < kGeo / 2; k++)
         {
@@ -996,55 +694,18 @@ __global__ void __launch_bounds__(64) kGdmHex8Ip(const RowArgs A, const GdmHex8T
             g[2 * k + 1] = w.y;
         }
     }
-    double Hu[3][3], he[3], eN;
-    GatherGradients(v, j, Hu, he, eN);
+    const double inv[3][3] = {{g[0], g[1], g[2]}, {g[3], g[4], g[5]}, {g[6], g[7], g[8]}};
+    GdmIp st;
+    double m3K, m2G, rec[kN];
+    GdmCellState<FULLDMG>(A, c, cell, v, sE + 8 * r, inv, st, m3K, m2G);
+    StateRecord<FULLDMG, DEC>(st, g[9], m3K, m2G, A.P, rec);
     __syncthreads();  // the records overwrite the geometry
-    if (valid)
     {
-        const double inv[3][3] = {{g[0], g[1], g[2]}, {g[3], g[4], g[5]}, {g[6], g[7], g[8]}};
-        const double s = g[9];
-        const double m3K = P.cK * E, m2G = P.cG * E;
-        GdmIp st;
-        GdmIpState<FULLDMG>(Hu, he, eN, inv, kh, m3K, m2G, k0, beta, P, st);
-        const double eV = st.I1 * kThird;
-        const double sV = (1.0 - st.om * st.H) * m3K * eV;
-        double am = P.K1, bm = 0.0;  // m = am [1,1,1,0,0,0] + bm e'' (A == 0: m = K1 [1,1,1,0,0,0])
-        if (st.Am != 0.0)
-        {
-            const double h = 0.5 / st.Am;
-            am = P.K1 + h * (2.0 * P.K1 * P.K1 * st.I1) - h * P.K2 * st.I1 * kThird;
-            bm = h * P.K2;
-        }
-        const double ct = s * st.dom * st.dk;
-        double rec[kN];
-        rec[rEps] = st.eps[0];
-        rec[rEps + 1] = st.eps[1];
-        rec[rEps + 2] = st.eps[2];
-        rec[rEps + 3] = 0.5 * st.eps[3];
-        rec[rEps + 4] = 0.5 * st.eps[4];
-        rec[rEps + 5] = 0.5 * st.eps[5];
-        rec[rSig] = s * (sV - st.d2G * eV);
-        rec[rSig + 1] = s * st.d2G;
-        rec[rT] = -ct * (m3K * st.H - m2G) * eV;
-        rec[rT + 1] = -ct * m2G;
-        rec[rM] = s * am;
-        rec[rM + 1] = s * bm;
-        rec[rC1] = FULLDMG ? s * (1.0 - st.om) : s * (m3K * (1.0 - st.om * st.H) - st.d2G) * kThird;
-        rec[rC2] = FULLDMG ? 0.0 : 0.5 * s * st.d2G;
-        rec[rRe] = s * (st.eN - st.eq);
-        rec[rGe] = s * P.c * st.ge[0];
-        rec[rGe + 1] = s * P.c * st.ge[1];
-        rec[rGe + 2] = s * P.c * st.ge[2];
-        if constexpr (DEC)
-        {
-            double gi, dgi;
-            NonlocalFactor(P, st.om, gi, dgi);
-            rec[rGi] = gi;
-            rec[rDg] = dgi * st.dom * st.dk;
-            rec[kN - 2] = rec[kN - 1] = 0.0;
-        }
-        // record (r, j) at row r * 8 + j: 9 or 11 chunks (odd), consecutive lanes on distinct bank groups
-        StoreRecord<kN>(stage + lane * kN, rec);
+        // record (r, ip) at row r * 8 + ip: 9 or 11 chunks (odd), consecutive lanes on distinct bank groups
+        double* dst = stage + (r * 8 + c.ip) * kN;
+#pragma unroll
+        for (int k = 0; k < kN; k += 2)
+            *reinterpret_cast<double2*>(dst + k) = make_double2(rec[k], rec[k + 1]);
     }
     __syncthreads();
     {
@@ -1054,9 +715,9 @@ __global__ void __launch_bounds__(64) kGdmHex8Ip(const RowArgs A, const GdmHex8T
 #pragma unroll
         for (int i = 0; i < (8 * kPerCell + 63) / 64; i++)
         {
-            const int c = lane + 64 * i;
-            if (c < nc * kPerCell)
-                dst[c] = src[c];
+            const int k = lane + 64 * i;
+            if (k < nc * kPerCell)
+                dst[k] = src[k];
         }
     }
 }

@@ -27,7 +27,6 @@
 
 #include "cell_vectors.hpp"
 #include "gdm_hex8.hpp"
-#include "hex8_lanes.hpp"
 
 namespace nuto_amd
 {
@@ -104,41 +103,38 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
     const double inv[3][3] = {{g[0], g[1], g[2]}, {g[3], g[4], g[5]}, {g[6], g[7], g[8]}};
     const double s = g[9];
     const double m3K = P.cK * E, m2G = P.cG * E;
-
-    double Hu[3][3], he[3], eN, unused;
+    double inv0[3][3];  // J^-1 with the gradients' factor
 #pragma unroll
     for (int i = 0; i < 3; i++)
-        NodesToPoint(c, v[i], unused, Hu[i]);
-    NodesToPoint(c, v[3], unused, he);
-    // kappa' jumps where eeq meets the history, as it does at every loading point after an update: eeq is bit
-    // for bit the value that the update and the matrix kernels form (N_n from ShapeAt's products, the nodes
-    // added in order), so that all take the same side and a residual does not change with the update
-    {
-        const double near = 1.0 + kGauss, far = 1.0 - kGauss;
-        const double fx[2] = {c.hx < 0.0 ? near : far, c.hx < 0.0 ? far : near};
-        const double fy[2] = {c.hy < 0.0 ? near : far, c.hy < 0.0 ? far : near};
-        const double fz[2] = {c.hz < 0.0 ? near : far, c.hz < 0.0 ? far : near};
-        eN = 0.0;
 #pragma unroll
-        for (int n = 0; n < 8; n++)
-            eN = fma(0.125 * fx[((n + 1) >> 1) & 1] * fy[(n >> 1) & 1] * fz[n >> 2], sE[8 * r + n], eN);
-    }
+        for (int k = 0; k < 3; k++)
+            inv0[i][k] = kGradScale * inv[i][k];
+    double Hu[3][3], he[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+        NodesToPoint(c, v[i], Hu[i]);
+    NodesToPoint(c, v[3], he);
+    // kappa' jumps where eeq meets the history, as it does at every loading point after an update: eeq is bit
+    // for bit the value that the update and the matrix kernels form, so that all take the same side and a
+    // residual does not change with the update
+    const double eN = NodeSum(c, sE + 8 * r);
     GdmIp st;
-    GdmIpState<FULLDMG>(Hu, he, eN, inv, kh, m3K, m2G, k0, beta, P, st);
+    GdmIpState<FULLDMG>(Hu, he, eN, inv0, kh, m3K, m2G, k0, beta, P, st);
 
     double sig[6], grad[3], value;  // s times the stress-like, gradient-like and value terms
     if constexpr (ADJ)
     {
-        double Hl[3][3], hl[3], lN, m[6];
+        double Hl[3][3], hl[3], m[6];
 #pragma unroll
         for (int i = 0; i < 3; i++)
-            NodesToPoint(c, l[i], unused, Hl[i]);
-        NodesToPoint(c, l[3], lN, hl);
+            NodesToPoint(c, l[i], Hl[i]);
+        NodesToPoint(c, l[3], hl);
+        const double lN = kValueScale * NodesToValue(l[3]);
         GdmMisesDerivative(st, P, m);
         double Gl[3][3];
 #pragma unroll
         for (int i = 0; i < 3; i++)
-            GradOf(Hl[i], inv, Gl[i]);
+            GradOf(Hl[i], inv0, Gl[i]);
         const double el[6] = {Gl[0][0], Gl[1][1], Gl[2][2], Gl[1][2] + Gl[2][1], Gl[2][0] + Gl[0][2],
                               Gl[0][1] + Gl[1][0]};
         const double elV = (el[0] + el[1] + el[2]) * kThird;
@@ -151,7 +147,7 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
             dsel += st.dsw[i] * el[i];
             sgel += st.sig[i] * el[i];
         }
-        GradOf(hl, inv, grad);
+        GradOf(hl, inv0, grad);
 #pragma unroll
         for (int i = 0; i < 3; i++)
             grad[i] *= s * P.c;
@@ -199,13 +195,13 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
     {
 #pragma unroll
         for (int k = 0; k < 3; k++)
-            p[k] = S[i][0] * inv[k][0] + S[i][1] * inv[k][1] + S[i][2] * inv[k][2];
+            p[k] = S[i][0] * inv0[k][0] + S[i][1] * inv0[k][1] + S[i][2] * inv0[k][2];
         res[i] = PointsToNode<false>(c, p, 0.0);
     }
 #pragma unroll
     for (int k = 0; k < 3; k++)
-        p[k] = grad[0] * inv[k][0] + grad[1] * inv[k][1] + grad[2] * inv[k][2];
-    res[3] = PointsToNode<true>(c, p, value);
+        p[k] = grad[0] * inv0[k][0] + grad[1] * inv0[k][1] + grad[2] * inv0[k][2];
+    res[3] = PointsToNode<true>(c, p, kValueScale * value);
     if (valid)
     {
         double2* dst = reinterpret_cast<double2*>(out + ((size_t)cell * 8 + c.node) * 4);
