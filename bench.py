@@ -281,7 +281,7 @@ def batched(n_meshes, steps, warmup, form=-1, tune=True):
         counts[k] = counts.get(k, 0) + 1
     names = {N.TET4: "tet4", N.TET10: "tet10", N.HEX8: "hex8", N.HEX20: "hex20"}
     forms = {0: "columns", 1: "gram, 1 row node per lane", 2: "gram, 2 row nodes per lane",
-             3: "gram on the matrix cores (MFMA)", -1: "default"}
+             3: "gram on the matrix cores (MFMA)", 4: "node tiles", -1: "default"}
     kernels = []
     for g in range(b.group_info(0)["groups"]):
         gi = b.group_info(g)

@@ -142,12 +142,284 @@ __device__ inline void StrainOfGradient(const double* R, const double inv[3][3],
     eps[5] = H[0][1] + H[1][0];
 }
 
+// What the integration of a cell reads: the coordinates and node values, the material (E, kappa0 = f_t / E,
+// beta = f_t / G_f) and the history column
+template <int KIND, int DIM, int NNC, int NND>
+struct CellNodes
+{
+    double X[NNC][DIM];
+    double U[NND][DIM];
+    double EE[KIND == kGradientDamage ? NND : 1];
+    double E, k0, beta;
+    int id;
+};
+
+template <int KIND, int DIM, int NNC, int NND>
+__device__ inline void LoadCellNodes(const RowArgs& A, int cell, CellNodes<KIND, DIM, NNC, NND>& c)
+{
+#pragma unroll
+    for (int k = 0; k < NNC; k++)
+    {
+        const int n = A.cconn[(size_t)cell * NNC + k];
+        c.X[k][0] = A.x[n];
+        c.X[k][1] = A.y[n];
+        if constexpr (DIM == 3)
+            c.X[k][2] = A.z[n];
+    }
+#pragma unroll
+    for (int b = 0; b < NND; b++)
+    {
+        const int q = A.dconn[(size_t)cell * NND + b];
+#pragma unroll
+        for (int i = 0; i < DIM; i++)
+            c.U[b][i] = A.u[(size_t)q * DIM + i];
+        if constexpr (KIND == kGradientDamage)
+            c.EE[b] = A.e[q];
+    }
+    c.E = A.P.E;
+    c.k0 = A.P.kappa0;
+    c.beta = A.P.beta;
+    if (A.thE)
+    {
+        c.E = A.thE[cell];
+        c.k0 = A.thFt[cell] / c.E;
+        c.beta = A.thFt[cell] / A.thGf[cell];
+    }
+    c.id = A.cellId ? A.cellId[cell] : cell;
+}
+
+// Integrates the rows of local node la of a cell over its IPs (Cell.h:108-117): kacc[bb] += the block of
+// column node b0 + bb (NB of them), racc += the R entries (with the first column block only)
+template <int KIND, int DIM, int NNC, int NND, int NIP, int NB, bool WR, bool WK>
+__device__ inline void CellRows(const RowArgs& A, const CellNodes<KIND, DIM, NNC, NND>& c, int la, int b0,
+                                double (*kacc)[(KIND == kGradientDamage ? 4 : DIM) * (KIND == kGradientDamage ? 4 : DIM)],
+                                double* racc)
+{
+    constexpr int F = KIND == kGradientDamage ? 4 : DIM;
+    constexpr int S = 1 + NNC * DIM + NND + NND * DIM;
+    const LawParams& P = A.P;
+    const double E = c.E, k0 = c.k0, beta = c.beta;
+                for (int ip = 0; ip < NIP; ip++)
+                {
+                    const double* t = A.tab + ip * S;
+                    const double w = t[0];
+                    const double* dNc = t + 1;
+                    const double* Nd = dNc + NNC * DIM;
+                    const double* dNd = Nd + NND;
+                    double J[DIM][DIM];
+    #pragma unroll
+                    for (int i = 0; i < DIM; i++)
+    #pragma unroll
+                        for (int j = 0; j < DIM; j++)
+                        {
+                            double s = 0.0;
+    #pragma unroll
+                            for (int k = 0; k < NNC; k++)
+                                s += c.X[k][i] * dNc[k * DIM + j];
+                            J[i][j] = s;
+                        }
+                    double inv[DIM][DIM];
+                    const double detJ = Inverse<DIM>(J, inv);
+                    const double s = detJ * w;
+
+                    // strain (Voigt 2D [xx,yy,xy], 3D [xx,yy,zz,yz,zx,xy]), nonlocal value and gradient
+                    constexpr int NV = DIM == 2 ? 3 : 6;
+                    double eps[NV];
+    #pragma unroll
+                    for (int i = 0; i < NV; i++)
+                        eps[i] = 0.0;
+                    double eN = 0.0, ge[3] = {0.0, 0.0, 0.0};
+    #pragma unroll
+                    for (int b = 0; b < NND; b++)
+                    {
+                        double g[DIM];
+                        Grad<DIM, NND>(dNd, b, inv, g);
+                        AddStrain<DIM>(g, c.U[b], eps);
+                        if constexpr (KIND == kGradientDamage)
+                        {
+                            eN += Nd[b] * c.EE[b];
+                            ge[0] += g[0] * c.EE[b];
+                            ge[1] += g[1] * c.EE[b];
+                            ge[2] += g[2] * c.EE[b];
+                        }
+                    }
+
+                    // row node a
+                    double ga[DIM];
+                    Grad<DIM, NND>(dNd, la, inv, ga);
+                    const double Na = Nd[la];
+
+                    // material response -> per-IP coefficients
+                    double sig[NV];
+                    double c1 = 0.0, c2 = 0.0, cm = 0.0;  // uu: c1 ga gb^T + c2 gb ga^T + c2 (ga.gb) I
+                    double t6[6] = {0, 0, 0, 0, 0, 0}, m6[6] = {0, 0, 0, 0, 0, 0};
+                    double rE = 0.0, cq = 0.0;  // cq: s c dg/dw dw/dk dk/de (grad eeq . g_a), the K_ee term of g'
+                    double C11 = 0, C12 = 0, C33 = 0;
+                    if constexpr (KIND == kLinearElastic)
+                    {
+                        if constexpr (DIM == 2)
+                        {
+                            if (P.plane_state == 0)
+                            {
+                                const double f = E / (1.0 - P.nu * P.nu);
+                                C11 = f;
+                                C12 = f * P.nu;
+                                C33 = f * 0.5 * (1.0 - P.nu);
+                            }
+                            else
+                            {
+                                const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
+                                C11 = f * (1.0 - P.nu);
+                                C12 = f * P.nu;
+                                C33 = E / (2.0 * (1.0 + P.nu));
+                            }
+                            sig[0] = C11 * eps[0] + C12 * eps[1];
+                            sig[1] = C12 * eps[0] + C11 * eps[1];
+                            sig[2] = C33 * eps[2];
+                        }
+                        else
+                        {
+                            const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
+                            const double lam = f * P.nu, mu = E / (2.0 * (1.0 + P.nu));
+                            const double tr = eps[0] + eps[1] + eps[2];
+                            for (int i = 0; i < 3; i++)
+                                sig[i] = lam * tr + 2.0 * mu * eps[i];
+                            for (int i = 3; i < 6; i++)
+                                sig[i] = mu * eps[i];
+                            c1 = s * lam;
+                            c2 = s * mu;
+                        }
+                    }
+                    else
+                    {
+                        double mdev[6];
+                        const double eq = Mises3(eps, P.nu, P.k, mdev);
+                        const double kh = A.kappa[(size_t)c.id + (size_t)ip * A.kappaLd];
+                        double kap, dk;
+                        if constexpr (KIND == kGradientDamage)
+                        {
+                            kap = kh < eN ? eN : kh;
+                            dk = eN >= kh ? 1.0 : 0.0;
+                        }
+                        else
+                        {
+                            kap = eq < kh ? kh : eq;
+                            dk = eq >= kh ? 1.0 : 0.0;
+                        }
+                        double om, dom;
+                        DamageExp(kap, k0, beta, P.alpha, om, dom);
+                        DamageStress3 ds;
+                        ElasticDamage3(eps, om, E, P.nu, P.damage_application, ds);
+                        for (int i = 0; i < 6; i++)
+                            sig[i] = ds.sig[i];
+                        c1 = s * (ds.alpha_v - ds.alpha_d) / 3.0;
+                        c2 = s * 0.5 * ds.alpha_d;
+                        const double ct = s * dom * dk;
+                        // gradient damage: K_eu = -N_a (B_b^T m) s; local damage: s dom dk (B_a^T dsdw)(B_b^T m)^T
+                        const double cmv = KIND == kGradientDamage ? s : 1.0;
+                        for (int i = 0; i < 6; i++)
+                        {
+                            t6[i] = ct * ds.dsdw[i];
+                            m6[i] = cmv * mdev[i];
+                        }
+                        cm = P.c * s;
+                        if constexpr (KIND == kGradientDamage)
+                        {
+                            double gi, dgi;
+                            NonlocalFactor(P, om, gi, dgi);
+                            const double gdot = ga[0] * ge[0] + ga[1] * ge[1] + ga[2] * ge[2];
+                            rE = s * (Na * (eN - eq) + P.c * gi * gdot);
+                            cm *= gi;
+                            cq = s * P.c * gdot * dgi * dom * dk;
+                        }
+                    }
+
+                    if constexpr (WR)
+                    {
+                        if (b0 == 0)
+                        {
+                            if constexpr (DIM == 2)
+                            {
+                                racc[0] += s * (ga[0] * sig[0] + ga[1] * sig[2]);
+                                racc[1] += s * (ga[1] * sig[1] + ga[0] * sig[2]);
+                            }
+                            else
+                            {
+                                double bt[3];
+                                BTv3(ga, sig, bt);
+                                racc[0] += s * bt[0];
+                                racc[1] += s * bt[1];
+                                racc[2] += s * bt[2];
+                            }
+                            if constexpr (KIND == kGradientDamage)
+                                racc[3] += rE;
+                        }
+                    }
+
+                    if constexpr (WK)
+                    {
+                        double va[3] = {0, 0, 0};
+                        if constexpr (KIND != kLinearElastic)
+                            BTv3(ga, t6, va);
+    #pragma unroll
+                        for (int bb = 0; bb < NB; bb++)
+                        {
+                            const int b = b0 + bb;
+                            if (b >= NND)
+                                break;
+                            double gb[DIM];
+                            Grad<DIM, NND>(dNd, b, inv, gb);
+                            double* kb = kacc[bb];
+                            if constexpr (DIM == 2)
+                            {
+                                const double sa0 = s * ga[0], sa1 = s * ga[1];
+                                kb[0] += C11 * sa0 * gb[0] + C33 * sa1 * gb[1];
+                                kb[1] += C12 * sa0 * gb[1] + C33 * sa1 * gb[0];
+                                kb[2] += C12 * sa1 * gb[0] + C33 * sa0 * gb[1];
+                                kb[3] += C11 * sa1 * gb[1] + C33 * sa0 * gb[0];
+                            }
+                            else
+                            {
+                                const double dot = ga[0] * gb[0] + ga[1] * gb[1] + ga[2] * gb[2];
+    #pragma unroll
+                                for (int i = 0; i < 3; i++)
+    #pragma unroll
+                                    for (int j = 0; j < 3; j++)
+                                        kb[i * F + j] += c1 * ga[i] * gb[j] + c2 * gb[i] * ga[j] + (i == j ? c2 * dot : 0.0);
+                                if constexpr (KIND == kLocalDamage)
+                                {
+                                    double wb[3];
+                                    BTv3(gb, m6, wb);
+    #pragma unroll
+                                    for (int i = 0; i < 3; i++)
+    #pragma unroll
+                                        for (int j = 0; j < 3; j++)
+                                            kb[i * F + j] += va[i] * wb[j];
+                                }
+                                if constexpr (KIND == kGradientDamage)
+                                {
+                                    double wb[3];
+                                    BTv3(gb, m6, wb);
+                                    const double Nb = Nd[b];
+                                    kb[0 * 4 + 3] += va[0] * Nb;
+                                    kb[1 * 4 + 3] += va[1] * Nb;
+                                    kb[2 * 4 + 3] += va[2] * Nb;
+                                    kb[3 * 4 + 0] -= Na * wb[0];
+                                    kb[3 * 4 + 1] -= Na * wb[1];
+                                    kb[3 * 4 + 2] -= Na * wb[2];
+                                    kb[15] += s * Na * Nb + cm * dot + cq * Nb;
+                                }
+                            }
+                        }
+                    }
+                }
+}
+
 // Rows of dof node p (p < pEnd <= A.nNodes): one lane per node, incident cells in group order.
 template <int KIND, int DIM, int NNC, int NND, int NIP, int BH, bool WR, bool WK>
 __device__ inline void AssembleRowsBody(const RowArgs& A, int p, int pEnd)
 {
     constexpr int F = KIND == kGradientDamage ? 4 : DIM;
-    constexpr int S = 1 + NNC * DIM + NND + NND * DIM;
     if (p >= pEnd)
         return;
     const int beg = A.incPtr[p], end = A.incPtr[p + 1];
@@ -155,7 +427,6 @@ __device__ inline void AssembleRowsBody(const RowArgs& A, int p, int pEnd)
     const int L = nA * F;
     const int ru0 = WK ? A.rowPtr[p * DIM] : 0;
     const int re0 = (WK && KIND == kGradientDamage) ? A.rowPtr[A.nU + p] : 0;
-    const LawParams& P = A.P;
 
     double racc[F];
 #pragma unroll
@@ -166,37 +437,8 @@ __device__ inline void AssembleRowsBody(const RowArgs& A, int p, int pEnd)
     {
         const int cell = A.incCell[r];
         const int la = A.incLocal[r];
-        double X[NNC][DIM];
-#pragma unroll
-        for (int k = 0; k < NNC; k++)
-        {
-            const int n = A.cconn[(size_t)cell * NNC + k];
-            X[k][0] = A.x[n];
-            X[k][1] = A.y[n];
-            if constexpr (DIM == 3)
-                X[k][2] = A.z[n];
-        }
-        double U[NND][DIM];
-        double EE[KIND == kGradientDamage ? NND : 1];
-#pragma unroll
-        for (int b = 0; b < NND; b++)
-        {
-            const int q = A.dconn[(size_t)cell * NND + b];
-#pragma unroll
-            for (int c = 0; c < DIM; c++)
-                U[b][c] = A.u[(size_t)q * DIM + c];
-            if constexpr (KIND == kGradientDamage)
-                EE[b] = A.e[q];
-        }
-        double E = P.E, k0 = P.kappa0, beta = P.beta;
-        if (A.thE)
-        {
-            E = A.thE[cell];
-            k0 = A.thFt[cell] / E;
-            beta = A.thFt[cell] / A.thGf[cell];
-        }
-        const int cid = A.cellId ? A.cellId[cell] : cell;
-
+        CellNodes<KIND, DIM, NNC, NND> nodes;
+        LoadCellNodes<KIND, DIM, NNC, NND>(A, cell, nodes);
 #pragma unroll
         for (int b0 = 0; b0 < NND; b0 += BH)
         {
@@ -208,220 +450,7 @@ __device__ inline void AssembleRowsBody(const RowArgs& A, int p, int pEnd)
                 for (int i = 0; i < F * F; i++)
                     kacc[bb][i] = 0.0;
 
-            for (int ip = 0; ip < NIP; ip++)
-            {
-                const double* t = A.tab + ip * S;
-                const double w = t[0];
-                const double* dNc = t + 1;
-                const double* Nd = dNc + NNC * DIM;
-                const double* dNd = Nd + NND;
-                double J[DIM][DIM];
-#pragma unroll
-                for (int i = 0; i < DIM; i++)
-#pragma unroll
-                    for (int j = 0; j < DIM; j++)
-                    {
-                        double s = 0.0;
-#pragma unroll
-                        for (int k = 0; k < NNC; k++)
-                            s += X[k][i] * dNc[k * DIM + j];
-                        J[i][j] = s;
-                    }
-                double inv[DIM][DIM];
-                const double detJ = Inverse<DIM>(J, inv);
-                const double s = detJ * w;
-
-                // strain (Voigt 2D [xx,yy,xy], 3D [xx,yy,zz,yz,zx,xy]), nonlocal value and gradient
-                constexpr int NV = DIM == 2 ? 3 : 6;
-                double eps[NV];
-#pragma unroll
-                for (int i = 0; i < NV; i++)
-                    eps[i] = 0.0;
-                double eN = 0.0, ge[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-                for (int b = 0; b < NND; b++)
-                {
-                    double g[DIM];
-                    Grad<DIM, NND>(dNd, b, inv, g);
-                    AddStrain<DIM>(g, U[b], eps);
-                    if constexpr (KIND == kGradientDamage)
-                    {
-                        eN += Nd[b] * EE[b];
-                        ge[0] += g[0] * EE[b];
-                        ge[1] += g[1] * EE[b];
-                        ge[2] += g[2] * EE[b];
-                    }
-                }
-
-                // row node a
-                double ga[DIM];
-                Grad<DIM, NND>(dNd, la, inv, ga);
-                const double Na = Nd[la];
-
-                // material response -> per-IP coefficients
-                double sig[NV];
-                double c1 = 0.0, c2 = 0.0, cm = 0.0;  // uu: c1 ga gb^T + c2 gb ga^T + c2 (ga.gb) I
-                double t6[6] = {0, 0, 0, 0, 0, 0}, m6[6] = {0, 0, 0, 0, 0, 0};
-                double rE = 0.0, cq = 0.0;  // cq: s c dg/dw dw/dk dk/de (grad eeq . g_a), the K_ee term of g'
-                double C11 = 0, C12 = 0, C33 = 0;
-                if constexpr (KIND == kLinearElastic)
-                {
-                    if constexpr (DIM == 2)
-                    {
-                        if (P.plane_state == 0)
-                        {
-                            const double f = E / (1.0 - P.nu * P.nu);
-                            C11 = f;
-                            C12 = f * P.nu;
-                            C33 = f * 0.5 * (1.0 - P.nu);
-                        }
-                        else
-                        {
-                            const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
-                            C11 = f * (1.0 - P.nu);
-                            C12 = f * P.nu;
-                            C33 = E / (2.0 * (1.0 + P.nu));
-                        }
-                        sig[0] = C11 * eps[0] + C12 * eps[1];
-                        sig[1] = C12 * eps[0] + C11 * eps[1];
-                        sig[2] = C33 * eps[2];
-                    }
-                    else
-                    {
-                        const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
-                        const double lam = f * P.nu, mu = E / (2.0 * (1.0 + P.nu));
-                        const double tr = eps[0] + eps[1] + eps[2];
-                        for (int i = 0; i < 3; i++)
-                            sig[i] = lam * tr + 2.0 * mu * eps[i];
-                        for (int i = 3; i < 6; i++)
-                            sig[i] = mu * eps[i];
-                        c1 = s * lam;
-                        c2 = s * mu;
-                    }
-                }
-                else
-                {
-                    double mdev[6];
-                    const double eq = Mises3(eps, P.nu, P.k, mdev);
-                    const double kh = A.kappa[(size_t)cid + (size_t)ip * A.kappaLd];
-                    double kap, dk;
-                    if constexpr (KIND == kGradientDamage)
-                    {
-                        kap = kh < eN ? eN : kh;
-                        dk = eN >= kh ? 1.0 : 0.0;
-                    }
-                    else
-                    {
-                        kap = eq < kh ? kh : eq;
-                        dk = eq >= kh ? 1.0 : 0.0;
-                    }
-                    double om, dom;
-                    DamageExp(kap, k0, beta, P.alpha, om, dom);
-                    DamageStress3 ds;
-                    ElasticDamage3(eps, om, E, P.nu, P.damage_application, ds);
-                    for (int i = 0; i < 6; i++)
-                        sig[i] = ds.sig[i];
-                    c1 = s * (ds.alpha_v - ds.alpha_d) / 3.0;
-                    c2 = s * 0.5 * ds.alpha_d;
-                    const double ct = s * dom * dk;
-                    // gradient damage: K_eu = -N_a (B_b^T m) s; local damage: s dom dk (B_a^T dsdw)(B_b^T m)^T
-                    const double cmv = KIND == kGradientDamage ? s : 1.0;
-                    for (int i = 0; i < 6; i++)
-                    {
-                        t6[i] = ct * ds.dsdw[i];
-                        m6[i] = cmv * mdev[i];
-                    }
-                    cm = P.c * s;
-                    if constexpr (KIND == kGradientDamage)
-                    {
-                        double gi, dgi;
-                        NonlocalFactor(P, om, gi, dgi);
-                        const double gdot = ga[0] * ge[0] + ga[1] * ge[1] + ga[2] * ge[2];
-                        rE = s * (Na * (eN - eq) + P.c * gi * gdot);
-                        cm *= gi;
-                        cq = s * P.c * gdot * dgi * dom * dk;
-                    }
-                }
-
-                if constexpr (WR)
-                {
-                    if (b0 == 0)
-                    {
-                        if constexpr (DIM == 2)
-                        {
-                            racc[0] += s * (ga[0] * sig[0] + ga[1] * sig[2]);
-                            racc[1] += s * (ga[1] * sig[1] + ga[0] * sig[2]);
-                        }
-                        else
-                        {
-                            double bt[3];
-                            BTv3(ga, sig, bt);
-                            racc[0] += s * bt[0];
-                            racc[1] += s * bt[1];
-                            racc[2] += s * bt[2];
-                        }
-                        if constexpr (KIND == kGradientDamage)
-                            racc[3] += rE;
-                    }
-                }
-
-                if constexpr (WK)
-                {
-                    double va[3] = {0, 0, 0};
-                    if constexpr (KIND != kLinearElastic)
-                        BTv3(ga, t6, va);
-#pragma unroll
-                    for (int bb = 0; bb < NB; bb++)
-                    {
-                        const int b = b0 + bb;
-                        if (b >= NND)
-                            break;
-                        double gb[DIM];
-                        Grad<DIM, NND>(dNd, b, inv, gb);
-                        double* kb = kacc[bb];
-                        if constexpr (DIM == 2)
-                        {
-                            const double sa0 = s * ga[0], sa1 = s * ga[1];
-                            kb[0] += C11 * sa0 * gb[0] + C33 * sa1 * gb[1];
-                            kb[1] += C12 * sa0 * gb[1] + C33 * sa1 * gb[0];
-                            kb[2] += C12 * sa1 * gb[0] + C33 * sa0 * gb[1];
-                            kb[3] += C11 * sa1 * gb[1] + C33 * sa0 * gb[0];
-                        }
-                        else
-                        {
-                            const double dot = ga[0] * gb[0] + ga[1] * gb[1] + ga[2] * gb[2];
-#pragma unroll
-                            for (int i = 0; i < 3; i++)
-#pragma unroll
-                                for (int j = 0; j < 3; j++)
-                                    kb[i * F + j] += c1 * ga[i] * gb[j] + c2 * gb[i] * ga[j] + (i == j ? c2 * dot : 0.0);
-                            if constexpr (KIND == kLocalDamage)
-                            {
-                                double wb[3];
-                                BTv3(gb, m6, wb);
-#pragma unroll
-                                for (int i = 0; i < 3; i++)
-#pragma unroll
-                                    for (int j = 0; j < 3; j++)
-                                        kb[i * F + j] += va[i] * wb[j];
-                            }
-                            if constexpr (KIND == kGradientDamage)
-                            {
-                                double wb[3];
-                                BTv3(gb, m6, wb);
-                                const double Nb = Nd[b];
-                                kb[0 * 4 + 3] += va[0] * Nb;
-                                kb[1 * 4 + 3] += va[1] * Nb;
-                                kb[2 * 4 + 3] += va[2] * Nb;
-                                kb[3 * 4 + 0] -= Na * wb[0];
-                                kb[3 * 4 + 1] -= Na * wb[1];
-                                kb[3 * 4 + 2] -= Na * wb[2];
-                                kb[15] += s * Na * Nb + cm * dot + cq * Nb;
-                            }
-                        }
-                    }
-                }
-            }  // ip
+            CellRows<KIND, DIM, NNC, NND, NIP, NB, WR, WK>(A, nodes, la, b0, kacc, racc);
 
             if constexpr (WK)
             {

@@ -40,16 +40,12 @@
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-#include <cstdlib>
-#include <string>
 #include <vector>
 
 #include "assemble_rows.hpp"
-#include "devbuf.hpp"
+#include "gdm_plan.hpp"
 #include "hex8_lanes.hpp"
 #include "laws.hpp"
-#include "mesh.hpp"
 #include "morton.hpp"
 
 namespace nuto_amd
@@ -57,32 +53,6 @@ namespace nuto_amd
 
 namespace gdm8
 {
-constexpr int kMaxInc = 8;   // incident cells per node
-constexpr int kMaxAdj = 32;  // neighbours per node
-constexpr int kGeo = 10;     // doubles per (cell, IP) geometry record: J^-1 (row-major), detJ * w
-// per (cell, IP) state record of the pre-pass (kGdmHex8Ip): with e'' = [e0, e1, e2, e3/2, e4/2, e5/2]
-// (tensor strain) the stress, t = s omega' kappa' d sigma / d omega and m = d eps_eq / d eps are all
-// of the form alpha [1, 1, 1, 0, 0, 0] + beta e'', so B_a^T of each is alpha g_a + beta (e'' g_a)
-constexpr int kSr = 18;
-// with the decreasing nonlocal interaction two more, the factor g and g' omega' kappa' (padded to an odd
-// number of 16-byte chunks)
-template <bool DEC>
-constexpr int kSrOf = DEC ? 22 : kSr;
-constexpr int rGi = 18;   // g(omega)
-constexpr int rDg = 19;   // dg / d omega * d omega / d kappa * d kappa / d eeq
-constexpr int rEps = 0;   // e'' (6)
-constexpr int rSig = 6;   // s alpha_sigma, s beta_sigma
-constexpr int rT = 8;     // alpha_t, beta_t (s and kValueScale included)
-constexpr int rM = 10;    // s alpha_m, s beta_m (kGradScale included, as in the next two)
-constexpr int rC1 = 12;   // FULL: s (1 - omega); UNILATERAL: s (3K (1 - omega H) - 2G (1 - omega)) / 3
-constexpr int rC2 = 13;   // UNILATERAL: s G (1 - omega); FULL: 0
-constexpr int rRe = 14;   // s (eeq - eps_eq)
-constexpr int rGe = 15;   // s c grad eeq (3)
-constexpr int kPs = 17;      // doubles per partial block (odd: 64 lanes spread over the banks)
-constexpr int kTab = 57;     // per-IP table row: w, dNc[8][3], N[8], dNd[8][3]
-
-constexpr int kRed = 1160;  // doubles of the reduction: partial blocks 64 x kPs, R sums 32, 8 unused, slot map 32
-
 constexpr double kGauss = 0.57735026918962573;  // sqrt(1/3), the 2-point Gauss abscissa
 constexpr double kThird = 1.0 / 3.0;
 constexpr double kSixth = 1.0 / 6.0;
@@ -213,24 +183,6 @@ __device__ inline void GdmMisesDerivative(const GdmIp& o, const LawParams& P, do
     }
 }
 
-// Per-node tables of the node kernel (built once per pattern, see GdmHex8Plan::Prepare), stored in
-// traversal order: position s holds the node order[s] (nodes sorted along a Morton curve).
-struct GdmHex8Tables
-{
-    const int4* nodeHead;           // [pos]: node p, first CSR entry of its displacement rows, their
-                                    //        length 4 nA, first CSR entry of its eeq row
-    const int* nodeCell;            // [pos][8]: r-th incident cell (group order), -1 past the last
-    const int* nodeHist;            // [pos][8]: history column Cell::Id of that cell (nullptr: the cell index)
-    const unsigned char* nodeLa;    // [pos][8]: local index of the node in that cell
-    const unsigned char* nodeSlot;  // [pos][8][8]: neighbour slot (column block) of local node j
-    const double* geo;              // [cell][ip][kGeo] geometry records
-    const double* ipState;          // [cell][ip][kSrOf] pre-pass state records (nullptr: recompute)
-    const double* geoCell;          // [cell][kGeo] IP 0's geometry record (affine meshes, else nullptr)
-    int xcdMap;                     // 1: contiguous node ranges per XCD
-    int pBegin, pEnd;               // launch indices [pBegin, pEnd)
-    const int* order;               // launch index -> position (nullptr: the index is the position)
-};
-
 // Table position of this workgroup, -1 past the end. Workgroups are dispatched round-robin over the
 // 8 XCDs; with xcdMap, XCD x takes the x-th contiguous eighth of the traversal, which follows space
 // (Morton order), so the nodes one XCD works on at a time share their cells' records in its L2.
@@ -247,6 +199,57 @@ __device__ inline int NodeOfBlock(const GdmHex8Tables& T)
     if (i >= T.pEnd)
         return -1;
     return T.order ? T.order[i] : i;
+}
+
+// Table entries of lane (r, m) for the node at a position: its r-th cell (-1 past the last), its local index
+// there and the neighbour slot of node c.node of that cell
+struct NodeTab
+{
+    int cell, la, slot;
+};
+
+__device__ inline NodeTab LoadNodeTab(const GdmHex8Tables& T, int pos, int r, const CornerLane& c)
+{
+    const size_t pr = (size_t)pos * 8 + r;
+    return NodeTab{T.nodeCell[pr], T.nodeLa[pr], T.nodeSlot[pr * 8 + c.node]};
+}
+
+// Geometry and state record of the lane's cell at its IP, and the cell's E. Lanes past the node's last cell
+// take cell 0's: their blocks are never read and their R terms are zeroed.
+template <bool DEC>
+struct NodeRecord
+{
+    double g[gdm8::kGeo], sr[gdm8::kSrOf<DEC>], E;
+};
+
+template <bool PRE, bool AFF, bool DEC>
+__device__ inline void LoadNodeRecord(const RowArgs& A, const GdmHex8Tables& T, const NodeTab& tab, const CornerLane& c,
+                                      NodeRecord<DEC>& f)
+{
+    using namespace gdm8;
+    constexpr int kN = kSrOf<DEC>, kUse = DEC ? 20 : kSr;  // record stride, doubles read
+    const int cell = tab.cell < 0 ? 0 : tab.cell;
+    const double2* gr =
+        reinterpret_cast<const double2*>(AFF ? T.geoCell + (size_t)cell * kGeo : T.geo + ((size_t)cell * 8 + c.ip) * kGeo);
+#pragma unroll
+    for (int k = 0; k < kGeo / 2; k++)
+    {
+        const double2 v = gr[k];
+        f.g[2 * k] = v.x;
+        f.g[2 * k + 1] = v.y;
+    }
+    if constexpr (PRE)
+    {
+        const double2* sp = reinterpret_cast<const double2*>(T.ipState + ((size_t)cell * 8 + c.ip) * kN);
+#pragma unroll
+        for (int k = 0; k < kUse / 2; k++)
+        {
+            const double2 v = sp[k];
+            f.sr[2 * k] = v.x;
+            f.sr[2 * k + 1] = v.y;
+        }
+    }
+    f.E = A.thE ? A.thE[cell] : A.P.E;
 }
 
 // The pre-pass state record of an integration point (kSrOf doubles)
@@ -478,68 +481,42 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
 {
     using namespace gdm8;
     constexpr bool PRE = MODE >= 1, AFF = MODE == 2;
-    constexpr int kN = kSrOf<DEC>, kUse = DEC ? 20 : kSr;  // record stride, doubles read
     static_assert(PRE || !DEC, "the decreasing interaction needs the pre-pass");
 
     const int lane = threadIdx.x;
     const int r = lane >> 3, m = lane & 7;
     const CornerLane c = CornerOf(lane);
     const LawParams& P = A.P;
+    const NodeTab tab = LoadNodeTab(T, pos, r, c);
     // node p at table position pos; its rows: 3 displacement rows (consecutive in the CSR) and the
     // eeq row, each 4 nA long
     const int4 head = T.nodeHead[pos];
     const int p = head.x, ru0 = head.y, L = head.z, re0 = head.w;
     const int nA = L >> 2;
-    const size_t pr = (size_t)pos * 8 + r;
-    const int cellOr = T.nodeCell[pr];
-    const int la = T.nodeLa[pr];
-    const int slot = T.nodeSlot[pr * 8 + c.node];
-    const bool valid = cellOr >= 0;  // r < number of cells incident to p
-    // lanes past the node's last cell work on cell 0: their blocks are never read, their R terms are zeroed
-    const int cell = valid ? cellOr : 0;
+    const bool valid = tab.cell >= 0;  // r < number of cells incident to p
+    const int slot = tab.slot;
 
     double Rv[4] = {0.0, 0.0, 0.0, 0.0};
     double acc[16];
     if (A.nCells > 0)
     {
-        double g[kGeo], sr[kN], m3K, m2G;
+        NodeRecord<DEC> rec;
+        LoadNodeRecord<PRE, AFF, DEC>(A, T, tab, c, rec);
+        double m3K = P.cK * rec.E, m2G = P.cG * rec.E;
+        if constexpr (!PRE)
         {
-            const double2* gr = reinterpret_cast<const double2*>(AFF ? T.geoCell + (size_t)cell * kGeo
-                                                                     : T.geo + ((size_t)cell * 8 + c.ip) * kGeo);
-#pragma unroll
-            for (int k = 0; k < kGeo / 2; k++)
-            {
-                const double2 v = gr[k];
-                g[2 * k] = v.x;
-                g[2 * k + 1] = v.y;
-            }
-        }
-        if constexpr (PRE)
-        {
-            const double2* sp = reinterpret_cast<const double2*>(T.ipState + ((size_t)cell * 8 + c.ip) * kN);
-#pragma unroll
-            for (int k = 0; k < kUse / 2; k++)
-            {
-                const double2 v = sp[k];
-                sr[2 * k] = v.x;
-                sr[2 * k + 1] = v.y;
-            }
-            const double E = A.thE ? A.thE[cell] : P.E;
-            m3K = P.cK * E;
-            m2G = P.cG * E;
-        }
-        else
-        {
+            const int cell = valid ? tab.cell : 0;
             const int q = A.dconn[(size_t)cell * 8 + c.node];
             const double v[4] = {A.u[(size_t)q * 3], A.u[(size_t)q * 3 + 1], A.u[(size_t)q * 3 + 2], A.e[q]};
             state[8 * r + c.node] = v[3];
             __syncthreads();
+            const double* g = rec.g;
             const double inv[3][3] = {{g[0], g[1], g[2]}, {g[3], g[4], g[5]}, {g[6], g[7], g[8]}};
             GdmIp st;
             GdmCellState<FULLDMG>(A, c, cell, v, state + 8 * r, inv, st, m3K, m2G);
-            StateRecord<FULLDMG, DEC>(st, g[9], m3K, m2G, P, sr);
+            StateRecord<FULLDMG, DEC>(st, g[9], m3K, m2G, P, rec.sr);
         }
-        CellBlock<FULLDMG, AFF, DEC>(c, sr, g, la, m3K, m2G, P, acc, Rv);
+        CellBlock<FULLDMG, AFF, DEC>(c, rec.sr, rec.g, tab.la, m3K, m2G, P, acc, Rv);
         if (!valid)
             Rv[0] = Rv[1] = Rv[2] = Rv[3] = 0.0;
     }
@@ -554,9 +531,9 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
 
     // ---- partial blocks, R sums and the slot map to LDS ----------------------------------------------
     double* part = state;               // [r][m][kPs]
-    double* rcell = state + 8 * 8 * kPs;  // [4][r]: R terms summed over the IPs of cell r
-    // slotOf[q][r] = lane m of neighbour q in cell r, 0xFF if q is not a node of cell r
-    unsigned char(*slotOf)[kMaxInc] = reinterpret_cast<unsigned char(*)[kMaxInc]>(rcell + 40);
+    double* rcell = state + 64 * kPs;  // [4][r]: R terms summed over the IPs of cell r
+    // slotOf[q][r] = lane of neighbour q in cell r, 0xFF if q is not a node of cell r
+    unsigned char(*slotOf)[kMaxInc] = reinterpret_cast<unsigned char(*)[kMaxInc]>(rcell + 32);
     {
         reinterpret_cast<unsigned int*>(slotOf)[lane] = 0xFFFFFFFFu;  // 64 x 4 bytes = the whole map
 #pragma unroll
@@ -571,7 +548,7 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
     }
     __syncthreads();
     if (valid)
-        slotOf[slot][r] = (unsigned char)m;
+        slotOf[slot][r] = (unsigned char)lane;
     __syncthreads();
 
     // ---- reduce: lane (q, half) sums its 8 block entries over the cells in order and writes them ----
@@ -593,7 +570,7 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
                 const unsigned b = (unsigned)(row >> (8 * rr)) & 0xFFu;
                 if (b != 0xFFu)
                 {
-                    const double* src = part + (rr * 8 + (int)b) * kPs + h * 8;
+                    const double* src = part + (int)b * kPs + h * 8;
 #pragma unroll
                     for (int k = 0; k < 8; k++)
                         sum[k] += src[k];
@@ -817,313 +794,5 @@ inline hipError_t MortonOrder(const NodeGraph& g, int nCells, int nCoord, const 
     MortonSort(n, 3, pts.data(), order, valid.data());
     return hipSuccess;
 }
-
-struct GdmHex8Plan
-{
-    bool ready = false;
-    int nNodes = 0;
-    int grid = 0;     // workgroups: one per node (rounded up to a multiple of 8 with the XCD mapping)
-    int xcdMap = 1;   // contiguous node ranges per XCD (env NUTO_AMD_GDM_XCD_MAP=0 switches it off)
-    DevBuf nodeHead, nodeCell, nodeHist, nodeLa, nodeSlot, geo;
-    DevBuf posOf;        // node -> table position (Morton order; NUTO_AMD_GDM_ORDER=0: node order, empty)
-    DevBuf ipState;      // pre-pass state records, or cell vectors (Work)
-    DevBuf geoCell;      // affine meshes: IP 0's geometry record per cell
-    DevBuf extra;        // nodes beyond the kernel's bounds (more than 8 cells or 32 neighbours)
-    int nExtra = 0;      // ... assembled by the generic row-owner kernel
-    bool prepass = true;
-    bool affine = false;  // every cell affine: MODE 2 of the node kernel
-    bool decreasing = false;  // NonlocalInteraction::Decreasing: longer pre-pass records
-    int nCells = 0;
-
-    void Release()
-    {
-        ready = false;
-        nNodes = 0;
-        for (DevBuf* b : {&nodeHead, &nodeCell, &nodeHist, &nodeLa, &nodeSlot, &geo, &ipState, &posOf, &geoCell, &extra})
-            b->Release();
-        nExtra = 0;
-    }
-
-    bool Usable(int kind, int coordType, int dofType, int nip) const
-    {
-        return ready && kind == kGradientDamage && coordType == kHex8 && dofType == kHex8 && nip == 8;
-    }
-
-    // Builds the per-node tables from the node graph and the geometry records from the device
-    // coordinates (x, y, z by coordinate node, cconn) and the IP table. Returns false (plan not
-    // used) when the mesh exceeds the kernel's bounds; a HIP failure is returned through `err`.
-    bool Prepare(int kind, int coordType, int dofType, int nip, const NodeGraph& g, int nCells, const int* cellIds,
-                 int nCoord, const double* x, const double* y, const double* z, const int* cconn, const double* tab,
-                 const int* rowPtr, int nRows, bool decreasingInteraction, hipStream_t stream, hipError_t& err)
-    {
-        Release();
-        err = hipSuccess;
-        if (kind != kGradientDamage || coordType != kHex8 || dofType != kHex8 || nip != 8)
-            return false;
-        const int n = g.nNodes;
-        if (nRows != 4 * n)  // 3 displacement rows and 1 eeq row per node
-            return false;
-        // nodes beyond the kernel's bounds stay out of the tables (the generic kernel assembles them)
-        std::vector<char> out(n, 0);
-        std::vector<int> extraNodes;
-        for (int p = 0; p < n; p++)
-        {
-            if (g.incPtr[p + 1] - g.incPtr[p] > gdm8::kMaxInc || g.adjPtr[p + 1] - g.adjPtr[p] > gdm8::kMaxAdj)
-            {
-                out[p] = 1;
-                extraNodes.push_back(p);
-            }
-        }
-        if (n > 0 && (int)extraNodes.size() == n)
-            return false;
-        // traversal order: position s holds node ord[s]
-        std::vector<int> ord(n);
-        bool reordered = false;
-        const char* ordEnv = std::getenv("NUTO_AMD_GDM_ORDER");
-        if (n > 0 && nCells > 0 && !(ordEnv && ordEnv[0] == '0'))
-        {
-            if ((err = MortonOrder(g, nCells, nCoord, x, y, z, cconn, stream, ord)) != hipSuccess)
-                return false;
-            reordered = true;
-        }
-        else
-        {
-            for (int s = 0; s < n; s++)
-                ord[s] = s;
-        }
-        if (!extraNodes.empty())
-        {
-            // drop the outside nodes from the traversal; they keep position -1
-            ord.erase(std::remove_if(ord.begin(), ord.end(), [&](int p) { return out[p] != 0; }), ord.end());
-            reordered = true;
-        }
-        const int nIn = (int)ord.size();
-        // CSR rows: displacement rows 3p .. 3p + 2, eeq row 3n + p
-        std::vector<int> rp((size_t)4 * n + 1);
-        if ((err = hipMemcpyAsync(rp.data(), rowPtr, rp.size() * sizeof(int), hipMemcpyDeviceToHost, stream)) !=
-                hipSuccess ||
-            (err = hipStreamSynchronize(stream)) != hipSuccess)
-            return false;
-        std::vector<int4> head(nIn);
-        std::vector<int> cell((size_t)nIn * 8, -1), hist(cellIds ? (size_t)nIn * 8 : 0, 0), pos(reordered ? n : 0, -1);
-        std::vector<unsigned char> la((size_t)nIn * 8, 0), slot((size_t)nIn * 64, 0);
-        for (int s = 0; s < nIn; s++)
-        {
-            const int p = ord[s];
-            head[s] = make_int4(p, rp[(size_t)3 * p], rp[(size_t)3 * p + 1] - rp[(size_t)3 * p], rp[(size_t)3 * n + p]);
-            if (reordered)
-                pos[p] = s;
-            for (int k = g.incPtr[p], r = 0; k < g.incPtr[p + 1]; k++, r++)
-            {
-                const size_t pr = (size_t)s * 8 + r;
-                cell[pr] = g.incCell[k];
-                la[pr] = g.incLocal[k];
-                if (cellIds)
-                    hist[pr] = cellIds[g.incCell[k]];
-                for (int j = 0; j < 8; j++)
-                    slot[pr * 8 + j] = (unsigned char)(g.slot[(size_t)k * 8 + j] & 0x7fff);
-            }
-        }
-        if ((err = nodeHead.Upload(head.data(), head.size() * sizeof(int4), stream)) != hipSuccess ||
-            (reordered && (err = posOf.Upload(pos.data(), pos.size() * sizeof(int), stream)) != hipSuccess) ||
-            (err = nodeCell.Upload(cell.data(), cell.size() * sizeof(int), stream)) != hipSuccess ||
-            (err = nodeLa.Upload(la.data(), la.size(), stream)) != hipSuccess ||
-            (!extraNodes.empty() &&
-             (err = extra.Upload(extraNodes.data(), extraNodes.size() * sizeof(int), stream)) != hipSuccess) ||
-            (err = nodeSlot.Upload(slot.data(), slot.size(), stream)) != hipSuccess ||
-            (cellIds && (err = nodeHist.Upload(hist.data(), hist.size() * sizeof(int), stream)) != hipSuccess) ||
-            (err = geo.Alloc((size_t)nCells * 8 * gdm8::kGeo * sizeof(double))) != hipSuccess)
-        {
-            Release();
-            return false;
-        }
-        if (nCells > 0)
-        {
-            const long long items = (long long)nCells * 8;
-            hipLaunchKernelGGL(kGdmHex8Geometry, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream, x, y,
-                               z, cconn, tab, nCells, geo.As<double>());
-            if ((err = hipGetLastError()) != hipSuccess || (err = hipStreamSynchronize(stream)) != hipSuccess)
-            {
-                Release();
-                return false;
-            }
-        }
-        const char* pre = std::getenv("NUTO_AMD_GDM_PREPASS");
-        prepass = !(pre && pre[0] == '0');
-        const char* aff = std::getenv("NUTO_AMD_GDM_AFFINE");
-        affine = false;
-        if (prepass && nCells > 0 && !(aff && aff[0] == '0'))
-        {
-            DevBuf cnt;
-            int h = -1;
-            if ((err = cnt.Alloc(sizeof(int))) != hipSuccess ||
-                (err = hipMemsetAsync(cnt.p, 0, sizeof(int), stream)) != hipSuccess)
-            {
-                Release();
-                return false;
-            }
-            hipLaunchKernelGGL(kGdmHex8CountNonAffine, dim3((unsigned)((nCells + 255) / 256)), dim3(256), 0, stream,
-                               geo.As<double>(), nCells, cnt.As<int>());
-            if ((err = hipGetLastError()) != hipSuccess ||
-                (err = hipMemcpyAsync(&h, cnt.p, sizeof(int), hipMemcpyDeviceToHost, stream)) != hipSuccess ||
-                (err = hipStreamSynchronize(stream)) != hipSuccess)
-            {
-                Release();
-                return false;
-            }
-            affine = h == 0;
-            if (affine && ((err = geoCell.Alloc((size_t)nCells * gdm8::kGeo * sizeof(double))) != hipSuccess ||
-                           (err = hipMemcpy2DAsync(geoCell.p, gdm8::kGeo * sizeof(double), geo.p,
-                                                   8 * gdm8::kGeo * sizeof(double), gdm8::kGeo * sizeof(double),
-                                                   nCells, hipMemcpyDeviceToDevice, stream)) != hipSuccess ||
-                           (err = hipStreamSynchronize(stream)) != hipSuccess))
-            {
-                Release();
-                return false;
-            }
-        }
-        decreasing = decreasingInteraction;
-        if ((err = ipState.Alloc((size_t)nCells * 8 * RecordDoubles() * sizeof(double))) != hipSuccess)
-        {
-            Release();
-            return false;
-        }
-        this->nCells = nCells;
-        nNodes = nIn;
-        nExtra = (int)extraNodes.size();
-        const char* env = std::getenv("NUTO_AMD_GDM_XCD_MAP");
-        xcdMap = env ? std::atoi(env) : 1;
-        grid = xcdMap ? (nNodes + 7) / 8 * 8 : nNodes;
-        ready = true;
-        return true;
-    }
-
-    GdmHex8Tables Tables() const
-    {
-        return GdmHex8Tables{nodeHead.As<int4>(), nodeCell.As<int>(), nodeHist.p ? nodeHist.As<int>() : nullptr,
-                             nodeLa.As<unsigned char>(), nodeSlot.As<unsigned char>(), geo.As<double>(),
-                             ipState.p ? ipState.As<double>() : nullptr, geoCell.p ? geoCell.As<double>() : nullptr,
-                             xcdMap, 0, nNodes, nullptr};
-    }
-
-    template <bool FULLDMG, int MODE, bool DEC>
-    void LaunchNodes(const RowArgs& a, const GdmHex8Tables& t, bool wr, int grid_, hipStream_t stream)
-    {
-        if (wr)
-            hipLaunchKernelGGL((kGdmHex8Node<true, FULLDMG, MODE, DEC>), dim3(grid_), dim3(64), 0, stream, a, t);
-        else
-            hipLaunchKernelGGL((kGdmHex8Node<false, FULLDMG, MODE, DEC>), dim3(grid_), dim3(64), 0, stream, a, t);
-    }
-
-    // doubles of a pre-pass record
-    int RecordDoubles() const
-    {
-        return decreasing ? gdm8::kSrOf<true> : gdm8::kSrOf<false>;
-    }
-
-    // doubles of the pre-pass state records (written in full by kGdmHex8Ip before the node kernel reads them)
-    size_t StateDoubles() const
-    {
-        return prepass ? (size_t)nCells * 8 * RecordDoubles() : 0;
-    }
-
-    template <bool FULLDMG, bool DEC>
-    void LaunchT(const RowArgs& a, bool wr, double* state, hipStream_t stream)
-    {
-        GdmHex8Tables t = Tables();
-        t.ipState = state;
-        const dim3 ipGrid((unsigned)(((long long)nCells * 8 + 63) / 64));
-        if (affine)
-        {
-            if (nCells > 0)
-                hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, true, DEC>), ipGrid, dim3(64), 0, stream, a, t, state);
-            LaunchNodes<FULLDMG, 2, DEC>(a, t, wr, grid, stream);
-        }
-        else
-        {
-            if (nCells > 0)
-                hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, false, DEC>), ipGrid, dim3(64), 0, stream, a, t, state);
-            LaunchNodes<FULLDMG, 1, DEC>(a, t, wr, grid, stream);
-        }
-    }
-
-    // the matrix of the plan's interaction can be assembled by the node kernel
-    bool Matrix() const
-    {
-        return prepass || !decreasing;
-    }
-
-    // K (and R, wr). state: device memory of StateDoubles() doubles for the pre-pass records (nullptr: the
-    // plan's own)
-    void Launch(const RowArgs& a, bool wr, hipStream_t stream, double* state = nullptr)
-    {
-        if (nNodes > 0)
-        {
-            if (!state)
-                state = Work();
-            const bool full = a.P.damage_application == 0;
-            if (!prepass)
-            {
-                if (full)
-                    LaunchNodes<true, 0, false>(a, Tables(), wr, grid, stream);
-                else
-                    LaunchNodes<false, 0, false>(a, Tables(), wr, grid, stream);
-            }
-            else if (decreasing)
-            {
-                if (full)
-                    LaunchT<true, true>(a, wr, state, stream);
-                else
-                    LaunchT<false, true>(a, wr, state, stream);
-            }
-            else if (full)
-                LaunchT<true, false>(a, wr, state, stream);
-            else
-                LaunchT<false, false>(a, wr, state, stream);
-        }
-        LaunchExtras(a, wr, stream);
-    }
-
-    // The plan's device memory: the pre-pass records of a matrix assembly (StateDoubles), or the cell
-    // vectors of a residual or an adjoint (32 doubles per cell, less than the records)
-    double* Work() const
-    {
-        return ipState.As<double>();
-    }
-
-    // K (and R) rows of the nodes beyond the node kernel's bounds (the generic row-owner body)
-    void LaunchExtras(const RowArgs& a, bool wr, hipStream_t stream)
-    {
-        if (nExtra > 0)
-        {
-            const dim3 grid((unsigned)((nExtra + 63) / 64));
-            const int* list = extra.As<int>();
-            if (wr)
-                hipLaunchKernelGGL((kAssembleRowsList<kGradientDamage, 3, 8, 8, 8, 4, true, true>), grid, dim3(64), 0,
-                                   stream, a, list, nExtra);
-            else
-                hipLaunchKernelGGL((kAssembleRowsList<kGradientDamage, 3, 8, 8, 8, 4, false, true>), grid, dim3(64), 0,
-                                   stream, a, list, nExtra);
-        }
-    }
-
-    // R + K of the nodes [first, end) only (one mesh of a batch), plain block order; the nodes beyond
-    // the bounds are not visited (LaunchExtras covers them for the whole plan)
-    void LaunchRange(const RowArgs& a, int first, int end, hipStream_t stream)
-    {
-        if (end <= first)
-            return;
-        GdmHex8Tables t = Tables();
-        t.xcdMap = 0;
-        t.pBegin = first;
-        t.pEnd = end;
-        t.order = posOf.p ? posOf.As<int>() : nullptr;  // launch index = node
-        // per-mesh launches recompute the IP state in the node kernel (no pre-pass over the mesh's cells)
-        if (a.P.damage_application == 0)
-            LaunchNodes<true, 0, false>(a, t, true, end - first, stream);
-        else
-            LaunchNodes<false, 0, false>(a, t, true, end - first, stream);
-    }
-};
 
 }  // namespace nuto_amd

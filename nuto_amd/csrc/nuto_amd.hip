@@ -16,8 +16,8 @@
 #include "../../include/nuto_amd.h"
 #include "assemble_rows.hpp"
 #include "elements.hpp"
-#include "gdm_hex8.hpp"
-#include "gdm_hex8_vectors.hpp"
+#include "gdm_plan.hpp"
+#include "node_tiles.hpp"
 #include "batch.hpp"
 #include "cell_fields.hpp"
 #include "cell_gram.hpp"
@@ -71,7 +71,6 @@ struct nuto_ctx
     bool cellsSet = false;
     int coordType = 0, dim = 0, nCells = 0, nCoordNodes = 0;
     DevBuf x, y, z, cconn, cellId;
-    std::vector<int> hcellId;  // host copy of the cell ids (pattern-time tables)
     bool hasCellIds = false;
     int maxCellId = 0;
     Field f[2];
@@ -120,8 +119,9 @@ struct nuto_ctx
     // staged cell matrices and vectors of the two-phase generic assembly
     DevBuf keStage, reStage;
     int maxAdj = -1;  // largest node neighbourhood (LDS rows of the wave gather), from the node graph
-    int cellGram = -1;  // cell-matrix kernel of the two-phase assembly: 0 by columns, 1 / 2 Gram form with 1 / 2
-                        // row nodes per lane, 3 Gram form on the matrix cores, -1 the element's default
+    long long maxWindow = -1;  // most neighbours of kTileNodes consecutive dof nodes (LDS of kNodeTile)
+    int cellGram = -1;  // form of the 3D matrix assembly: 0 cell matrices by columns, 1 / 2 in Gram form with 1 / 2
+                        // row nodes per lane, 3 on the matrix cores, 4 node tiles (tet4), -1 the element's default
 };
 
 namespace
@@ -241,7 +241,10 @@ void InvalidatePattern(nuto_ctx* ctx)
     ctx->gdmTried = false;
     ctx->consBuilt = false;
     ctx->maxAdj = -1;
+    ctx->maxWindow = -1;
 }
+
+size_t TileLds(nuto_ctx* ctx);
 
 // Staging of the cells' vectors (every dof of every cell); false when it cannot be allocated (the error
 // state is cleared). It only grows: two-phase matrix assemblies stage their vectors there too.
@@ -388,13 +391,44 @@ bool TryStage(nuto_ctx* ctx, int nd, long long cells)
 
 // Two-phase assembly of the cells [c0, c1) and the rows of the dof nodes [p0, p1) (the rows'
 // incident cells must lie in [c0, c1): a whole mesh of a batch, or the whole group).
-// NUTO_AMD_CELL_GRAM=0 / 1 / 2 / 3 forces the cell-matrix form of every two-phase launch: by columns
+// NUTO_AMD_CELL_GRAM=0 / 1 / 2 / 3 / 4 forces the form of every 3D matrix launch: cell matrices by columns
 // (kCellMatrices), Gram form with one or two row nodes per lane (kCellGram), Gram form on the
-// matrix cores (kCellMfma); -1 when unset
+// matrix cores (kCellMfma), node tiles (kNodeTile, tet4); -1 when unset
 int CellFormEnv()
 {
     const char* v = std::getenv("NUTO_AMD_CELL_GRAM");
-    return v && v[0] >= '0' && v[0] <= '3' ? v[0] - '0' : -1;
+    return v && v[0] >= '0' && v[0] <= '4' ? v[0] - '0' : -1;
+}
+
+// LDS of kNodeTile for any launch over the context's nodes: the rows of the kTileNodes consecutive nodes
+// with the most neighbours
+size_t TileLds(nuto_ctx* ctx)
+{
+    if (ctx->maxWindow < 0)
+    {
+        const std::vector<int>& ptr = ctx->graph.adjPtr;
+        long long m = 0;
+        for (int p = 0; p < ctx->graph.nNodes; p++)
+            m = std::max<long long>(m, (long long)ptr[std::min(p + kTileNodes, ctx->graph.nNodes)] - ptr[p]);
+        ctx->maxWindow = m;
+    }
+    return (size_t)ctx->maxWindow * ctx->dim * ctx->dim * sizeof(double);
+}
+
+// Rows of the nodes [p0, p1) by node tiles; false when a tile's rows do not fit in LDS
+template <int KIND, int DIM, int NNC, int NND, int NIP>
+bool LaunchTiles(nuto_ctx* ctx, const RowArgs& a, bool wr, int p0, int p1, hipStream_t stream)
+{
+    const size_t lds = TileLds(ctx);
+    if (lds > kTileMaxLds)
+        return false;
+    const dim3 grid((unsigned)((p1 - p0 + kTileNodes - 1) / kTileNodes));
+    if (wr)
+        hipLaunchKernelGGL((kNodeTile<KIND, DIM, NNC, NND, NIP, true>), grid, dim3(64), lds, stream, a, p0, p1);
+    else
+        hipLaunchKernelGGL((kNodeTile<KIND, DIM, NNC, NND, NIP, false>), grid, dim3(64), lds, stream, a, p0, p1);
+    Check(hipGetLastError(), "node tile launch");
+    return true;
 }
 
 // kCellGram's shape per element and row nodes per lane (AP): cells per workgroup, threads, IPs per
@@ -453,9 +487,10 @@ void LaunchGram(const RowArgs& a, int c0, int c1, double* ke, double* re, hipStr
 }
 
 // form: 0 by columns (kCellMatrices), 1 Gram form with one row node per lane, 2 with two (four
-// accumulated blocks per lane), 3 Gram form on the matrix cores (kCellMfma). UNILATERAL damage
-// application, which needs a second Gram, runs forms 2 and 3 as 1.
-constexpr int kCellForms = 4;
+// accumulated blocks per lane), 3 Gram form on the matrix cores (kCellMfma); 4, where node tiles are not
+// provided or do not fit, as 1. UNILATERAL damage application, which needs a second Gram, runs forms 2
+// and 3 as 1.
+constexpr int kCellForms = 5;
 template <int KIND, int NNC, int NND, int NIP>
 void LaunchCellMatrices(const RowArgs& a, int form, int c0, int c1, double* ke, double* re, hipStream_t stream)
 {
@@ -484,13 +519,18 @@ void LaunchTwoPhaseT(nuto_ctx* ctx, const RowArgs& a, bool wr, int c0, int c1, i
     constexpr int ND = NND * 3;
     if (c1 <= c0 || p1 <= p0)
         return;
+    // the Gram form wins on the hexahedra (32 and 200 lanes per cell), the column kernel on the ten-node
+    // tetrahedra, node tiles on the four-node ones (a batch's autotune measures every form)
+    const int env = CellFormEnv();
+    const int form = env >= 0 ? env : (ctx->cellGram >= 0 ? ctx->cellGram : (NND == 4 ? 4 : (NND == 10 ? 0 : 1)));
+    if constexpr (NND == 4)
+    {
+        if (form == 4 && LaunchTiles<KIND, 3, NNC, NND, NIP>(ctx, a, wr, p0, p1, stream))
+            return;
+    }
     EnsureStage(ctx, ND, c1 - c0);  // cell c's matrix at staging position c - c0
     double* ke = ctx->keStage.As<double>();
     double* re = ctx->reStage.As<double>();
-    // the Gram form wins on the hexahedra (32 and 200 lanes per cell); the column kernel is as fast or
-    // faster on the tetrahedra, whose cell matrices are small (a batch's autotune measures every form)
-    const int env = CellFormEnv();
-    const int form = env >= 0 ? env : (ctx->cellGram >= 0 ? ctx->cellGram : (NND >= 8 ? 1 : 0));
     LaunchCellMatrices<KIND, NNC, NND, NIP>(a, form, c0, c1, ke, re, stream);
     if (ctx->maxAdj < 0)
     {
@@ -548,6 +588,15 @@ void LaunchRowsT(nuto_ctx* ctx, const RowArgs& a, bool wr, bool wk)
         Check(hipGetLastError(), "vector assembly launch");
         SyncCheck(ctx, "vector assembly");
         return;
+    }
+    if constexpr (DIM == 2)
+    {
+        if (wk && !ForceGeneric() && !ctx->f[1].set &&
+            LaunchTiles<KIND, DIM, NNC, NND, NIP>(ctx, a, wr, 0, n, ctx->stream))
+        {
+            SyncCheck(ctx, "assembly kernel");
+            return;
+        }
     }
     // (the staging kernels keep every IP's state in LDS: rules up to 27 points)
     if constexpr (DIM == 3 && KIND != kGradientDamage && NND * 3 <= 64 && NIP <= 27)
@@ -684,7 +733,7 @@ void PrepareGdm(nuto_ctx* ctx)
         return;
     hipError_t err = hipSuccess;
     ctx->gdm.Prepare(ctx->params.kind, ctx->coordType, ctx->f[0].type, ctx->nip, ctx->graph, ctx->nCells,
-                     ctx->hasCellIds ? ctx->hcellId.data() : nullptr, ctx->nCoordNodes, ctx->x.As<double>(),
+                     ctx->nCoordNodes, ctx->x.As<double>(),
                      ctx->y.As<double>(), ctx->z.As<double>(), ctx->cconn.As<int>(), ctx->tab.As<double>(),
                      ctx->rowPtr.As<int>(), ctx->nRows, ctx->params.interaction != 0, ctx->stream, err);
     if (err == hipErrorOutOfMemory && ctx->params.interaction != 0)
@@ -791,7 +840,7 @@ void Assemble(nuto_ctx* ctx, const double* u, const double* e, const double* kap
         if (wk)
             ctx->gdm.Launch(a, wr, ctx->stream);
         else
-            LaunchGdmHex8Vector<false>(ctx->gdm, a, nullptr, R, nullptr, ctx->gdm.Work(), ctx->stream);
+            ctx->gdm.LaunchVector(a, R, ctx->stream);
         Check(hipGetLastError(), "gdm hex8 launch");
         SyncCheck(ctx, "gdm hex8 kernel");
         return;
@@ -945,9 +994,6 @@ int nuto_set_cells(nuto_ctx* ctx, int coord_type, int n_cells, int n_coord_nodes
         if (dim == 3)
             Upload(ctx, ctx->z, sz.data(), sz.size(), "coords");
         Upload(ctx, ctx->cconn, coord_conn, (size_t)n_cells * nn, "connectivity");
-        ctx->hcellId.clear();
-        if (cell_ids)
-            ctx->hcellId.assign(cell_ids, cell_ids + n_cells);
         ctx->hasCellIds = cell_ids != nullptr;
         ctx->maxCellId = n_cells - 1;
         if (cell_ids)
@@ -1132,6 +1178,7 @@ int nuto_build_pattern(nuto_ctx* ctx, long long* nnz, int* n_rows)
         ctx->nRows = (int)(rp.size() - 1);
         ctx->patternBuilt = true;
         (void)TryVectorStage(ctx);  // here, so that vector assemblies allocate nothing
+        (void)TileLds(ctx);
         // gradient damage with the integrand and the rule already set: the IP tables and the node
         // kernel's tables now, so that assemblies (nuto_build_vector_matrix_noalloc) allocate nothing
         if (ctx->integrandSet && ctx->ruleSet && ctx->params.kind == kGradientDamage && !ForceGeneric())
@@ -1736,7 +1783,7 @@ int nuto_vjp(nuto_ctx* ctx, const double* u, const double* e, const double* kapp
         Require(ctx->gdm.Usable(ctx->params.kind, ctx->coordType, ctx->f[0].type, ctx->nip), NUTO_ERR_UNSUPPORTED,
                 "the adjoint needs hex8 cells and dofs and 2x2x2 Gauss points");
         RowArgs a = MakeRowArgs(ctx, u, e, kappa, nullptr, nullptr);
-        LaunchGdmHex8Vector<true>(ctx->gdm, a, lambda, d_state, d_theta, ctx->gdm.Work(), ctx->stream);
+        ctx->gdm.LaunchAdjoint(a, lambda, d_state, d_theta, ctx->stream);
         Check(hipGetLastError(), "vjp launch");
         SyncCheck(ctx, "vjp kernel");
     });
@@ -2152,8 +2199,7 @@ void LaunchVjp(nuto_batch* b, const double* u, const double* e, const double* ka
     for (BatchGroup& g : b->groups)
     {
         RowArgs a = MakeRowArgs(g.ctx, u + g.uOff, e + g.eOff, kappa + g.hOff, nullptr, nullptr);
-        LaunchGdmHex8Vector<true>(g.ctx->gdm, a, lam + g.ROff, dstate + g.ROff, dtheta ? dtheta + g.tOff : nullptr,
-                                  g.ctx->gdm.Work(), b->stream);
+        g.ctx->gdm.LaunchAdjoint(a, lam + g.ROff, dstate + g.ROff, dtheta ? dtheta + g.tOff : nullptr, b->stream);
     }
     Check(hipGetLastError(), "batch vjp launch");
 }
@@ -2713,6 +2759,8 @@ int nuto_batch_autotune(nuto_batch* b, const double* u, const double* e, const d
                 for (int gram = 0; gram < kCellForms; gram++)
                     for (long long c : chunks)
                     {
+                        if (gram == 4 && g.type != kBtTet4)
+                            continue;
                         g.ctx->cellGram = gram;
                         g.stageCells = c;
                         const double t = median([&] {
