@@ -106,10 +106,10 @@ bool GdmHex8Plan::Prepare(int kind, int coordType, int dofType, int nip, const N
         }
     }
     const char* pre = std::getenv("NUTO_AMD_GDM_PREPASS");
-    prepass = !(pre && pre[0] == '0');
+    prepass = pre ? (pre[0] == '0' ? 0 : 1) : -1;
     const char* aff = std::getenv("NUTO_AMD_GDM_AFFINE");
     affine = false;
-    if (prepass && nCells > 0 && !(aff && aff[0] == '0'))
+    if (nCells > 0 && !(aff && aff[0] == '0'))
     {
         DevBuf cnt;
         int h = -1;
@@ -155,60 +155,62 @@ bool GdmHex8Plan::Prepare(int kind, int coordType, int dofType, int nip, const N
     return true;
 }
 
-template <bool FULLDMG, int MODE, bool DEC>
-static void LaunchNodes(const RowArgs& a, const GdmHex8Tables& t, bool wr, int grid, hipStream_t stream)
+template <bool FULLDMG, bool PRE, bool DEC>
+static void LaunchNodes(const RowArgs& a, const GdmHex8Tables& t, bool affine, bool wr, int grid, hipStream_t stream)
 {
-    if (wr)
-        hipLaunchKernelGGL((kGdmHex8Node<true, FULLDMG, MODE, DEC>), dim3(grid), dim3(64), 0, stream, a, t);
+    if (wr && affine)
+        hipLaunchKernelGGL((kGdmHex8Node<true, FULLDMG, PRE, true, DEC>), dim3(grid), dim3(64), 0, stream, a, t);
+    else if (wr)
+        hipLaunchKernelGGL((kGdmHex8Node<true, FULLDMG, PRE, false, DEC>), dim3(grid), dim3(64), 0, stream, a, t);
+    else if (affine)
+        hipLaunchKernelGGL((kGdmHex8Node<false, FULLDMG, PRE, true, DEC>), dim3(grid), dim3(64), 0, stream, a, t);
     else
-        hipLaunchKernelGGL((kGdmHex8Node<false, FULLDMG, MODE, DEC>), dim3(grid), dim3(64), 0, stream, a, t);
+        hipLaunchKernelGGL((kGdmHex8Node<false, FULLDMG, PRE, false, DEC>), dim3(grid), dim3(64), 0, stream, a, t);
 }
 
+// all nodes of the plan; state: the pre-pass records' memory (nullptr: no pre-pass)
 template <bool FULLDMG, bool DEC>
 static void LaunchT(const GdmHex8Plan& plan, const RowArgs& a, bool wr, double* state, hipStream_t stream)
 {
     GdmHex8Tables t = plan.Tables();
+    if (!state)
+    {
+        LaunchNodes<FULLDMG, false, DEC>(a, t, plan.affine, wr, plan.grid, stream);
+        return;
+    }
     t.ipState = state;
-    const dim3 ipGrid((unsigned)(((long long)plan.nCells * 8 + 63) / 64));
-    if (plan.affine)
+    if (plan.nCells > 0)
     {
-        if (plan.nCells > 0)
-            hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, true, DEC>), ipGrid, dim3(64), 0, stream, a, t, state);
-        LaunchNodes<FULLDMG, 2, DEC>(a, t, wr, plan.grid, stream);
+        const dim3 grid((unsigned)((plan.nCells + 7) / 8));
+        if (plan.affine)
+            hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, true, DEC>), grid, dim3(64), 0, stream, a, t, state);
+        else
+            hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, false, DEC>), grid, dim3(64), 0, stream, a, t, state);
     }
-    else
-    {
-        if (plan.nCells > 0)
-            hipLaunchKernelGGL((kGdmHex8Ip<FULLDMG, false, DEC>), ipGrid, dim3(64), 0, stream, a, t, state);
-        LaunchNodes<FULLDMG, 1, DEC>(a, t, wr, plan.grid, stream);
-    }
+    LaunchNodes<FULLDMG, true, DEC>(a, t, plan.affine, wr, plan.grid, stream);
 }
+
+// A mesh whose nodes' workgroups are all on the chip at once (16 per CU) takes one launch without the
+// pre-pass: its time is the latency of one workgroup, which the pre-pass would only precede. Measured, R + K,
+// with / without pre-pass: 125 nodes 9.7 / 7.0 us, 3375 nodes 14.7 / 12.6 us (affine) and 16.0 / 12.5 us
+// (jittered); 9261 nodes 24.4 / 24.1 and 28.2 / 24.7 us, 24,389 nodes 47.7 / 56.1 and 52.8 / 55.9 us.
+constexpr int kOneLaunchNodes = 16 * 256;
 
 void GdmHex8Plan::Launch(const RowArgs& a, bool wr, hipStream_t stream, double* state) const
 {
     if (nNodes > 0)
     {
-        if (!state)
-            state = Work();
+        const bool pre = prepass < 0 ? nNodes > kOneLaunchNodes : prepass != 0;
+        double* records = !pre ? nullptr : (state ? state : Work());
         const bool full = a.P.damage_application == 0;
-        if (!prepass)
-        {
-            if (full)
-                LaunchNodes<true, 0, false>(a, Tables(), wr, grid, stream);
-            else
-                LaunchNodes<false, 0, false>(a, Tables(), wr, grid, stream);
-        }
-        else if (decreasing)
-        {
-            if (full)
-                LaunchT<true, true>(*this, a, wr, state, stream);
-            else
-                LaunchT<false, true>(*this, a, wr, state, stream);
-        }
+        if (full && decreasing)
+            LaunchT<true, true>(*this, a, wr, records, stream);
         else if (full)
-            LaunchT<true, false>(*this, a, wr, state, stream);
+            LaunchT<true, false>(*this, a, wr, records, stream);
+        else if (decreasing)
+            LaunchT<false, true>(*this, a, wr, records, stream);
         else
-            LaunchT<false, false>(*this, a, wr, state, stream);
+            LaunchT<false, false>(*this, a, wr, records, stream);
     }
     LaunchExtras(a, wr, stream);
 }
@@ -237,11 +239,11 @@ void GdmHex8Plan::LaunchRange(const RowArgs& a, int first, int end, hipStream_t 
     t.pBegin = first;
     t.pEnd = end;
     t.order = posOf.p ? posOf.As<int>() : nullptr;  // launch index = node
-    // per-mesh launches recompute the IP state in the node kernel (no pre-pass over the mesh's cells)
+    // without the pre-pass, which runs over all cells of the plan
     if (a.P.damage_application == 0)
-        LaunchNodes<true, 0, false>(a, t, true, end - first, stream);
+        LaunchNodes<true, false, false>(a, t, affine, true, end - first, stream);
     else
-        LaunchNodes<false, 0, false>(a, t, true, end - first, stream);
+        LaunchNodes<false, false, false>(a, t, affine, true, end - first, stream);
 }
 
 void GdmHex8Plan::LaunchVector(const RowArgs& a, double* vec, hipStream_t stream) const

@@ -19,10 +19,12 @@
 // UNILATERAL damage application keeps the volumetric factor per IP, so uu is accumulated in the
 // general form c1 g_a g_b^T + c2 g_b g_a^T + c2 (g_a . g_b) I.
 //
-// Modes: 2 (every cell affine: one J^-1 per cell), 1 (J^-1 per IP), both with the IP states from the
-// pre-pass kGdmHex8Ip; 0 evaluates the IP states in the node kernel (launches over one mesh of a batch).
+// AFF: every cell of the mesh is affine, one J^-1 per cell; otherwise J^-1 per IP. PRE: the IP states come
+// from the pre-pass kGdmHex8Ip; otherwise every node's workgroup evaluates its cells' IPs itself (8 times
+// the physics, one launch less), with the same functions on the same operands, so that both give the same
+// bits. GdmHex8Plan::Launch says when.
 //
-// What bounds it: the FP64 and exchange instructions of the vector units, 701 per wave in mode 2 (334
+// What bounds it: the FP64 and exchange instructions of the vector units, 676 per wave with AFF (334
 // FP64), with the latency of the record gather and of the reduction's LDS reads behind them (4 waves per
 // SIMD: 9.3 KB of LDS per workgroup). Summing the blocks from records in LDS instead (each lane reading
 // the 8 points' records of its cell) took 732 instructions and kept the LDS busy 78 % of the time.
@@ -72,12 +74,26 @@ __device__ inline void ShapeAt(int n, int ip, double d[3], double& N)
     N = e * f0 * f1 * f2;
 }
 
+// In the functions below that the pre-pass and the node kernel share, every fused multiply-add is named and
+// the compiler's own contraction is off: a record gives the same bits whichever kernel evaluates it.
+__device__ inline double Dot3(double a0, double a1, double a2, double b0, double b1, double b2)
+{
+    return fma(a2, b2, fma(a1, b1, a0 * b0));
+}
+
+__device__ inline void ElasticFactors(const LawParams& P, double E, double& m3K, double& m2G)
+{
+#pragma clang fp contract(off)
+    m3K = P.cK * E;
+    m2G = P.cG * E;
+}
+
 // g = J^-T d  (dN/dX = dN/dxi J^-1, Jacobian.h:100-103)
 __device__ inline void GradOf(const double d[3], const double inv[3][3], double g[3])
 {
 #pragma unroll
     for (int c = 0; c < 3; c++)
-        g[c] = d[0] * inv[0][c] + d[1] * inv[1][c] + d[2] * inv[2][c];
+        g[c] = fma(d[2], inv[2][c], fma(d[1], inv[1][c], d[0] * inv[0][c]));
 }
 }  // namespace gdm8
 
@@ -102,14 +118,13 @@ __device__ inline void GdmIpState(const double Hu[3][3], const double he[3], dou
                                   double kh, double m3K, double m2G, double k0, double beta, const LawParams& P,
                                   GdmIp& o)
 {
+#pragma clang fp contract(off)
     using namespace gdm8;
     // displacement gradient Gu = Hu J^-1
     double Gu[3][3];
 #pragma unroll
     for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-            Gu[i][c] = Hu[i][0] * inv[0][c] + Hu[i][1] * inv[1][c] + Hu[i][2] * inv[2][c];
+        GradOf(Hu[i], inv, Gu[i]);
     o.eps[0] = Gu[0][0];
     o.eps[1] = Gu[1][1];
     o.eps[2] = Gu[2][2];
@@ -129,21 +144,21 @@ __device__ inline void GdmIpState(const double Hu[3][3], const double he[3], dou
         const double ik = 1.0 / o.kap;
         const double ex = exp(beta * (k0 - o.kap));
         const double rr = k0 * ik;
-        o.om = 1.0 - rr * (1.0 - P.alpha + P.alpha * ex);
-        o.dom = rr * ((ik + beta) * P.alpha * ex + (1.0 - P.alpha) * ik);
+        o.om = fma(-rr, fma(P.alpha, ex, 1.0 - P.alpha), 1.0);
+        o.dom = rr * fma((ik + beta) * P.alpha, ex, (1.0 - P.alpha) * ik);
     }
     // LinearElasticDamage<3> stress and dStress/dOmega (LinearElasticDamage.h:65-91)
     const double* eps = o.eps;
     const double eV = (eps[0] + eps[1] + eps[2]) * kThird;
     o.H = (!FULLDMG && eV < 0.0) ? 0.0 : 1.0;
-    const double sV = (1.0 - o.om * o.H) * m3K * eV;
+    const double sV = fma(-o.om, o.H, 1.0) * m3K * eV;
     o.d2G = (1.0 - o.om) * m2G;
 #pragma unroll
     for (int i = 0; i < 3; i++)
     {
         const double dev = eps[i] - eV;
-        o.sig[i] = sV + o.d2G * dev;
-        o.dsw[i] = -m3K * eV * o.H - m2G * dev;
+        o.sig[i] = fma(o.d2G, dev, sV);
+        o.dsw[i] = fma(-m2G, dev, -m3K * eV * o.H);
     }
 #pragma unroll
     for (int i = 3; i < 6; i++)
@@ -155,9 +170,9 @@ __device__ inline void GdmIpState(const double Hu[3][3], const double he[3], dou
     o.I1 = eps[0] + eps[1] + eps[2];
     const double a0 = eps[0] - eps[1], a1 = eps[1] - eps[2], a2 = eps[2] - eps[0];
     const double J2 =
-        (a0 * a0 + a1 * a1 + a2 * a2) * kSixth + 0.25 * (eps[3] * eps[3] + eps[4] * eps[4] + eps[5] * eps[5]);
-    o.Am = sqrt(P.K1 * P.K1 * o.I1 * o.I1 + P.K2 * J2);
-    o.eq = P.K1 * o.I1 + o.Am;
+        fma(0.25, Dot3(eps[3], eps[4], eps[5], eps[3], eps[4], eps[5]), Dot3(a0, a1, a2, a0, a1, a2) * kSixth);
+    o.Am = sqrt(fma(P.K1 * P.K1 * o.I1, o.I1, P.K2 * J2));
+    o.eq = fma(P.K1, o.I1, o.Am);
 }
 
 // d eps_eq / d eps of the modified Mises norm (ModifiedMisesStrainNorm.h:231-268, A == 0 branch)
@@ -256,14 +271,15 @@ __device__ inline void LoadNodeRecord(const RowArgs& A, const GdmHex8Tables& T, 
 template <bool FULLDMG, bool DEC>
 __device__ inline void StateRecord(const GdmIp& st, double s, double m3K, double m2G, const LawParams& P, double* rec)
 {
+#pragma clang fp contract(off)
     using namespace gdm8;
     const double eV = st.I1 * kThird;
-    const double sV = (1.0 - st.om * st.H) * m3K * eV;
+    const double sV = fma(-st.om, st.H, 1.0) * m3K * eV;
     double am = P.K1, bm = 0.0;  // m = am [1,1,1,0,0,0] + bm e'' (A == 0: m = K1 [1,1,1,0,0,0])
     if (st.Am != 0.0)
     {
         const double h = 0.5 / st.Am;
-        am = P.K1 + h * (2.0 * P.K1 * P.K1 * st.I1) - h * P.K2 * st.I1 * kThird;
+        am = fma(-h * P.K2 * st.I1, kThird, fma(h, 2.0 * P.K1 * P.K1 * st.I1, P.K1));
         bm = h * P.K2;
     }
     const double ct = kValueScale * s * st.dom * st.dk, sg = kGradScale * s;
@@ -273,13 +289,13 @@ __device__ inline void StateRecord(const GdmIp& st, double s, double m3K, double
     rec[rEps + 3] = 0.5 * st.eps[3];
     rec[rEps + 4] = 0.5 * st.eps[4];
     rec[rEps + 5] = 0.5 * st.eps[5];
-    rec[rSig] = s * (sV - st.d2G * eV);
+    rec[rSig] = s * fma(-st.d2G, eV, sV);
     rec[rSig + 1] = s * st.d2G;
     rec[rT] = -ct * (m3K * st.H - m2G) * eV;
     rec[rT + 1] = -ct * m2G;
     rec[rM] = sg * am;
     rec[rM + 1] = sg * bm;
-    rec[rC1] = FULLDMG ? sg * (1.0 - st.om) : sg * (m3K * (1.0 - st.om * st.H) - st.d2G) * kThird;
+    rec[rC1] = FULLDMG ? sg * (1.0 - st.om) : sg * fma(m3K, fma(-st.om, st.H, 1.0), -st.d2G) * kThird;
     rec[rC2] = FULLDMG ? 0.0 : 0.5 * sg * st.d2G;
     rec[rRe] = s * (st.eN - st.eq);
     rec[rGe] = s * P.c * st.ge[0];
@@ -317,8 +333,7 @@ __device__ inline void GdmCellState(const RowArgs& A, const CornerLane& c, int c
 {
     double E, k0, beta;
     GdmMaterial(A, cell, E, k0, beta);
-    m3K = A.P.cK * E;
-    m2G = A.P.cG * E;
+    gdm8::ElasticFactors(A.P, E, m3K, m2G);
     const int hist = A.cellId ? A.cellId[cell] : cell;
     const double kh = A.kappa[(size_t)hist + (size_t)c.ip * A.kappaLd];
     double Hu[3][3], he[3], inv0[3][3];
@@ -356,6 +371,7 @@ template <bool FULLDMG, bool AFF, bool DEC>
 __device__ inline void CellBlock(const CornerLane& c, const double* sr, const double* g, int la, double m3K, double m2G,
                                  const LawParams& P, double acc[16], double Rv[4])
 {
+#pragma clang fp contract(off)
     using namespace gdm8;
     const double inv[3][3] = {{g[0], g[1], g[2]}, {g[3], g[4], g[5]}, {g[6], g[7], g[8]}};
     const double s = g[9];
@@ -365,16 +381,16 @@ __device__ inline void CellBlock(const CornerLane& c, const double* sr, const do
     const double E[3][3] = {{sr[rEps], sr[rEps + 5], sr[rEps + 4]},
                             {sr[rEps + 5], sr[rEps + 1], sr[rEps + 3]},
                             {sr[rEps + 4], sr[rEps + 3], sr[rEps + 2]}};
-    const double gdot = ga[0] * sr[rGe] + ga[1] * sr[rGe + 1] + ga[2] * sr[rGe + 2];
+    const double gdot = Dot3(ga[0], ga[1], ga[2], sr[rGe], sr[rGe + 1], sr[rGe + 2]);
     const double cs = kGradScale * P.c * (DEC ? s * sr[DEC ? rGi : 0] : s);
-    Rv[3] = Na * sr[rRe] + (DEC ? sr[DEC ? rGi : 0] * gdot : gdot);
+    Rv[3] = fma(Na, sr[rRe], DEC ? sr[DEC ? rGi : 0] * gdot : gdot);
 #pragma unroll
     for (int i = 0; i < 3; i++)
     {
         // e'' g_a: B_a^T of the Voigt vector e''
-        const double Eg = E[i][0] * ga[0] + E[i][1] * ga[1] + E[i][2] * ga[2];
-        Rv[i] = sr[rSig] * ga[i] + sr[rSig + 1] * Eg;
-        acc[4 * i + 3] = ValuesToNode(sr[rT] * ga[i] + sr[rT + 1] * Eg);  // ue: (B_a^T t) N_b
+        const double Eg = Dot3(E[i][0], E[i][1], E[i][2], ga[0], ga[1], ga[2]);
+        Rv[i] = fma(sr[rSig], ga[i], sr[rSig + 1] * Eg);
+        acc[4 * i + 3] = ValuesToNode(fma(sr[rT], ga[i], sr[rT + 1] * Eg));  // ue: (B_a^T t) N_b
     }
     double p[3];
     {
@@ -385,15 +401,15 @@ __device__ inline void CellBlock(const CornerLane& c, const double* sr, const do
         {
 #pragma unroll
             for (int k = 0; k < 3; k++)
-                p[k] = am * inv[k][i] + bm * (E[i][0] * inv[k][0] + E[i][1] * inv[k][1] + E[i][2] * inv[k][2]);
+                p[k] = fma(am, inv[k][i], bm * Dot3(E[i][0], E[i][1], E[i][2], inv[k][0], inv[k][1], inv[k][2]));
             acc[12 + i] = PointsToNode<false>(c, p, 0.0);
         }
     }
     // ee: s N_a N_b + c s g_a . g_b
 #pragma unroll
     for (int k = 0; k < 3; k++)
-        p[k] = cs * (ga[0] * inv[k][0] + ga[1] * inv[k][1] + ga[2] * inv[k][2]);
-    acc[15] = PointsToNode<true>(c, p, kValueScale * (DEC ? s * Na + sr[DEC ? rDg : 0] * gdot : s * Na));
+        p[k] = cs * Dot3(ga[0], ga[1], ga[2], inv[k][0], inv[k][1], inv[k][2]);
+    acc[15] = PointsToNode<true>(c, p, kValueScale * (DEC ? fma(s, Na, sr[DEC ? rDg : 0] * gdot) : s * Na));
     // S = sum h g_a g_b^T for the factor h of the displacement block
     auto gram = [&](double h, double S[3][3]) {
 #pragma unroll
@@ -431,7 +447,7 @@ __device__ inline void CellBlock(const CornerLane& c, const double* sr, const do
 #pragma unroll
             for (int k = 0; k < 3; k++)
             {
-                acc[4 * i + k] = lam * S[i][k] + mu * S[k][i];
+                acc[4 * i + k] = fma(lam, S[i][k], mu * S[k][i]);
                 if (i == k)
                     acc[4 * i + k] += tr;
             }
@@ -476,13 +492,10 @@ __device__ inline void StoreRows(double* dst, const double* src, int n, int lane
 
 // The rows of node p (one 64-lane workgroup); `state` is the workgroup's LDS (kRed doubles): partial
 // blocks, R sums and the slot map.
-template <bool WR, bool FULLDMG, int MODE, bool DEC>
+template <bool WR, bool FULLDMG, bool PRE, bool AFF, bool DEC>
 __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int pos, double* state)
 {
     using namespace gdm8;
-    constexpr bool PRE = MODE >= 1, AFF = MODE == 2;
-    static_assert(PRE || !DEC, "the decreasing interaction needs the pre-pass");
-
     const int lane = threadIdx.x;
     const int r = lane >> 3, m = lane & 7;
     const CornerLane c = CornerOf(lane);
@@ -502,7 +515,8 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
     {
         NodeRecord<DEC> rec;
         LoadNodeRecord<PRE, AFF, DEC>(A, T, tab, c, rec);
-        double m3K = P.cK * rec.E, m2G = P.cG * rec.E;
+        double m3K, m2G;
+        ElasticFactors(P, rec.E, m3K, m2G);
         if constexpr (!PRE)
         {
             const int cell = valid ? tab.cell : 0;
@@ -610,16 +624,16 @@ __device__ inline void NodeBody(const RowArgs& A, const GdmHex8Tables& T, int po
     }
 }
 
-// MODE >= 1 targets 4 waves per SIMD (<= 128 VGPRs; the LDS of modes 1 and 2 allows 16 workgroups per CU)
-template <bool WR, bool FULLDMG, int MODE, bool DEC>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE >= 1 ? 4 : 1)))
+// 4 waves per SIMD (<= 128 VGPRs; the LDS allows 17 workgroups per CU)
+template <bool WR, bool FULLDMG, bool PRE, bool AFF, bool DEC>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
 kGdmHex8Node(const RowArgs A, const GdmHex8Tables T)
 {
     __shared__ __align__(16) double state[gdm8::kRed];
     const int pos = NodeOfBlock(T);
     if (pos < 0)
         return;
-    NodeBody<WR, FULLDMG, MODE, DEC>(A, T, pos, state);
+    NodeBody<WR, FULLDMG, PRE, AFF, DEC>(A, T, pos, state);
 }
 
 // Pre-pass: the state of every (cell, IP) once, for the node kernel (which would otherwise evaluate

@@ -73,8 +73,8 @@ struct GdmHex8Plan
     DevBuf geoCell;      // affine meshes: IP 0's geometry record per cell
     DevBuf extra;        // nodes beyond the kernel's bounds (more than 8 cells or 32 neighbours)
     int nExtra = 0;      // ... assembled by the generic row-owner kernel
-    bool prepass = true;
-    bool affine = false;  // every cell affine: MODE 2 of the node kernel
+    int prepass = -1;     // NUTO_AMD_GDM_PREPASS=0 / 1: never / always run the pre-pass; -1: by the mesh's size
+    bool affine = false;  // every cell affine: one J^-1 per cell
     bool decreasing = false;  // NonlocalInteraction::Decreasing: longer pre-pass records
     int nCells = 0;
 
@@ -117,12 +117,6 @@ struct GdmHex8Plan
     size_t StateDoubles() const
     {
         return prepass ? (size_t)nCells * 8 * RecordDoubles() : 0;
-    }
-
-    // the matrix of the plan's interaction can be assembled by the node kernel
-    bool Matrix() const
-    {
-        return prepass || !decreasing;
     }
 
     // K (and R, wr). state: device memory of StateDoubles() doubles for the pre-pass records (nullptr: the

@@ -833,8 +833,7 @@ void Assemble(nuto_ctx* ctx, const double* u, const double* e, const double* kap
     const bool nodeKernel = !ForceGeneric();
     if (nodeKernel)
         PrepareGdm(ctx);
-    if (nodeKernel && ctx->gdm.Usable(ctx->params.kind, ctx->coordType, ctx->f[0].type, ctx->nip) &&
-        (!wk || ctx->gdm.Matrix()))
+    if (nodeKernel && ctx->gdm.Usable(ctx->params.kind, ctx->coordType, ctx->f[0].type, ctx->nip))
     {
         RowArgs a = MakeRowArgs(ctx, u, e, kappa, R, K);
         if (wk)

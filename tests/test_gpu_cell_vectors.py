@@ -54,9 +54,11 @@ def test_gradient_damage(n, jitter, app):
 @pytest.mark.parametrize("n,jitter", [((1, 1, 1), 0.0), ((3, 3, 1), 0.1), ((5, 3, 3), 0.0), ((4, 3, 3), 0.1)])
 @pytest.mark.parametrize("app", [N.FULL, N.UNILATERAL])
 @pytest.mark.parametrize("r", [0.005, 0.0])
-def test_decreasing_interaction(n, jitter, app, r):
+@pytest.mark.parametrize("prepass", ["0", "1"])
+def test_decreasing_interaction(n, jitter, app, r, prepass, monkeypatch):
     """R and K of the decreasing nonlocal interaction (node kernel and cell vectors) against the oracle,
     also with a factor that reaches zero at omega = 1, and the residual alone."""
+    monkeypatch.setenv("NUTO_AMD_GDM_PREPASS", prepass)
     X, C = make_mesh(N.HEX8, n, lengths=tuple(float(v) for v in n), jitter=jitter)
     dev = N.gradient_damage_params(damage_application=app, interaction=N.DECREASING, interaction_r=r)
     orc = O.Params(kind=1, dim=3, E=30000.0, nu=0.2, k=10.0, kappa0=1e-4, beta=100.0, alpha=0.99, c=4.0,
@@ -155,3 +157,21 @@ def test_local_damage_loads_at_the_updated_history(ct, dt, n, rule, forms, monke
         K, want = (ctx.build_matrix(du, None, k).cpu().numpy() for k in (dk, low))
         # points that the update did not raise (history above the strain) load in neither
         assert np.abs(K - want).max() <= 1e-7 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("n,jitter", [((15, 15, 15), 0.0), ((15, 15, 15), 0.1), ((16, 15, 15), 0.0)])
+@pytest.mark.parametrize("app", [N.FULL, N.UNILATERAL])
+def test_one_launch_gives_the_same_bits(n, jitter, app, monkeypatch):
+    """Meshes on either side of the size from which on the pre-pass runs (4096 nodes): with and without it
+    the same bits, so a mesh gives the same result alone and in a large batch."""
+    X, C = make_mesh(N.HEX8, n, lengths=tuple(float(v) for v in n), jitter=jitter)
+    p = Pair(N.HEX8, N.HEX8, X, C, N.gradient_damage_params(damage_application=app), gdm_params(app)[1], True)
+    state = [to_dev(v) for v in p.inputs()]
+    out = []
+    for prepass in ("0", "1", None):
+        monkeypatch.delenv("NUTO_AMD_GDM_PREPASS", raising=False)
+        if prepass:
+            monkeypatch.setenv("NUTO_AMD_GDM_PREPASS", prepass)
+        out.append([v.cpu().numpy() for v in p.context().build_vector_matrix(*state)])
+    for R, K in out[1:]:
+        assert np.array_equal(R, out[0][0]) and np.array_equal(K, out[0][1])
