@@ -12,22 +12,25 @@
 //
 // Solvers: Jacobi-preconditioned conjugate gradients and BiCGSTAB (the iterative solvers NuTo selects
 // by name, EigenSparseSolve.cpp:44-49, whose default preconditioner is the diagonal). An iteration is
-// three (CG) or five (BiCGSTAB) kernels. Dot products ride on the kernels that make their operands:
+// two (CG) or three (BiCGSTAB) kernels in small systems, three or five in larger ones (kFormNodes). Dot products ride on the kernels that make their operands:
 // each block leaves its partial sum, and every block of the next kernel adds the partials itself, all
 // in the same fixed order, so no kernel exists only to finish a reduction and solves are
-// bit-reproducible. The scalars, the convergence test and the iteration count stay on the device
+// bit-reproducible. A kernel loads all that does not depend on those sums, the test of the status
+// included, before it waits for them. The scalars, the convergence test and the iteration count stay on the device
 // (KrylovState); once the test is met the remaining launches return at once. The host queues
 // kSolveChunk iterations at a time and reads the state of a chunk while the next one runs, so the
 // device never waits for it.
 // Measured, per iteration: BiCGSTAB in a load step on 1536 hex8 gradient-damage cells (K of 5.8 MB) 61
-// us with 14 kernels and a host read, 23 us like this (4 us of latency per kernel); conjugate gradients
-// on 24,480 elastic tet10 cells (K of 69 MB) 55 us with 9 kernels and a host read, 29 us like this.
+// us with 14 kernels and a host read, 23 us with five kernels, 15.3 us with three (the two products 5.8 us
+// each, the update 3.7 us, without gaps between them); conjugate gradients on 24,480 elastic tet10 cells (K
+// of 69 MB) 55 us with 9 kernels and a host read, 29 us with three.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <vector>
 
 #include "devbuf.hpp"
@@ -39,6 +42,15 @@ namespace nuto_amd
 constexpr int kDotBlocks = 1024;    // blocks (= partial sums) of the vector kernels
 constexpr int kSpmvBlocks = 2048;   // blocks of the K product: 8 of 4 waves on each of 256 CUs
 constexpr int kSolveChunk = 4;      // iterations the host queues before it reads a state
+
+// Up to this size a wave of the K product has one node, and an iteration takes as long as its chain of
+// launches and dependent loads: there the product forms its input vector where it gathers it, and the
+// kernels that made the vectors are left out. In larger systems the product is bound by its reads, and two
+// or three gathers in place of one cost more than a pass over the vectors. Measured, us per iteration with
+// stored / formed vectors, hex8 gradient damage (K of 4 rows per node): CG 125 nodes 12.0 / 9.3, 2025 nodes
+// 13.6 / 11.1, 9261 nodes 16.0 / 15.4, 226,981 nodes 234 / 248; BiCGSTAB 18.6 / 16.1, 20.4 / 17.5, 27.6 / 28.5,
+// 465 / 530; elastic hex8, 15,625 nodes: 17.5 / 17.0 and 30.5 / 33.3.
+constexpr int kFormNodes = 4 * kSpmvBlocks;
 
 enum SolveStatus : int
 {
@@ -115,6 +127,127 @@ __device__ inline void StorePartials(double v[N], double* __restrict__ part, dou
     }
 }
 
+// What the first kernel of an iteration needs: its launch number seq (copy seq & 1 of the state is read, the
+// other written), the iteration `it`, the partials of the dots that the iteration before left, the
+// tolerance. first: the state of a new solve; forced: no tests (the iteration after a restart, whose
+// (r . r) becomes |r0|^2); check: the test alone, no iteration follows. tell: where the host reads the
+// outcome (pinned memory, or nullptr): the kernel writes it there itself, since a copy command between the
+// kernels holds the stream up for longer than an iteration of a small system takes.
+struct StepArgs
+{
+    int seq, it;
+    bool first, forced, check;
+    double tol2;
+    const double* part;
+    int np;
+    KrylovState* st;
+    KrylovState* tell;
+};
+
+__device__ inline void Tell(KrylovState* host, double rr, double bb, int status, int iters)
+{
+    if (!host)
+        return;
+    host->rr = rr;
+    host->bb = bb;
+    host->status = status;
+    host->iters = iters;
+}
+
+// CG: the test |r|^2 < tol^2 |b|^2, then beta = (r . z) / (r . z of the iteration before); false when the
+// solve has ended
+__device__ inline bool CgStep(const StepArgs& a, double* sh, double& beta)
+{
+    const KrylovState* in = a.st + (a.seq & 1);
+    KrylovState* out = a.st + ((a.seq + 1) & 1);
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const int status = in->status, iters = in->iters;
+    const double oldRr = in->rr, oldRho = in->rho, oldBb = in->bb;
+    double s[2];
+    SumPartials<2, kDotBlocks>(a.part, a.np, s, sh);
+    if (status != kRunning)
+    {
+        if (lead)
+        {
+            out->rr = oldRr;
+            out->bb = oldBb;
+            out->status = status;
+            out->iters = iters;
+            Tell(a.tell, oldRr, oldBb, status, iters);
+        }
+        return false;
+    }
+    const double bb = a.first ? s[0] : oldBb;
+    const bool done = s[0] < fmax(a.tol2 * bb, 1e-300);
+    if (lead)
+    {
+        const int now = done ? kDone : kRunning;
+        const int before = done && a.it > 0 ? a.it - 1 : a.it;  // the iterations before the converging one
+        out->rr = s[0];
+        out->bb = bb;
+        out->rho = s[1];
+        out->status = now;
+        out->iters = before;
+        Tell(a.tell, s[0], bb, now, before);
+    }
+    beta = a.first ? 0.0 : s[1] / oldRho;
+    return !done;
+}
+
+// BiCGSTAB: the tests !(|r|^2 > tol^2 |b|^2) and |rho| < eps^2 |r0|^2 (a restart, done by the host), then
+// beta; false when the solve has ended or waits for the restart
+__device__ inline bool BicgStep(const StepArgs& a, double* sh, double& beta)
+{
+    const KrylovState* in = a.st + (a.seq & 1);
+    KrylovState* out = a.st + ((a.seq + 1) & 1);
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const int status = in->status, iters = in->iters;
+    const double oldRr = in->rr, oldBb = in->bb, oldRho = in->rho, alpha = in->alpha, w = in->w, oldR0 = in->r0sq;
+    double s[2];
+    SumPartials<2, kDotBlocks>(a.part, a.np, s, sh);
+    if (status == kDone || (status == kRestart && !a.forced))
+    {
+        if (lead)
+        {
+            out->rr = oldRr;
+            out->bb = oldBb;
+            out->rho = oldRho;
+            out->alpha = alpha;
+            out->w = w;
+            out->r0sq = oldR0;
+            out->status = status;
+            out->iters = iters;
+            Tell(a.tell, oldRr, oldBb, status, iters);
+        }
+        return false;
+    }
+    const double bb = a.first ? s[0] : oldBb, r0sq = a.first || a.forced ? s[0] : oldR0;
+    int now = kRunning;
+    if (!a.forced)
+    {
+        const double eps2 = 2.220446049250313e-16 * 2.220446049250313e-16;
+        if (!(s[0] > a.tol2 * bb))
+            now = kDone;
+        else if (!a.check && fabs(s[1]) < eps2 * r0sq)
+            now = kRestart;
+    }
+    if (lead)
+    {
+        const double rr = a.forced ? oldRr : s[0];  // after a restart the residual's norm is the one that was tested
+        Tell(a.tell, rr, bb, now, a.it);
+        out->rr = rr;
+        out->bb = bb;
+        out->rho = now == kRestart ? oldRho : s[1];  // the restarted iteration's beta divides by the last rho
+        out->alpha = alpha;
+        out->w = w;
+        out->r0sq = r0sq;
+        out->status = now;
+        out->iters = a.it;
+    }
+    beta = (s[1] / oldRho) * (alpha / w);
+    return now == kRunning;
+}
+
 // Dots of the K product: none, (d . y) (CG: p . q, BiCGSTAB: r0 . v), or (y . y) and (d . y)
 // (BiCGSTAB: t . t, t . s)
 enum SpmvDots : int
@@ -122,6 +255,26 @@ enum SpmvDots : int
     kNoDots = 0,
     kOneDot = 1,
     kTwoDots = 2
+};
+
+// The vector that the K product multiplies: x itself, or formed entry by entry where it is gathered (every
+// block forms the entries it needs; `own` receives the vector before the preconditioner at the block's rows):
+// CG p = x + beta x2 (z, the last p), BiCGSTAB invd p with p = x + beta x2 (r, the last p - w v) or invd s with
+// s = x - alpha x2 (r, v)
+enum SpmvInput : int
+{
+    kStored = 0,
+    kCgDirection = 1,
+    kBicgDirection = 2,
+    kBicgHalfStep = 3
+};
+struct FormedInput
+{
+    const double *x, *x2, *invd;
+    double* own;
+    StepArgs step;            // the directions: the iteration begins here
+    const double* dotPart;    // the half step: partials of (r0 . v)
+    int nDot;
 };
 
 // y = A x for a CSR matrix, 16 lanes per row: lane l sums the entries l, l + 16, ... of its row in
@@ -153,17 +306,20 @@ __global__ void __launch_bounds__(256) kCsrSpmv(int nRows, const int* __restrict
 // 128 entries of every row in flight while it works on this one's, and the row offsets of the node
 // after that: only the gather of x is waited for. mask (one byte per node, bit i: row i is a dependent
 // dof) zeroes those rows of y; DOTS: the block's partial sums of the dots over its rows.
-// Bound by the reads of the values.
-template <int C0, int C1, int DOTS>
+// Bound by the reads of the values; in small systems by the latency of its launch and of its dependent
+// loads. IN != kStored: the kernel that would make x is left out, see SpmvInput; the first node's entries
+// are in flight while the block adds the partials.
+template <int C0, int C1, int DOTS, int IN>
 __global__ void __launch_bounds__(256) kNodeSpmv(int nNodes, int nU, const int* __restrict__ rowPtr,
                                                  const int* __restrict__ col, const double* __restrict__ val,
                                                  const double* __restrict__ x, double* __restrict__ y,
                                                  const unsigned char* __restrict__ mask, const double* __restrict__ d,
-                                                 double* __restrict__ part, const KrylovState* __restrict__ st)
+                                                 double* __restrict__ part, KrylovState* __restrict__ st,
+                                                 const FormedInput in)
 {
     constexpr int F = C0 + C1;
-    if (DOTS != kNoDots && st->status != kRunning)
-        return;
+    __shared__ double sh[8];
+    const int status = IN == kStored && DOTS != kNoDots ? st->status : kRunning;
     const int l = (int)(threadIdx.x & 63);
     const int step = (int)gridDim.x * 4;
     const int last = nNodes - 1;
@@ -204,6 +360,40 @@ __global__ void __launch_bounds__(256) kNodeSpmv(int nNodes, int nU, const int* 
     Head now = head(p), next = head(p + step);
     if (p < nNodes && now.L > 0)
         load(now);
+    if (status != kRunning)
+        return;
+    double f = 0.0;  // beta or -alpha
+    if constexpr (IN == kCgDirection)
+    {
+        if (!CgStep(in.step, sh, f))
+            return;
+    }
+    if constexpr (IN == kBicgDirection)
+    {
+        if (!BicgStep(in.step, sh, f))
+            return;
+    }
+    if constexpr (IN == kBicgHalfStep)
+    {
+        const int status = st->status;
+        const double rho = st->rho;
+        double rv[1];
+        SumPartials<1, kSpmvBlocks>(in.dotPart, in.nDot, rv, sh);
+        if (status != kRunning)
+            return;
+        const double alpha = rho / rv[0];
+        if (blockIdx.x == 0 && threadIdx.x == 0)
+            st->alpha = alpha;
+        f = -alpha;
+    }
+    auto entry = [&](int j) {
+        if constexpr (IN == kStored)
+            return x[j];
+        else if constexpr (IN == kCgDirection)
+            return fma(f, in.x2[j], in.x[j]);
+        else
+            return in.invd[j] * fma(f, in.x2[j], in.x[j]);
+    };
     for (; p < nNodes; p += step)
     {
         double acc[4] = {0.0, 0.0, 0.0, 0.0};
@@ -211,12 +401,15 @@ __global__ void __launch_bounds__(256) kNodeSpmv(int nNodes, int nU, const int* 
         // this lane's row of y after the exchanges
         const int row = l < C0 ? C0 * p + l : nU + p;
         const bool dep = mask && ((mask[p] >> (l & 7)) & 1);
-        const double dv = DOTS != kNoDots && l < F ? d[row] : 0.0;
+        const bool formsD = IN == kCgDirection || IN == kBicgHalfStep;  // d is the formed vector
+        const double dr = DOTS != kNoDots && !formsD && l < F ? d[row] : 0.0;
+        const double ov = IN != kStored && l < F ? fma(f, in.x2[row], in.x[row]) : 0.0;
+        const double dv = formsD ? ov : dr;
         double xa = 0.0, xb = 0.0, wa[F], wb[F];
         if (h.L > 0)
         {
-            xa = x[ca];
-            xb = x[cb];
+            xa = entry(ca);
+            xb = entry(cb);
 #pragma unroll
             for (int i = 0; i < F; i++)
             {
@@ -239,7 +432,7 @@ __global__ void __launch_bounds__(256) kNodeSpmv(int nNodes, int nU, const int* 
         }
         for (int k = l + 128; k < h.L; k += 64)
         {
-            const double xk = x[col[h.r0 + k]];
+            const double xk = entry(col[h.r0 + k]);
 #pragma unroll
             for (int i = 0; i < C0; i++)
                 acc[i] += val[h.r0 + i * h.L + k] * xk;
@@ -265,6 +458,8 @@ __global__ void __launch_bounds__(256) kNodeSpmv(int nNodes, int nU, const int* 
         {
             a = dep ? 0.0 : a;
             y[row] = a;
+            if constexpr (IN != kStored)
+                in.own[row] = ov;
             if constexpr (DOTS == kOneDot)
                 dots[0] += a * dv;
             if constexpr (DOTS == kTwoDots)
@@ -275,10 +470,7 @@ __global__ void __launch_bounds__(256) kNodeSpmv(int nNodes, int nU, const int* 
         }
     }
     if constexpr (DOTS != kNoDots)
-    {
-        __shared__ double sh[8];
         StorePartials<DOTS>(dots, part, sh);
-    }
 }
 
 // the dots of a finished product y (the path with constraint terms, whose C^T changes y after the
@@ -475,47 +667,16 @@ __global__ void __launch_bounds__(256) kKrylovStart(int n, const int* __restrict
         st[0] = KrylovState{0.0, 0.0, 1.0, 1.0, 1.0, 0.0, kRunning, 0};
 }
 
-// First kernel of CG iteration `it` (copy seq & 1 of the state read, the other written): the test
-// |r|^2 < tol^2 |b|^2, then p = z + beta p, beta = (r . z) / (r . z of the iteration before). `check`:
-// the test alone (after the last iteration that the caller allows).
-__global__ void __launch_bounds__(256) kCgP(int n, int it, bool check, double tol2, const double* __restrict__ part,
-                                            int np, const double* __restrict__ z, double* __restrict__ p,
-                                            KrylovState* __restrict__ st)
+// First kernel of CG iteration `it` where the K product does not begin the iteration itself: p = z + beta p.
+// `check`: the test alone (after the last iteration that the caller allows).
+__global__ void __launch_bounds__(256) kCgP(int n, const StepArgs a, const double* __restrict__ z, double* __restrict__ p)
 {
     __shared__ double sh[8];
-    const KrylovState* in = st + (it & 1);
-    KrylovState* out = st + ((it + 1) & 1);
-    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    const int status = in->status, iters = in->iters;
-    const double oldRr = in->rr, oldRho = in->rho, oldBb = in->bb;
-    if (status != kRunning)
-    {
-        if (lead)
-        {
-            out->rr = oldRr;
-            out->bb = oldBb;
-            out->status = status;
-            out->iters = iters;
-        }
+    double beta;
+    if (!CgStep(a, sh, beta) || a.check)
         return;
-    }
-    double s[2];
-    SumPartials<2, kDotBlocks>(part, np, s, sh);
-    const double bb = it == 0 ? s[0] : oldBb;
-    const bool done = s[0] < fmax(tol2 * bb, 1e-300);
-    if (lead)
-    {
-        out->rr = s[0];
-        out->bb = bb;
-        out->rho = s[1];
-        out->status = done ? kDone : kRunning;
-        out->iters = done && it > 0 ? it - 1 : it;  // the iterations before the converging one
-    }
-    if (done || check)
-        return;
-    const double beta = it == 0 ? 0.0 : s[1] / oldRho;
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
-        p[i] = z[i] + (it == 0 ? 0.0 : beta * p[i]);
+        p[i] = fma(beta, p[i], z[i]);
 }
 
 // CG's alpha = (r . z) / (p . q), x += alpha p, r -= alpha q, z = invd r, and the partials of (r . r)
@@ -527,85 +688,54 @@ __global__ void __launch_bounds__(256) kCgUpdate(int n, const double* __restrict
                                                  double* __restrict__ part, const KrylovState* __restrict__ st)
 {
     __shared__ double sh[8];
-    if (st->status != kRunning)
-        return;
+    // the operands of a lane's first entry are in flight while the block adds the partials
+    long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    const long long i0 = i < n ? i : n - 1;
+    double pi = p[i0], qi = q[i0], xi = x[i0], ri = r[i0], di = invd[i0];
+    const int status = st->status;
+    const double rho = st->rho;
     double pq[1];
     SumPartials<1, kSpmvBlocks>(dotPart, np, pq, sh);
-    const double alpha = st->rho / pq[0];
+    if (status != kRunning)
+        return;
+    const double alpha = rho / pq[0];
     double s[2] = {0.0, 0.0};
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
+    while (i < n)
     {
-        x[i] = alpha * p[i] + x[i];
-        const double ri = -alpha * q[i] + r[i];
+        x[i] = fma(alpha, pi, xi);
+        ri = fma(-alpha, qi, ri);
         r[i] = ri;
-        const double zi = invd[i] * ri;
+        const double zi = di * ri;
         z[i] = zi;
-        s[0] += ri * ri;
-        s[1] += ri * zi;
+        s[0] = fma(ri, ri, s[0]);
+        s[1] = fma(ri, zi, s[1]);
+        i += (long long)gridDim.x * 256;
+        if (i < n)
+        {
+            pi = p[i];
+            qi = q[i];
+            xi = x[i];
+            ri = r[i];
+            di = invd[i];
+        }
     }
     StorePartials<2>(s, part, sh);
 }
 
-// First kernel of a BiCGSTAB iteration (launch number seq, iteration `it`): the tests
-// !(|r|^2 > tol^2 |b|^2) and |rho| < eps^2 |r0|^2 (a restart, done by the host), then
-// p = r + beta (p - w v), y = invd p. first: the state of a new solve; forced: no tests (the iteration
-// after a restart, whose (r . r) becomes |r0|^2); check: the tests alone.
-__global__ void __launch_bounds__(256) kBicgP(int n, int seq, int it, bool first, bool forced, bool check, double tol2,
-                                              const double* __restrict__ part, int np, const double* __restrict__ r,
+// First kernel of a BiCGSTAB iteration where the K product does not begin it itself: p = r + beta (p - w v),
+// y = invd p. check: the tests alone.
+__global__ void __launch_bounds__(256) kBicgP(int n, const StepArgs a, const double* __restrict__ r,
                                               const double* __restrict__ v, const double* __restrict__ invd,
-                                              double* __restrict__ p, double* __restrict__ y,
-                                              KrylovState* __restrict__ st)
+                                              double* __restrict__ p, double* __restrict__ y)
 {
     __shared__ double sh[8];
-    const KrylovState* in = st + (seq & 1);
-    KrylovState* out = st + ((seq + 1) & 1);
-    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    const int status = in->status, iters = in->iters;
-    const double oldRr = in->rr, oldBb = in->bb, oldRho = in->rho, alpha = in->alpha, w = in->w, oldR0 = in->r0sq;
-    if (status == kDone || (status == kRestart && !forced))
-    {
-        if (lead)
-        {
-            out->rr = oldRr;
-            out->bb = oldBb;
-            out->rho = oldRho;
-            out->alpha = alpha;
-            out->w = w;
-            out->r0sq = oldR0;
-            out->status = status;
-            out->iters = iters;
-        }
+    double beta;
+    const double w = a.st[a.seq & 1].w;
+    if (!BicgStep(a, sh, beta) || a.check)
         return;
-    }
-    double s[2];
-    SumPartials<2, kDotBlocks>(part, np, s, sh);
-    const double bb = first ? s[0] : oldBb, r0sq = first || forced ? s[0] : oldR0;
-    int now = kRunning;
-    if (!forced)
-    {
-        const double eps2 = 2.220446049250313e-16 * 2.220446049250313e-16;
-        if (!(s[0] > tol2 * bb))
-            now = kDone;
-        else if (!check && fabs(s[1]) < eps2 * r0sq)
-            now = kRestart;
-    }
-    if (lead)
-    {
-        out->rr = forced ? oldRr : s[0];  // after a restart the residual's norm is the one that was tested
-        out->bb = bb;
-        out->rho = now == kRestart ? oldRho : s[1];  // the restarted iteration's beta divides by the last rho
-        out->alpha = alpha;
-        out->w = w;
-        out->r0sq = r0sq;
-        out->status = now;
-        out->iters = it;
-    }
-    if (now != kRunning || check)
-        return;
-    const double beta = (s[1] / oldRho) * (alpha / w);
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
     {
-        const double pi = r[i] + beta * (p[i] - w * v[i]);
+        const double pi = fma(beta, fma(-w, v[i], p[i]), r[i]);
         p[i] = pi;
         y[i] = invd[i] * pi;
     }
@@ -618,48 +748,83 @@ __global__ void __launch_bounds__(256) kBicgS(int n, const double* __restrict__ 
                                               double* __restrict__ z, KrylovState* __restrict__ st)
 {
     __shared__ double sh[8];
-    if (st->status != kRunning)
-        return;
+    long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    const long long i0 = i < n ? i : n - 1;
+    double vi = v[i0], ri = r[i0], di = invd[i0];
+    const int status = st->status;
+    const double rho = st->rho;
     double d[1];
     SumPartials<1, kSpmvBlocks>(dotPart, np, d, sh);
-    const double alpha = st->rho / d[0];
+    if (status != kRunning)
+        return;
+    const double alpha = rho / d[0];
     if (blockIdx.x == 0 && threadIdx.x == 0)
         st->alpha = alpha;
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
+    while (i < n)
     {
-        const double si = -alpha * v[i] + r[i];
+        const double si = fma(-alpha, vi, ri);
         s[i] = si;
-        z[i] = invd[i] * si;
+        z[i] = di * si;
+        i += (long long)gridDim.x * 256;
+        if (i < n)
+        {
+            vi = v[i];
+            ri = r[i];
+            di = invd[i];
+        }
     }
 }
 
 // BiCGSTAB's w = (t . s) / (t . t) (0 when t = 0), x += alpha y + w z, r = s - w t, and the partials of
-// (r . r) and (r0 . r)
+// (r . r) and (r0 . r). FORM: y = invd p and z = invd s are formed here, and h = p - w v is left for the
+// next direction.
+template <bool FORM>
 __global__ void __launch_bounds__(256) kBicgUpdate(int n, const double* __restrict__ dotPart, int np,
                                                    const double* __restrict__ y, const double* __restrict__ z,
                                                    double* __restrict__ x, const double* __restrict__ s,
                                                    const double* __restrict__ t, double* __restrict__ r,
                                                    const double* __restrict__ r0, double* __restrict__ part,
-                                                   KrylovState* __restrict__ st)
+                                                   KrylovState* __restrict__ st, const double* __restrict__ invd,
+                                                   const double* __restrict__ p, const double* __restrict__ v,
+                                                   double* __restrict__ h)
 {
     __shared__ double sh[8];
-    if (st->status != kRunning)
-        return;
+    // the operands of a lane's first entry are in flight while the block adds the partials
+    long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    const long long i0 = i < n ? i : n - 1;
+    double si = s[i0], ti = t[i0], xi = x[i0], r0i = r0[i0];
+    double a = FORM ? p[i0] : y[i0], b = FORM ? v[i0] : z[i0], di = FORM ? invd[i0] : 0.0;
+    const int status = st->status;
+    const double alpha = st->alpha;
     double d[2];
     SumPartials<2, kSpmvBlocks>(dotPart, np, d, sh);
-    const double alpha = st->alpha, w = d[0] > 0.0 ? d[1] / d[0] : 0.0;
+    if (status != kRunning)
+        return;
+    const double w = d[0] > 0.0 ? d[1] / d[0] : 0.0;
     if (blockIdx.x == 0 && threadIdx.x == 0)
         st->w = w;
     double q[2] = {0.0, 0.0};
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
+    while (i < n)
     {
-        double xi = alpha * y[i] + x[i];
-        xi = w * z[i] + xi;
-        x[i] = xi;
-        const double ri = -w * t[i] + s[i];
+        const double yi = FORM ? di * a : a, zi = FORM ? di * si : b;
+        if constexpr (FORM)
+            h[i] = fma(-w, b, a);
+        x[i] = fma(w, zi, fma(alpha, yi, xi));
+        const double ri = fma(-w, ti, si);
         r[i] = ri;
-        q[0] += ri * ri;
-        q[1] += r0[i] * ri;
+        q[0] = fma(ri, ri, q[0]);
+        q[1] = fma(r0i, ri, q[1]);
+        i += (long long)gridDim.x * 256;
+        if (i < n)
+        {
+            si = s[i];
+            ti = t[i];
+            xi = x[i];
+            r0i = r0[i];
+            a = FORM ? p[i] : y[i];
+            b = FORM ? v[i] : z[i];
+            di = FORM ? invd[i] : 0.0;
+        }
     }
     StorePartials<2>(q, part, sh);
 }
@@ -796,12 +961,14 @@ public:
         const double tol2 = tol * tol;
         hipLaunchKernelGGL(kInvDiag, dim3((unsigned)((mN + 255) / 256)), blk, 0, mS, mN, mRev, mCt.row, mCt.col,
                            mCt.val, mK.row, mK.col, mK.val, invd);
+        const bool formed = Formed();
+        double* H = Y;  // BiCGSTAB, formed: p - w v
         if (cg)
             hipLaunchKernelGGL(kKrylovStart<true>, g, blk, 0, mS, mN, mRev, mCt.row, mCt.col, mCt.val, f, invd, b, x, R,
                                R0, P, V, part, state);
         else
             hipLaunchKernelGGL(kKrylovStart<false>, g, blk, 0, mS, mN, mRev, mCt.row, mCt.col, mCt.val, f, invd, b, x,
-                               R, R0, P, V, part, state);
+                               R, R0, formed ? H : P, V, part, state);
         int it = 0, seq = 0, restarts = 0, queued = 0;
         bool first = true, forced = false;
         KrylovState last{};
@@ -813,35 +980,59 @@ public:
             for (; it < end; it++, seq++)
             {
                 KrylovState* st = state + ((seq + 1) & 1);
+                KrylovState* tell = it + 1 == end && end < maxIt ? mBuf.host + (queued & 1) : nullptr;
+                const StepArgs step{seq, it, first, forced, false, tol2, part, np, state, tell};
+                first = forced = false;
                 if (cg)
                 {
-                    hipLaunchKernelGGL(kCgP, g, blk, 0, mS, mN, it, false, tol2, part, np, R0, P, state);
-                    const int nd = Product<kOneDot>(P, V, P, st, dotPart);
-                    hipLaunchKernelGGL(kCgUpdate, g, blk, 0, mS, mN, dotPart, nd, P, V, x, R, invd, R0, part, st);
+                    double* p = P;
+                    int nd;
+                    if (formed)
+                    {
+                        // the product reads the last p at other rows than it writes: two copies in turn
+                        double* old = it & 1 ? Y : P;
+                        p = it & 1 ? P : Y;
+                        nd = NodeProduct<kOneDot, kCgDirection>(nullptr, V, mMask, nullptr, dotPart, st,
+                                                                {R0, old, nullptr, p, step, nullptr, 0});
+                    }
+                    else
+                    {
+                        hipLaunchKernelGGL(kCgP, g, blk, 0, mS, mN, step, R0, P);
+                        nd = Product<kOneDot>(P, V, P, st, dotPart);
+                    }
+                    hipLaunchKernelGGL(kCgUpdate, g, blk, 0, mS, mN, dotPart, nd, p, V, x, R, invd, R0, part, st);
                     continue;
                 }
-                hipLaunchKernelGGL(kBicgP, g, blk, 0, mS, mN, seq, it, first, forced, false, tol2, part, np, R, V, invd,
-                                   P, Y, state);
-                first = forced = false;
+                if (formed)
+                {
+                    double* part2 = Z;  // 2 sums per block; dotPart is read by the kernel that writes these
+                    int nd = NodeProduct<kOneDot, kBicgDirection>(nullptr, V, mMask, R0, dotPart, st,
+                                                                  {R, H, invd, P, step, nullptr, 0});
+                    nd = NodeProduct<kTwoDots, kBicgHalfStep>(nullptr, T, mMask, nullptr, part2, st,
+                                                              {R, V, invd, S, {}, dotPart, nd});
+                    hipLaunchKernelGGL(kBicgUpdate<true>, g, blk, 0, mS, mN, part2, nd, nullptr, nullptr, x, S, T, R, R0,
+                                       part, st, invd, P, V, H);
+                    continue;
+                }
+                hipLaunchKernelGGL(kBicgP, g, blk, 0, mS, mN, step, R, V, invd, P, Y);
                 int nd = Product<kOneDot>(Y, V, R0, st, dotPart);
                 hipLaunchKernelGGL(kBicgS, g, blk, 0, mS, mN, dotPart, nd, R, V, invd, S, Z, st);
                 nd = Product<kTwoDots>(Z, T, S, st, dotPart);
-                hipLaunchKernelGGL(kBicgUpdate, g, blk, 0, mS, mN, dotPart, nd, Y, Z, x, S, T, R, R0, part, st);
+                hipLaunchKernelGGL(kBicgUpdate<false>, g, blk, 0, mS, mN, dotPart, nd, Y, Z, x, S, T, R, R0, part, st,
+                                   nullptr, nullptr, nullptr, nullptr);
             }
             const bool atEnd = it >= maxIt;
             if (atEnd)
             {
+                const StepArgs step{seq, it, first, forced, true, tol2, part, np, state, mBuf.host + (queued & 1)};
                 if (cg)
-                    hipLaunchKernelGGL(kCgP, dim3(1), blk, 0, mS, mN, it, true, tol2, part, np, R0, P, state);
+                    hipLaunchKernelGGL(kCgP, dim3(1), blk, 0, mS, mN, step, R0, P);
                 else
-                    hipLaunchKernelGGL(kBicgP, dim3(1), blk, 0, mS, mN, seq, it, first, forced, true, tol2, part, np, R,
-                                       V, invd, P, Y, state);
+                    hipLaunchKernelGGL(kBicgP, dim3(1), blk, 0, mS, mN, step, R, V, invd, P, Y);
                 seq++;
             }
             const int slot = queued & 1;
             if ((err = hipGetLastError()) != hipSuccess ||
-                (err = hipMemcpyAsync(mBuf.host + slot, state + (seq & 1), sizeof(KrylovState), hipMemcpyDeviceToHost,
-                                      mS)) != hipSuccess ||
                 (err = hipEventRecord(mBuf.arrived[slot], mS)) != hipSuccess)
                 break;
             queued++;
@@ -889,11 +1080,19 @@ private:
     {
         return std::max(1, std::min(kDotBlocks, (mN + 255) / 256));
     }
+    // whether the K products form the vectors they multiply
+    bool Formed() const
+    {
+        const char* v = std::getenv("NUTO_AMD_SOLVE_FORM");  // 0 / 1: never / wherever possible (tests)
+        if (!mFused || (v && v[0] == '0'))
+            return false;
+        return (v && v[0] == '1') || mNodes.nNodes <= kFormNodes;
+    }
     // y = C^T K C x for a full-length x whose dependent entries this fills
     void Operator(double* x, double* y)
     {
         if (mFused)
-            NodeProduct<kNoDots>(x, y, mMask, nullptr, nullptr, nullptr);
+            NodeProduct<kNoDots, kStored>(x, y, mMask, nullptr, nullptr, nullptr);
         else
             Constrained(x, y);
     }
@@ -911,12 +1110,12 @@ private:
     }
     // DOTS: the operator C^T K C with the dots' partials in `out`, their number returned; kNoDots: K alone
     template <int DOTS>
-    int Product(const double* x, double* y, const double* d, const KrylovState* st, double* out)
+    int Product(const double* x, double* y, const double* d, KrylovState* st, double* out)
     {
         if constexpr (DOTS == kNoDots)
         {
             if (mNode)
-                NodeProduct<kNoDots>(x, y, nullptr, nullptr, nullptr, nullptr);
+                NodeProduct<kNoDots, kStored>(x, y, nullptr, nullptr, nullptr, nullptr);
             else if (mN > 0)
                 hipLaunchKernelGGL(kCsrSpmv, dim3((unsigned)(((long long)mN * 16 + 255) / 256)), dim3(256), 0, mS, mN,
                                    mK.row, mK.col, mK.val, x, y);
@@ -925,28 +1124,28 @@ private:
         else
         {
             if (mFused)
-                return NodeProduct<DOTS>(x, y, mMask, d, out, st);
+                return NodeProduct<DOTS, kStored>(x, y, mMask, d, out, st);
             Constrained(const_cast<double*>(x), y);
             hipLaunchKernelGGL(kSpmvDots<DOTS>, dim3((unsigned)Grid()), dim3(256), 0, mS, (long long)mN, y, d, out, st);
             return Grid();
         }
     }
-    template <int DOTS>
+    template <int DOTS, int IN>
     int NodeProduct(const double* x, double* y, const unsigned char* mask, const double* d, double* out,
-                    const KrylovState* st)
+                    KrylovState* st, const FormedInput& in = {})
     {
         const NodeRows& nr = mNodes;
         const int g = std::min(kSpmvBlocks, (nr.nNodes + 3) / 4);
         const dim3 grid((unsigned)g), block(256);
         if (nr.c0 == 3 && nr.c1 == 1)
-            hipLaunchKernelGGL((kNodeSpmv<3, 1, DOTS>), grid, block, 0, mS, nr.nNodes, nr.nU, mK.row, mK.col, mK.val, x,
-                               y, mask, d, out, st);
+            hipLaunchKernelGGL((kNodeSpmv<3, 1, DOTS, IN>), grid, block, 0, mS, nr.nNodes, nr.nU, mK.row, mK.col, mK.val, x,
+                               y, mask, d, out, st, in);
         else if (nr.c0 == 3)
-            hipLaunchKernelGGL((kNodeSpmv<3, 0, DOTS>), grid, block, 0, mS, nr.nNodes, nr.nU, mK.row, mK.col, mK.val, x,
-                               y, mask, d, out, st);
+            hipLaunchKernelGGL((kNodeSpmv<3, 0, DOTS, IN>), grid, block, 0, mS, nr.nNodes, nr.nU, mK.row, mK.col, mK.val, x,
+                               y, mask, d, out, st, in);
         else
-            hipLaunchKernelGGL((kNodeSpmv<2, 0, DOTS>), grid, block, 0, mS, nr.nNodes, nr.nU, mK.row, mK.col, mK.val, x,
-                               y, mask, d, out, st);
+            hipLaunchKernelGGL((kNodeSpmv<2, 0, DOTS, IN>), grid, block, 0, mS, nr.nNodes, nr.nU, mK.row, mK.col, mK.val, x,
+                               y, mask, d, out, st, in);
         return g;
     }
 

@@ -12,7 +12,7 @@ import pytest
 
 import nuto_amd as N
 from pairs import Pair, make_mesh, to_dev
-from test_gpu_parity import le_params
+from test_gpu_parity import gdm_params, le_params
 
 pytestmark = pytest.mark.gpu
 
@@ -118,3 +118,33 @@ def test_bicgstab_restart(seed):
     want = np.linalg.solve(A, f)
     assert info["iterations"] < 200 and info["relative_residual"] <= 1e-13
     assert np.abs(x.cpu().numpy() - want).max() <= 1e-9 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("case,n", [("quad4", (1, 1)), ("quad4", (5, 4)), ("quad4", (100, 90)), ("hex8", (1, 1, 1)),
+                                    ("hex8", (21, 21, 20)), ("hex20", (2, 1, 2)), ("gdm", (1, 2, 1)),
+                                    ("gdm", (21, 21, 20))])
+@pytest.mark.parametrize("method", [N.SOLVER_CG, N.SOLVER_BICGSTAB])
+def test_formed_vectors_give_the_same_bits(case, n, method, monkeypatch):
+    """The K product that forms its input where it gathers it, against the same iteration with a kernel of
+    its own for every vector: one node per wave and several (more than 8192 nodes), every row structure,
+    limits inside and beyond a queued group. The operations and the order of the sums are the same."""
+    ct = N.QUAD4 if case == "quad4" else N.HEX8
+    dt = {"quad4": N.QUAD4, "hex20": N.HEX20}.get(case, N.HEX8)
+    X, C = make_mesh(ct, n, (1.0, 1.2, 0.9), jitter=0.1 if max(n) > 2 else 0.0)
+    dim = N.DIM[ct]
+    params = gdm_params() if case == "gdm" else le_params(dim)
+    p = Pair(ct, dt, X, C, *params, two_fields=case == "gdm")
+    ctx = p.context()
+    K = ctx.build_vector_matrix(*[to_dev(v) for v in p.inputs()])[1] if case == "gdm" else \
+        ctx.build_matrix(to_dev(np.zeros(p.n_u)))
+    xs = np.ones((p.nn, dim))
+    xs[p.ranks[:, :C.shape[1]].ravel()] = X[C.ravel(), :dim]
+    ctx.set_constraints(0, [(int(dim * r + c), []) for r in np.nonzero(xs[:, 0] < 1e-12)[0] for c in range(dim)])
+    f = to_dev(np.random.default_rng(4).uniform(-1.0, 1.0, len(ctx.pattern()[0]) - 1))
+    for k in (1, 2, 4, 7):
+        out = []
+        for form in ("0", "1"):
+            monkeypatch.setenv("NUTO_AMD_SOLVE_FORM", form)
+            x, info = ctx.solve(K, f, method=method, tol=1e-12, max_iter=k)
+            out.append((x.cpu().numpy(), info["iterations"], info["relative_residual"]))
+        assert out[0][1:] == out[1][1:] and np.array_equal(out[0][0], out[1][0])
