@@ -92,7 +92,9 @@ int nuto_create(nuto_ctx** ctx, int device);
 int nuto_destroy(nuto_ctx* ctx);
 const char* nuto_last_error(const nuto_ctx* ctx);
 /* Run subsequent kernels on this HIP stream (hipStream_t); NULL is the device's default (null)
- * stream. A new context uses a stream of its own until this is called. */
+ * stream. A new context uses a stream of its own until this is called. The calls of one context share
+ * its work memory (states and cell vectors of R, K and the adjoint, staged cell matrices, vectors of a
+ * solve): a caller that puts them on different streams orders the streams. */
 int nuto_set_stream(nuto_ctx* ctx, void* stream);
 int nuto_synchronize(nuto_ctx* ctx);
 
@@ -344,8 +346,8 @@ int nuto_batch_mesh_info(nuto_batch* batch, int mesh, long long* info /* 17 */);
 int nuto_batch_copy_pattern(nuto_batch* batch, int mesh, int* row_ptr, int* col);
 /* info[7] of a group: dof element type, meshes, dof nodes, cells, cell-matrix kernel of its
  * two-phase launch (0 by columns, 1 / 2 Gram form with one / two row nodes per lane, 3 Gram form
- * on the FP64 matrix cores, -1 the element's default until nuto_batch_autotune times each),
- * number of groups, cells per staging
+ * on the FP64 matrix cores, 4 rows by node tiles without cell matrices (tet4), -1 the element's
+ * default until nuto_batch_autotune times each), number of groups, cells per staging
  * chunk (0: the whole group, -1: not chosen yet) */
 int nuto_batch_group_info(nuto_batch* batch, int group, long long* info /* 7 */);
 /* per-cell (E, f_t, G_f) over all cells, meshes in the order they were added (host arrays) */

@@ -1,15 +1,16 @@
 // Row assembly of elements with few nodes and points (quad4; tet4) without staged cell matrices: a wave owns
-// the rows of 16 consecutive dof nodes.
+// the rows of 16 (quad4) or 8 (tet4) consecutive dof nodes.
 //
 // The rows of consecutive nodes are one segment of the CSR; it is built in LDS and written once, in
-// consecutive stores. Four lanes per node take its incident cells in turn: each forms the row blocks of one
-// cell (CellRows, the integration of the row-owner kernel), then the four add theirs to the segment one after
+// consecutive stores. Four (eight) lanes per node take its incident cells in turn: each forms the row blocks of one
+// cell (CellRows, the integration of the row-owner kernel), then they add theirs to the segment one after
 // the other, so every entry sums its cells in group order as setFromTriplets does (SimpleAssembler.cpp:149-155).
 // A node's blocks of all its cells would fit one lane, as in kAssembleRows, but that kernel has a quarter of
 // the lanes and reads and rewrites each entry in memory, 8 bytes at a time; a cell matrix kernel and a gather
 // (kCellMatrices, kGatherRowsWave) write and read 8 ND^2 bytes per cell more.
 // Measured, R + K of 40,000 quad4 cells, linear elasticity: row-owner kernel 26.5 us, tiles 11.9 us (14 MB
-// moved; 2526 waves, bound by the chain of the gathers and the four turns).
+// moved; 2526 waves, bound by the chain of the gathers and the four turns); tet4, 1350 cells, local damage, with 4
+// lanes per node 33 us, with 8 27 us, 33,000 cells 35.3 and 33.9 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -19,8 +20,15 @@
 namespace nuto_amd
 {
 
-constexpr int kTileLanes = 4;                  // lanes per node
-constexpr int kTileNodes = 64 / kTileLanes;    // nodes per wave
+// lanes per node (an inner node of a quad4 mesh has 4 cells, of a tet4 mesh about 24), nodes per wave
+constexpr int TileLanes(int dim)
+{
+    return dim == 2 ? 4 : 8;
+}
+constexpr int TileNodes(int dim)
+{
+    return 64 / TileLanes(dim);
+}
 constexpr size_t kTileMaxLds = 40 * 1024;      // segments beyond this leave too few waves per CU
 
 // Rows of the nodes [p0, p1); dynamic LDS: the largest segment of kTileNodes consecutive nodes.
@@ -28,6 +36,7 @@ template <int KIND, int DIM, int NNC, int NND, int NIP, bool WR>
 __global__ void __launch_bounds__(64) kNodeTile(const RowArgs A, int p0, int p1)
 {
     static_assert(KIND != kGradientDamage, "one dof type");
+    constexpr int kTileLanes = TileLanes(DIM), kTileNodes = TileNodes(DIM);
     extern __shared__ double seg[];
     __shared__ double sR[kTileNodes * DIM];
     const int lane = (int)threadIdx.x;

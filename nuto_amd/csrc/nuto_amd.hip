@@ -119,7 +119,7 @@ struct nuto_ctx
     // staged cell matrices and vectors of the two-phase generic assembly
     DevBuf keStage, reStage;
     int maxAdj = -1;  // largest node neighbourhood (LDS rows of the wave gather), from the node graph
-    long long maxWindow = -1;  // most neighbours of kTileNodes consecutive dof nodes (LDS of kNodeTile)
+    long long maxWindow = -1;  // most neighbours of a node tile's consecutive dof nodes (LDS of kNodeTile)
     int cellGram = -1;  // form of the 3D matrix assembly: 0 cell matrices by columns, 1 / 2 in Gram form with 1 / 2
                         // row nodes per lane, 3 on the matrix cores, 4 node tiles (tet4), -1 the element's default
 };
@@ -400,16 +400,17 @@ int CellFormEnv()
     return v && v[0] >= '0' && v[0] <= '4' ? v[0] - '0' : -1;
 }
 
-// LDS of kNodeTile for any launch over the context's nodes: the rows of the kTileNodes consecutive nodes
+// LDS of kNodeTile for any launch over the context's nodes: the rows of a tile's consecutive nodes
 // with the most neighbours
 size_t TileLds(nuto_ctx* ctx)
 {
     if (ctx->maxWindow < 0)
     {
         const std::vector<int>& ptr = ctx->graph.adjPtr;
+        const int nodes = TileNodes(ctx->dim);
         long long m = 0;
         for (int p = 0; p < ctx->graph.nNodes; p++)
-            m = std::max<long long>(m, (long long)ptr[std::min(p + kTileNodes, ctx->graph.nNodes)] - ptr[p]);
+            m = std::max<long long>(m, (long long)ptr[std::min(p + nodes, ctx->graph.nNodes)] - ptr[p]);
         ctx->maxWindow = m;
     }
     return (size_t)ctx->maxWindow * ctx->dim * ctx->dim * sizeof(double);
@@ -422,7 +423,8 @@ bool LaunchTiles(nuto_ctx* ctx, const RowArgs& a, bool wr, int p0, int p1, hipSt
     const size_t lds = TileLds(ctx);
     if (lds > kTileMaxLds)
         return false;
-    const dim3 grid((unsigned)((p1 - p0 + kTileNodes - 1) / kTileNodes));
+    constexpr int nodes = TileNodes(DIM);
+    const dim3 grid((unsigned)((p1 - p0 + nodes - 1) / nodes));
     if (wr)
         hipLaunchKernelGGL((kNodeTile<KIND, DIM, NNC, NND, NIP, true>), grid, dim3(64), lds, stream, a, p0, p1);
     else
@@ -513,16 +515,34 @@ void LaunchCellMatrices(const RowArgs& a, int form, int c0, int c1, double* ke, 
         LaunchGram<KIND, NNC, NND, NIP, 1, false>(a, c0, c1, ke, re, stream);
 }
 
+// The form of a launch over `nodes` dof nodes (a batch's autotune measures every form). Four-node tetrahedra:
+// node tiles, but in small meshes a node's 24 or so cells in turns of 8 take longer than two launches.
+// Measured, R + K, us, elasticity / local damage, tiles against columns and gather: 105 nodes 13.8 / 15.4
+// against 10.6 / 11.5, 990 nodes 24.6 / 26.9 against 22.8 / 23.6, 2184 nodes 25.3 / 27.7 against 26.7 / 28.1,
+// 6460 nodes 31.3 / 33.9 against 38.3 / 40.4.
+// Ten- and twenty-node elements with local damage: the matrix cores, which take the LDS reads out of its two
+// products; with one product (elasticity), two Grams (UNILATERAL damage application) and on hex8 the Gram
+// lanes are as fast or faster. Measured, R + K, us, Gram / matrix cores / columns: hex20 local damage, 12,144
+// cells 394 / 367 / 600, 1320 cells 58.5 / 52.4 / 93.9, 120 cells 24.2 / 21.7 / 56.6; elasticity 315 / 340 / 461,
+// 46.0 / 44.5 / 71.4, 19.3 / 19.7 / 43.8; tet10 local damage, 20,160 cells 139 / 132 / 155, 5940 cells 47.2 / 44.2 /
+// 50.3; elasticity 124 / 126 / 126, 43.2 / 40.6 / 42.8; hex8 local damage, 63,960 cells 302 / 316 / 391.
+template <int KIND, int NND>
+int DefaultForm(const RowArgs& a, int nodes)
+{
+    if (NND == 4)
+        return nodes >= 2048 ? 4 : 0;
+    const bool two = KIND == kLocalDamage && a.P.damage_application == 0;
+    return (NND == 20 || NND == 10) && two ? 3 : 1;
+}
+
 template <int KIND, int NNC, int NND, int NIP>
 void LaunchTwoPhaseT(nuto_ctx* ctx, const RowArgs& a, bool wr, int c0, int c1, int p0, int p1, hipStream_t stream)
 {
     constexpr int ND = NND * 3;
     if (c1 <= c0 || p1 <= p0)
         return;
-    // the Gram form wins on the hexahedra (32 and 200 lanes per cell), the column kernel on the ten-node
-    // tetrahedra, node tiles on the four-node ones (a batch's autotune measures every form)
     const int env = CellFormEnv();
-    const int form = env >= 0 ? env : (ctx->cellGram >= 0 ? ctx->cellGram : (NND == 4 ? 4 : (NND == 10 ? 0 : 1)));
+    const int form = env >= 0 ? env : (ctx->cellGram >= 0 ? ctx->cellGram : DefaultForm<KIND, NND>(a, p1 - p0));
     if constexpr (NND == 4)
     {
         if (form == 4 && LaunchTiles<KIND, 3, NNC, NND, NIP>(ctx, a, wr, p0, p1, stream))

@@ -1,4 +1,4 @@
-"""Node tiles (rows of 16 consecutive nodes built in LDS) at the edges of the tiles: fewer nodes than one
+"""Node tiles (rows of 16 or 8 consecutive nodes built in LDS) at the edges of the tiles: fewer nodes than one
 tile, exactly one, one node more; nodes with more cells than the lanes of a node take in one turn; and a node
 whose rows do not fit in LDS, which leaves the tiles for the kernels behind them. R and K against the oracle.
 """
@@ -40,9 +40,13 @@ def test_quad4(mesh, rule):
     check(p, u, None)
 
 
-@pytest.mark.parametrize("n", [(1, 1, 1), (3, 1, 1), (3, 3, 3)])
+@pytest.mark.parametrize("n", [(1, 1, 1), (3, 1, 1), (3, 3, 3), (15, 11, 9), (15, 12, 9)])
 @pytest.mark.parametrize("kind", ["elastic", "local", "unilateral"])
-def test_tet4(n, kind):
+@pytest.mark.parametrize("form", ["", "4"])
+def test_tet4(n, kind, form, monkeypatch):
+    """on either side of the size from which on the tiles are taken (2048 nodes), and the tiles at every size"""
+    if form:
+        monkeypatch.setenv("NUTO_AMD_CELL_GRAM", form)
     X, C = make_mesh(N.TET4, n, lengths=tuple(float(v) for v in n), jitter=0.1)
     par = {"elastic": lambda: le_params(3), "local": ld_params, "unilateral": lambda: ld_params(N.UNILATERAL)}[kind]()
     p = Pair(N.TET4, N.TET4, X, C, *par, two_fields=False)
