@@ -51,16 +51,39 @@ struct RowArgs
     double* K;
 };
 
-// The strain of a local-damage point decides whether it loads (kappa' is 1 where the equivalent strain
-// equals the history, as it does right after an update). Every kernel that forms that strain goes through
-// the functions of this file and Mises3, which name each fused multiply-add: left to the compiler, a b + c d
-// is contracted one way in one kernel and the other way in the next, and the last bit differs.
+// The strain of a local-damage point, and the nonlocal strain of a gradient-damage point, decide whether it
+// loads (kappa' is 1 where they equal the history, as they do right after an update). So every kernel forms
+// them alike, bit for bit: J and the reference gradient R = sum u_n dN_n/dxi^T node by node (NodalGradient, or
+// the same products in the same order where one lane sums one entry), Inverse<3>, StrainOfGradient and Mises3;
+// the nonlocal strain as the sum of N_n e_n node by node. Each names its fused multiply-adds: left to the
+// compiler, a b + c d is contracted one way in one kernel and the other way in the next, and the last bit differs.
+// g_ij = sum_n v_n[i] dN_n[j]; v: node n's DIM values at v[STRIDE n]
+template <int DIM, int N, int STRIDE>
+__device__ inline void NodalGradient(const double* v, const double* dN, double g[DIM][DIM])
+{
+#pragma unroll
+    for (int i = 0; i < DIM; i++)
+#pragma unroll
+        for (int j = 0; j < DIM; j++)
+            g[i][j] = 0.0;
+#pragma unroll
+    for (int n = 0; n < N; n++)
+#pragma unroll
+        for (int i = 0; i < DIM; i++)
+        {
+            const double x = v[STRIDE * n + i];
+#pragma unroll
+            for (int j = 0; j < DIM; j++)
+                g[i][j] = fma(x, dN[n * DIM + j], g[i][j]);
+        }
+}
+
 template <int DIM>
 __device__ inline double Inverse(const double J[DIM][DIM], double inv[DIM][DIM])
 {
     if constexpr (DIM == 2)
     {
-        const double det = J[0][0] * J[1][1] - J[1][0] * J[0][1];
+        const double det = fma(J[0][0], J[1][1], -(J[1][0] * J[0][1]));
         const double id = 1.0 / det;
         inv[0][0] = J[1][1] * id;
         inv[0][1] = -J[0][1] * id;
@@ -96,10 +119,10 @@ __device__ inline void Grad(const double* dNd, int b, const double inv[DIM][DIM]
 #pragma unroll
     for (int j = 0; j < DIM; j++)
     {
-        double s = 0.0;
+        double s = dNd[b * DIM] * inv[0][j];
 #pragma unroll
-        for (int i = 0; i < DIM; i++)
-            s += dNd[b * DIM + i] * inv[i][j];
+        for (int i = 1; i < DIM; i++)
+            s = fma(dNd[b * DIM + i], inv[i][j], s);
         g[j] = s;
     }
 }
@@ -206,42 +229,41 @@ __device__ inline void CellRows(const RowArgs& A, const CellNodes<KIND, DIM, NNC
                     const double* dNc = t + 1;
                     const double* Nd = dNc + NNC * DIM;
                     const double* dNd = Nd + NND;
-                    double J[DIM][DIM];
-    #pragma unroll
-                    for (int i = 0; i < DIM; i++)
-    #pragma unroll
-                        for (int j = 0; j < DIM; j++)
-                        {
-                            double s = 0.0;
-    #pragma unroll
-                            for (int k = 0; k < NNC; k++)
-                                s += c.X[k][i] * dNc[k * DIM + j];
-                            J[i][j] = s;
-                        }
-                    double inv[DIM][DIM];
+                    double J[DIM][DIM], inv[DIM][DIM];
+                    NodalGradient<DIM, NNC, DIM>(&c.X[0][0], dNc, J);
                     const double detJ = Inverse<DIM>(J, inv);
                     const double s = detJ * w;
 
                     // strain (Voigt 2D [xx,yy,xy], 3D [xx,yy,zz,yz,zx,xy]), nonlocal value and gradient
                     constexpr int NV = DIM == 2 ? 3 : 6;
                     double eps[NV];
-    #pragma unroll
-                    for (int i = 0; i < NV; i++)
-                        eps[i] = 0.0;
                     double eN = 0.0, ge[3] = {0.0, 0.0, 0.0};
-    #pragma unroll
-                    for (int b = 0; b < NND; b++)
+                    if constexpr (KIND != kLocalDamage)
                     {
-                        double g[DIM];
-                        Grad<DIM, NND>(dNd, b, inv, g);
-                        AddStrain<DIM>(g, c.U[b], eps);
-                        if constexpr (KIND == kGradientDamage)
+                        // the strain decides nothing here, and every dN_n/dX is needed anyway
+    #pragma unroll
+                        for (int i = 0; i < NV; i++)
+                            eps[i] = 0.0;
+    #pragma unroll
+                        for (int b = 0; b < NND; b++)
                         {
-                            eN += Nd[b] * c.EE[b];
-                            ge[0] += g[0] * c.EE[b];
-                            ge[1] += g[1] * c.EE[b];
-                            ge[2] += g[2] * c.EE[b];
+                            double g[DIM];
+                            Grad<DIM, NND>(dNd, b, inv, g);
+                            AddStrain<DIM>(g, c.U[b], eps);
+                            if constexpr (KIND == kGradientDamage)
+                            {
+                                eN = fma(Nd[b], c.EE[b], eN);
+                                ge[0] += g[0] * c.EE[b];
+                                ge[1] += g[1] * c.EE[b];
+                                ge[2] += g[2] * c.EE[b];
+                            }
                         }
+                    }
+                    else
+                    {
+                        double Ru[DIM][DIM];
+                        NodalGradient<DIM, NND, DIM>(&c.U[0][0], dNd, Ru);
+                        StrainOfGradient(&Ru[0][0], inv, eps);
                     }
 
                     // row node a
@@ -373,19 +395,25 @@ __device__ inline void CellRows(const RowArgs& A, const CellNodes<KIND, DIM, NNC
                             if constexpr (DIM == 2)
                             {
                                 const double sa0 = s * ga[0], sa1 = s * ga[1];
-                                kb[0] += C11 * sa0 * gb[0] + C33 * sa1 * gb[1];
-                                kb[1] += C12 * sa0 * gb[1] + C33 * sa1 * gb[0];
-                                kb[2] += C12 * sa1 * gb[0] + C33 * sa0 * gb[1];
-                                kb[3] += C11 * sa1 * gb[1] + C33 * sa0 * gb[0];
+                                // named, so that K has the same bits with and without R
+                                kb[0] = fma(C33 * sa1, gb[1], fma(C11 * sa0, gb[0], kb[0]));
+                                kb[1] = fma(C33 * sa1, gb[0], fma(C12 * sa0, gb[1], kb[1]));
+                                kb[2] = fma(C33 * sa0, gb[1], fma(C12 * sa1, gb[0], kb[2]));
+                                kb[3] = fma(C33 * sa0, gb[0], fma(C11 * sa1, gb[1], kb[3]));
                             }
                             else
                             {
-                                const double dot = ga[0] * gb[0] + ga[1] * gb[1] + ga[2] * gb[2];
+                                const double dot = fma(ga[2], gb[2], fma(ga[1], gb[1], ga[0] * gb[0]));
     #pragma unroll
                                 for (int i = 0; i < 3; i++)
     #pragma unroll
                                     for (int j = 0; j < 3; j++)
-                                        kb[i * F + j] += c1 * ga[i] * gb[j] + c2 * gb[i] * ga[j] + (i == j ? c2 * dot : 0.0);
+                                    {
+                                        double& k = kb[i * F + j];
+                                        k = fma(c2 * gb[i], ga[j], fma(c1 * ga[i], gb[j], k));
+                                        if (i == j)
+                                            k = fma(c2, dot, k);
+                                    }
                                 if constexpr (KIND == kLocalDamage)
                                 {
                                     double wb[3];
@@ -394,7 +422,7 @@ __device__ inline void CellRows(const RowArgs& A, const CellNodes<KIND, DIM, NNC
                                     for (int i = 0; i < 3; i++)
     #pragma unroll
                                         for (int j = 0; j < 3; j++)
-                                            kb[i * F + j] += va[i] * wb[j];
+                                            kb[i * F + j] = fma(va[i], wb[j], kb[i * F + j]);
                                 }
                                 if constexpr (KIND == kGradientDamage)
                                 {

@@ -41,17 +41,7 @@ __device__ inline double CellJacobian(const RowArgs& A, int cell, const double* 
             X[k][2] = A.z[n];
     }
     double J[DIM][DIM];
-#pragma unroll
-    for (int i = 0; i < DIM; i++)
-#pragma unroll
-        for (int j = 0; j < DIM; j++)
-        {
-            double s = 0.0;
-#pragma unroll
-            for (int k = 0; k < NNC; k++)
-                s += X[k][i] * dNc[k * DIM + j];
-            J[i][j] = s;
-        }
+    NodalGradient<DIM, NNC, DIM>(&X[0][0], dNc, J);
     return Inverse<DIM>(J, inv);
 }
 

@@ -92,7 +92,7 @@ __device__ inline void CellIpRecords(const RowArgs& A, int c1, int cellBase, dou
             const int row = e / 3, m = e - 3 * row;
 #pragma unroll
             for (int n = 0; n < NNC; n++)
-                v += sX[cl][n * 3 + row] * dNc[n * 3 + m];
+                v = fma(sX[cl][n * 3 + row], dNc[n * 3 + m], v);
         }
         else
         {
@@ -100,7 +100,7 @@ __device__ inline void CellIpRecords(const RowArgs& A, int c1, int cellBase, dou
             const int row = (e - 9) / 3, m = e - 9 - 3 * row;
 #pragma unroll
             for (int n = 0; n < NND; n++)
-                v += sU[cl][n * 3 + row] * dNd[n * 3 + m];
+                v = fma(sU[cl][n * 3 + row], dNd[n * 3 + m], v);
         }
         sJG[cl][ip][e] = v;
     }

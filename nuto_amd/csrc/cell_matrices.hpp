@@ -74,14 +74,14 @@ __global__ void __launch_bounds__(64) kCellMatrices(const RowArgs A, int c0, int
                 const int i = k / 3, m = k - 3 * i;
 #pragma unroll
                 for (int n = 0; n < NNC; n++)
-                    v += sX[grp][n * 4 + i] * dNc[n * 3 + m];
+                    v = fma(sX[grp][n * 4 + i], dNc[n * 3 + m], v);
             }
             else
             {
                 const int i = (k - 9) / 3, m = k - 9 - 3 * i;
 #pragma unroll
                 for (int n = 0; n < NND; n++)
-                    v += sU[grp][n * 4 + i] * dNd[n * 3 + m];
+                    v = fma(sU[grp][n * 4 + i], dNd[n * 3 + m], v);
             }
             sJG[grp][tt] = v;
         }

@@ -70,10 +70,6 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
     constexpr int NV = DIM == 2 ? 3 : 6;
     constexpr int SX = NNC * DIM | 1, SU = NND * F | 1;  // odd strides: consecutive cells on other banks
     constexpr int PR = GD ? DIM * DIM + DIM + 1 : (DIM == 2 ? 5 : 9);  // doubles per point in LDS (odd)
-    // the strain: the gradient H = (sum u_n dN_n/dxi^T) J^-1 as the cell-matrix kernels form it, or the sum
-    // of B_n u_n as the row-owner kernel does, whichever assembles this rule's matrix: a history that was
-    // just updated then counts as loading there too (kappa' is 1 where the two are equal)
-    constexpr bool kSumForm = DIM == 2 || GD || NIP > 27;
     static_assert(CPW >= 1, "a wave holds a cell's points");
     constexpr int IN = CPW * (SX + SU), RES = CPW * NIP * PR;
     __shared__ double pool[IN > RES ? IN : RES];  // the cells' nodes, then the points' results
@@ -153,29 +149,15 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
         {
 #pragma unroll
             for (int b = 0; b < NND; b++)
-                eN += Nd[b] * U[b * F + DIM];
+                eN = fma(Nd[b], U[b * F + DIM], eN);
         }
         double eps[NV], inv[DIM][DIM], ge[3] = {0.0, 0.0, 0.0}, s = 0.0;
         if constexpr (kGeometry)
         {
             double J[DIM][DIM];
-#pragma unroll
-            for (int i = 0; i < DIM; i++)
-#pragma unroll
-                for (int k = 0; k < DIM; k++)
-                    J[i][k] = 0.0;
-#pragma unroll
-            for (int n = 0; n < NNC; n++)
-#pragma unroll
-                for (int i = 0; i < DIM; i++)
-                {
-                    const double x = sX[cl * SX + n * DIM + i];
-#pragma unroll
-                    for (int k = 0; k < DIM; k++)
-                        J[i][k] += x * dNc[n * DIM + k];
-                }
+            NodalGradient<DIM, NNC, DIM>(sX + cl * SX, dNc, J);
             s = Inverse<DIM>(J, inv) * t[0];
-            if constexpr (kSumForm)
+            if constexpr (DIM == 2 || GD)
             {
 #pragma unroll
                 for (int i = 0; i < NV; i++)
@@ -197,21 +179,9 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
             }
             else
             {
-                double R[9];
-#pragma unroll
-                for (int i = 0; i < 9; i++)
-                    R[i] = 0.0;
-#pragma unroll
-                for (int n = 0; n < NND; n++)
-#pragma unroll
-                    for (int i = 0; i < 3; i++)
-                    {
-                        const double u = U[n * F + i];
-#pragma unroll
-                        for (int k = 0; k < 3; k++)
-                            R[3 * i + k] += u * dNd[n * 3 + k];
-                    }
-                StrainOfGradient(R, inv, eps);
+                double R[DIM][DIM];
+                NodalGradient<DIM, NND, F>(U, dNd, R);
+                StrainOfGradient(&R[0][0], inv, eps);
             }
         }
 

@@ -56,17 +56,23 @@ inline LawParams MakeDerived(LawParams p)
     return p;
 }
 
+// The functions below name each fused multiply-add and keep the compiler from fusing more: it would fuse one
+// way in one kernel and the other way in the next, and a matrix assembled with and without R, or a point's
+// side of a comparison, would differ in the last bit.
+
 // B_a^T v for a 3D strain-type 6-vector v: component i collects the rows of B_a that act on u_i
 __device__ __host__ inline void BTv3(const double g[3], const double v[6], double o[3])
 {
-    o[0] = g[0] * v[0] + g[2] * v[4] + g[1] * v[5];
-    o[1] = g[1] * v[1] + g[2] * v[3] + g[0] * v[5];
-    o[2] = g[2] * v[2] + g[1] * v[3] + g[0] * v[4];
+#pragma clang fp contract(off)
+    o[0] = fma(g[1], v[5], fma(g[2], v[4], g[0] * v[0]));
+    o[1] = fma(g[0], v[5], fma(g[2], v[3], g[1] * v[1]));
+    o[2] = fma(g[0], v[4], fma(g[1], v[3], g[2] * v[2]));
 }
 
 // DamageLawExponential (DamageLawExponential.h:39-52)
 __device__ __host__ inline void DamageExp(double kappa, double k0, double beta, double alpha, double& w, double& dw)
 {
+#pragma clang fp contract(off)
     if (kappa < k0)
     {
         w = 0.0;
@@ -76,13 +82,14 @@ __device__ __host__ inline void DamageExp(double kappa, double k0, double beta, 
     const double ex = exp(beta * (k0 - kappa));
     const double ik = 1.0 / kappa;
     const double r = k0 * ik;
-    w = 1.0 - r * (1.0 - alpha + alpha * ex);
-    dw = r * ((ik + beta) * alpha * ex + (1.0 - alpha) * ik);
+    w = fma(-r, fma(alpha, ex, 1.0 - alpha), 1.0);
+    dw = r * fma((ik + beta) * alpha, ex, (1.0 - alpha) * ik);
 }
 
 // ModifiedMisesStrainNorm<3> value and derivative (ModifiedMisesStrainNorm.h:70-84,136-146,231-268)
 __device__ __host__ inline double Mises3(const double e[6], double nu, double k, double d[6])
 {
+#pragma clang fp contract(off)
     const double K1 = (k - 1.0) / (2.0 * k * (1.0 - 2.0 * nu));
     const double K2 = 3.0 / (k * (1.0 + nu) * (1.0 + nu));
     const double I1 = e[0] + e[1] + e[2];
@@ -100,9 +107,9 @@ __device__ __host__ inline double Mises3(const double e[6], double nu, double k,
         const double h = 0.5 / A;
         const double t = 2.0 * K1 * K1 * I1;
         const double K23 = K2 * (1.0 / 3.0);
-        d[0] = K1 + h * (t + K23 * (2.0 * e[0] - e[1] - e[2]));
-        d[1] = K1 + h * (t + K23 * (2.0 * e[1] - e[0] - e[2]));
-        d[2] = K1 + h * (t + K23 * (2.0 * e[2] - e[0] - e[1]));
+        d[0] = fma(h, fma(K23, 2.0 * e[0] - e[1] - e[2], t), K1);
+        d[1] = fma(h, fma(K23, 2.0 * e[1] - e[0] - e[2], t), K1);
+        d[2] = fma(h, fma(K23, 2.0 * e[2] - e[0] - e[1], t), K1);
         d[3] = h * K2 * 0.5 * e[3];
         d[4] = h * K2 * 0.5 * e[4];
         d[5] = h * K2 * 0.5 * e[5];
@@ -121,22 +128,23 @@ struct DamageStress3
 __device__ __host__ inline void ElasticDamage3K(const double e[6], double omega, double m3K, double m2G, int app,
                                                 DamageStress3& o)
 {
+#pragma clang fp contract(off)
     const double eV = (e[0] + e[1] + e[2]) * (1.0 / 3.0);
     const double H = (app == 1 && eV < 0.0) ? 0.0 : 1.0;
-    const double sV = (1.0 - omega * H) * m3K * eV;
+    const double wV = fma(-omega, H, 1.0), sV = wV * m3K * eV;
     const double d2G = (1.0 - omega) * m2G;
     for (int i = 0; i < 3; i++)
     {
         const double dev = e[i] - eV;
-        o.sig[i] = sV + d2G * dev;
-        o.dsdw[i] = -m3K * eV * H - m2G * dev;
+        o.sig[i] = fma(d2G, dev, sV);
+        o.dsdw[i] = fma(-m2G, dev, -m3K * eV * H);
     }
     for (int i = 3; i < 6; i++)
     {
         o.sig[i] = d2G * 0.5 * e[i];
         o.dsdw[i] = -m2G * 0.5 * e[i];
     }
-    o.alpha_v = m3K * (1.0 - omega * H);
+    o.alpha_v = m3K * wV;
     o.alpha_d = d2G;
 }
 

@@ -138,25 +138,93 @@ def test_generic_vectors_history_and_fields(ct, dt, n, rule, kind, monkeypatch):
     assert np.array_equal(state[2].view(p.nip, p.ncells).T.cpu().numpy(), kappa[:, :, 0].cpu().numpy())
 
 
-@pytest.mark.parametrize("ct,dt,n,rule,forms", [(N.HEX8, N.HEX8, (4, 3, 3), (0, 2), "0123"), (N.HEX8, N.HEX8, (2, 2, 2), (0, 4), "0"),
-                                                (N.HEX8, N.HEX20, (3, 2, 2), (0, 3), "0123"), (N.TET4, N.TET4, (3, 3, 3), (1, 1), "0123"),
-                                                (N.TET4, N.TET10, (2, 2, 2), (1, 2), "0123")])
-def test_local_damage_loads_at_the_updated_history(ct, dt, n, rule, forms, monkeypatch):
-    """Right after a history update every point it raised is loading: the tangent there equals the tangent
-    at a history lower by 1e-10 of itself (omega differs by at most 1e-8 of the entries' magnitude), in every
-    form of the cell matrices."""
-    X, C = make_mesh(ct, n, lengths=tuple(float(v) for v in n), jitter=0.1)
+# local damage: (coordinate element, dof element, cells, rule, forms of the matrix assembly)
+LOCAL = [(N.HEX8, N.HEX8, (4, 3, 3), (0, 2), "0123"), (N.HEX8, N.HEX8, (2, 2, 2), (0, 3), "0123"),
+         (N.HEX8, N.HEX8, (2, 2, 2), (0, 4), "0"), (N.HEX8, N.HEX20, (3, 2, 2), (0, 3), "0123"),
+         (N.TET4, N.TET4, (3, 3, 3), (1, 1), "01234"), (N.TET4, N.TET10, (2, 2, 2), (1, 2), "0123"),
+         (N.TET10, N.TET10, (2, 2, 2), (1, 2), "0123")]
+
+
+def tet10_mesh(n):
+    """quadratic tetrahedra with curved edges"""
+    X, C = make_mesh(N.TET4, n, lengths=tuple(float(v) for v in n), jitter=0.1)
+    C10, nn = N.dof_layer(N.TET4, C, N.TET10)
+    mid = X[C[:, [0, 1, 0, 0, 2, 1]]] + X[C[:, [1, 2, 2, 3, 3, 3]]]
+    X10 = np.zeros((nn, 3))
+    X10[C10[:, :4]] = X[C]
+    X10[C10[:, 4:]] = 0.5 * mid
+    edge = np.unique(C10[:, 4:])
+    X10[edge] += S.uniform(0x53, 3 * len(edge), -0.02, 0.02).reshape(-1, 3)
+    return X10, C10
+
+
+def at_updated_history(ct, dt, n, rule):
+    """A context, displacements, the history right after an update with them, and a history lower by 1e-10 of
+    itself, at which every point that the update raised is loading for certain."""
+    X, C = tet10_mesh(n) if ct == N.TET10 else make_mesh(ct, n, lengths=tuple(float(v) for v in n), jitter=0.1)
     p = Pair(ct, dt, X, C, *ld_params(), two_fields=False, rule=rule)
     u, _, kap = p.inputs()
     ctx = p.context()
     du, dk = to_dev(u), to_dev(kap)
     ctx.update_history(du, None, dk)
-    low = dk * (1.0 - 1e-10)
-    for form in forms:
-        monkeypatch.setenv("NUTO_AMD_CELL_GRAM", form)
-        K, want = (ctx.build_matrix(du, None, k).cpu().numpy() for k in (dk, low))
-        # points that the update did not raise (history above the strain) load in neither
-        assert np.abs(K - want).max() <= 1e-7 * np.abs(want).max()
+    return p, ctx, du, dk, dk * (1.0 - 1e-10)
+
+
+def check_loading(matrix, updated, low):
+    """omega differs by at most 1e-8 of the entries' magnitude between the two histories; points that the update
+    did not raise (history above the strain) load in neither"""
+    K, want = matrix(updated), matrix(low)
+    assert np.abs(K - want).max() <= 1e-7 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("ct,dt,n,rule,forms", LOCAL)
+def test_local_damage_loads_at_the_updated_history(ct, dt, n, rule, forms, monkeypatch):
+    """Right after a history update every point it raised is loading: the tangent there equals the tangent
+    at a history lower by 1e-10 of itself, in every form of the cell matrices and in the row-owner kernel."""
+    _, ctx, du, dk, low = at_updated_history(ct, dt, n, rule)
+    for form in forms + "r":
+        if form == "r":
+            monkeypatch.setenv("NUTO_AMD_TWO_PHASE", "0")
+        else:
+            monkeypatch.setenv("NUTO_AMD_CELL_GRAM", form)
+        check_loading(lambda k: ctx.build_matrix(du, None, k).cpu().numpy(), dk, low)
+
+
+def test_local_damage_loads_at_the_updated_history_in_large_tet4_meshes():
+    """beyond 2048 nodes, where the rows come from node tiles by default"""
+    _, ctx, du, dk, low = at_updated_history(N.TET4, N.TET4, (15, 12, 9), (1, 1))
+    check_loading(lambda k: ctx.build_matrix(du, None, k).cpu().numpy(), dk, low)
+
+
+@pytest.mark.parametrize("ct,dt,n,rule,forms", [v for v in LOCAL if v[:2] != (N.TET10, N.TET10) and v[3] not in ((0, 4),) and
+                                                (v[1] == N.HEX20 or v[3] != (0, 3))])
+def test_local_damage_loads_at_the_updated_history_in_batches(ct, dt, n, rule, forms, monkeypatch):
+    """the launch modes of a batch (its meshes take each element's default rule)"""
+    p, _, du, dk, low = at_updated_history(ct, dt, n, rule)
+    b = N.Batch()
+    b.set_integrand(p.params_dev)
+    b.add_mesh(ct, dt, p.X, p.C, p.ranks, p.nn)
+    b.build()
+    for mode in range(7):
+        for form in forms if mode >= 5 else forms[:1]:
+            monkeypatch.setenv("NUTO_AMD_CELL_GRAM", form)
+            check_loading(lambda k: b.assemble(du, None, k, mode=mode)[1].cpu().numpy(), dk, low)
+
+
+@pytest.mark.parametrize("rule", [(0, 2), (0, 3), (0, 4)])
+@pytest.mark.parametrize("env", [{}, {"NUTO_AMD_GDM_PREPASS": "0"}, {"NUTO_AMD_GDM_PREPASS": "1"}, {"NUTO_AMD_GENERIC": "1"}])
+def test_gradient_damage_loads_at_the_updated_history(rule, env, monkeypatch):
+    """The same for gradient damage, whose nonlocal strain decides: the node kernel with and without the
+    pre-pass, the row-owner kernel, and the rules that only the latter has."""
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    X, C = make_mesh(N.HEX8, (4, 3, 3), lengths=(4.0, 3.0, 3.0), jitter=0.1)
+    p = Pair(N.HEX8, N.HEX8, X, C, *gdm_params(), two_fields=True, rule=rule)
+    u, e, kap = p.inputs()
+    ctx = p.context()
+    du, de, dk = to_dev(u), to_dev(e), to_dev(kap)
+    ctx.update_history(du, de, dk)
+    check_loading(lambda k: ctx.build_matrix(du, de, k).cpu().numpy(), dk, dk * (1.0 - 1e-10))
 
 
 @pytest.mark.parametrize("n,jitter", [((15, 15, 15), 0.0), ((15, 15, 15), 0.1), ((16, 15, 15), 0.0)])
