@@ -94,7 +94,8 @@ const char* nuto_last_error(const nuto_ctx* ctx);
 /* Run subsequent kernels on this HIP stream (hipStream_t); NULL is the device's default (null)
  * stream. A new context uses a stream of its own until this is called. The calls of one context share
  * its work memory (states and cell vectors of R, K and the adjoint, staged cell matrices, vectors of a
- * solve): a caller that puts them on different streams orders the streams. */
+ * solve): work on a newly set stream waits for the work on the last one. Graphs captured from these calls
+ * share that memory as well; a caller that launches several orders them. */
 int nuto_set_stream(nuto_ctx* ctx, void* stream);
 int nuto_synchronize(nuto_ctx* ctx);
 
@@ -317,7 +318,8 @@ typedef struct nuto_batch nuto_batch;
 int nuto_batch_create(nuto_batch** batch, int device);
 int nuto_batch_destroy(nuto_batch* batch);
 const char* nuto_batch_last_error(const nuto_batch* batch);
-int nuto_batch_set_stream(nuto_batch* batch, void* stream); /* non-NULL for graph replay (mode -1) */
+/* non-NULL for graph replay (mode -1); ordered after the last stream's work like nuto_set_stream */
+int nuto_batch_set_stream(nuto_batch* batch, void* stream);
 int nuto_batch_synchronize(nuto_batch* batch);
 int nuto_batch_set_integrand(nuto_batch* batch, const nuto_params* params); /* dim 3 integrands */
 /* cell_ranks: n_cells x nodes(dof_type) dof node ranks (nuto_dof_layer); mesh receives its index */

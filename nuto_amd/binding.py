@@ -487,7 +487,8 @@ class Context:
             raise NutoError(r, lib().nuto_last_error(self.h).decode())
 
     def set_stream(self, stream):
-        # 0 / None selects the null stream (torch's default stream)
+        """Run the next calls on this stream (0 / None: the null stream, torch's default). They wait for this
+        context's calls on the last stream, whose work memory they share."""
         self._chk(lib().nuto_set_stream(self.h, ctypes.c_void_p(stream) if stream else None))
 
     def synchronize(self):

@@ -62,6 +62,7 @@ struct nuto_ctx
     int device = 0;
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;
+    hipEvent_t moved = nullptr;  // orders a newly set stream after the last one (FollowStream)
     std::string err;
     // the constrained solves' vectors, and the pinned states with the events of their arrival, kept
     // between solves (a Newton step solves once per iteration); grown when a solve needs more
@@ -208,6 +209,30 @@ void SyncCheck(nuto_ctx* ctx, const char* what)
         Check(hipStreamSynchronize(ctx->stream), what);
         Check(hipGetLastError(), what);
     }
+}
+
+// The calls of a context share its work memory (records, cell vectors, staged matrices, solve vectors), so
+// when they move to another stream it first waits for what the last one holds. No wait where one of the two
+// is being captured without the other: nothing runs then, the order is that of the graph's launches; nor where
+// the last stream is gone (its handle is refused).
+void FollowStream(nuto_ctx* ctx, hipStream_t next)
+{
+    const hipStream_t last = ctx->stream;
+    if (next == last)
+        return;
+    hipStreamCaptureStatus nextStatus = hipStreamCaptureStatusNone, lastStatus = hipStreamCaptureStatusNone;
+    unsigned long long nextId = 0, lastId = 0;
+    if (hipStreamGetCaptureInfo(next, &nextStatus, &nextId) == hipSuccess &&
+        hipStreamGetCaptureInfo(last, &lastStatus, &lastId) == hipSuccess && nextStatus == lastStatus &&
+        nextStatus != hipStreamCaptureStatusInvalidated &&
+        (nextStatus == hipStreamCaptureStatusNone || nextId == lastId))
+    {
+        if (!ctx->moved)
+            Check(hipEventCreateWithFlags(&ctx->moved, hipEventDisableTiming), "stream event");
+        if (hipEventRecord(ctx->moved, last) == hipSuccess)
+            Check(hipStreamWaitEvent(next, ctx->moved, 0), "stream order");
+    }
+    (void)hipGetLastError();
 }
 
 // NUTO_AMD_GENERIC=1 routes every call through the generic row-owner kernel (used by the tests
@@ -959,7 +984,7 @@ int nuto_destroy(nuto_ctx* ctx)
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->solveBuf.host)
         (void)hipHostFree(ctx->solveBuf.host);
-    for (hipEvent_t e : ctx->solveBuf.arrived)
+    for (hipEvent_t e : {ctx->solveBuf.arrived[0], ctx->solveBuf.arrived[1], ctx->moved})
         if (e)
             (void)hipEventDestroy(e);
     if (ctx->own)
@@ -976,7 +1001,10 @@ const char* nuto_last_error(const nuto_ctx* ctx)
 int nuto_set_stream(nuto_ctx* ctx, void* stream)
 {
     // NULL is HIP's default (null) stream, which orders with every blocking stream of the device
-    return Guard(ctx, [&] { ctx->stream = (hipStream_t)stream; });
+    return Guard(ctx, [&] {
+        FollowStream(ctx, (hipStream_t)stream);
+        ctx->stream = (hipStream_t)stream;
+    });
 }
 
 int nuto_synchronize(nuto_ctx* ctx)
