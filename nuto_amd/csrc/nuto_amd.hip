@@ -120,6 +120,7 @@ struct nuto_ctx
     // staged cell matrices and vectors of the two-phase generic assembly
     DevBuf keStage, reStage;
     int maxAdj = -1;  // largest node neighbourhood (LDS rows of the wave gather), from the node graph
+    bool batchGroup = false;  // the super-mesh of a batch's group
     long long maxWindow = -1;  // most neighbours of a node tile's consecutive dof nodes (LDS of kNodeTile)
     int cellGram = -1;  // form of the 3D matrix assembly: 0 cell matrices by columns, 1 / 2 in Gram form with 1 / 2
                         // row nodes per lane, 3 on the matrix cores, 4 node tiles (tet4), -1 the element's default
@@ -271,16 +272,27 @@ void InvalidatePattern(nuto_ctx* ctx)
 
 size_t TileLds(nuto_ctx* ctx);
 
-// Staging of the cells' vectors (every dof of every cell); false when it cannot be allocated (the error
-// state is cleared). It only grows: two-phase matrix assemblies stage their vectors there too.
-bool TryVectorStage(nuto_ctx* ctx)
+// Staging of the cells' vectors (every dof of every cell); two-phase matrix assemblies stage theirs there too
+size_t VectorStageBytes(const nuto_ctx* ctx)
 {
-    const size_t bytes = (size_t)ctx->nCells * NodesOf(ctx->f[0].type) *
-                         (ctx->f[0].ncomp + (ctx->f[1].set ? ctx->f[1].ncomp : 0)) * sizeof(double);
-    if (ctx->reStage.bytes >= bytes || ctx->reStage.Alloc(bytes) == hipSuccess)
-        return true;
-    (void)hipGetLastError();
-    return false;
+    return (size_t)ctx->nCells * NodesOf(ctx->f[0].type) *
+           (ctx->f[0].ncomp + (ctx->f[1].set ? ctx->f[1].ncomp : 0)) * sizeof(double);
+}
+
+// Reserves it once the pattern, the integrand and the rule are known, so that vector assemblies allocate
+// nothing; without room they take the single-pass kernel. Not where nothing would use it: the hex8
+// gradient-damage plan has work memory of its own, and a batch's group assembles no vector alone.
+void ReserveVectorStage(nuto_ctx* ctx)
+{
+    if (!ctx->patternBuilt || !ctx->integrandSet || !ctx->ruleSet || ctx->batchGroup)
+        return;
+    const bool planned = ctx->params.kind == kGradientDamage && ctx->coordType == kHex8 && ctx->f[0].type == kHex8 &&
+                         ctx->ruleKind == 0 && ctx->ruleN == 2;
+    if (planned && (!ctx->gdmTried || ctx->gdm.ready))
+        return;
+    const size_t bytes = VectorStageBytes(ctx);
+    if (ctx->reStage.bytes < bytes && ctx->reStage.Alloc(bytes) != hipSuccess)
+        (void)hipGetLastError();
 }
 
 // IP tables: per IP w, dNc[nnC][dim], N[nnD], dNd[nnD][dim] (shape tables of the coordinate
@@ -623,8 +635,8 @@ void LaunchRowsT(nuto_ctx* ctx, const RowArgs& a, bool wr, bool wk)
     if (n == 0)
         return;
     // a vector alone: the cells' vectors, then the sum per node; the single-pass kernel serves when they
-    // do not fit in device memory
-    if (!wk && !ForceGeneric() && TryVectorStage(ctx))
+    // did not fit in device memory
+    if (!wk && !ForceGeneric() && ctx->reStage.bytes >= VectorStageBytes(ctx))
     {
         constexpr int F = KIND == kGradientDamage ? DIM + 1 : DIM;
         double* cv = ctx->reStage.As<double>();
@@ -790,6 +802,7 @@ void PrepareGdm(nuto_ctx* ctx)
     }
     Check(err, "hex8 node tables");
     ctx->gdmTried = true;
+    ReserveVectorStage(ctx);  // where the plan does not serve the mesh
 }
 
 // Block (slot i, slot j) of the monolithic matrix, row by row: the monolithic row of dof row0 + r
@@ -1118,6 +1131,7 @@ int nuto_set_integrand(nuto_ctx* ctx, const nuto_params* params)
         ctx->integrandSet = true;
         ctx->gdm.Release();
         ctx->gdmTried = false;
+        ReserveVectorStage(ctx);
     });
 }
 
@@ -1133,6 +1147,7 @@ int nuto_set_rule(nuto_ctx* ctx, int kind, int n)
         ctx->tabValid = false;
         ctx->gdm.Release();
         ctx->gdmTried = false;
+        ReserveVectorStage(ctx);
     });
 }
 
@@ -1224,8 +1239,8 @@ int nuto_build_pattern(nuto_ctx* ctx, long long* nnz, int* n_rows)
         ctx->nnz = nz;
         ctx->nRows = (int)(rp.size() - 1);
         ctx->patternBuilt = true;
-        (void)TryVectorStage(ctx);  // here, so that vector assemblies allocate nothing
         (void)TileLds(ctx);
+        ReserveVectorStage(ctx);
         // gradient damage with the integrand and the rule already set: the IP tables and the node
         // kernel's tables now, so that assemblies (nuto_build_vector_matrix_noalloc) allocate nothing
         if (ctx->integrandSet && ctx->ruleSet && ctx->params.kind == kGradientDamage && !ForceGeneric())
@@ -2533,6 +2548,7 @@ int nuto_batch_build(nuto_batch* b)
             b->groups.push_back(g);
             BatchGroup& G = b->groups.back();
             nuto_ctx* c = G.ctx;
+            c->batchGroup = true;
             CheckCtx(c, nuto_set_stream(c, b->stream));
             CheckCtx(c, nuto_set_cells(c, G.ct, G.nCells, G.nCoord, X.data(), C.data(), nullptr));
             std::vector<int> cd(Rk.size() * 3);
