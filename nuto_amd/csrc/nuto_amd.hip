@@ -453,13 +453,17 @@ size_t TileLds(nuto_ctx* ctx)
     return (size_t)ctx->maxWindow * ctx->dim * ctx->dim * sizeof(double);
 }
 
-// Rows of the nodes [p0, p1) by node tiles; false when a tile's rows do not fit in LDS
+// one dof type (its rows are a tile's segment), and every tile's rows fit in LDS
+bool TilesFit(nuto_ctx* ctx)
+{
+    return !ctx->f[1].set && TileLds(ctx) <= kTileMaxLds;
+}
+
+// Rows of the nodes [p0, p1) by node tiles (TilesFit); they need no staging
 template <int KIND, int DIM, int NNC, int NND, int NIP>
-bool LaunchTiles(nuto_ctx* ctx, const RowArgs& a, bool wr, int p0, int p1, hipStream_t stream)
+void LaunchTiles(nuto_ctx* ctx, const RowArgs& a, bool wr, int p0, int p1, hipStream_t stream)
 {
     const size_t lds = TileLds(ctx);
-    if (lds > kTileMaxLds)
-        return false;
     constexpr int nodes = TileNodes(DIM);
     const dim3 grid((unsigned)((p1 - p0 + nodes - 1) / nodes));
     if (wr)
@@ -467,7 +471,6 @@ bool LaunchTiles(nuto_ctx* ctx, const RowArgs& a, bool wr, int p0, int p1, hipSt
     else
         hipLaunchKernelGGL((kNodeTile<KIND, DIM, NNC, NND, NIP, false>), grid, dim3(64), lds, stream, a, p0, p1);
     Check(hipGetLastError(), "node tile launch");
-    return true;
 }
 
 // kCellGram's shape per element and row nodes per lane (AP): cells per workgroup, threads, IPs per
@@ -563,13 +566,26 @@ void LaunchCellMatrices(const RowArgs& a, int form, int c0, int c1, double* ke, 
 // cells 394 / 367 / 600, 1320 cells 58.5 / 52.4 / 93.9, 120 cells 24.2 / 21.7 / 56.6; elasticity 315 / 340 / 461,
 // 46.0 / 44.5 / 71.4, 19.3 / 19.7 / 43.8; tet10 local damage, 20,160 cells 139 / 132 / 155, 5940 cells 47.2 / 44.2 /
 // 50.3; elasticity 124 / 126 / 126, 43.2 / 40.6 / 42.8; hex8 local damage, 63,960 cells 302 / 316 / 391.
-template <int KIND, int NND>
-int DefaultForm(const RowArgs& a, int nodes)
+int DefaultForm(int kind, int damageApplication, int nnd, int nodes)
 {
-    if (NND == 4)
+    if (nnd == 4)
         return nodes >= 2048 ? 4 : 0;
-    const bool two = KIND == kLocalDamage && a.P.damage_application == 0;
-    return (NND == 20 || NND == 10) && two ? 3 : 1;
+    const bool two = kind == kLocalDamage && damageApplication == 0;
+    return (nnd == 20 || nnd == 10) && two ? 3 : 1;
+}
+
+// the form that a launch over `nodes` dof nodes of the context takes: forced, tuned, or the default
+int FormOf(const nuto_ctx* ctx, int nodes)
+{
+    const int env = CellFormEnv();
+    if (env >= 0 || ctx->cellGram >= 0)
+        return env >= 0 ? env : ctx->cellGram;
+    return DefaultForm(ctx->params.kind, ctx->params.damage_application, NodesOf(ctx->f[0].type), nodes);
+}
+
+bool TakesTiles(nuto_ctx* ctx, int nodes)
+{
+    return ctx->f[0].type == kTet4 && FormOf(ctx, nodes) == 4 && TilesFit(ctx);
 }
 
 template <int KIND, int NNC, int NND, int NIP>
@@ -578,17 +594,18 @@ void LaunchTwoPhaseT(nuto_ctx* ctx, const RowArgs& a, bool wr, int c0, int c1, i
     constexpr int ND = NND * 3;
     if (c1 <= c0 || p1 <= p0)
         return;
-    const int env = CellFormEnv();
-    const int form = env >= 0 ? env : (ctx->cellGram >= 0 ? ctx->cellGram : DefaultForm<KIND, NND>(a, p1 - p0));
     if constexpr (NND == 4)
     {
-        if (form == 4 && LaunchTiles<KIND, 3, NNC, NND, NIP>(ctx, a, wr, p0, p1, stream))
+        if (TakesTiles(ctx, p1 - p0))
+        {
+            LaunchTiles<KIND, 3, NNC, NND, NIP>(ctx, a, wr, p0, p1, stream);
             return;
+        }
     }
     EnsureStage(ctx, ND, c1 - c0);  // cell c's matrix at staging position c - c0
     double* ke = ctx->keStage.As<double>();
     double* re = ctx->reStage.As<double>();
-    LaunchCellMatrices<KIND, NNC, NND, NIP>(a, form, c0, c1, ke, re, stream);
+    LaunchCellMatrices<KIND, NNC, NND, NIP>(a, FormOf(ctx, p1 - p0), c0, c1, ke, re, stream);
     if (ctx->maxAdj < 0)
     {
         int m = 0;
@@ -648,9 +665,9 @@ void LaunchRowsT(nuto_ctx* ctx, const RowArgs& a, bool wr, bool wk)
     }
     if constexpr (DIM == 2)
     {
-        if (wk && !ForceGeneric() && !ctx->f[1].set &&
-            LaunchTiles<KIND, DIM, NNC, NND, NIP>(ctx, a, wr, 0, n, ctx->stream))
+        if (wk && !ForceGeneric() && TilesFit(ctx))
         {
+            LaunchTiles<KIND, DIM, NNC, NND, NIP>(ctx, a, wr, 0, n, ctx->stream);
             SyncCheck(ctx, "assembly kernel");
             return;
         }
@@ -659,7 +676,7 @@ void LaunchRowsT(nuto_ctx* ctx, const RowArgs& a, bool wr, bool wk)
     if constexpr (DIM == 3 && KIND != kGradientDamage && NND * 3 <= 64 && NIP <= 27)
     {
         // the single-pass kernel serves when the staging does not fit in device memory
-        if (wk && !TwoPhaseOff() && TryStage(ctx, NND * 3, a.nCells))
+        if (wk && !TwoPhaseOff() && (TakesTiles(ctx, n) || TryStage(ctx, NND * 3, a.nCells)))
         {
             LaunchTwoPhaseT<KIND, NNC, NND, NIP>(ctx, a, wr, 0, a.nCells, 0, n, ctx->stream);
             SyncCheck(ctx, "assembly kernel");
@@ -2133,13 +2150,15 @@ long long MaxChunkCells(const nuto_batch* b, const BatchGroup& g)
 }
 
 // Staging of every group's two-phase launch (mode 5) allocated now, before a graph capture of the
-// launch (which must not allocate); the chunk defaults where none is chosen yet
+// launch (which must not allocate); the chunk defaults where none is chosen yet. Node tiles have none.
 void PrepareStaging(nuto_batch* b)
 {
     if (IsGdm(b))
         return;
     for (BatchGroup& g : b->groups)
     {
+        if (TakesTiles(g.ctx, g.nNodes))
+            continue;
         if (g.stageCells < 0)
             g.stageCells = DefaultStageCells(g);
         EnsureStage(g.ctx, 3 * NodesOf(g.dt), MaxChunkCells(b, g));
@@ -2149,13 +2168,14 @@ void PrepareStaging(nuto_batch* b)
 // Two-phase launches of a group in chunks of consecutive meshes whose cells fit stageCells (0: the
 // whole group at once; a mesh larger than the chunk is a chunk of its own). The rows of a mesh only
 // touch its own cells, so each chunk's staging is consumed by its gather before the next chunk
-// rewrites it (same stream).
+// rewrites it (same stream). Node tiles stage nothing: the whole group at once.
 template <int KIND>
 void LaunchTwoPhaseGroup(nuto_batch* b, BatchGroup& g, const RowArgs& a)
 {
-    if (g.stageCells < 0)
+    const bool tiles = TakesTiles(g.ctx, g.nNodes);
+    if (!tiles && g.stageCells < 0)
         g.stageCells = DefaultStageCells(g);
-    if (g.stageCells == 0 || g.nCells <= g.stageCells)
+    if (tiles || g.stageCells == 0 || g.nCells <= g.stageCells)
     {
         LaunchTwoPhaseType<KIND>(g.ctx, a, g.type, 0, g.nCells, 0, g.nNodes, b->stream);
         return;
@@ -2822,10 +2842,11 @@ int nuto_batch_autotune(nuto_batch* b, const double* u, const double* e, const d
                 for (int gram = 0; gram < kCellForms; gram++)
                     for (long long c : chunks)
                     {
-                        if (gram == 4 && g.type != kBtTet4)
-                            continue;
                         g.ctx->cellGram = gram;
                         g.stageCells = c;
+                        // node tiles: no chunks
+                        if (gram == 4 && (c != chunks[0] || !TakesTiles(g.ctx, g.nNodes)))
+                            continue;
                         const double t = median([&] {
                             if (b->params.kind == kLinearElastic)
                                 LaunchTwoPhaseGroup<kLinearElastic>(b, g, a);
@@ -2843,7 +2864,7 @@ int nuto_batch_autotune(nuto_batch* b, const double* u, const double* e, const d
                 g.stageCells = bestChunk;
                 // staging of the chosen chunk only, allocated here: a graph capture of the tuned launch
                 // must not allocate
-                const long long keep = MaxChunkCells(b, g);
+                const long long keep = TakesTiles(g.ctx, g.nNodes) ? 0 : MaxChunkCells(b, g);
                 if (g.ctx->keStage.bytes > (size_t)keep * nd * nd * sizeof(double))
                 {
                     Check(hipStreamSynchronize(b->stream), "staging release");

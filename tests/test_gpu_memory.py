@@ -71,6 +71,25 @@ def test_generic_vector_allocates_nothing():
     assert got == 0
 
 
+def test_tet4_tiles_stage_nothing():
+    """the matrix of a tet4 mesh that takes node tiles, alone and in a batch"""
+    ctx, X, C, ranks, nn = prepared(N.TET4, (30, 30, 30), N.local_damage_params(), False)
+    ctx.build_pattern()
+    u, kap = to_dev(S.uniform(S.SEED_U, 3 * nn, -5e-3, 5e-3)), to_dev(S.uniform(S.SEED_KAPPA, len(C), 0.0, 3e-4))
+    R = torch.empty(ctx.n_rows, dtype=torch.float64, device="cuda")
+    K = torch.empty(ctx.nnz, dtype=torch.float64, device="cuda")
+    _, got = taken(lambda: ctx.build_vector_matrix(u, None, kap, R, K))
+    assert got <= SPARE
+    b = N.Batch()
+    b.set_integrand(N.local_damage_params())
+    b.add_mesh(N.TET4, N.TET4, X, C, ranks, nn)
+    b.build()
+    Rb, Kb = torch.empty_like(R), torch.empty_like(K)
+    _, got = taken(lambda: b.assemble(u, None, kap, Rb, Kb, mode=5))
+    assert got <= SPARE
+    assert torch.equal(Rb, R) and torch.equal(Kb, K)
+
+
 def test_batch_reserves_no_vectors():
     """a batch assembles no vector alone: its groups hold less than a context of the same mesh"""
     params = N.linear_elastic_params(3, 30000.0, 0.2)
