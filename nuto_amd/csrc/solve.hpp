@@ -12,10 +12,11 @@
 //
 // Solvers: Jacobi-preconditioned conjugate gradients and BiCGSTAB (the iterative solvers NuTo selects
 // by name, EigenSparseSolve.cpp:44-49, whose default preconditioner is the diagonal). An iteration is
-// two (CG) or three (BiCGSTAB) kernels in small systems, three or five in larger ones (kFormNodes). Dot products ride on the kernels that make their operands:
-// each block leaves its partial sum, and every block of the next kernel adds the partials itself, all
-// in the same fixed order, so no kernel exists only to finish a reduction and solves are
-// bit-reproducible. A kernel loads all that does not depend on those sums, the test of the status
+// two (CG) or three (BiCGSTAB) kernels in small systems, three or five in larger ones (kFormNodes). Dot
+// products ride on the kernels that make their operands: each block leaves its partial sum, and every
+// block of the next kernel adds the partials itself, all in the same fixed order, so solves are
+// bit-reproducible and no kernel exists only to finish a reduction (but for the K product of the largest
+// systems, kFoldRows). A kernel loads all that does not depend on those sums, the test of the status
 // included, before it waits for them. The scalars, the convergence test and the iteration count stay on the device
 // (KrylovState); once the test is met the remaining launches return at once. The host queues
 // kSolveChunk iterations at a time and reads the state of a chunk while the next one runs, so the
@@ -51,6 +52,16 @@ constexpr int kSolveChunk = 4;      // iterations the host queues before it read
 // 13.6 / 11.1, 9261 nodes 16.0 / 15.4, 226,981 nodes 234 / 248; BiCGSTAB 18.6 / 16.1, 20.4 / 17.5, 27.6 / 28.5,
 // 465 / 530; elastic hex8, 15,625 nodes: 17.5 / 17.0 and 30.5 / 33.3.
 constexpr int kFormNodes = 4 * kSpmvBlocks;
+
+// From this many rows on a wave of the K product has one node, and one more kernel adds the many blocks'
+// partials up to kFoldBlocks: waves that stride over the nodes keep the partials few, but 2048 blocks of 72
+// VGPRs are one and a third rounds of resident blocks, and a wave that ends early leaves its place empty.
+// Below, the fold's launch costs more than that. Measured, us per iteration, striding / one node per wave:
+// hex8 gradient damage (4 rows per node), BiCGSTAB 157,216 rows 67.0 / 68.3, 202,612 rows 85.7 / 82.5,
+// 4,121,204 rows 2122 / 1687, CG there 1064 / 857; elastic hex8, BiCGSTAB 151,959 rows 62.3 / 63.1, 206,763
+// rows 79.6 / 78.0, 3,090,903 rows 1451 / 1219; elastic quad4 181,202 rows 70.3 / 72.7, 722,402 rows 235 / 225.
+constexpr int kFoldRows = 24 * 4 * kSpmvBlocks;
+constexpr int kFoldBlocks = 512;
 
 enum SolveStatus : int
 {
@@ -302,9 +313,9 @@ __global__ void __launch_bounds__(256) kCsrSpmv(int nRows, const int* __restrict
 // field-1 row (nU + p, when C1 = 1) hold the same L columns, so one wave per node reads each x entry
 // once for all of them. Lane l sums the entries l, l + 64, ... of each row in order; the 64 partial
 // sums are added by exchanges in which the lanes share out the rows, a fixed order, without LDS.
-// A wave strides over the nodes (so that the dots' partials stay few) and keeps the next node's first
-// 128 entries of every row in flight while it works on this one's, and the row offsets of the node
-// after that: only the gather of x is waited for. mask (one byte per node, bit i: row i is a dependent
+// A wave strides over the nodes (so that the dots' partials stay few; not in the largest systems, kFoldRows)
+// and keeps the next node's first 128 entries of every row in flight while it works on this one's, and
+// the row offsets of the node after that: only the gather of x is waited for. mask (one byte per node, bit i: row i is a dependent
 // dof) zeroes those rows of y; DOTS: the block's partial sums of the dots over its rows.
 // Bound by the reads of the values; in small systems by the latency of its launch and of its dependent
 // loads. IN != kStored: the kernel that would make x is left out, see SpmvInput; the first node's entries
@@ -628,6 +639,27 @@ __global__ void __launch_bounds__(256) kSumPartials(int np, const double* __rest
     }
 }
 
+// out[N][gridDim.x] = the sums of consecutive runs of the K product's partials part[N][np]
+template <int N>
+__global__ void __launch_bounds__(256) kFoldPartials(int np, const double* __restrict__ part, double* __restrict__ out,
+                                                     const KrylovState* __restrict__ st)
+{
+    __shared__ double sh[8];
+    if (st->status != kRunning)
+        return;
+    const int run = (np + (int)gridDim.x - 1) / (int)gridDim.x;
+    const int beg = (int)blockIdx.x * run, end = beg + run < np ? beg + run : np;
+    double v[N];
+#pragma unroll
+    for (int i = 0; i < N; i++)
+    {
+        v[i] = 0.0;
+        for (int k = beg + (int)threadIdx.x; k < end; k += 256)
+            v[i] += part[(size_t)i * np + k];
+    }
+    StorePartials<N>(v, out, sh);
+}
+
 // Start of a solve from x = 0: b = C^T f, r = b, and for BiCGSTAB r0 = b, p = v = 0 with the partials
 // of (r . r) and (r0 . r), for CG z = invd b with those of (r . r) and (r . z); the state
 template <bool CG>
@@ -895,10 +927,11 @@ class ReducedSolver
 {
 public:
     // doubles of the workspace: 11 vectors of a solve (x and the preconditioner's diagonal included) and
-    // 2 of its caller, the partial sums of the vector kernels and of the K product, the two states
+    // 2 of its caller, the partial sums of the vector kernels and of the K product, the two states, and the
+    // partials of one block per four nodes (a node has two rows at least)
     static size_t WorkDoubles(long long n)
     {
-        return 13 * (size_t)n + 2 * kDotBlocks + 2 * kSpmvBlocks + 32;
+        return 13 * (size_t)n + 2 * kDotBlocks + 2 * kSpmvBlocks + 32 + (n >= kFoldRows ? 2 * (size_t)(n / 8 + 1) : 0);
     }
     ReducedSolver(hipStream_t s, Csr K, Csr Ct, const int* rev, const unsigned char* mask, ConstraintView cons,
                   NodeRows nodes, const SolveBuffers& buf)
@@ -908,6 +941,7 @@ public:
         part = vecs + 13 * (size_t)mN;
         dotPart = part + 2 * kDotBlocks;
         state = reinterpret_cast<KrylovState*>(dotPart + 2 * kSpmvBlocks);
+        blockPart = dotPart + 2 * kSpmvBlocks + 32;
         const bool known = (nodes.c0 == 3 && nodes.c1 <= 1) || (nodes.c0 == 2 && nodes.c1 == 0);
         mNode = nodes.nNodes > 0 && known;
         mFused = mNode && cons.nTermDofs == 0;
@@ -1135,7 +1169,12 @@ private:
                     KrylovState* st, const FormedInput& in = {})
     {
         const NodeRows& nr = mNodes;
-        const int g = std::min(kSpmvBlocks, (nr.nNodes + 3) / 4);
+        const int all = (nr.nNodes + 3) / 4;
+        const bool fold = IN == kStored && mN >= kFoldRows;
+        const int g = fold ? all : std::min(kSpmvBlocks, all);
+        double* const sums = out;
+        if (fold && DOTS != kNoDots)
+            out = blockPart;
         const dim3 grid((unsigned)g), block(256);
         if (nr.c0 == 3 && nr.c1 == 1)
             hipLaunchKernelGGL((kNodeSpmv<3, 1, DOTS, IN>), grid, block, 0, mS, nr.nNodes, nr.nU, mK.row, mK.col, mK.val, x,
@@ -1146,6 +1185,14 @@ private:
         else
             hipLaunchKernelGGL((kNodeSpmv<2, 0, DOTS, IN>), grid, block, 0, mS, nr.nNodes, nr.nU, mK.row, mK.col, mK.val, x,
                                y, mask, d, out, st, in);
+        if constexpr (DOTS != kNoDots)
+        {
+            if (fold)
+            {
+                hipLaunchKernelGGL(kFoldPartials<DOTS>, dim3(kFoldBlocks), block, 0, mS, g, blockPart, sums, st);
+                return kFoldBlocks;
+            }
+        }
         return g;
     }
 
@@ -1158,7 +1205,7 @@ private:
     NodeRows mNodes;
     SolveBuffers mBuf;
     bool mNode = false, mFused = false;
-    double *vecs = nullptr, *part = nullptr, *dotPart = nullptr;
+    double *vecs = nullptr, *part = nullptr, *dotPart = nullptr, *blockPart = nullptr;
     KrylovState* state = nullptr;
 };
 

@@ -17,8 +17,20 @@ from test_gpu_parity import gdm_params, le_params
 pytestmark = pytest.mark.gpu
 
 
+class Masked:
+    """rows and columns `ind` of a sparse matrix, with its diagonal"""
+
+    def __init__(self, K, ind, diag):
+        self.K, self.ind, self.diag = K, ind, diag[ind]
+
+    def __matmul__(self, v):
+        full = np.zeros(self.K.shape[0])
+        full[self.ind] = v
+        return (self.K @ full)[self.ind]
+
+
 def cg(A, b, k):
-    d = 1.0 / np.diag(A)
+    d = 1.0 / (A.diag if isinstance(A, Masked) else np.diag(A))
     x, r = np.zeros_like(b), b.copy()
     z = d * r
     p, rz = z.copy(), r @ z
@@ -33,7 +45,7 @@ def cg(A, b, k):
 
 
 def bicgstab(A, b, k):
-    d = 1.0 / np.diag(A)
+    d = 1.0 / (A.diag if isinstance(A, Masked) else np.diag(A))
     x, r, r0 = np.zeros_like(b), b.copy(), b.copy()
     p = v = np.zeros_like(b)
     rho = alpha = w = 1.0
@@ -148,3 +160,50 @@ def test_formed_vectors_give_the_same_bits(case, n, method, monkeypatch):
             x, info = ctx.solve(K, f, method=method, tol=1e-12, max_iter=k)
             out.append((x.cpu().numpy(), info["iterations"], info["relative_residual"]))
         assert out[0][1:] == out[1][1:] and np.array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("case,n", [("quad4", (382, 255)), ("quad4", (383, 255)), ("quad4", (400, 300)), ("hex8", (41, 40, 40)),
+                                    ("gdm", (37, 37, 36))])
+@pytest.mark.parametrize("method", [N.SOLVER_CG, N.SOLVER_BICGSTAB])
+def test_large_systems(case, n, method):
+    """On either side of 196,608 rows, from where on a wave of the K product has one node and its partial sums
+    are added by a kernel of their own; the same iterations in numpy on the sparse matrix."""
+    from scipy.sparse import csr_matrix
+
+    ct = N.QUAD4 if case == "quad4" else N.HEX8
+    dim = N.DIM[ct]
+    X, C = make_mesh(ct, n, tuple(float(v) for v in n) + (0.0,) * (3 - dim))
+    ranks, nn = N.dof_layer(ct, C, ct)
+    ctx = N.Context()
+    ctx.set_cells(ct, X, C)
+    ctx.set_dof_type(0, ct, dim, dim * nn, N.cell_dofs(ranks, dim))
+    u = to_dev(np.random.default_rng(5).uniform(-1e-4, 1e-4, dim * nn))
+    if case == "gdm":
+        ctx.set_dof_type(1, ct, 1, nn, N.cell_dofs(ranks, 1))
+        ctx.set_integrand(N.gradient_damage_params())
+        ctx.set_rule(0, 2)
+        ctx.build_pattern()
+        K = ctx.build_matrix(u, to_dev(np.full(nn, 5e-5)), to_dev(np.zeros(8 * len(C))))
+    else:
+        ctx.set_integrand(N.linear_elastic_params(dim, 30000.0, 0.2))
+        ctx.set_rule(0, 2)
+        ctx.build_pattern()
+        K = ctx.build_matrix(u)
+    left = np.unique(ranks.ravel()[X[C.ravel(), 0] < 1e-12])
+    dep = (dim * left[:, None] + np.arange(dim)).ravel()
+    ctx.set_constraints(0, [(int(d), []) for d in dep])
+    rp, ci = ctx.pattern()
+    keep = np.ones(len(rp) - 1)
+    keep[dep] = 0.0
+    ind = np.nonzero(keep)[0]
+    val = K.cpu().numpy()
+    diag = csr_matrix((val, ci, rp)).diagonal()
+    A = Masked(csr_matrix((val, ci, rp)), ind, diag)
+    f = np.random.default_rng(4).uniform(-1.0, 1.0, len(keep))
+    for k in (1, 5):
+        x, info = ctx.solve(K, to_dev(f), method=method, tol=1e-300, max_iter=k)
+        want, rel = (cg if method == N.SOLVER_CG else bicgstab)(A, f[ind], k)
+        assert info["iterations"] == k
+        assert np.abs(x.cpu().numpy()[ind] - want).max() <= 1e-9 * np.abs(want).max()
+        assert not x.cpu().numpy()[dep].any()
+        assert abs(info["relative_residual"] - rel) <= 1e-9 * max(rel, 1.0)
