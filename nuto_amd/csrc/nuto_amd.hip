@@ -697,11 +697,15 @@ void LaunchRowsT(nuto_ctx* ctx, const RowArgs& a, bool wr, bool wk)
 template <int KIND, int DIM, int NNC, int NND, int NIP>
 void LaunchHistoryT(nuto_ctx* ctx, const RowArgs& a, double* kappa)
 {
-    if constexpr (KIND != kLinearElastic && DIM == 3)
+    if constexpr (KIND == kGradientDamage)
     {
-        LaunchPoints<KIND, DIM, NNC, NND, NIP, kPointHistory>(ctx, a, 0, kappa);
-        Check(hipGetLastError(), "history launch");
+        if (a.nCells > 0)
+            hipLaunchKernelGGL((kNonlocalHistory<NNC, NND, NIP>), dim3((unsigned)((a.nCells + 255) / 256), NIP), dim3(256),
+                               0, ctx->stream, a, kappa);
     }
+    else if constexpr (KIND == kLocalDamage)
+        LaunchPoints<KIND, DIM, NNC, NND, NIP, kPointHistory>(ctx, a, 0, kappa);
+    Check(hipGetLastError(), "history launch");
 }
 
 template <int DIM, int NNC, int NND, int NIP>

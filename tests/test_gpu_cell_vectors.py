@@ -218,12 +218,14 @@ def test_gradient_damage_loads_at_the_updated_history(rule, env, monkeypatch):
     pre-pass, the row-owner kernel, and the rules that only the latter has."""
     for k, v in env.items():
         monkeypatch.setenv(k, v)
-    X, C = make_mesh(N.HEX8, (4, 3, 3), lengths=(4.0, 3.0, 3.0), jitter=0.1)
+    X, C = make_mesh(N.HEX8, (9, 6, 5), lengths=(9.0, 6.0, 5.0), jitter=0.1)  # more than one block of 256 cells
     p = Pair(N.HEX8, N.HEX8, X, C, *gdm_params(), two_fields=True, rule=rule)
     u, e, kap = p.inputs()
     ctx = p.context()
     du, de, dk = to_dev(u), to_dev(e), to_dev(kap)
+    kappa = ctx.eval_ip(N.IP_KAPPA, du, de, dk)
     ctx.update_history(du, de, dk)
+    assert np.array_equal(dk.view(p.nip, p.ncells).T.cpu().numpy(), kappa[:, :, 0].cpu().numpy())
     check_loading(lambda k: ctx.build_matrix(du, de, k).cpu().numpy(), dk, dk * (1.0 - 1e-10))
 
 
