@@ -272,6 +272,18 @@ void InvalidatePattern(nuto_ctx* ctx)
 
 size_t TileLds(nuto_ctx* ctx);
 
+// Whether a vector alone goes through the cells' vectors and a gather (else the row-owner kernel). In 3D
+// always; a quad4 node has four cells only, each of a few points, and the row-owner kernel integrates them
+// in one launch until there are many points per cell, or so many nodes that evaluating each point four times
+// is what bounds it. Measured, us, cell vectors / row-owner: 1 point 961 nodes 8.1 / 5.6, 160,801 nodes
+// 18.8 / 10.5, 361,201 nodes 23.8 / 27.7; 4 points 8.3 / 8.0, 20.3 / 16.4, 31.6 / 34.5; 9 points 961 nodes 8.2 / 12.3,
+// 22,801 nodes 9.0 / 12.7, 40,401 nodes 12.7 / 12.8, 160,801 nodes 29.4 / 26.3; 25 points 8.0 / 27.0, 19.9 / 27.1,
+// 31.5 / 27.5, 104.8 / 57.8.
+bool StagesVector(int dim, int nip, int nodes)
+{
+    return dim == 3 || (nip <= 4 ? nodes >= 262144 : nodes < 32768);
+}
+
 // Staging of the cells' vectors (every dof of every cell); two-phase matrix assemblies stage theirs there too
 size_t VectorStageBytes(const nuto_ctx* ctx)
 {
@@ -289,6 +301,9 @@ void ReserveVectorStage(nuto_ctx* ctx)
     const bool planned = ctx->params.kind == kGradientDamage && ctx->coordType == kHex8 && ctx->f[0].type == kHex8 &&
                          ctx->ruleKind == 0 && ctx->ruleN == 2;
     if (planned && (!ctx->gdmTried || ctx->gdm.ready))
+        return;
+    Rule r;
+    if (!MakeRule(ctx->ruleKind, ctx->dim, ctx->ruleN, r) || !StagesVector(ctx->dim, r.Num(), ctx->f[0].nNodes))
         return;
     const size_t bytes = VectorStageBytes(ctx);
     if (ctx->reStage.bytes < bytes && ctx->reStage.Alloc(bytes) != hipSuccess)
@@ -653,7 +668,7 @@ void LaunchRowsT(nuto_ctx* ctx, const RowArgs& a, bool wr, bool wk)
         return;
     // a vector alone: the cells' vectors, then the sum per node; the single-pass kernel serves when they
     // did not fit in device memory
-    if (!wk && !ForceGeneric() && ctx->reStage.bytes >= VectorStageBytes(ctx))
+    if (!wk && !ForceGeneric() && StagesVector(DIM, NIP, n) && ctx->reStage.bytes >= VectorStageBytes(ctx))
     {
         constexpr int F = KIND == kGradientDamage ? DIM + 1 : DIM;
         double* cv = ctx->reStage.As<double>();

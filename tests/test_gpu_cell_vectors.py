@@ -138,6 +138,27 @@ def test_generic_vectors_history_and_fields(ct, dt, n, rule, kind, monkeypatch):
     assert np.array_equal(state[2].view(p.nip, p.ncells).T.cpu().numpy(), kappa[:, :, 0].cpu().numpy())
 
 
+@pytest.mark.parametrize("n,order", [((511, 511), 1), ((600, 500), 2), ((180, 180), 3), ((255, 127), 5)])
+def test_quad4_vectors_at_the_limits(n, order, monkeypatch):
+    """quad4 residuals on either side of the sizes between cell vectors and the row-owner kernel: the same as the
+    row-owner kernel's (forced), within 1e-13 of the largest entry"""
+    for m in ((n[0] - 1, n[1]), n):
+        X, C = make_mesh(N.QUAD4, m)
+        ranks, nn = N.dof_layer(N.QUAD4, C, N.QUAD4)
+        ctx = N.Context()
+        ctx.set_cells(N.QUAD4, X, C)
+        ctx.set_dof_type(0, N.QUAD4, 2, 2 * nn, N.cell_dofs(ranks, 2))
+        ctx.set_integrand(N.linear_elastic_params(2, 30000.0, 0.2))
+        ctx.set_rule(0, order)
+        ctx.build_pattern()
+        u = to_dev(S.uniform(S.SEED_U, 2 * nn, -1e-3, 1e-3))
+        R = ctx.build_vector(u).cpu().numpy()
+        monkeypatch.setenv("NUTO_AMD_GENERIC", "1")
+        want = ctx.build_vector(u).cpu().numpy()
+        monkeypatch.delenv("NUTO_AMD_GENERIC")
+        assert np.abs(R - want).max() <= 1e-13 * np.abs(want).max()
+
+
 # local damage: (coordinate element, dof element, cells, rule, forms of the matrix assembly)
 LOCAL = [(N.HEX8, N.HEX8, (4, 3, 3), (0, 2), "0123"), (N.HEX8, N.HEX8, (2, 2, 2), (0, 3), "0123"),
          (N.HEX8, N.HEX8, (2, 2, 2), (0, 4), "0"), (N.HEX8, N.HEX20, (3, 2, 2), (0, 3), "0123"),
