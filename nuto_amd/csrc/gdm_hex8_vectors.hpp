@@ -18,7 +18,8 @@
 //
 // Two kernels: kGdmHex8CellVec evaluates every integration point once, sums the cell's vector over its
 // points and writes it (32 doubles per cell) and d_theta; kGatherCellVectors adds the cells' entries of
-// every dof node in group order. Nothing limits the number of cells or neighbours of a node.
+// every dof node in group order. Nothing limits the number of cells or neighbours of a node. The adjoint of a
+// small mesh takes one kernel, kGdmHex8NodeVec.
 // Measured on 262,144 cells, affine: adjoint 66 us for the cells + 23 us for the gather, residual 41 + 23
 // us (120 and 110 MB moved; the vector arithmetic, about 650 and 450 instructions per wave, takes as long
 // as the memory). With every node's workgroup evaluating the points of its own 8 cells the adjoint took
@@ -31,75 +32,55 @@
 namespace nuto_amd
 {
 
-// One wave per 8 cells (lane (r, m): cell 8 w + r, corner m). The geometry records of the wave's cells are
-// contiguous and pass through LDS, so that they are read with 16 contiguous bytes per lane; the 4
-// values of the lane's node go to out[cell][node][4].
-template <bool FULLDMG, bool AFF, bool ADJ>
-__global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const GdmHex8Tables T,
-                                                       const double* __restrict__ lam, double* __restrict__ out,
-                                                       double* __restrict__ dtheta)
+// What lane (r, m) reads of its cell: the state and lambda at the lane's node q, the history at its point and the
+// material (scalar parameters map to f_t = kappa0 E, G_f = f_t / beta)
+struct CellPoint
 {
-    using namespace gdm8;
-    constexpr int kPerCell = AFF ? kGeo / 2 : 8 * kGeo / 2;  // 16-byte chunks of geometry per cell
-    __shared__ __align__(16) double stage[16 * kPerCell];
-    __shared__ double sE[64];  // eeq of the cells' nodes
-    const int lane = (int)threadIdx.x, r = lane >> 3;
-    const CornerLane c = CornerOf(lane);
-    const long long cell0 = (long long)blockIdx.x * 8;
-    const int nc = (int)(A.nCells - cell0 < 8 ? A.nCells - cell0 : 8);  // cells of this block, >= 1
-    const bool valid = r < nc;
-    const int cell = (int)cell0 + (valid ? r : 0);
+    double v[4], l[4], kh, E, k0, beta, gf;
+};
+
+template <bool ADJ>
+__device__ inline void LoadCellPoint(const RowArgs& A, const CornerLane& c, int cell, int q,
+                                     const double* __restrict__ lam, CellPoint& o)
+{
     const LawParams& P = A.P;
-    const int q = A.dconn[(size_t)cell * 8 + c.node];
-    {
-        const double2* src =
-            reinterpret_cast<const double2*>(AFF ? T.geoCell + cell0 * kGeo : T.geo + cell0 * 8 * kGeo);
-        double2* dst = reinterpret_cast<double2*>(stage);
-#pragma unroll
-        for (int i = 0; i < (8 * kPerCell + 63) / 64; i++)
-        {
-            const int k = lane + 64 * i;
-            if (k < nc * kPerCell)
-                dst[k] = src[k];
-        }
-    }
     const int hist = A.cellId ? A.cellId[cell] : cell;
-    const double kh = A.kappa[(size_t)hist + (size_t)c.ip * A.kappaLd];
-    // scalar parameters map to f_t = kappa0 E, G_f = f_t / beta
-    double E = P.E, k0 = P.kappa0, beta = P.beta, gf = k0 * E / beta;
+    o.kh = A.kappa[(size_t)hist + (size_t)c.ip * A.kappaLd];
+    o.E = P.E;
+    o.k0 = P.kappa0;
+    o.beta = P.beta;
+    o.gf = o.k0 * o.E / o.beta;
     if (A.thE)
     {
-        E = A.thE[cell];
+        o.E = A.thE[cell];
         const double ft = A.thFt[cell];
-        gf = A.thGf[cell];
-        k0 = ft / E;
-        beta = ft / gf;
+        o.gf = A.thGf[cell];
+        o.k0 = ft / o.E;
+        o.beta = ft / o.gf;
     }
-    double v[4], l[4];
 #pragma unroll
     for (int i = 0; i < 3; i++)
-        v[i] = A.u[(size_t)q * 3 + i];
-    v[3] = A.e[q];
+        o.v[i] = A.u[(size_t)q * 3 + i];
+    o.v[3] = A.e[q];
     if constexpr (ADJ)
     {
 #pragma unroll
         for (int i = 0; i < 3; i++)
-            l[i] = lam[(size_t)q * 3 + i];
-        l[3] = lam[(size_t)A.nU + q];
+            o.l[i] = lam[(size_t)q * 3 + i];
+        o.l[3] = lam[(size_t)A.nU + q];
     }
-    sE[8 * r + c.node] = v[3];
-    __syncthreads();
-    double g[kGeo];
-    {
-        const double2* gs = reinterpret_cast<const double2*>(stage + (AFF ? r : r * 8 + c.ip) * kGeo);
-#pragma unroll
-        for (int k = 0; k < kGeo / 2; k++)
-        {
-            const double2 w = gs[k];
-            g[2 * k] = w.x;
-            g[2 * k + 1] = w.y;
-        }
-    }
+}
+
+// The cell's vector at the lane's node, summed over the cell's points, into res. sE: eeq of the cell's nodes (LDS,
+// written before a barrier); g: the geometry record of the lane's point. ADJ: theta (if wanted) = the cell's
+// d_theta, known to every lane of the group.
+template <bool FULLDMG, bool ADJ>
+__device__ inline void CellVectorTerms(const LawParams& P, const CornerLane& c, const CellPoint& pt, const double* sE,
+                                       const double* g, bool wantTheta, double res[4], double theta[3])
+{
+    using namespace gdm8;
+    const double *v = pt.v, *l = pt.l;
+    const double kh = pt.kh, E = pt.E, k0 = pt.k0, beta = pt.beta, gf = pt.gf;
     const double inv[3][3] = {{g[0], g[1], g[2]}, {g[3], g[4], g[5]}, {g[6], g[7], g[8]}};
     const double s = g[9];
     const double m3K = P.cK * E, m2G = P.cG * E;
@@ -117,7 +98,7 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
     // kappa' jumps where eeq meets the history, as it does at every loading point after an update: eeq is bit
     // for bit the value that the update and the matrix kernels form, so that all take the same side and a
     // residual does not change with the update
-    const double eN = NodeSum(c, sE + 8 * r);
+    const double eN = NodeSum(c, sE);
     GdmIp st;
     GdmIpState<FULLDMG>(Hu, he, eN, inv0, kh, m3K, m2G, k0, beta, P, st);
 
@@ -152,7 +133,7 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
         for (int i = 0; i < 3; i++)
             grad[i] *= s * P.c;
         value = s * (st.dom * st.dk * dsel + lN);
-        if (dtheta)
+        if (wantTheta)
         {
             // d omega / d kappa0 and d omega / d beta of DamageLawExponential (zero below kappa0)
             double dwk = 0.0, dwb = 0.0;
@@ -163,15 +144,9 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
                 dwk = -ik * (1.0 - P.alpha + P.alpha * ex) - k0 * ik * P.alpha * beta * ex;
                 dwb = -k0 * ik * P.alpha * ex * (k0 - st.kap);
             }
-            const double t0 = CornerSum(s * (sgel / E + dsel * dwk * (-k0 / E)));
-            const double t1 = CornerSum(s * dsel * (dwk / E + dwb / gf));
-            const double t2 = CornerSum(s * dsel * dwb * (-beta / gf));
-            if (valid && (lane & 7) == 0)
-            {
-                dtheta[cell] = t0;
-                dtheta[(size_t)A.nCells + cell] = t1;
-                dtheta[(size_t)2 * A.nCells + cell] = t2;
-            }
+            theta[0] = CornerSum(s * (sgel / E + dsel * dwk * (-k0 / E)));
+            theta[1] = CornerSum(s * dsel * (dwk / E + dwb / gf));
+            theta[2] = CornerSum(s * dsel * dwb * (-beta / gf));
         }
     }
     else
@@ -189,7 +164,7 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
     }
     // sigma g_a = (sigma J^-T) dN_a/dxi: the reference-space terms of this point, then the node's sums
     const double S[3][3] = {{sig[0], sig[5], sig[4]}, {sig[5], sig[1], sig[3]}, {sig[4], sig[3], sig[2]}};
-    double res[4], p[3];
+    double p[3];
 #pragma unroll
     for (int i = 0; i < 3; i++)
     {
@@ -202,11 +177,124 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
     for (int k = 0; k < 3; k++)
         p[k] = grad[0] * inv0[k][0] + grad[1] * inv0[k][1] + grad[2] * inv0[k][2];
     res[3] = PointsToNode<true>(c, p, kValueScale * value);
+}
+
+__device__ inline void StoreTheta(const RowArgs& A, int cell, const double theta[3], double* __restrict__ dtheta)
+{
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        dtheta[(size_t)k * A.nCells + cell] = theta[k];
+}
+
+// One wave per 8 cells (lane (r, m): cell 8 w + r, corner m). The geometry records of the wave's cells are
+// contiguous and pass through LDS, so that they are read with 16 contiguous bytes per lane; the 4
+// values of the lane's node go to out[cell][node][4].
+template <bool FULLDMG, bool AFF, bool ADJ>
+__global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const GdmHex8Tables T,
+                                                       const double* __restrict__ lam, double* __restrict__ out,
+                                                       double* __restrict__ dtheta)
+{
+    using namespace gdm8;
+    constexpr int kPerCell = AFF ? kGeo / 2 : 8 * kGeo / 2;  // 16-byte chunks of geometry per cell
+    __shared__ __align__(16) double stage[16 * kPerCell];
+    __shared__ double sE[64];  // eeq of the cells' nodes
+    const int lane = (int)threadIdx.x, r = lane >> 3;
+    const CornerLane c = CornerOf(lane);
+    const long long cell0 = (long long)blockIdx.x * 8;
+    const int nc = (int)(A.nCells - cell0 < 8 ? A.nCells - cell0 : 8);  // cells of this block, >= 1
+    const bool valid = r < nc;
+    const int cell = (int)cell0 + (valid ? r : 0);
+    const int q = A.dconn[(size_t)cell * 8 + c.node];
+    {
+        const double2* src =
+            reinterpret_cast<const double2*>(AFF ? T.geoCell + cell0 * kGeo : T.geo + cell0 * 8 * kGeo);
+        double2* dst = reinterpret_cast<double2*>(stage);
+#pragma unroll
+        for (int i = 0; i < (8 * kPerCell + 63) / 64; i++)
+        {
+            const int k = lane + 64 * i;
+            if (k < nc * kPerCell)
+                dst[k] = src[k];
+        }
+    }
+    CellPoint pt;
+    LoadCellPoint<ADJ>(A, c, cell, q, lam, pt);
+    sE[8 * r + c.node] = pt.v[3];
+    __syncthreads();
+    double g[kGeo];
+    {
+        const double2* gs = reinterpret_cast<const double2*>(stage + (AFF ? r : r * 8 + c.ip) * kGeo);
+#pragma unroll
+        for (int k = 0; k < kGeo / 2; k++)
+        {
+            const double2 w = gs[k];
+            g[2 * k] = w.x;
+            g[2 * k + 1] = w.y;
+        }
+    }
+    double res[4], theta[3];
+    CellVectorTerms<FULLDMG, ADJ>(A.P, c, pt, sE + 8 * r, g, dtheta != nullptr, res, theta);
+    if (ADJ && dtheta && valid && (lane & 7) == 0)
+        StoreTheta(A, cell, theta, dtheta);
     if (valid)
     {
         double2* dst = reinterpret_cast<double2*>(out + ((size_t)cell * 8 + c.node) * 4);
         dst[0] = make_double2(res[0], res[1]);
         dst[1] = make_double2(res[2], res[3]);
+    }
+}
+
+// The adjoint in one launch, for small meshes: one wave per dof node, lane (r, m) corner m of the r-th cell
+// incident to it. Every cell is evaluated for each of its 8 nodes, but up to 16 waves per CU the time is about
+// the latency of one wave, and a second launch costs more. d_theta is the entry of the wave whose node is the
+// cell's local node 0. Measured, the whole call, one launch / two: 27 to 4096 nodes 10.3 / 12.8 us, 4913 nodes
+// 11.5 / 12.8 us, 6859 nodes 14.6 / 12.8 us.
+constexpr int kNodeVecNodes = 16 * 256;
+template <bool FULLDMG, bool AFF>
+__global__ void __launch_bounds__(64) kGdmHex8NodeVec(const RowArgs A, const GdmHex8Tables T,
+                                                       const double* __restrict__ lam, double* __restrict__ vec,
+                                                       double* __restrict__ dtheta)
+{
+    using namespace gdm8;
+    __shared__ double sE[64], sV[32];
+    const int pos = NodeOfBlock(T);
+    if (pos < 0)
+        return;
+    const int lane = (int)threadIdx.x, r = lane >> 3;
+    const CornerLane c = CornerOf(lane);
+    const NodeTab tab = LoadNodeTab(T, pos, r, c);
+    const int p = T.nodeHead[pos].x;
+    const bool valid = tab.cell >= 0;
+    const int cell = valid ? tab.cell : 0;
+    if (lane < 32)
+        sV[lane] = 0.0;
+    if (A.nCells > 0)
+    {
+        NodeRecord<false> rec;
+        LoadNodeRecord<false, AFF, false>(A, T, tab, c, rec);
+        CellPoint pt;
+        LoadCellPoint<true>(A, c, cell, A.dconn[(size_t)cell * 8 + c.node], lam, pt);
+        sE[8 * r + c.node] = pt.v[3];
+        __syncthreads();
+        double res[4], theta[3];
+        CellVectorTerms<FULLDMG, true>(A.P, c, pt, sE + 8 * r, rec.g, dtheta != nullptr, res, theta);
+        if (valid && c.node == tab.la)
+        {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                sV[4 * r + k] = res[k];
+            if (dtheta && tab.la == 0)
+                StoreTheta(A, cell, theta, dtheta);
+        }
+    }
+    __syncthreads();
+    if (lane < 4)
+    {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            s += sV[4 * k + lane];
+        vec[lane < 3 ? (size_t)p * 3 + lane : (size_t)A.nU + p] = s;
     }
 }
 
@@ -217,10 +305,28 @@ inline void LaunchGdmHex8Vector(const GdmHex8Plan& plan, const RowArgs& a, const
                                 double* dtheta, double* work, hipStream_t stream)
 {
     const GdmHex8Tables t = plan.Tables();
+    const bool full = a.P.damage_application == 0;
+    if constexpr (ADJ)
+    {
+        if (plan.nExtra == 0 && plan.nNodes <= kNodeVecNodes)
+        {
+            const dim3 grid((unsigned)plan.grid), block(64);
+            if (plan.nNodes == 0)
+                return;
+            if (full && plan.affine)
+                hipLaunchKernelGGL((kGdmHex8NodeVec<true, true>), grid, block, 0, stream, a, t, lam, vec, dtheta);
+            else if (full)
+                hipLaunchKernelGGL((kGdmHex8NodeVec<true, false>), grid, block, 0, stream, a, t, lam, vec, dtheta);
+            else if (plan.affine)
+                hipLaunchKernelGGL((kGdmHex8NodeVec<false, true>), grid, block, 0, stream, a, t, lam, vec, dtheta);
+            else
+                hipLaunchKernelGGL((kGdmHex8NodeVec<false, false>), grid, block, 0, stream, a, t, lam, vec, dtheta);
+            return;
+        }
+    }
     if (a.nCells > 0)
     {
         const dim3 grid((unsigned)((a.nCells + 7) / 8)), block(64);
-        const bool full = a.P.damage_application == 0;
         if (full && plan.affine)
             hipLaunchKernelGGL((kGdmHex8CellVec<true, true, ADJ>), grid, block, 0, stream, a, t, lam, work, dtheta);
         else if (full)

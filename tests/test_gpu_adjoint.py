@@ -184,3 +184,39 @@ def test_vjp_is_K_transpose_lambda_at_full_size():
     kb = torch.zeros(n_rows, dtype=torch.float64, device="cuda").index_add_(0, col, K.abs() * lam.abs()[rows])
     err = (d_state - kt).abs()
     assert bool((err <= 1e-12 * kb).all()), f"max err/bound {float((err / kb).max()):.3e}"
+
+
+@pytest.mark.parametrize("n", [(1, 1, 1), (5, 4, 3), (15, 15, 15), (16, 15, 15)])
+@pytest.mark.parametrize("app", [N.FULL, N.UNILATERAL])
+@pytest.mark.parametrize("jitter", [0.0, 0.1])
+def test_one_launch_adjoint_against_cell_vectors(n, app, jitter):
+    """A mesh alone (one launch up to 4096 nodes) against the same mesh in a batch with a larger one (cell vectors and a
+    gather): K^T lambda and d_theta, the same operations in the same order, within 1e-13 of the largest entry."""
+    p, th = gdm_pair(n, app, jitter=jitter)
+    q, tq = gdm_pair((17, 16, 15), app, jitter=0.1 if n[0] % 2 else 0.0)
+    u, e, kap = p.inputs()
+    ctx = p.context()
+    ctx.set_material_fields(*th)
+    lam = S.uniform(0x55, p.n_u + p.n_e, -1.0, 1.0)
+    ds, dt = (t.cpu().numpy() for t in ctx.vjp(to_dev(u), to_dev(e), to_dev(kap), to_dev(lam)))
+    b = N.Batch()
+    b.set_integrand(p.params_dev)
+    for m in (p, q):
+        b.add_mesh(N.HEX8, N.HEX8, m.X, m.C, m.ranks, m.nn)
+    sz = b.build()
+    b.set_material_fields(*(np.concatenate([x, y]) for x, y in zip(th, tq)))
+    i = b.mesh_info(0)
+    ub, eb, kb, lb = (S.uniform(s, sz[k], 0.0, h) for s, k, h in ((1, "u", 1e-3), (2, "e", 5e-4), (3, "history", 3e-4), (4, "R", 1.0)))
+    ub[i["u"]:i["u"] + p.n_u] = u
+    eb[i["e"]:i["e"] + p.nn] = e
+    cells = np.arange(p.ncells)
+    for ip in range(8):
+        kb[i["history"] + cells + ip * i["history_ld"]] = kap[cells + ip * p.ncells]
+    lb[i["R_u"]:i["R_u"] + p.n_u] = lam[:p.n_u]
+    lb[i["R_e"]:i["R_e"] + p.nn] = lam[p.n_u:]
+    bs, bt = (t.cpu().numpy() for t in b.vjp(to_dev(ub), to_dev(eb), to_dev(kb), to_dev(lb)))
+    got = np.concatenate([bs[i["R_u"]:i["R_u"] + p.n_u], bs[i["R_e"]:i["R_e"] + p.nn]])
+    assert np.abs(got - ds).max() <= 1e-13 * np.abs(ds).max()
+    for k in range(3):
+        f = bt[i["theta"] + k * i["theta_stride"] + cells]
+        assert np.abs(f - dt[k]).max() <= 1e-13 * np.abs(dt[k]).max()
