@@ -3,10 +3,11 @@
 // (GradientDamage::Update, GradientDamage.h:122-125; EvolutionImplicit::Update,
 // LocalIsotropicDamage.h:130-133) and the fields of Cell::Eval (Cell.h:80-93).
 //
-// One wave takes 64 / NIP cells: their coordinates and node values go to LDS once, lane (cell, IP) forms
-// the point's state, and for R_e lane (cell, node) adds the points in rule order from LDS. A point is
-// evaluated once; the row-owner kernel evaluates it for every node of its cell. The sum over the cells is
-// kGatherCellVectors. Bound by the latency of the gathers and the two passes over LDS.
+// One workgroup takes as many whole cells as its threads have points: their coordinates and node values go to
+// LDS once, lane (cell, IP) forms the point's state, and for R_e lane (cell, node) adds the points in rule order
+// from LDS. A point is evaluated once; the row-owner kernel evaluates it for every node of its cell. The sum
+// over the cells is kGatherCellVectors. Bound by the latency of the gathers and the two passes over LDS. Where
+// a cell has one point (kOwn) its lane is the only reader of its nodes, which then stay in registers.
 // Measured on 47,880 ten-node tetrahedra with local damage: residual 267 us by the row-owner kernel, 22 +
 // 10 us (gather) here; history 15 -> 13 us, stresses 17 -> 15 us (one lane per point with its own gathers
 // before). 2993 waves, three per SIMD: the chain of loads, not a rate, is what is left.
@@ -60,6 +61,16 @@ __device__ inline void PointTerms(double s, const double* sig, const double inv[
         }
 }
 
+// threads of a workgroup: four waves where a lane has a cell (fewer workgroups to dispatch; 384,000 tet4 cells with
+// local damage: history 12.1 us with a wave and LDS, 8.8 with a wave and registers, 8.1 with four waves; kappa 13.2,
+// 9.0, 8.4 us), and where a wave's whole cells would leave more than a fifth of its lanes idle (25 points; 10^6
+// quad4 cells: strain 414 -> 334 us). Elsewhere one wave: four take longer at their barriers (27 points, 125,000
+// hex8 cells: strain 114 -> 131 us).
+constexpr int PointThreads(int nip)
+{
+    return nip == 1 || 64 % nip * 5 > 64 ? 256 : 64;
+}
+
 // kappa = max(history, eeq) of gradient damage. It needs no geometry: a lane per cell, the grid's second
 // dimension the point, so that the shape values are scalars and the history, stored point by point, is read and
 // written in consecutive lanes. Measured, kCellPoints / this kernel: 13,824 cells with 64 points 23.1 / 7.1 us,
@@ -83,17 +94,19 @@ __global__ void __launch_bounds__(256) kNonlocalHistory(const RowArgs A, double*
 }
 
 template <int KIND, int DIM, int NNC, int NND, int NIP, int OUT>
-__global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, double* __restrict__ out)
+__global__ void __launch_bounds__(PointThreads(NIP)) kCellPoints(const RowArgs A, int field, double* __restrict__ out)
 {
-    constexpr int CPW = 64 / NIP;                       // cells per wave
+    constexpr int NT = PointThreads(NIP);
+    constexpr int CPW = NT / NIP;                       // cells per workgroup
+    constexpr bool kOwn = NIP == 1;                     // a lane has its cell to itself: nodes in registers
     constexpr bool GD = KIND == kGradientDamage;
     constexpr int F = GD ? DIM + 1 : DIM;               // values per node
     constexpr int S = 1 + NNC * DIM + NND + NND * DIM;  // IP table row: w, dNc, N, dNd
     constexpr int NV = DIM == 2 ? 3 : 6;
     constexpr int SX = NNC * DIM | 1, SU = NND * F | 1;  // odd strides: consecutive cells on other banks
     constexpr int PR = GD ? DIM * DIM + DIM + 1 : (DIM == 2 ? 5 : 9);  // doubles per point in LDS (odd)
-    static_assert(CPW >= 1, "a wave holds a cell's points");
-    constexpr int IN = CPW * (SX + SU), RES = CPW * NIP * PR;
+    static_assert(CPW >= 1, "a workgroup holds a cell's points");
+    constexpr int IN = kOwn ? 0 : CPW * (SX + SU), RES = OUT == kPointHistory ? 1 : CPW * NIP * PR;
     __shared__ double pool[IN > RES ? IN : RES];  // the cells' nodes, then the points' results
     double* sX = pool;
     double* sU = pool + CPW * SX;
@@ -104,16 +117,46 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
     const LawParams& P = A.P;
     static_assert(!(GD && OUT == kPointHistory), "kNonlocalHistory");
     // every node number, then every node value is loaded before the first of them is waited for
-    constexpr int ITX = (CPW * NNC + 63) / 64, ITU = (CPW * NND + 63) / 64;
+    constexpr int ITX = (CPW * NNC + NT - 1) / NT, ITU = (CPW * NND + NT - 1) / NT;
+    double rX[kOwn ? NNC * DIM : 1], rU[kOwn ? NND * F : 1];
+    if constexpr (kOwn)
+    {
+        const size_t cell = (size_t)cell0 + (lane < nc ? lane : 0);
+        int nx[NNC], nu[NND];
+#pragma unroll
+        for (int k = 0; k < NNC; k++)
+            nx[k] = A.cconn[cell * NNC + k];
+#pragma unroll
+        for (int k = 0; k < NND; k++)
+            nu[k] = A.dconn[cell * NND + k];
+#pragma unroll
+        for (int k = 0; k < NNC; k++)
+        {
+            rX[k * DIM] = A.x[nx[k]];
+            rX[k * DIM + 1] = A.y[nx[k]];
+            if constexpr (DIM == 3)
+                rX[k * DIM + 2] = A.z[nx[k]];
+        }
+#pragma unroll
+        for (int k = 0; k < NND; k++)
+        {
+#pragma unroll
+            for (int i = 0; i < DIM; i++)
+                rU[k * F + i] = A.u[(size_t)nu[k] * DIM + i];
+            if constexpr (GD)
+                rU[k * F + DIM] = A.e[nu[k]];
+        }
+    }
+    else
     {
         int nx[ITX], nu[ITU];
         double x[ITX][DIM], v[ITU][F];
 #pragma unroll
         for (int i = 0; i < ITX; i++)
-            nx[i] = A.cconn[(size_t)cell0 * NNC + (lane + 64 * i < nc * NNC ? lane + 64 * i : 0)];
+            nx[i] = A.cconn[(size_t)cell0 * NNC + (lane + NT * i < nc * NNC ? lane + NT * i : 0)];
 #pragma unroll
         for (int i = 0; i < ITU; i++)
-            nu[i] = A.dconn[(size_t)cell0 * NND + (lane + 64 * i < nc * NND ? lane + 64 * i : 0)];
+            nu[i] = A.dconn[(size_t)cell0 * NND + (lane + NT * i < nc * NND ? lane + NT * i : 0)];
 #pragma unroll
         for (int i = 0; i < ITX; i++)
         {
@@ -134,7 +177,7 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
 #pragma unroll
         for (int i = 0; i < ITX; i++)
         {
-            const int k = lane + 64 * i;
+            const int k = lane + NT * i;
             if (k < nc * NNC)
             {
 #pragma unroll
@@ -145,7 +188,7 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
 #pragma unroll
         for (int i = 0; i < ITU; i++)
         {
-            const int k = lane + 64 * i;
+            const int k = lane + NT * i;
             if (k < nc * NND)
             {
 #pragma unroll
@@ -153,8 +196,8 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
                     sU[k / NND * SU + k % NND * F + m] = v[i][m];
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
 
     const int cl = lane / NIP, ip = lane - cl * NIP;
     double o[PR];  // the point's results
@@ -165,7 +208,8 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
         const double* dNc = t + 1;
         const double* Nd = dNc + NNC * DIM;
         const double* dNd = Nd + NND;
-        const double* U = sU + cl * SU;
+        const double* X = kOwn ? rX : sX + cl * SX;
+        const double* U = kOwn ? rU : sU + cl * SU;
         double eN = 0.0;
         if constexpr (GD)
         {
@@ -175,7 +219,7 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
         }
         double eps[NV], inv[DIM][DIM], ge[3] = {0.0, 0.0, 0.0}, s = 0.0;
         double J[DIM][DIM];
-        NodalGradient<DIM, NNC, DIM>(sX + cl * SX, dNc, J);
+        NodalGradient<DIM, NNC, DIM>(X, dNc, J);
         s = Inverse<DIM>(J, inv) * t[0];
         if constexpr (DIM == 2 || GD)
         {
@@ -298,7 +342,17 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
     }
     if constexpr (OUT == kPointHistory)
         return;
-    __syncthreads();  // the results overwrite the nodes
+    if constexpr (kOwn && OUT == kPointField)
+    {
+        if (field > kIpStress)
+        {
+            if (cl < nc)
+                out[cell0 + cl] = o[0];
+            return;
+        }
+    }
+    if constexpr (!kOwn)
+        __syncthreads();  // the results overwrite the nodes
     if (cl < nc)
     {
 #pragma unroll
@@ -311,12 +365,12 @@ __global__ void __launch_bounds__(64) kCellPoints(const RowArgs A, int field, do
         // the block's values are contiguous: written with consecutive lanes on consecutive doubles
         const int w = field <= kIpStress ? NV : 1;
         double* dst = out + (size_t)cell0 * NIP * w;
-        for (int k = lane; k < nc * NIP * w; k += 64)
+        for (int k = lane; k < nc * NIP * w; k += NT)
             dst[k] = sP[(k / w) * PR + k % w];
         return;
     }
     // R_e: the points' reference-space terms against dN_a/dxi (and N_a), in rule order
-    for (int k = lane; k < nc * NND; k += 64)
+    for (int k = lane; k < nc * NND; k += NT)
     {
         const int c = k / NND, a = k - c * NND;
         double r[F];

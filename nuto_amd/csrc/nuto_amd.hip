@@ -654,10 +654,10 @@ void LaunchTwoPhaseT(nuto_ctx* ctx, const RowArgs& a, bool wr, int c0, int c1, i
 template <int KIND, int DIM, int NNC, int NND, int NIP, int OUT>
 void LaunchPoints(nuto_ctx* ctx, const RowArgs& a, int field, double* out)
 {
-    constexpr int CPW = 64 / NIP;
+    constexpr int CPW = PointThreads(NIP) / NIP;
     if (a.nCells > 0)
         hipLaunchKernelGGL((kCellPoints<KIND, DIM, NNC, NND, NIP, OUT>), dim3((unsigned)((a.nCells + CPW - 1) / CPW)),
-                           dim3(64), 0, ctx->stream, a, field, out);
+                           dim3(PointThreads(NIP)), 0, ctx->stream, a, field, out);
 }
 
 template <int KIND, int DIM, int NNC, int NND, int NIP, int BH>

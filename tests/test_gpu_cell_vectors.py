@@ -97,8 +97,9 @@ def test_adjoint_at_the_updated_history():
     assert (np.abs(got - kt) <= 1e-12 * kb + 1e-300).all()
 
 
-# (coordinate element, dof element, cells, rule); a wave takes 64, 16, 8, 4, 2 or 1 cells
+# (coordinate element, dof element, cells, rule); a workgroup takes 256 (one point), 16, 10 (25 points), 8, 4, 2 or 1 cells
 GENERIC = [(N.QUAD4, N.QUAD4, (1, 1), (0, 1)), (N.QUAD4, N.QUAD4, (5, 4), (0, 2)), (N.QUAD4, N.QUAD4, (3, 3), (0, 5)),
+           (N.QUAD4, N.QUAD4, (4, 3), (0, 5)), (N.QUAD4, N.QUAD4, (17, 16), (0, 1)), (N.TET4, N.TET4, (4, 4, 3), (1, 1)),
            (N.HEX8, N.HEX8, (3, 3, 1), (0, 2)), (N.HEX8, N.HEX8, (1, 1, 1), (0, 3)), (N.HEX8, N.HEX8, (2, 1, 1), (0, 4)),
            (N.HEX8, N.HEX20, (3, 1, 1), (0, 3)), (N.TET4, N.TET4, (1, 1, 1), (1, 1)), (N.TET4, N.TET4, (3, 2, 2), (1, 1)),
            (N.TET4, N.TET10, (3, 1, 1), (1, 2))]
