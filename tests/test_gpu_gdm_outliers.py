@@ -3,9 +3,11 @@ around a vertical axis in two layers, so the axis node of the middle level has 1
 and 33 neighbours (the node kernel takes at most 8 and 32). That node's rows come from the generic
 row-owner kernel, every other node's from the node kernel; R and K against the oracle, the
 outside node's rows bit-identical to the all-generic assembly, and the allocation-free entry point
-on the same mesh. The adjoint of that node (and d_theta of the cells whose local node 0 it is) comes
-from the adjoint's list kernel: d_state against K^T lambda of the oracle's K, d_theta against
-central finite differences of the oracle's R. Batches holding this mesh: tests/test_gpu_batch.py."""
+on the same mesh, each with one launch for the node kernel, as a mesh of this size takes it, and with the
+pre-pass of large meshes forced. The residual alone and the adjoint go through cell vectors, which know no
+bounds: d_state of that node against K^T lambda of the oracle's K, d_theta of the cells whose local
+node 0 it is against central finite differences of the oracle's R. Batches holding this mesh:
+tests/test_gpu_batch.py."""
 import numpy as np
 import pytest
 import torch
@@ -18,6 +20,12 @@ from test_gpu_adjoint import kt_lambda
 from test_gpu_parity import gdm_params
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(params=["", "1"], ids=["one launch", "prepass"])
+def path(request, monkeypatch):
+    if request.param:
+        monkeypatch.setenv("NUTO_AMD_GDM_PREPASS", request.param)
 
 
 def fan_mesh(sectors=5, layers=2, outer=1.2):
@@ -42,7 +50,7 @@ def fan_mesh(sectors=5, layers=2, outer=1.2):
     return np.array(X), np.array(C, np.int32)
 
 
-def test_outside_node_by_the_generic_kernel(monkeypatch):
+def test_outside_node_by_the_generic_kernel(path, monkeypatch):
     X, C = fan_mesh()
     p = Pair(N.HEX8, N.HEX8, X, C, *gdm_params(), True)
     u, e, kap = p.inputs(u_range=4e-4, k_range=1.5e-4)
@@ -53,6 +61,7 @@ def test_outside_node_by_the_generic_kernel(monkeypatch):
     assert np.array_equal(rp, ref["row_ptr"]) and np.array_equal(ci, ref["col"])
     check_values(R.cpu().numpy(), ref["R"], ref["R_bound"], "R")
     check_values(K.cpu().numpy(), ref["val"], ref["bound"], "K")
+    check_values(ctx.build_vector(to_dev(u), to_dev(e), to_dev(kap)).cpu().numpy(), ref["R"], ref["R_bound"], "R alone")
     # the axis node of the middle level (dof rank of coordinate node 11) is the one outside
     axis = int(p.ranks[np.argwhere(C == 11)[0][0], np.argwhere(C == 11)[0][1]])
     monkeypatch.setenv("NUTO_AMD_GENERIC", "1")
@@ -107,7 +116,7 @@ def test_outside_node_adjoint(app):
     assert (np.abs(got_t - fd) <= 1e-6 * scale).all(), f"max rel {np.max(np.abs(got_t - fd) / scale):.3e}"
 
 
-def test_outside_node_allocation_free():
+def test_outside_node_allocation_free(path):
     X, C = fan_mesh()
     p = Pair(N.HEX8, N.HEX8, X, C, *gdm_params(), True)
     u, e, kap = (to_dev(a) for a in p.inputs(u_range=4e-4, k_range=1.5e-4))

@@ -69,4 +69,11 @@ def test_cell_ids_select_history_columns(path):
             ctx.set_history_ld(hld)
         ctx.build_pattern()
         out.append([t.cpu().numpy() for t in ctx.build_vector_matrix(to_dev(u), to_dev(e), to_dev(kk))])
+        dk = to_dev(kk)
+        ctx.update_history(to_dev(u), to_dev(e), dk)
+        out[-1].append(dk.cpu().numpy())
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    # the update writes the cells' own columns and nothing else
+    updated, by_id = out[0][2].reshape(8, nc), out[1][2].reshape(8, ld)
+    assert np.array_equal(by_id[:, ids], updated) and (updated > kap.reshape(8, nc)).any()
+    assert np.isnan(np.delete(by_id, ids, axis=1)).all()

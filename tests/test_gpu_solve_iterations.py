@@ -112,9 +112,13 @@ def test_stops_at_the_limit(element, n, terms, method):
 
 
 @pytest.mark.parametrize("seed", [0, 1, 2])
-def test_bicgstab_restart(seed):
+@pytest.mark.parametrize("form", ["0", "1", "terms"])
+def test_bicgstab_restart(seed, form, monkeypatch):
     """A lower triangular matrix on one quad4 cell (all its dofs are coupled) with f = e_0: after the
-    first iteration the residual has no entry at dof 0, so rho = 0 and the solver must restart."""
+    first iteration the residual has no entry at dof 0, so rho = 0 and the solver must restart: with stored
+    vectors, with the products forming theirs, and with a constraint term (dof 7 = half of dof 6)."""
+    if form != "terms":
+        monkeypatch.setenv("NUTO_AMD_SOLVE_FORM", form)
     X, C = make_mesh(N.QUAD4, (1, 1), (1.0, 1.0, 1.0))
     p = Pair(N.QUAD4, N.QUAD4, X, C, *le_params(2), two_fields=False)
     ctx = p.context()
@@ -123,11 +127,14 @@ def test_bicgstab_restart(seed):
     rng = np.random.default_rng(seed)
     A = np.tril(rng.uniform(-0.5, 0.5, (8, 8)), -1) + np.diag(rng.uniform(1.0, 2.0, 8))
     K = to_dev(A[np.repeat(np.arange(8), np.diff(rp)), ci])
-    ctx.set_constraints(0, [])
+    ctx.set_constraints(0, [(7, [(6, -0.5)])] if form == "terms" else [])
+    Cm = np.eye(8)[:, :7] if form == "terms" else np.eye(8)
+    if form == "terms":
+        Cm[7, 6] = 0.5
     f = np.zeros(8)
     f[0] = 1.0
     x, info = ctx.solve(K, to_dev(f), method=N.SOLVER_BICGSTAB, tol=1e-13, max_iter=200)
-    want = np.linalg.solve(A, f)
+    want = Cm @ np.linalg.solve(Cm.T @ A @ Cm, Cm.T @ f)
     assert info["iterations"] < 200 and info["relative_residual"] <= 1e-13
     assert np.abs(x.cpu().numpy() - want).max() <= 1e-9 * np.abs(want).max()
 
