@@ -72,11 +72,12 @@ __device__ inline void LoadCellPoint(const RowArgs& A, const CornerLane& c, int 
 }
 
 // The cell's vector at the lane's node, summed over the cell's points, into res. sE: eeq of the cell's nodes (LDS,
-// written before a barrier); g: the geometry record of the lane's point. ADJ: theta (if wanted) = the cell's
-// d_theta, known to every lane of the group.
+// written before a barrier); g: the geometry record of the lane's point. ADJ: the cell's d_theta (nCells apart) goes
+// to dtheta, if given, from the lane with `own`.
 template <bool FULLDMG, bool ADJ>
 __device__ inline void CellVectorTerms(const LawParams& P, const CornerLane& c, const CellPoint& pt, const double* sE,
-                                       const double* g, bool wantTheta, double res[4], double theta[3])
+                                       const double* g, double* __restrict__ dtheta, size_t nCells, bool own,
+                                       double res[4])
 {
     using namespace gdm8;
     const double *v = pt.v, *l = pt.l;
@@ -133,7 +134,7 @@ __device__ inline void CellVectorTerms(const LawParams& P, const CornerLane& c, 
         for (int i = 0; i < 3; i++)
             grad[i] *= s * P.c;
         value = s * (st.dom * st.dk * dsel + lN);
-        if (wantTheta)
+        if (dtheta)
         {
             // d omega / d kappa0 and d omega / d beta of DamageLawExponential (zero below kappa0)
             double dwk = 0.0, dwb = 0.0;
@@ -144,9 +145,15 @@ __device__ inline void CellVectorTerms(const LawParams& P, const CornerLane& c, 
                 dwk = -ik * (1.0 - P.alpha + P.alpha * ex) - k0 * ik * P.alpha * beta * ex;
                 dwb = -k0 * ik * P.alpha * ex * (k0 - st.kap);
             }
-            theta[0] = CornerSum(s * (sgel / E + dsel * dwk * (-k0 / E)));
-            theta[1] = CornerSum(s * dsel * (dwk / E + dwb / gf));
-            theta[2] = CornerSum(s * dsel * dwb * (-beta / gf));
+            const double t0 = CornerSum(s * (sgel / E + dsel * dwk * (-k0 / E)));
+            const double t1 = CornerSum(s * dsel * (dwk / E + dwb / gf));
+            const double t2 = CornerSum(s * dsel * dwb * (-beta / gf));
+            if (own)
+            {
+                dtheta[0] = t0;
+                dtheta[nCells] = t1;
+                dtheta[2 * nCells] = t2;
+            }
         }
     }
     else
@@ -177,13 +184,6 @@ __device__ inline void CellVectorTerms(const LawParams& P, const CornerLane& c, 
     for (int k = 0; k < 3; k++)
         p[k] = grad[0] * inv0[k][0] + grad[1] * inv0[k][1] + grad[2] * inv0[k][2];
     res[3] = PointsToNode<true>(c, p, kValueScale * value);
-}
-
-__device__ inline void StoreTheta(const RowArgs& A, int cell, const double theta[3], double* __restrict__ dtheta)
-{
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-        dtheta[(size_t)k * A.nCells + cell] = theta[k];
 }
 
 // One wave per 8 cells (lane (r, m): cell 8 w + r, corner m). The geometry records of the wave's cells are
@@ -232,10 +232,9 @@ __global__ void __launch_bounds__(64) kGdmHex8CellVec(const RowArgs A, const Gdm
             g[2 * k + 1] = w.y;
         }
     }
-    double res[4], theta[3];
-    CellVectorTerms<FULLDMG, ADJ>(A.P, c, pt, sE + 8 * r, g, dtheta != nullptr, res, theta);
-    if (ADJ && dtheta && valid && (lane & 7) == 0)
-        StoreTheta(A, cell, theta, dtheta);
+    double res[4];
+    CellVectorTerms<FULLDMG, ADJ>(A.P, c, pt, sE + 8 * r, g, dtheta ? dtheta + cell : nullptr, A.nCells,
+                                  valid && (lane & 7) == 0, res);
     if (valid)
     {
         double2* dst = reinterpret_cast<double2*>(out + ((size_t)cell * 8 + c.node) * 4);
@@ -276,15 +275,15 @@ __global__ void __launch_bounds__(64) kGdmHex8NodeVec(const RowArgs A, const Gdm
         LoadCellPoint<true>(A, c, cell, A.dconn[(size_t)cell * 8 + c.node], lam, pt);
         sE[8 * r + c.node] = pt.v[3];
         __syncthreads();
-        double res[4], theta[3];
-        CellVectorTerms<FULLDMG, true>(A.P, c, pt, sE + 8 * r, rec.g, dtheta != nullptr, res, theta);
-        if (valid && c.node == tab.la)
+        double res[4];
+        const bool own = valid && c.node == tab.la;  // this lane's corner is the node
+        CellVectorTerms<FULLDMG, true>(A.P, c, pt, sE + 8 * r, rec.g, dtheta ? dtheta + cell : nullptr, A.nCells,
+                                       own && tab.la == 0, res);
+        if (own)
         {
 #pragma unroll
             for (int k = 0; k < 4; k++)
                 sV[4 * r + k] = res[k];
-            if (dtheta && tab.la == 0)
-                StoreTheta(A, cell, theta, dtheta);
         }
     }
     __syncthreads();
