@@ -57,6 +57,7 @@ struct RowArgs
 // the same products in the same order where one lane sums one entry), Inverse<3>, StrainOfGradient and Mises3;
 // the nonlocal strain as the sum of N_n e_n node by node. Each names its fused multiply-adds: left to the
 // compiler, a b + c d is contracted one way in one kernel and the other way in the next, and the last bit differs.
+
 // g_ij = sum_n v_n[i] dN_n[j]; v: node n's DIM values at v[STRIDE n]
 template <int DIM, int N, int STRIDE>
 __device__ inline void NodalGradient(const double* v, const double* dN, double g[DIM][DIM])
@@ -222,225 +223,225 @@ __device__ inline void CellRows(const RowArgs& A, const CellNodes<KIND, DIM, NNC
     constexpr int S = 1 + NNC * DIM + NND + NND * DIM;
     const LawParams& P = A.P;
     const double E = c.E, k0 = c.k0, beta = c.beta;
-                for (int ip = 0; ip < NIP; ip++)
+    for (int ip = 0; ip < NIP; ip++)
+    {
+        const double* t = A.tab + ip * S;
+        const double w = t[0];
+        const double* dNc = t + 1;
+        const double* Nd = dNc + NNC * DIM;
+        const double* dNd = Nd + NND;
+        double J[DIM][DIM], inv[DIM][DIM];
+        NodalGradient<DIM, NNC, DIM>(&c.X[0][0], dNc, J);
+        const double detJ = Inverse<DIM>(J, inv);
+        const double s = detJ * w;
+
+        // strain (Voigt 2D [xx,yy,xy], 3D [xx,yy,zz,yz,zx,xy]), nonlocal value and gradient
+        constexpr int NV = DIM == 2 ? 3 : 6;
+        double eps[NV];
+        double eN = 0.0, ge[3] = {0.0, 0.0, 0.0};
+        if constexpr (KIND != kLocalDamage)
+        {
+            // the strain decides nothing here, and every dN_n/dX is needed anyway
+#pragma unroll
+            for (int i = 0; i < NV; i++)
+                eps[i] = 0.0;
+#pragma unroll
+            for (int b = 0; b < NND; b++)
+            {
+                double g[DIM];
+                Grad<DIM, NND>(dNd, b, inv, g);
+                AddStrain<DIM>(g, c.U[b], eps);
+                if constexpr (KIND == kGradientDamage)
                 {
-                    const double* t = A.tab + ip * S;
-                    const double w = t[0];
-                    const double* dNc = t + 1;
-                    const double* Nd = dNc + NNC * DIM;
-                    const double* dNd = Nd + NND;
-                    double J[DIM][DIM], inv[DIM][DIM];
-                    NodalGradient<DIM, NNC, DIM>(&c.X[0][0], dNc, J);
-                    const double detJ = Inverse<DIM>(J, inv);
-                    const double s = detJ * w;
+                    eN = fma(Nd[b], c.EE[b], eN);
+                    ge[0] += g[0] * c.EE[b];
+                    ge[1] += g[1] * c.EE[b];
+                    ge[2] += g[2] * c.EE[b];
+                }
+            }
+        }
+        else
+        {
+            double Ru[DIM][DIM];
+            NodalGradient<DIM, NND, DIM>(&c.U[0][0], dNd, Ru);
+            StrainOfGradient(&Ru[0][0], inv, eps);
+        }
 
-                    // strain (Voigt 2D [xx,yy,xy], 3D [xx,yy,zz,yz,zx,xy]), nonlocal value and gradient
-                    constexpr int NV = DIM == 2 ? 3 : 6;
-                    double eps[NV];
-                    double eN = 0.0, ge[3] = {0.0, 0.0, 0.0};
-                    if constexpr (KIND != kLocalDamage)
-                    {
-                        // the strain decides nothing here, and every dN_n/dX is needed anyway
-    #pragma unroll
-                        for (int i = 0; i < NV; i++)
-                            eps[i] = 0.0;
-    #pragma unroll
-                        for (int b = 0; b < NND; b++)
-                        {
-                            double g[DIM];
-                            Grad<DIM, NND>(dNd, b, inv, g);
-                            AddStrain<DIM>(g, c.U[b], eps);
-                            if constexpr (KIND == kGradientDamage)
-                            {
-                                eN = fma(Nd[b], c.EE[b], eN);
-                                ge[0] += g[0] * c.EE[b];
-                                ge[1] += g[1] * c.EE[b];
-                                ge[2] += g[2] * c.EE[b];
-                            }
-                        }
-                    }
-                    else
-                    {
-                        double Ru[DIM][DIM];
-                        NodalGradient<DIM, NND, DIM>(&c.U[0][0], dNd, Ru);
-                        StrainOfGradient(&Ru[0][0], inv, eps);
-                    }
+        // row node a
+        double ga[DIM];
+        Grad<DIM, NND>(dNd, la, inv, ga);
+        const double Na = Nd[la];
 
-                    // row node a
-                    double ga[DIM];
-                    Grad<DIM, NND>(dNd, la, inv, ga);
-                    const double Na = Nd[la];
+        // material response -> per-IP coefficients
+        double sig[NV];
+        double c1 = 0.0, c2 = 0.0, cm = 0.0;  // uu: c1 ga gb^T + c2 gb ga^T + c2 (ga.gb) I
+        double t6[6] = {0, 0, 0, 0, 0, 0}, m6[6] = {0, 0, 0, 0, 0, 0};
+        double rE = 0.0, cq = 0.0;  // cq: s c dg/dw dw/dk dk/de (grad eeq . g_a), the K_ee term of g'
+        double C11 = 0, C12 = 0, C33 = 0;
+        if constexpr (KIND == kLinearElastic)
+        {
+            if constexpr (DIM == 2)
+            {
+                if (P.plane_state == 0)
+                {
+                    const double f = E / (1.0 - P.nu * P.nu);
+                    C11 = f;
+                    C12 = f * P.nu;
+                    C33 = f * 0.5 * (1.0 - P.nu);
+                }
+                else
+                {
+                    const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
+                    C11 = f * (1.0 - P.nu);
+                    C12 = f * P.nu;
+                    C33 = E / (2.0 * (1.0 + P.nu));
+                }
+                sig[0] = C11 * eps[0] + C12 * eps[1];
+                sig[1] = C12 * eps[0] + C11 * eps[1];
+                sig[2] = C33 * eps[2];
+            }
+            else
+            {
+                const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
+                const double lam = f * P.nu, mu = E / (2.0 * (1.0 + P.nu));
+                const double tr = eps[0] + eps[1] + eps[2];
+                for (int i = 0; i < 3; i++)
+                    sig[i] = lam * tr + 2.0 * mu * eps[i];
+                for (int i = 3; i < 6; i++)
+                    sig[i] = mu * eps[i];
+                c1 = s * lam;
+                c2 = s * mu;
+            }
+        }
+        else
+        {
+            double mdev[6];
+            const double eq = Mises3(eps, P.nu, P.k, mdev);
+            const double kh = A.kappa[(size_t)c.id + (size_t)ip * A.kappaLd];
+            double kap, dk;
+            if constexpr (KIND == kGradientDamage)
+            {
+                kap = kh < eN ? eN : kh;
+                dk = eN >= kh ? 1.0 : 0.0;
+            }
+            else
+            {
+                kap = eq < kh ? kh : eq;
+                dk = eq >= kh ? 1.0 : 0.0;
+            }
+            double om, dom;
+            DamageExp(kap, k0, beta, P.alpha, om, dom);
+            DamageStress3 ds;
+            ElasticDamage3(eps, om, E, P.nu, P.damage_application, ds);
+            for (int i = 0; i < 6; i++)
+                sig[i] = ds.sig[i];
+            c1 = s * (ds.alpha_v - ds.alpha_d) / 3.0;
+            c2 = s * 0.5 * ds.alpha_d;
+            const double ct = s * dom * dk;
+            // gradient damage: K_eu = -N_a (B_b^T m) s; local damage: s dom dk (B_a^T dsdw)(B_b^T m)^T
+            const double cmv = KIND == kGradientDamage ? s : 1.0;
+            for (int i = 0; i < 6; i++)
+            {
+                t6[i] = ct * ds.dsdw[i];
+                m6[i] = cmv * mdev[i];
+            }
+            cm = P.c * s;
+            if constexpr (KIND == kGradientDamage)
+            {
+                double gi, dgi;
+                NonlocalFactor(P, om, gi, dgi);
+                const double gdot = ga[0] * ge[0] + ga[1] * ge[1] + ga[2] * ge[2];
+                rE = s * (Na * (eN - eq) + P.c * gi * gdot);
+                cm *= gi;
+                cq = s * P.c * gdot * dgi * dom * dk;
+            }
+        }
 
-                    // material response -> per-IP coefficients
-                    double sig[NV];
-                    double c1 = 0.0, c2 = 0.0, cm = 0.0;  // uu: c1 ga gb^T + c2 gb ga^T + c2 (ga.gb) I
-                    double t6[6] = {0, 0, 0, 0, 0, 0}, m6[6] = {0, 0, 0, 0, 0, 0};
-                    double rE = 0.0, cq = 0.0;  // cq: s c dg/dw dw/dk dk/de (grad eeq . g_a), the K_ee term of g'
-                    double C11 = 0, C12 = 0, C33 = 0;
-                    if constexpr (KIND == kLinearElastic)
-                    {
-                        if constexpr (DIM == 2)
-                        {
-                            if (P.plane_state == 0)
-                            {
-                                const double f = E / (1.0 - P.nu * P.nu);
-                                C11 = f;
-                                C12 = f * P.nu;
-                                C33 = f * 0.5 * (1.0 - P.nu);
-                            }
-                            else
-                            {
-                                const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
-                                C11 = f * (1.0 - P.nu);
-                                C12 = f * P.nu;
-                                C33 = E / (2.0 * (1.0 + P.nu));
-                            }
-                            sig[0] = C11 * eps[0] + C12 * eps[1];
-                            sig[1] = C12 * eps[0] + C11 * eps[1];
-                            sig[2] = C33 * eps[2];
-                        }
-                        else
-                        {
-                            const double f = E / ((1.0 + P.nu) * (1.0 - 2.0 * P.nu));
-                            const double lam = f * P.nu, mu = E / (2.0 * (1.0 + P.nu));
-                            const double tr = eps[0] + eps[1] + eps[2];
-                            for (int i = 0; i < 3; i++)
-                                sig[i] = lam * tr + 2.0 * mu * eps[i];
-                            for (int i = 3; i < 6; i++)
-                                sig[i] = mu * eps[i];
-                            c1 = s * lam;
-                            c2 = s * mu;
-                        }
-                    }
-                    else
-                    {
-                        double mdev[6];
-                        const double eq = Mises3(eps, P.nu, P.k, mdev);
-                        const double kh = A.kappa[(size_t)c.id + (size_t)ip * A.kappaLd];
-                        double kap, dk;
-                        if constexpr (KIND == kGradientDamage)
-                        {
-                            kap = kh < eN ? eN : kh;
-                            dk = eN >= kh ? 1.0 : 0.0;
-                        }
-                        else
-                        {
-                            kap = eq < kh ? kh : eq;
-                            dk = eq >= kh ? 1.0 : 0.0;
-                        }
-                        double om, dom;
-                        DamageExp(kap, k0, beta, P.alpha, om, dom);
-                        DamageStress3 ds;
-                        ElasticDamage3(eps, om, E, P.nu, P.damage_application, ds);
-                        for (int i = 0; i < 6; i++)
-                            sig[i] = ds.sig[i];
-                        c1 = s * (ds.alpha_v - ds.alpha_d) / 3.0;
-                        c2 = s * 0.5 * ds.alpha_d;
-                        const double ct = s * dom * dk;
-                        // gradient damage: K_eu = -N_a (B_b^T m) s; local damage: s dom dk (B_a^T dsdw)(B_b^T m)^T
-                        const double cmv = KIND == kGradientDamage ? s : 1.0;
-                        for (int i = 0; i < 6; i++)
-                        {
-                            t6[i] = ct * ds.dsdw[i];
-                            m6[i] = cmv * mdev[i];
-                        }
-                        cm = P.c * s;
-                        if constexpr (KIND == kGradientDamage)
-                        {
-                            double gi, dgi;
-                            NonlocalFactor(P, om, gi, dgi);
-                            const double gdot = ga[0] * ge[0] + ga[1] * ge[1] + ga[2] * ge[2];
-                            rE = s * (Na * (eN - eq) + P.c * gi * gdot);
-                            cm *= gi;
-                            cq = s * P.c * gdot * dgi * dom * dk;
-                        }
-                    }
+        if constexpr (WR)
+        {
+            if (b0 == 0)
+            {
+                if constexpr (DIM == 2)
+                {
+                    racc[0] += s * (ga[0] * sig[0] + ga[1] * sig[2]);
+                    racc[1] += s * (ga[1] * sig[1] + ga[0] * sig[2]);
+                }
+                else
+                {
+                    double bt[3];
+                    BTv3(ga, sig, bt);
+                    racc[0] += s * bt[0];
+                    racc[1] += s * bt[1];
+                    racc[2] += s * bt[2];
+                }
+                if constexpr (KIND == kGradientDamage)
+                    racc[3] += rE;
+            }
+        }
 
-                    if constexpr (WR)
-                    {
-                        if (b0 == 0)
+        if constexpr (WK)
+        {
+            double va[3] = {0, 0, 0};
+            if constexpr (KIND != kLinearElastic)
+                BTv3(ga, t6, va);
+#pragma unroll
+            for (int bb = 0; bb < NB; bb++)
+            {
+                const int b = b0 + bb;
+                if (b >= NND)
+                    break;
+                double gb[DIM];
+                Grad<DIM, NND>(dNd, b, inv, gb);
+                double* kb = kacc[bb];
+                if constexpr (DIM == 2)
+                {
+                    const double sa0 = s * ga[0], sa1 = s * ga[1];
+                    // named, so that K has the same bits with and without R
+                    kb[0] = fma(C33 * sa1, gb[1], fma(C11 * sa0, gb[0], kb[0]));
+                    kb[1] = fma(C33 * sa1, gb[0], fma(C12 * sa0, gb[1], kb[1]));
+                    kb[2] = fma(C33 * sa0, gb[1], fma(C12 * sa1, gb[0], kb[2]));
+                    kb[3] = fma(C33 * sa0, gb[0], fma(C11 * sa1, gb[1], kb[3]));
+                }
+                else
+                {
+                    const double dot = fma(ga[2], gb[2], fma(ga[1], gb[1], ga[0] * gb[0]));
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+#pragma unroll
+                        for (int j = 0; j < 3; j++)
                         {
-                            if constexpr (DIM == 2)
-                            {
-                                racc[0] += s * (ga[0] * sig[0] + ga[1] * sig[2]);
-                                racc[1] += s * (ga[1] * sig[1] + ga[0] * sig[2]);
-                            }
-                            else
-                            {
-                                double bt[3];
-                                BTv3(ga, sig, bt);
-                                racc[0] += s * bt[0];
-                                racc[1] += s * bt[1];
-                                racc[2] += s * bt[2];
-                            }
-                            if constexpr (KIND == kGradientDamage)
-                                racc[3] += rE;
+                            double& k = kb[i * F + j];
+                            k = fma(c2 * gb[i], ga[j], fma(c1 * ga[i], gb[j], k));
+                            if (i == j)
+                                k = fma(c2, dot, k);
                         }
+                    if constexpr (KIND == kLocalDamage)
+                    {
+                        double wb[3];
+                        BTv3(gb, m6, wb);
+#pragma unroll
+                        for (int i = 0; i < 3; i++)
+#pragma unroll
+                            for (int j = 0; j < 3; j++)
+                                kb[i * F + j] = fma(va[i], wb[j], kb[i * F + j]);
                     }
-
-                    if constexpr (WK)
+                    if constexpr (KIND == kGradientDamage)
                     {
-                        double va[3] = {0, 0, 0};
-                        if constexpr (KIND != kLinearElastic)
-                            BTv3(ga, t6, va);
-    #pragma unroll
-                        for (int bb = 0; bb < NB; bb++)
-                        {
-                            const int b = b0 + bb;
-                            if (b >= NND)
-                                break;
-                            double gb[DIM];
-                            Grad<DIM, NND>(dNd, b, inv, gb);
-                            double* kb = kacc[bb];
-                            if constexpr (DIM == 2)
-                            {
-                                const double sa0 = s * ga[0], sa1 = s * ga[1];
-                                // named, so that K has the same bits with and without R
-                                kb[0] = fma(C33 * sa1, gb[1], fma(C11 * sa0, gb[0], kb[0]));
-                                kb[1] = fma(C33 * sa1, gb[0], fma(C12 * sa0, gb[1], kb[1]));
-                                kb[2] = fma(C33 * sa0, gb[1], fma(C12 * sa1, gb[0], kb[2]));
-                                kb[3] = fma(C33 * sa0, gb[0], fma(C11 * sa1, gb[1], kb[3]));
-                            }
-                            else
-                            {
-                                const double dot = fma(ga[2], gb[2], fma(ga[1], gb[1], ga[0] * gb[0]));
-    #pragma unroll
-                                for (int i = 0; i < 3; i++)
-    #pragma unroll
-                                    for (int j = 0; j < 3; j++)
-                                    {
-                                        double& k = kb[i * F + j];
-                                        k = fma(c2 * gb[i], ga[j], fma(c1 * ga[i], gb[j], k));
-                                        if (i == j)
-                                            k = fma(c2, dot, k);
-                                    }
-                                if constexpr (KIND == kLocalDamage)
-                                {
-                                    double wb[3];
-                                    BTv3(gb, m6, wb);
-    #pragma unroll
-                                    for (int i = 0; i < 3; i++)
-    #pragma unroll
-                                        for (int j = 0; j < 3; j++)
-                                            kb[i * F + j] = fma(va[i], wb[j], kb[i * F + j]);
-                                }
-                                if constexpr (KIND == kGradientDamage)
-                                {
-                                    double wb[3];
-                                    BTv3(gb, m6, wb);
-                                    const double Nb = Nd[b];
-                                    kb[0 * 4 + 3] += va[0] * Nb;
-                                    kb[1 * 4 + 3] += va[1] * Nb;
-                                    kb[2 * 4 + 3] += va[2] * Nb;
-                                    kb[3 * 4 + 0] -= Na * wb[0];
-                                    kb[3 * 4 + 1] -= Na * wb[1];
-                                    kb[3 * 4 + 2] -= Na * wb[2];
-                                    kb[15] += s * Na * Nb + cm * dot + cq * Nb;
-                                }
-                            }
-                        }
+                        double wb[3];
+                        BTv3(gb, m6, wb);
+                        const double Nb = Nd[b];
+                        kb[0 * 4 + 3] += va[0] * Nb;
+                        kb[1 * 4 + 3] += va[1] * Nb;
+                        kb[2 * 4 + 3] += va[2] * Nb;
+                        kb[3 * 4 + 0] -= Na * wb[0];
+                        kb[3 * 4 + 1] -= Na * wb[1];
+                        kb[3 * 4 + 2] -= Na * wb[2];
+                        kb[15] += s * Na * Nb + cm * dot + cq * Nb;
                     }
                 }
+            }
+        }
+    }
 }
 
 // Rows of dof node p (p < pEnd <= A.nNodes): one lane per node, incident cells in group order.

@@ -24,7 +24,7 @@
 // the physics, one launch less), with the same functions on the same operands, so that both give the same
 // bits. GdmHex8Plan::Launch says when.
 //
-// What bounds it: the FP64 and exchange instructions of the vector units, 676 per wave with AFF (334
+// What bounds it: the FP64 and exchange instructions of the vector units, 672 per wave with AFF (333
 // FP64), with the latency of the record gather and of the reduction's LDS reads behind them (4 waves per
 // SIMD: 9.3 KB of LDS per workgroup). Summing the blocks from records in LDS instead (each lane reading
 // the 8 points' records of its cell) took 732 instructions and kept the LDS busy 78 % of the time.
@@ -349,8 +349,7 @@ __device__ inline void GdmCellState(const RowArgs& A, const CornerLane& c, int c
     GdmIpState<FULLDMG>(Hu, he, NodeSum(c, sE), inv0, kh, m3K, m2G, k0, beta, A.P, st);
 }
 
-// v of lane i + dpp-selected lane (CTRL: a DPP control word; out-of-row reads give 0): the sum over the
-// 8 lanes of a group, ((t0 + t1) + (t2 + t3)) + ((t4 + t5) + (t6 + t7)), valid in the group's lane 0
+// the sum over the 8 lanes of a group, ((t0 + t1) + (t2 + t3)) + ((t4 + t5) + (t6 + t7)), valid in its lane 0
 __device__ inline double GroupSum0(double v)
 {
     v += LaneDpp<kDppXor1>(v);
@@ -638,7 +637,7 @@ kGdmHex8Node(const RowArgs A, const GdmHex8Tables T)
 
 // Pre-pass: the state of every (cell, IP) once, for the node kernel (which would otherwise evaluate
 // it in each of the cell's 8 node workgroups). Lane (c, ip) of 8-lane group c; node j of the cell is
-// gathered by lane (c, j) and shared by swizzle, as in the node kernel.
+// gathered by lane (c, j); the lanes exchange their values (NodesToPoint), as in the node kernel.
 // AFF: affine cells, IP 0's geometry (T.geoCell) at every IP.
 // Workgroup w handles cells 8w .. 8w + 7 (lane (r, j): cell 8w + r, IP j). Their geometry and their
 // records are contiguous blocks in memory; both pass through LDS so that every global load and

@@ -8,7 +8,7 @@
 // A node's blocks of all its cells would fit one lane, as in kAssembleRows, but that kernel has a quarter of
 // the lanes and reads and rewrites each entry in memory, 8 bytes at a time; a cell matrix kernel and a gather
 // (kCellMatrices, kGatherRowsWave) write and read 8 ND^2 bytes per cell more.
-// Measured, R + K of 40,000 quad4 cells, linear elasticity: row-owner kernel 26.5 us, tiles 11.9 us (14 MB
+// Measured, R + K of 40,000 quad4 cells, linear elasticity: row-owner kernel 26.5 us, tiles 10.7 us (14 MB
 // moved; 2526 waves, bound by the chain of the gathers and the four turns); tet4, 1350 cells, local damage, with 4
 // lanes per node 33 us, with 8 27 us, 33,000 cells 35.3 and 33.9 us.
 #pragma once
@@ -35,7 +35,8 @@ constexpr size_t kTileMaxLds = 40 * 1024;      // segments beyond this leave too
 // per SIMD (at most 168 VGPRs): left alone, tet4 with local damage takes 176 and two, 546,750 cells 234 us
 // instead of 213 us.
 template <int KIND, int DIM, int NNC, int NND, int NIP, bool WR>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KIND == kLocalDamage ? 3 : 1))) kNodeTile(const RowArgs A, int p0, int p1)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KIND == kLocalDamage ? 3 : 1)))
+kNodeTile(const RowArgs A, int p0, int p1)
 {
     static_assert(KIND != kGradientDamage, "one dof type");
     constexpr int kTileLanes = TileLanes(DIM), kTileNodes = TileNodes(DIM);

@@ -2835,9 +2835,9 @@ int nuto_batch_autotune(nuto_batch* b, const double* u, const double* e, const d
             std::sort(rep.begin(), rep.end());
             return (double)rep[rep.size() / 2];
         };
-        // the two-phase modes (not for gradient damage): each group's cell-matrix kernel (by columns, Gram
-        // form with one or two row nodes per lane or on the matrix cores) and staging chunk (the whole group when it fits, 1 GiB, 256 MiB, 64 MiB of staging),
-        // timed on the group's two-phase launch
+        // the two-phase modes (not for gradient damage): each group's form (cell matrices by columns, in Gram
+        // form with one or two row nodes per lane or on the matrix cores; node tiles) and staging chunk (the
+        // whole group when it fits, 1 GiB, 256 MiB, 64 MiB of staging), timed on the group's two-phase launch
         const bool staged = !IsGdm(b);
         if (staged)
         {

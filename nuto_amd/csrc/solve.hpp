@@ -315,8 +315,9 @@ __global__ void __launch_bounds__(256) kCsrSpmv(int nRows, const int* __restrict
 // sums are added by exchanges in which the lanes share out the rows, a fixed order, without LDS.
 // A wave strides over the nodes (so that the dots' partials stay few; not in the largest systems, kFoldRows)
 // and keeps the next node's first 128 entries of every row in flight while it works on this one's, and
-// the row offsets of the node after that: only the gather of x is waited for. mask (one byte per node, bit i: row i is a dependent
-// dof) zeroes those rows of y; DOTS: the block's partial sums of the dots over its rows.
+// the row offsets of the node after that: only the gather of x is waited for. mask (one byte per node,
+// bit i: row i is a dependent dof) zeroes those rows of y; DOTS: the block's partial sums of the dots over
+// its rows.
 // Bound by the reads of the values; in small systems by the latency of its launch and of its dependent
 // loads. IN != kStored: the kernel that would make x is left out, see SpmvInput; the first node's entries
 // are in flight while the block adds the partials.
