@@ -58,8 +58,8 @@ struct RowArgs
 // the nonlocal strain as the sum of N_n e_n node by node. Each names its fused multiply-adds: left to the
 // compiler, a b + c d is contracted one way in one kernel and the other way in the next, and the last bit differs.
 
-// g_ij = sum_n v_n[i] dN_n[j]; v: node n's DIM values at v[STRIDE n]
-template <int DIM, int N, int STRIDE>
+// g_ij = sum_n v_n[i] dN_n[j]; v: node n's DIM values at v[STRIDE n], in LDS where UNROLL < N
+template <int DIM, int N, int STRIDE, int UNROLL = N>
 __device__ inline void NodalGradient(const double* v, const double* dN, double g[DIM][DIM])
 {
 #pragma unroll
@@ -67,7 +67,7 @@ __device__ inline void NodalGradient(const double* v, const double* dN, double g
 #pragma unroll
         for (int j = 0; j < DIM; j++)
             g[i][j] = 0.0;
-#pragma unroll
+#pragma unroll UNROLL
     for (int n = 0; n < N; n++)
 #pragma unroll
         for (int i = 0; i < DIM; i++)

@@ -244,7 +244,9 @@ __global__ void __launch_bounds__(PointThreads(NIP)) kCellPoints(const RowArgs A
         else
         {
             double R[DIM][DIM];
-            NodalGradient<DIM, NND, F>(U, dNd, R);
+            // five nodes at a time on twenty: all at once the shape derivatives take 350 registers and leave one
+            // wave per SIMD (64,000 hex20 cells, stress 152 -> 105 us); a residual of few cells would wait longer
+            NodalGradient<DIM, NND, F, NND == 20 && OUT != kPointVector ? 5 : NND>(U, dNd, R);
             StrainOfGradient(&R[0][0], inv, eps);
         }
 
